@@ -40,6 +40,20 @@ namespace sph {
     const int t_ = first_ + (int)threadIdx.x;             \
     if (t_ >= cd.n - cd.n_heavy) return;                  \
     const int i = cd.porder ? cd.porder[t_] : t_;
+// GROUP lanes a particle (g_: the lane in its group)
+#define SEG_GROUP(sg)                                     \
+    int first_;                                           \
+    const int cid_ = seg_case((sg), first_);              \
+    const CaseDesc& cd = (sg).cd[cid_];                   \
+    const int i = first_ + (int)threadIdx.x / GROUP, g_ = (int)threadIdx.x % GROUP; \
+    if (i >= cd.n) return;
+#define SEG_GROUP_LIGHT(sg)                               \
+    int first_;                                           \
+    const int cid_ = seg_case((sg), first_);              \
+    const CaseDesc& cd = (sg).cd[cid_];                   \
+    const int t_ = first_ + (int)threadIdx.x / GROUP, g_ = (int)threadIdx.x % GROUP; \
+    if (t_ >= cd.n - cd.n_heavy) return;                  \
+    const int i = cd.porder ? cd.porder[t_] : t_;
 #define SEG_HEAVY(sg)                                         \
     int first_;                                               \
     const int cid_ = seg_case((sg), first_);                  \
@@ -138,40 +152,10 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_snapshot(Seg sg, int which, int n
 
 // ------------------------------------------------------------------------
 // KERNEL_clc_gradient_correction_3D, functions_KNL.cuh:216-324
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr(Seg sg) {
-    SEG_PARTICLE(sg);
-    if (cd.gc_fresh) return;   // unchanged since the last step of this search
-    const KConst kc = cd.kc;
-    const PView S = cd.S;
-    const QView Q = cd.Q;
-    const NList nl = cd.nl;
-    int ptype_i = S.p_type[i];
-    R hi = (R)S.h[i];
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double tmpxx = 0, tmpyy = 0, tmpzz = 0, tmpxy = 0, tmpyz = 0, tmpzx = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_B)) continue;
-        int j = e & NB_IDX;
-        R dx = (R)(xi - S.x[j]), dy = (R)(yi - S.y[j]), dz = (R)(zi - S.z[j]);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz);
-        R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-        R mj = (R)S.m[j], rhoj = (R)S.rho[j];
-        R mtd = mj * tdwij;
-        R rtd = (R)1.0 / (rhoj * tdist);
-        R txx = -mtd * dx * dx; txx *= rtd;
-        R txy = -mtd * dy * dx; txy *= rtd;
-        R tyy = -mtd * dy * dy; tyy *= rtd;
-        R tzx = -mtd * dx * dz; tzx *= rtd;
-        R tyz = -mtd * dy * dz; tyz *= rtd;
-        R tzz = -mtd * dz * dz; tzz *= rtd;
-        R f = (R)(S.p_type[j] == 1);
-        tmpxx += (double)(txx * f); tmpxy += (double)(txy * f); tmpyy += (double)(tyy * f);
-        tmpzx += (double)(tzx * f); tmpyz += (double)(tyz * f); tmpzz += (double)(tzz * f);
-    }
+// the inverse of the moment matrix of a fluid particle's fluid neighbours
+// (the identity where it is singular, and for every other particle)
+__device__ __forceinline__ void grad_corr_store(const QView& Q, int i, int ptype_i, double tmpxx, double tmpyy,
+                                                double tmpzz, double tmpxy, double tmpyz, double tmpzx) {
     double tmpcmd = tmpxx * (tmpyy * tmpzz - tmpyz * tmpyz);
     tmpcmd -= tmpxy * (tmpxy * tmpzz - tmpyz * tmpzx);
     tmpcmd += tmpzx * (tmpxy * tmpyz - tmpyy * tmpzx);
@@ -187,6 +171,71 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr(Seg sg) {
         Q.inv_xx[i] = 1.0; Q.inv_xy[i] = 0.0; Q.inv_zx[i] = 0.0;
         Q.inv_yy[i] = 1.0; Q.inv_yz[i] = 0.0; Q.inv_zz[i] = 1.0;
     }
+}
+
+__global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr(Seg sg) {
+    SEG_PARTICLE(sg);
+    if (cd.gc_fresh) return;   // unchanged since the last step of this search
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    const QView Q = cd.Q;
+    const NList nl = cd.nl;
+    int ptype_i = S.p_type[i];
+    double hi = (double)S.h[i];
+    double tmp_A = calc_tmpA<double>(kc, hi);
+    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    double tmpxx = 0, tmpyy = 0, tmpzz = 0, tmpxy = 0, tmpyz = 0, tmpzx = 0;
+    NLRow row = nl_row(nl, i);
+    for (int k = 0; k < row.cnt; k++) {
+        unsigned e = NB_AT(row, k);
+        if (!(e & F_B)) continue;
+        int j = e & NB_IDX;
+        double dx = (double)(xi - S.x[j]), dy = (double)(yi - S.y[j]), dz = (double)(zi - S.z[j]);
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz);
+        double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+        double mj = (double)S.m[j], rhoj = (double)S.rho[j];
+        double mtd = mj * tdwij;
+        double rtd = (double)1.0 / (rhoj * tdist);
+        double txx = -mtd * dx * dx; txx *= rtd;
+        double txy = -mtd * dy * dx; txy *= rtd;
+        double tyy = -mtd * dy * dy; tyy *= rtd;
+        double tzx = -mtd * dx * dz; tzx *= rtd;
+        double tyz = -mtd * dy * dz; tyz *= rtd;
+        double tzz = -mtd * dz * dz; tzz *= rtd;
+        double f = (double)(S.p_type[j] == 1);
+        tmpxx += txx * f; tmpxy += txy * f; tmpyy += tyy * f;
+        tmpzx += tzx * f; tmpyz += tyz * f; tmpzz += tzz * f;
+    }
+    grad_corr_store(Q, i, ptype_i, tmpxx, tmpyy, tmpzz, tmpxy, tmpyz, tmpzx);
+}
+// MIXED: GROUP lanes a particle (SEG_GROUP), the pair arithmetic in float,
+// the sums in double
+__global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr_mixed(Seg sg) {
+    SEG_GROUP(sg);
+    if (cd.gc_fresh) return;   // unchanged since the last step of this search
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    const float hi = (float)S.h[i], tmp_A = calc_tmpA<float>(kc, hi), f = dw_factor<float>(kc, hi);
+    const HScale hs(kc, hi);
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    double txx = 0, tyy = 0, tzz = 0, txy = 0, tyz = 0, tzx = 0;
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = g_; k < row.cnt; k += GROUP) {
+        const unsigned e = NB_AT(row, k);
+        if (!(e & F_B)) continue;
+        const int j = e & NB_IDX;
+        if (S.p_type[j] != 1) continue;
+        const float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
+        const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+        const float w = -((float)S.m[j] * kernel_dw_t<float>(kc, tmp_A, f, hs.tR(d.r)));
+        const float rtd = recip((float)S.rho[j] * d.r);
+        txx += (double)(w * dx * dx * rtd); txy += (double)(w * dy * dx * rtd); tyy += (double)(w * dy * dy * rtd);
+        tzx += (double)(w * dx * dz * rtd); tyz += (double)(w * dy * dz * rtd); tzz += (double)(w * dz * dz * rtd);
+    }
+    group_fold<GROUP>(txx); group_fold<GROUP>(tyy); group_fold<GROUP>(tzz);
+    group_fold<GROUP>(txy); group_fold<GROUP>(tyz); group_fold<GROUP>(tzx);
+    if (g_ != 0) return;
+    grad_corr_store(cd.Q, i, S.p_type[i], txx, tyy, tzz, txy, tyz, tzx);
 }
 
 // ------------------------------------------------------------------------
@@ -232,89 +281,13 @@ __global__ void __launch_bounds__(BLOCK) k_pack_records(Seg sg) {
     r[6] = make_double2(S.temp[i], S.concn[i]);
 }
 
-// W = 64 (MIXED, a heavy list): the calling wave's lanes take entries lane,
-// lane + 64, ... and wave_fold adds their sums; lane 0 writes.
-template <class R, class Src, int W = 1>
-__device__ __forceinline__ void prep_body(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
-                                          int lane = 0) {
-    const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
+// A particle's strain rate and eddy viscosity from its sums.
+__device__ __forceinline__ void prep_store(const CaseDesc& cd, int i, bool les, bool filt, double ki, double nui,
+                                           double hi_d, double tmp_flt, double tmp_sigma, double st11, double st12,
+                                           double st22, double st23, double st31, double st33) {
+    const sph_params& pr = cd.pr;
     const PView S = cd.S;
     const P2View S2 = cd.S2;
-    const QView Q = cd.Q;
-    const int count = cd.count;
-    const double dt = cd.dt;
-    if (S.i_type[i] > 2) return;
-    if (S.p_type[i] >= 1000) return;
-    if (S.p_type[i] <= 0) return;
-    double ki = fmax(S.k_turb[i], 0.0);
-    double nui = S.vis_t[i];
-    R gc11 = (R)Q.inv_xx[i], gc12 = (R)Q.inv_xy[i], gc22 = (R)Q.inv_yy[i];
-    R gc23 = (R)Q.inv_yz[i], gc31 = (R)Q.inv_zx[i], gc33 = (R)Q.inv_zz[i];
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    double hi_d = S.h[i];
-    R hi = (R)hi_d;
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    double tmp_flt = 0.0, tmp_sigma = 0.0;
-    double st11 = 0, st12 = 0, st22 = 0, st23 = 0, st31 = 0, st33 = 0;
-    const bool filt = (count % pr.freq_filt) == 0;
-    const bool les = (pr.fv_solve != 0) && (pr.turbulence_model != SPH_LAMINAR);
-    const bool compact = Src::lds || (sizeof(R) == 4 && src.ok());
-    const NLRow row = nl_row(nl, li);
-    for (int k = W > 1 ? lane : 0; k < row.cnt; k += W) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_HP)) continue;
-        int j = e & NB_IDX;
-        // the neighbour's position, m, rho and type from the compact record
-        // (the same values as the field arrays hold) or the field arrays
-        double xj, yj, zj, mj_d, rhoj_d;
-        int ptj;
-        const float* C = compact ? src.at(j) : nullptr;
-        if (compact) {
-            const rec_f4 a = Src::f4(C), b = Src::f4(src.piece(C, 1));
-            xj = a.x; yj = a.y; zj = a.z; mj_d = a.w; rhoj_d = b.x; ptj = crec_ptype(b.w);
-        } else {
-            if constexpr (Src::lds) continue;   // staged records are compact
-            xj = S.x[j]; yj = S.y[j]; zj = S.z[j]; mj_d = S.m[j]; rhoj_d = S.rho[j]; ptj = S.p_type[j];
-        }
-        R dx = (R)(xi - xj), dy = (R)(yi - yj), dz = (R)(zi - zj);
-        R mj = (R)mj_d, rhoj = (R)rhoj_d;
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) + (R)1e-20;
-        R tmp_wij = kernel_w<R>(kc, tmp_A, hi, tdist);
-        R tmp_dwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-        R tdwx = tmp_dwij * dx / tdist;
-        R tdwy = tmp_dwij * dy / tdist;
-        R tdwz = tmp_dwij * dz / tdist;
-        if (filt) tmp_flt += (double)(mj / rhoj * tmp_wij);
-        if (les) {
-            tmp_sigma += (double)(tdist * tdist * tmp_wij * mj / rhoj);
-            if (ptj == 1) {
-                R tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
-                R tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
-                R tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
-                double uxj, uyj, uzj;
-                if (compact) {
-                    const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
-                    uxj = u.x; uyj = u.y; uzj = w.x;
-                } else {
-                    uxj = S.ux[j]; uyj = S.uy[j]; uzj = S.uz[j];
-                }
-                R dux = (R)(uxj - uxi), duy = (R)(uyj - uyi), duz = (R)(uzj - uzi);
-                st11 += (double)(mj / rhoj * dux * tdwxc);
-                st12 += (double)((R)0.5 * mj / rhoj * (dux * tdwyc + duy * tdwxc));
-                st22 += (double)(mj / rhoj * duy * tdwyc);
-                st23 += (double)((R)0.5 * mj / rhoj * (duy * tdwzc + duz * tdwyc));
-                st31 += (double)((R)0.5 * mj / rhoj * (dux * tdwzc + duz * tdwxc));
-                st33 += (double)(mj / rhoj * duz * tdwzc);
-            }
-        }
-    }
-    if constexpr (W > 1) {
-        wave_fold(tmp_flt); wave_fold(tmp_sigma);
-        wave_fold(st11); wave_fold(st12); wave_fold(st22); wave_fold(st23); wave_fold(st31); wave_fold(st33);
-        if (lane != 0) return;
-    }
     if (les) {
         double tmp_SR = 2 * (st11 * st11 + st22 * st22 + st33 * st33 + 2 * st12 * st12 + 2 * st31 * st31 + 2 * st23 * st23);
         tmp_SR = sqrt(tmp_SR);
@@ -330,31 +303,176 @@ __device__ __forceinline__ void prep_body(const CaseDesc& cd, int i, const NList
             double b = 0.0;
             double eps = pr.Ce_sgs * ki * sqrt(ki) / tmp_cl;
             double dk = p + b - eps + 0.0;
-            ki += dk * dt;
+            ki += dk * cd.dt;
             ki = ki > 1e-4 ? ki : 1e-4;
             double tvis_t = pr.Ck_sgs * tmp_cl * sqrt(ki);
             if (S.buffer_type[i] != 1) { S.vis_t[i] = tvis_t; S.k_turb[i] = ki; S.e_turb[i] = eps; }
         }
     }
-    if (count == 0) S2.rho_ref[i] = S.rho[i];
+    if (cd.count == 0) S2.rho_ref[i] = S.rho[i];
     if (filt) S.flt_s[i] = tmp_flt;
 }
-template <class R>
 __global__ void __launch_bounds__(MAX_BLOCK) k_prep(Seg sg) {
     SEG_PARTICLE_LIGHT(sg);
-    prep_body<R>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{sizeof(R) == 4 ? &cd.crec_adv : nullptr});
+    const KConst kc = cd.kc;
+    const sph_params pr = cd.pr;
+    const PView S = cd.S;
+    const QView Q = cd.Q;
+    if (S.i_type[i] > 2) return;
+    if (S.p_type[i] >= 1000) return;
+    if (S.p_type[i] <= 0) return;
+    const double ki = fmax(S.k_turb[i], 0.0), nui = S.vis_t[i];
+    double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
+    double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
+    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    double hi = S.h[i];
+    double tmp_A = calc_tmpA<double>(kc, hi);
+    double tmp_flt = 0.0, tmp_sigma = 0.0;
+    double st11 = 0, st12 = 0, st22 = 0, st23 = 0, st31 = 0, st33 = 0;
+    const bool filt = (cd.count % pr.freq_filt) == 0;
+    const bool les = (pr.fv_solve != 0) && (pr.turbulence_model != SPH_LAMINAR);
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = 0; k < row.cnt; k++) {
+        unsigned e = NB_AT(row, k);
+        if (!(e & F_HP)) continue;
+        int j = e & NB_IDX;
+        double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+        double mj = S.m[j], rhoj = S.rho[j];
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+        double tmp_wij = kernel_w<double>(kc, tmp_A, hi, tdist);
+        double tmp_dwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+        double tdwx = tmp_dwij * dx / tdist;
+        double tdwy = tmp_dwij * dy / tdist;
+        double tdwz = tmp_dwij * dz / tdist;
+        if (filt) tmp_flt += mj / rhoj * tmp_wij;
+        if (les) {
+            tmp_sigma += tdist * tdist * tmp_wij * mj / rhoj;
+            if (S.p_type[j] == 1) {
+                double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
+                double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
+                double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
+                double dux = S.ux[j] - uxi, duy = S.uy[j] - uyi, duz = S.uz[j] - uzi;
+                st11 += mj / rhoj * dux * tdwxc;
+                st12 += 0.5 * mj / rhoj * (dux * tdwyc + duy * tdwxc);
+                st22 += mj / rhoj * duy * tdwyc;
+                st23 += 0.5 * mj / rhoj * (duy * tdwzc + duz * tdwyc);
+                st31 += 0.5 * mj / rhoj * (dux * tdwzc + duz * tdwxc);
+                st33 += mj / rhoj * duz * tdwzc;
+            }
+        }
+    }
+    prep_store(cd, i, les, filt, ki, nui, hi, tmp_flt, tmp_sigma, st11, st12, st22, st23, st31, st33);
+}
+
+// MIXED passes over the neighbours of particle i: the pair arithmetic in
+// float, the sums in double.  REC: the pair's fields come from the compact
+// records (float positions, whose float difference is the rounded exact
+// difference), else from the field arrays (prep, which runs before the
+// 128-byte double records are packed) or those records.
+template <bool REC, class Src, int W>
+__device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow row, const Src src, int g, bool filt,
+                                          bool les, double& flt, double& sigma, double (&st)[6]) {
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    const QView Q = cd.Q;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const float gc11 = (float)Q.inv_xx[i], gc12 = (float)Q.inv_xy[i], gc22 = (float)Q.inv_yy[i];
+    const float gc23 = (float)Q.inv_yz[i], gc31 = (float)Q.inv_zx[i], gc33 = (float)Q.inv_zz[i];
+    const float hi = (float)S.h[i], tmp_A = calc_tmpA<float>(kc, hi), f = dw_factor<float>(kc, hi);
+    const HScale hs(kc, hi);
+    // consecutive neighbours mostly share rho: its reciprocal is kept
+    float rho_c = -1.0f, yrho = 0.0f;
+    for (int k = g; k < row.cnt; k += W) {
+        const unsigned e = NB_AT(row, k);
+        if (!(e & F_HP)) continue;
+        const int j = e & NB_IDX;
+        float dx, dy, dz, mj, rhoj;
+        int ptj;
+        const float* C = nullptr;
+        if constexpr (REC) {
+            C = src.at(j);
+            const rec_f4 a = Src::f4(C), b = Src::f4(src.piece(C, 1));
+            dx = xf - a.x; dy = yf - a.y; dz = zf - a.z; mj = a.w; rhoj = b.x;
+            ptj = crec_ptype(b.w);
+        } else {
+            dx = (float)(xi - S.x[j]); dy = (float)(yi - S.y[j]); dz = (float)(zi - S.z[j]);
+            mj = (float)S.m[j]; rhoj = (float)S.rho[j];
+            ptj = S.p_type[j];
+        }
+        if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
+        const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+        const float tR = hs.tR(d.r);
+        const float wij = kernel_w_t<float>(kc, tmp_A, tR);
+        const float vj = quot(mj, rhoj, yrho);
+        if (filt) flt += (double)(vj * wij);
+        if (les) {
+            sigma += (double)quot(d.r * d.r * wij * mj, rhoj, yrho);
+            if (ptj == 1) {
+                double uxj, uyj, uzj;
+                if constexpr (REC) {
+                    const rec_d2 p = Src::d2(src.piece(C, 2)), q = Src::d2(src.piece(C, 3));
+                    uxj = p.x; uyj = p.y; uzj = q.x;
+                } else {
+                    uxj = S.ux[j]; uyj = S.uy[j]; uzj = S.uz[j];
+                }
+                const float dw = kernel_dw_t<float>(kc, tmp_A, f, tR);
+                const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
+                const float cx = gc11 * tx + gc12 * ty + gc31 * tz, cy = gc12 * tx + gc22 * ty + gc23 * tz,
+                            cz = gc31 * tx + gc23 * ty + gc33 * tz;
+                const float dux = (float)(uxj - uxi), duy = (float)(uyj - uyi), duz = (float)(uzj - uzi);
+                st[0] += (double)(vj * dux * cx);
+                st[1] += (double)(0.5f * vj * (dux * cy + duy * cx));
+                st[2] += (double)(vj * duy * cy);
+                st[3] += (double)(0.5f * vj * (duy * cz + duz * cy));
+                st[4] += (double)(0.5f * vj * (dux * cz + duz * cx));
+                st[5] += (double)(vj * duz * cz);
+            }
+        }
+    }
+}
+template <class Src, int W = 1>
+__device__ __forceinline__ void prep_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
+                                           int g = 0) {
+    const sph_params& pr = cd.pr;
+    const PView S = cd.S;
+    if (S.i_type[i] > 2) return;
+    if (S.p_type[i] >= 1000) return;
+    if (S.p_type[i] <= 0) return;
+    const bool filt = (cd.count % pr.freq_filt) == 0;
+    const bool les = (pr.fv_solve != 0) && (pr.turbulence_model != SPH_LAMINAR);
+    double flt = 0.0, sigma = 0.0, st[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const NLRow row = nl_row(nl, li);
+    if constexpr (Src::lds) {
+        prep_sums<true, Src, W>(cd, i, row, src, g, filt, les, flt, sigma, st);
+    } else {
+        if (src.ok()) prep_sums<true, Src, W>(cd, i, row, src, g, filt, les, flt, sigma, st);
+        else prep_sums<false, Src, W>(cd, i, row, src, g, filt, les, flt, sigma, st);
+    }
+    if constexpr (W > 1) {
+        group_fold<W>(flt); group_fold<W>(sigma);
+        for (double& v : st) group_fold<W>(v);
+        if (g != 0) return;
+    }
+    prep_store(cd, i, les, filt, fmax(S.k_turb[i], 0.0), S.vis_t[i], S.h[i], flt, sigma, st[0], st[1], st[2], st[3],
+               st[4], st[5]);
+}
+__global__ void __launch_bounds__(MAX_BLOCK) k_prep_mixed(Seg sg) {
+    SEG_GROUP_LIGHT(sg);
+    prep_mixed<GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
 }
 __global__ void __launch_bounds__(WAVE_BLOCK) k_prep_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    prep_body<float, GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
+    prep_mixed<GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
 }
-__global__ void __launch_bounds__(TILE_MAX) k_prep_tile(Seg sg) {
-    TILE_PARTICLE(sg, cd.crec_adv, CREC_ADV_FLOATS);
-    if (chunk_.y >= 0)
-        prep_body<float>(cd, i, cd.tile.nl, lane_, LSrc<CREC_ADV_FLOATS>{(const float*)tile_lds_, chunk_.y,
-                                                     cd.tile.halo + chunk_.x,
-                                             cd.tile.self[lane_]});
-    else prep_body<float>(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv});
+__global__ void __launch_bounds__(TILE_THREADS) k_prep_tile(Seg sg, int width) {
+    TILE_CHUNK(sg, width, cd.crec_adv, CREC_ADV_FLOATS);
+    TILE_LANES(width) {
+        if (chunk_.y >= 0) prep_mixed<LSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_);
+        else prep_mixed<GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -419,8 +537,8 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_wave(Seg sg) {
     if (p_type_i != 0 && p_type_i != 9) return;
     const KConst kc = cd.kc;
     const NList nl = cd.nl;
-    float hi = (float)S.h[i];
-    float tmp_A = calc_tmpA<float>(kc, hi);
+    const float hi = (float)S.h[i], tmp_A = calc_tmpA<float>(kc, hi);
+    const HScale hs(kc, hi);
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     double t[4] = {0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
@@ -431,8 +549,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_wave(Seg sg) {
         const int p_type_j = S.p_type[j];
         if (!((p_type_j > 0) && (p_type_j != 9))) continue;
         float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
-        float tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20f;
-        float twij = kernel_w<float>(kc, tmp_A, hi, tdist);
+        const float twij = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
         t[0] += (double)((float)S.ux[j] * twij);
         t[1] += (double)((float)S.uy[j] * twij);
         t[2] += (double)((float)S.uz[j] * twij);
@@ -708,39 +825,41 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
         // (pairs lane, lane + 64, ... in list order), then a fixed butterfly
         // adds the 64 lane sums; lane 0's total is used, so the sums are the
         // same on every call, alone or in a batch
+        const HScale hs(kc, (float)hi);
+        const float dwf = dw_factor<float>(kc, (float)hi);
+        float rho_c = -1.0f, yrho = 0.0f;
         double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         const long long e0 = cd.nmp_off[u], e1 = cd.nmp_off[u + 1];
         const float* const nrec = cd.nm_rec;   // the same values, packed (float-exact positions)
         for (long long e = e0 + lane; e < e1; e += 64) {
             double xj, yj, zj, presj;
-            R mj, rhoj, uxj, uyj, uzj;
+            float mj, rhoj, uxj, uyj, uzj;
             if (nrec) {
                 const float* C = nrec + (size_t)cd.nmp_cent[e] * NMREC_FLOATS;
                 const rec_f4 a = ld_f4(C), b = ld_f4(C + 4);
-                xj = a.x; yj = a.y; zj = a.z; mj = (R)a.w; rhoj = (R)b.x; uxj = (R)b.y; uyj = (R)b.z; uzj = (R)b.w;
+                xj = a.x; yj = a.y; zj = a.z; mj = a.w; rhoj = b.x; uxj = b.y; uyj = b.z; uzj = b.w;
                 presj = ld_d2(C + 8).x;
             } else {
                 const int j = cd.nmp_ent[e];
-                xj = A.x[j]; yj = A.y[j]; zj = A.z[j]; mj = (R)A.m[j]; rhoj = (R)A.rho[j];
-                uxj = (R)A.ux[j]; uyj = (R)A.uy[j]; uzj = (R)A.uz[j];
+                xj = A.x[j]; yj = A.y[j]; zj = A.z[j]; mj = (float)A.m[j]; rhoj = (float)A.rho[j];
+                uxj = (float)A.ux[j]; uyj = (float)A.uy[j]; uzj = (float)A.uz[j];
                 presj = pold[j];
             }
-            R dx = (R)(xg - xj), dy = (R)(yg - yj), dz = (R)(zg - zj);
-            R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-            if (!(tdist < search_range)) continue;
-            R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-            s[0] += (double)(mj / rhoj * (R)presj * twij);
-            s[1] += (double)(mj / rhoj * uxj * twij);
-            s[2] += (double)(mj / rhoj * uyj * twij);
-            s[3] += (double)(mj / rhoj * uzj * twij);
-            s[4] += (double)(mj / rhoj * twij);
+            if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
+            // (the list holds exactly the pairs inside the search range)
+            const float dx = (float)(xg - xj), dy = (float)(yg - yj), dz = (float)(zg - zj);
+            const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+            const float tR = hs.tR(d.r), w = kernel_w_t<float>(kc, (float)tmp_A, tR), vj = quot(mj, rhoj, yrho);
+            s[0] += (double)(vj * (float)presj * w);
+            s[1] += (double)(vj * uxj * w);
+            s[2] += (double)(vj * uyj * w);
+            s[3] += (double)(vj * uzj * w);
+            s[4] += (double)(vj * w);
             if (inlet) {
-                R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-                R tdwx = dx / tdist * tdwij, tdwy = dy / tdist * tdwij, tdwz = dz / tdist * tdwij;
-                R dp = (R)(presj - pres_g);
-                s[5] += (double)(mj / rhoj * dp * tdwx);
-                s[6] += (double)(mj / rhoj * dp * tdwy);
-                s[7] += (double)(mj / rhoj * dp * tdwz);
+                const float dw = kernel_dw_t<float>(kc, (float)tmp_A, dwf, tR), dp = vj * (float)(presj - pres_g);
+                s[5] += (double)(dp * (quot(dx, d.r, d.y) * dw));
+                s[6] += (double)(dp * (quot(dy, d.r, d.y) * dw));
+                s[7] += (double)(dp * (quot(dz, d.r, d.y) * dw));
             }
         }
         for (int off = 32; off > 0; off >>= 1)
@@ -829,15 +948,33 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
 // SCAL: some case of the launch transports temperature or concentration or
 // uses the Boussinesq buoyancy; without them (the canyon) those terms and
 // their registers are compiled out (130 -> fewer VGPRs, more waves per SIMD)
-template <class R, bool SCAL, class Src, int W = 1>
-__device__ __forceinline__ void advection_body(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
-                                               int lane = 0) {
+struct AdvSums {   // viscous and artificial (t), convective (c) terms; scalars
+    double tx = 0, ty = 0, tz = 0, cx = 0, cy = 0, cz = 0, rc = 0, rd = 0, ct = 0, temp = 0, flt = 0;
+};
+__device__ __forceinline__ void advection_store(const CaseDesc& cd, int i, const AdvSums& a, bool con_solve,
+                                                bool concn_solve, bool boussinesq_solve, double cpi) {
+    const sph_params& pr = cd.pr;
+    const QView Q = cd.Q;
+    const int ptypei = cd.S.p_type[i];
+    double tz = a.tz;
+    if (pr.fg_solve) tz += -pr.gravity;
+    if ((boussinesq_solve) && (ptypei > 0) && (ptypei < 1000))
+        tz = 1.0 / pr.T_ini * pr.gravity * (a.temp / a.flt - pr.tempb);
+    Q.ftotalx[i] = a.tx - a.cx;
+    Q.ftotaly[i] = a.ty - a.cy;
+    Q.ftotalz[i] = tz - a.cz;
+    if (con_solve) Q.dtemp[i] += a.rc / cpi - a.ct;
+    Q.ftotal[i] = sqrt(a.tx * a.tx + a.ty * a.ty + tz * tz);
+    if (concn_solve) Q.dconcn[i] = a.rd;
+}
+template <bool SCAL>
+__global__ void __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(SCAL ? 1 : 4))) k_advection(Seg sg) {
+    SEG_PARTICLE_LIGHT(sg);
     const KConst kc = cd.kc;
     const sph_params pr = cd.pr;
     const bool con_solve = SCAL && pr.con_solve, concn_solve = SCAL && pr.concn_solve;
     const bool boussinesq_solve = SCAL && pr.boussinesq_solve;
     const PView S = cd.S;
-    const QView Q = cd.Q;
     if (S.i_type[i] > 2) return;
     int ptypei = S.p_type[i];
     if (ptypei == 1000) return;
@@ -845,167 +982,287 @@ __device__ __forceinline__ void advection_body(const CaseDesc& cd, int i, const 
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
     double tempi = SCAL ? S.temp[i] : 0.0;
-    R hi = (R)S.h[i], mi = (R)S.m[i], rhoi = (R)S.rho[i];
-    double hi_d = S.h[i];
+    double hi = S.h[i], mi = S.m[i], rhoi = S.rho[i];
     double eli = S.eli[i];
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    R kci = 0, cpi = 1, concni = 0, diffi = 0;
+    double tmp_A = calc_tmpA<double>(kc, hi);
+    double kci = 0, cpi = 1, concni = 0, diffi = 0;
     if (con_solve) {
-        kci = (R)(pr.solid_k * (ptypei == 0 || ptypei == 1000) + pr.air_k * (ptypei == 1 || ptypei == -1));
-        cpi = (R)(pr.solid_cp * (ptypei == 0 || ptypei == 1000) + pr.air_cp * (ptypei == 1 || ptypei == -1));
+        kci = pr.solid_k * (ptypei == 0 || ptypei == 1000) + pr.air_k * (ptypei == 1 || ptypei == -1);
+        cpi = pr.solid_cp * (ptypei == 0 || ptypei == 1000) + pr.air_cp * (ptypei == 1 || ptypei == -1);
     }
-    if (concn_solve) { concni = (R)S.concn[i]; diffi = (R)pr.diff_coef; }
-    R visi = (R)(viscosity2(pr, ptypei) + S.vis_t[i] * S.rho[i]);
-    double betai = 1.0 / pr.T_ini;
-    double tmpx = 0, tmpy = 0, tmpz = 0, tmp_Rc = 0, tmp_Rd = 0;
-    double eulerx = 0, eulery = 0, eulerz = 0, eulert = 0, tmp_temp = 0, tmp_flt = 0;
-    const R Alpha = (R)pr.av_alpha, Beta = (R)pr.av_beta, soundspeed = (R)pr.av_c;
-    const R ome = (R)(1 - eli);
-    const bool compact = Src::lds || (sizeof(R) == 4 && src.ok());
-    const NLRow row = nl_row(nl, li);
-    for (int k = W > 1 ? lane : 0; k < row.cnt; k += W) {
+    if (concn_solve) { concni = S.concn[i]; diffi = pr.diff_coef; }
+    double visi = viscosity2(pr, ptypei) + S.vis_t[i] * S.rho[i];
+    AdvSums a;
+    const double Alpha = pr.av_alpha, Beta = pr.av_beta, soundspeed = pr.av_c;
+    const double ome = 1 - eli;
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = 0; k < row.cnt; k++) {
         unsigned e = NB_AT(row, k);
         if (!(e & F_DP)) continue;
         int j = e & NB_IDX;
-        double hj_d, visj_d, xj, yj, zj, mj_d, uxj, uyj, uzj, rhoj_d;
+        double hj, vis_tj, xj, yj, zj, mj, uxj, uyj, uzj, rhoj, pqj_;
+        int ptypej, itj_;
+        rec_aux(cd.rec, j, vis_tj, ptypej, itj_);
+        if (ptypej >= 1000) continue;
+        rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pqj_);
+        rec_vel(cd.rec, j, uxj, uyj, uzj, hj);
+        double visj = viscosity2(pr, ptypej) + vis_tj * rhoj;
+        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+        double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
+        double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+        double tdwx = tdwij * dx / tdist;
+        double tdwy = tdwij * dy / tdist;
+        double tdwz = tdwij * dz / tdist;
+        double dux = uxi - uxj, duy = uyi - uyj, duz = uzi - uzj;   // u_i - u_j
+        double tempj = 0.0, concnj = 0.0;
+        if (con_solve || concn_solve || boussinesq_solve) rec_scalar(cd.rec, j, tempj, concnj);
+        if (pr.fv_solve == SPH_FV_CLEARY) {
+            double C_v = dx * tdwx + dy * tdwy + dz * tdwz;
+            C_v *= (visi * visj) / (visi + visj);
+            C_v *= 4.0 * (mj / (rhoi * rhoj));
+            C_v /= tdist;
+            C_v /= tdist;
+            a.tx += C_v * dux; a.ty += C_v * duy; a.tz += C_v * duz;
+        } else if (pr.fv_solve == SPH_FV_MONAGHAN) {
+            double uij_xij = dux * dx + duy * dy + duz * dz;
+            double phi_ij = uij_xij;
+            phi_ij /= (tdist * tdist + 0.01 * hi * hi);
+            double P_ij = -2.0 * (3 + 2.0) * phi_ij * mj / rhoj;
+            double C_v = 2.0 * (visi * visj) / (visi + visj - 1e-20);
+            double nui = C_v / rhoi;
+            P_ij *= nui;
+            if (ptypei <= 0 || ptypei >= 1000) P_ij = 0;
+            if (ptypej <= 0 || ptypei >= 1000) P_ij = 0;
+            a.tx += -(P_ij)*tdwx; a.ty += -(P_ij)*tdwy; a.tz += -(P_ij)*tdwz;
+        }
+        if (eli < 1.0) {
+            double vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
+            a.cx += (uxi * vx * tdwx + uyi * vx * tdwy + uzi * vx * tdwz) * mj / rhoj * ome;
+            a.cy += (uxi * vy * tdwx + uyi * vy * tdwy + uzi * vy * tdwz) * mj / rhoj * ome;
+            a.cz += (uxi * vz * tdwx + uyi * vz * tdwy + uzi * vz * tdwz) * mj / rhoj * ome;
+            if (con_solve)
+                a.ct -= 2.0 * mj / (rhoi + rhoj) * (tempj - tempi) * (dux * tdwx + duy * tdwy + duz * tdwz) * ome;
+            if (concn_solve) {
+                double dc = concnj - concni;
+                a.rd -= (uxi * dc * tdwx + uyi * dc * tdwy + uzi * dc * tdwz) * mj / rhoj * ome;
+            }
+        }
+        if (con_solve) {
+            double kcj = pr.solid_k * (ptypej == 0 || ptypej == 1000) + pr.air_k * (ptypej == 1 || ptypej == -1);
+            double rhoj_temp = (ptypej == 1 || ptypej == -1) ? rhoj : pr.solid_rho;
+            double mj_temp = mj * rhoj_temp / rhoj;
+            double sum_con_H = 4.0 * mj_temp * kcj * kci * (tempi - tempj) * tdwij;
+            sum_con_H /= (tdist + 1e-10) * rhoi * rhoj_temp * (kci + kcj);
+            a.rc += sum_con_H;
+        }
+        if (concn_solve) {
+            double diffj = pr.diff_coef;
+            double tmprd = mi * (diffi * rhoi + diffj * rhoj);
+            tmprd *= (dx * tdwx + dy * tdwy + dz * tdwz);
+            tmprd /= (rhoi * rhoj * (tdist * tdist + 0.01 * hi * hi));
+            double tmprd1 = tmprd * (concni - concnj) * (double)(ptypei == ptypej);
+            a.rd += tmprd1;
+        }
+        if (boussinesq_solve) {
+            a.temp += (mj / rhoj) * tempj * twij;
+            a.flt += (mj / rhoj) * twij;
+        }
+        if (pr.artificial_viscosity) {
+            double uij_xij = dux * dx + duy * dy + duz * dz;
+            if (uij_xij < 0) {
+                double h_ij = (hi + hj) * 0.5;
+                double phi_ij = h_ij * uij_xij;
+                phi_ij /= (tdist * tdist + 0.01 * h_ij * h_ij);
+                double P_ij = mi * phi_ij * (-Alpha * soundspeed + Beta * phi_ij);
+                P_ij /= (rhoi + rhoj);
+                P_ij *= 0.5;
+                a.tx += -(P_ij)*tdwx; a.ty += -(P_ij)*tdwy; a.tz += -(P_ij)*tdwz;
+            }
+        }
+    }
+    advection_store(cd, i, a, con_solve, concn_solve, boussinesq_solve, cpi);
+}
+
+// MIXED (see prep_sums)
+template <bool SCAL, bool REC, class Src, int W>
+__device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const NLRow row, const Src src, int g,
+                                               bool con_solve, bool concn_solve, bool boussinesq_solve, AdvSums& a) {
+    const KConst kc = cd.kc;
+    const sph_params& pr = cd.pr;
+    const PView S = cd.S;
+    const double* const rec = cd.rec;
+    const int ptypei = S.p_type[i];
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const float fux = (float)uxi, fuy = (float)uyi, fuz = (float)uzi;
+    const double tempi = SCAL ? S.temp[i] : 0.0;
+    const float concni = SCAL ? (float)S.concn[i] : 0.0f;
+    const double hi_d = S.h[i], eli = S.eli[i];
+    const float hi = (float)hi_d, mi = (float)S.m[i], rhoi = (float)S.rho[i];
+    const float tmp_A = calc_tmpA<float>(kc, hi), f = dw_factor<float>(kc, hi);
+    const HScale hs(kc, hi);
+    const float kci = SCAL ? (float)(pr.solid_k * (ptypei == 0 || ptypei == 1000) + pr.air_k * (ptypei == 1 || ptypei == -1)) : 0.0f;
+    const float visi = (float)(viscosity2(pr, ptypei) + S.vis_t[i] * S.rho[i]);
+    const float ome = (float)(1 - eli);
+    const bool conv = eli < 1.0, av = pr.artificial_viscosity != 0;
+    const int fv = pr.fv_solve;
+    const float Alpha = (float)pr.av_alpha, Beta = (float)pr.av_beta, soundspeed = (float)pr.av_c;
+    // consecutive neighbours mostly share rho: the reciprocals it enters are kept
+    float rho_c = -1.0f, yrho = 0.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
+    for (int k = g; k < row.cnt; k += W) {
+        const unsigned e = NB_AT(row, k);
+        if (!(e & F_DP)) continue;
+        const int j = e & NB_IDX;
+        float dx, dy, dz, mj, rhoj, visj;
+        double uxj, uyj, uzj, hj_d;
         int ptypej;
-        if (compact) {
+        if constexpr (REC) {
             const float* C = src.at(j);
             const rec_f4 b = Src::f4(src.piece(C, 1));
             ptypej = crec_ptype(b.w);
             if (ptypej >= 1000) continue;
-            const rec_f4 a = Src::f4(C);
+            const rec_f4 p = Src::f4(C);
             const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
-            xj = a.x; yj = a.y; zj = a.z; mj_d = a.w;
-            rhoj_d = b.x; hj_d = b.y; visj_d = b.z;
+            dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
+            rhoj = b.x; hj_d = b.y; visj = b.z;
             uxj = u.x; uyj = u.y; uzj = w.x;
         } else {
-            if constexpr (Src::lds) continue;   // staged records are compact
-            double vis_tj, pqj_;
+            double vis_tj, xj, yj, zj, mj_d, rhoj_d, pqj_;
             int itj_;
-            rec_aux(cd.rec, j, vis_tj, ptypej, itj_);
+            rec_aux(rec, j, vis_tj, ptypej, itj_);
             if (ptypej >= 1000) continue;
-            rec_pos(cd.rec, j, xj, yj, zj, mj_d, rhoj_d, pqj_);
-            rec_vel(cd.rec, j, uxj, uyj, uzj, hj_d);
-            visj_d = viscosity2(pr, ptypej) + vis_tj * rhoj_d;
+            rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, pqj_);
+            rec_vel(rec, j, uxj, uyj, uzj, hj_d);
+            dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
+            mj = (float)mj_d; rhoj = (float)rhoj_d;
+            visj = (float)(viscosity2(pr, ptypej) + vis_tj * rhoj_d);
         }
-        R dx = (R)(xi - xj), dy = (R)(yi - yj), dz = (R)(zi - zj);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) + (R)1e-20;
-        R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-        R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-        R tdwx = tdwij * dx / tdist;
-        R tdwy = tdwij * dy / tdist;
-        R tdwz = tdwij * dz / tdist;
-        R mj = (R)mj_d, rhoj = (R)rhoj_d;
-        R dux = (R)(uxi - uxj), duy = (R)(uyi - uyj), duz = (R)(uzi - uzj);   // u_i - u_j
-        double tempj = 0.0, concnj_d = 0.0;
-        if (con_solve || concn_solve || boussinesq_solve) {
-            if (compact) { tempj = S.temp[src.gidx(j)]; concnj_d = S.concn[src.gidx(j)]; }
-            else rec_scalar(cd.rec, j, tempj, concnj_d);
+        if (rhoj != rho_c) {
+            rho_c = rhoj;
+            yrho = recip(rhoj);
+            rr = rhoi * rhoj; yrr = recip(rr);
+            rs = rhoi + rhoj; yrs = recip(rs);
         }
-        if (pr.fv_solve == SPH_FV_CLEARY) {
-            R visj = (R)visj_d;
-            R C_v = dx * tdwx + dy * tdwy + dz * tdwz;
-            C_v *= (visi * visj) / (visi + visj);
-            C_v *= (R)4 * (mj / (rhoi * rhoj));
-            C_v /= tdist;
-            C_v /= tdist;
-            tmpx += (double)(C_v * dux); tmpy += (double)(C_v * duy); tmpz += (double)(C_v * duz);
-        } else if (pr.fv_solve == SPH_FV_MONAGHAN) {
-            R uij_xij = dux * dx + duy * dy + duz * dz;
-            R visj = (R)visj_d;
-            R phi_ij = uij_xij;
-            phi_ij /= (tdist * tdist + (R)0.01 * hi * hi);
-            R P_ij = (R)(-2.0) * (R)(3 + 2.0) * phi_ij * mj / rhoj;
-            R C_v = (R)2.0 * (visi * visj) / (visi + visj - (R)1e-20);
-            R nui = C_v / rhoi;
-            P_ij *= nui;
-            if (ptypei <= 0 || ptypei >= 1000) P_ij = 0;
-            if (ptypej <= 0 || ptypei >= 1000) P_ij = 0;
-            tmpx += (double)(-(P_ij)*tdwx); tmpy += (double)(-(P_ij)*tdwy); tmpz += (double)(-(P_ij)*tdwz);
+        const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+        const float tR = hs.tR(d.r), dw = kernel_dw_t<float>(kc, tmp_A, f, tR);
+        const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
+        const float dux = (float)(uxi - uxj), duy = (float)(uyi - uyj), duz = (float)(uzi - uzj);   // u_i - u_j
+        if (fv == SPH_FV_CLEARY) {
+            float C_v = dx * tx + dy * ty + dz * tz;
+            const float vs = visi + visj;
+            C_v *= quot(visi * visj, vs, recip(vs));
+            C_v *= 4.0f * quot(mj, rr, yrr);
+            C_v = quot(quot(C_v, d.r, d.y), d.r, d.y);
+            a.tx += (double)(C_v * dux); a.ty += (double)(C_v * duy); a.tz += (double)(C_v * duz);
+        } else if (fv == SPH_FV_MONAGHAN) {
+            const float phi = (dux * dx + duy * dy + duz * dz) / (d.r * d.r + 0.01f * hi * hi);
+            float P = -10.0f * phi * mj / rhoj;
+            const float C_v = 2.0f * (visi * visj) / (visi + visj - 1e-20f);
+            P *= C_v / rhoi;
+            if (ptypei <= 0 || ptypei >= 1000 || ptypej <= 0) P = 0;
+            a.tx += (double)(-P * tx); a.ty += (double)(-P * ty); a.tz += (double)(-P * tz);
         }
-        if (eli < 1.0) {
-            R Rux = (R)uxi, Ruy = (R)uyi, Ruz = (R)uzi;
-            R vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
-            eulerx += (double)((Rux * vx * tdwx + Ruy * vx * tdwy + Ruz * vx * tdwz) * mj / rhoj * ome);
-            eulery += (double)((Rux * vy * tdwx + Ruy * vy * tdwy + Ruz * vy * tdwz) * mj / rhoj * ome);
-            eulerz += (double)((Rux * vz * tdwx + Ruy * vz * tdwy + Ruz * vz * tdwz) * mj / rhoj * ome);
-            if (con_solve)
-                eulert -= (double)((R)2.0 * mj / (rhoi + rhoj) * (R)(tempj - tempi) * (dux * tdwx + duy * tdwy + duz * tdwz) * ome);
+        if (conv) {
+            const float vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
+            a.cx += (double)(quot((fux * vx * tx + fuy * vx * ty + fuz * vx * tz) * mj, rhoj, yrho) * ome);
+            a.cy += (double)(quot((fux * vy * tx + fuy * vy * ty + fuz * vy * tz) * mj, rhoj, yrho) * ome);
+            a.cz += (double)(quot((fux * vz * tx + fuy * vz * ty + fuz * vz * tz) * mj, rhoj, yrho) * ome);
+        }
+        if (SCAL && (con_solve || concn_solve || boussinesq_solve)) {
+            double tempj, concnj_d;
+            if constexpr (REC) { tempj = S.temp[src.gidx(j)]; concnj_d = S.concn[src.gidx(j)]; }
+            else rec_scalar(rec, j, tempj, concnj_d);
+            if (conv && con_solve)
+                a.ct -= (double)(2.0f * mj / rs * (float)(tempj - tempi) * (dux * tx + duy * ty + duz * tz) * ome);
+            if (conv && concn_solve) {
+                const float dc = (float)(concnj_d - (double)concni);
+                a.rd -= (double)((fux * dc * tx + fuy * dc * ty + fuz * dc * tz) * mj / rhoj * ome);
+            }
+            if (con_solve) {
+                const float kcj = (float)(pr.solid_k * (ptypej == 0 || ptypej == 1000) + pr.air_k * (ptypej == 1 || ptypej == -1));
+                const float rhoj_temp = (ptypej == 1 || ptypej == -1) ? rhoj : (float)pr.solid_rho;
+                const float mj_temp = mj * rhoj_temp / rhoj;
+                float H = 4.0f * mj_temp * kcj * kci * (float)(tempi - tempj) * dw;
+                H /= (d.r + 1e-10f) * rhoi * rhoj_temp * (kci + kcj);
+                a.rc += (double)H;
+            }
             if (concn_solve) {
-                R dc = (R)(concnj_d - (double)concni);
-                tmp_Rd -= (double)((Rux * dc * tdwx + Ruy * dc * tdwy + Ruz * dc * tdwz) * mj / rhoj * ome);
+                const float diff = (float)pr.diff_coef;
+                float D = mi * (diff * rhoi + diff * rhoj);
+                D *= (dx * tx + dy * ty + dz * tz);
+                D /= (rhoi * rhoj * (d.r * d.r + 0.01f * hi * hi));
+                a.rd += (double)(D * (concni - (float)concnj_d) * (float)(ptypei == ptypej));
+            }
+            if (boussinesq_solve) {
+                const float vj = mj / rhoj, twij = kernel_w_t<float>(kc, tmp_A, tR);
+                a.temp += (double)(vj * (float)tempj * twij);
+                a.flt += (double)(vj * twij);
             }
         }
-        if (con_solve) {
-            R kcj = (R)(pr.solid_k * (ptypej == 0 || ptypej == 1000) + pr.air_k * (ptypej == 1 || ptypej == -1));
-            R rhoj_temp = (ptypej == 1 || ptypej == -1) ? rhoj : (R)pr.solid_rho;
-            R mj_temp = mj * rhoj_temp / rhoj;
-            R sum_con_H = (R)4.0 * mj_temp * kcj * kci * (R)(tempi - tempj) * tdwij;
-            sum_con_H /= (tdist + (R)1e-10) * rhoi * rhoj_temp * (kci + kcj);
-            tmp_Rc += (double)sum_con_H;
-        }
-        if (concn_solve) {
-            R concnj = (R)concnj_d;
-            R diffj = (R)pr.diff_coef;
-            R tmprd = mi * (diffi * rhoi + diffj * rhoj);
-            tmprd *= (dx * tdwx + dy * tdwy + dz * tdwz);
-            tmprd /= (rhoi * rhoj * (tdist * tdist + (R)0.01 * hi * hi));
-            R tmprd1 = tmprd * (concni - concnj) * (R)(ptypei == ptypej);
-            tmp_Rd += (double)tmprd1;
-        }
-        if (boussinesq_solve) {
-            tmp_temp += (double)((mj / rhoj) * (R)tempj * twij);
-            tmp_flt += (double)((mj / rhoj) * twij);
-        }
-        if (pr.artificial_viscosity) {
-            R uij_xij = dux * dx + duy * dy + duz * dz;
-            if (uij_xij < 0) {
-                R h_ij = (R)((hi_d + hj_d) * 0.5);
-                R phi_ij = h_ij * uij_xij;
-                phi_ij /= (tdist * tdist + (R)0.01 * h_ij * h_ij);
-                R P_ij = mi * phi_ij * (-Alpha * soundspeed + Beta * phi_ij);
-                P_ij /= (rhoi + rhoj);
-                P_ij *= (R)0.5;
-                tmpx += (double)(-(P_ij)*tdwx); tmpy += (double)(-(P_ij)*tdwy); tmpz += (double)(-(P_ij)*tdwz);
+        if (av) {
+            const float ud = dux * dx + duy * dy + duz * dz;
+            if (ud < 0) {
+                const float h_ij = (float)((hi_d + hj_d) * 0.5);
+                const float den = d.r * d.r + 0.01f * h_ij * h_ij;
+                const float phi = quot(h_ij * ud, den, recip(den));
+                const float P = quot(mi * phi * (-Alpha * soundspeed + Beta * phi), rs, yrs) * 0.5f;
+                a.tx += (double)(-P * tx); a.ty += (double)(-P * ty); a.tz += (double)(-P * tz);
             }
         }
+    }
+}
+template <bool SCAL, class Src, int W = 1>
+__device__ __forceinline__ void advection_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
+                                                int g = 0) {
+    const sph_params& pr = cd.pr;
+    const bool con = SCAL && pr.con_solve, concn = SCAL && pr.concn_solve, bous = SCAL && pr.boussinesq_solve;
+    const int ptypei = cd.S.p_type[i];
+    if (cd.S.i_type[i] > 2) return;
+    if (ptypei == 1000) return;
+    if (ptypei <= 0) return;
+    AdvSums a;
+    const NLRow row = nl_row(nl, li);
+    if constexpr (Src::lds) {
+        advection_sums<SCAL, true, Src, W>(cd, i, row, src, g, con, concn, bous, a);
+    } else {
+        if (src.ok()) advection_sums<SCAL, true, Src, W>(cd, i, row, src, g, con, concn, bous, a);
+        else advection_sums<SCAL, false, Src, W>(cd, i, row, src, g, con, concn, bous, a);
     }
     if constexpr (W > 1) {
-        wave_fold(tmpx); wave_fold(tmpy); wave_fold(tmpz); wave_fold(tmp_Rc); wave_fold(tmp_Rd);
-        wave_fold(eulerx); wave_fold(eulery); wave_fold(eulerz); wave_fold(eulert);
-        wave_fold(tmp_temp); wave_fold(tmp_flt);
-        if (lane != 0) return;
+        group_fold<W>(a.tx); group_fold<W>(a.ty); group_fold<W>(a.tz);
+        group_fold<W>(a.cx); group_fold<W>(a.cy); group_fold<W>(a.cz);
+        if (SCAL) {
+            group_fold<W>(a.rc); group_fold<W>(a.rd); group_fold<W>(a.ct); group_fold<W>(a.temp); group_fold<W>(a.flt);
+        }
+        if (g != 0) return;
     }
-    if (pr.fg_solve) tmpz += -pr.gravity;
-    if ((boussinesq_solve) && (ptypei > 0) && (ptypei < 1000))
-        tmpz = betai * pr.gravity * (tmp_temp / tmp_flt - pr.tempb);
-    Q.ftotalx[i] = tmpx - eulerx;
-    Q.ftotaly[i] = tmpy - eulery;
-    Q.ftotalz[i] = tmpz - eulerz;
-    if (con_solve) Q.dtemp[i] += tmp_Rc / (double)cpi - eulert;
-    Q.ftotal[i] = sqrt(tmpx * tmpx + tmpy * tmpy + tmpz * tmpz);
-    if (concn_solve) Q.dconcn[i] = tmp_Rd;
+    double cpi = 1.0;
+    if (con)
+        cpi = (double)(float)(pr.solid_cp * (ptypei == 0 || ptypei == 1000) + pr.air_cp * (ptypei == 1 || ptypei == -1));
+    advection_store(cd, i, a, con, concn, bous, cpi);
 }
-template <class R, bool SCAL>
-__global__ void __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(SCAL ? 1 : 4)))
-k_advection(Seg sg) {
-    SEG_PARTICLE_LIGHT(sg);
-    advection_body<R, SCAL>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{sizeof(R) == 4 ? &cd.crec_adv : nullptr});
+template <bool SCAL>
+__global__ void __launch_bounds__(MAX_BLOCK) k_advection_mixed(Seg sg) {
+    SEG_GROUP_LIGHT(sg);
+    advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
 }
 template <bool SCAL>
 __global__ void __launch_bounds__(WAVE_BLOCK) k_advection_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    advection_body<float, SCAL, GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
+    advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
 }
 template <bool SCAL>
-__global__ void __launch_bounds__(TILE_MAX) k_advection_tile(Seg sg) {
-    TILE_PARTICLE(sg, cd.crec_adv, CREC_ADV_FLOATS);
-    if (chunk_.y >= 0)
-        advection_body<float, SCAL>(cd, i, cd.tile.nl, lane_, LSrc<CREC_ADV_FLOATS>{(const float*)tile_lds_, chunk_.y,
-                                                     cd.tile.halo + chunk_.x,
-                                                         cd.tile.self[lane_]});
-    else advection_body<float, SCAL>(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv});
+__global__ void __launch_bounds__(TILE_THREADS) k_advection_tile(Seg sg, int width) {
+    TILE_CHUNK(sg, width, cd.crec_adv, CREC_ADV_FLOATS);
+    TILE_LANES(width) {
+        if (chunk_.y >= 0)
+            advection_mixed<SCAL, LSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_);
+        else
+            advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_,
+                                                                GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -1152,8 +1409,9 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_wave(Seg sg, int which)
     if (A.p_type[i] != -1) return;
     const KConst kc = cd.kc;
     const NList nl = cd.nl;
-    float hi = (float)A.h[i];
-    float tmp_A = calc_tmpA<float>(kc, hi);
+    const float hi = (float)A.h[i], tmp_A = calc_tmpA<float>(kc, hi);
+    const HScale hs(kc, hi);
+    float rho_c = -1.0f, yrho = 0.0f;
     double xg = A.x[i], yg = A.y[i], zg = A.z[i];
     double t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
@@ -1163,15 +1421,16 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_wave(Seg sg, int which)
         int j = e & NB_IDX;
         if (A.p_type[j] != 1) continue;
         float dx = (float)(xg - A.x[j]), dy = (float)(yg - A.y[j]), dz = (float)(zg - A.z[j]);
-        float tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20f;
-        float mj = (float)A.m[j], rhoj = (float)A.rho[j];
-        float twij = kernel_w<float>(kc, tmp_A, hi, tdist);
-        t[0] += (double)((float)A.ux[j] * (mj / rhoj) * twij);
-        t[1] += (double)((float)A.uy[j] * (mj / rhoj) * twij);
-        t[2] += (double)((float)A.uz[j] * (mj / rhoj) * twij);
-        t[3] += (double)((float)A.pres[j] * (mj / rhoj) * twij);
-        t[4] += (double)((float)A.temp[j] * (mj / rhoj) * twij);
-        t[5] += (double)((mj / rhoj) * twij);
+        const float rhoj = (float)A.rho[j];
+        if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
+        const float vj = quot((float)A.m[j], rhoj, yrho);
+        const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
+        t[0] += (double)((float)A.ux[j] * vj * w);
+        t[1] += (double)((float)A.uy[j] * vj * w);
+        t[2] += (double)((float)A.uz[j] * vj * w);
+        t[3] += (double)((float)A.pres[j] * vj * w);
+        t[4] += (double)((float)A.temp[j] * vj * w);
+        t[5] += (double)(vj * w);
     }
     for (int off = 32; off > 0; off >>= 1)
         for (int q = 0; q < 6; q++) t[q] += __shfl_xor(t[q], off, 64);
@@ -1224,106 +1483,140 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_outlet(Seg sg, int which) {
 }
 
 // ------------------------------------------------------------------------
-// KERNEL_pressureforce3D, functions_PPE.cuh:482-647.  row: i's neighbour
-// entries; src: where their records are (compact records in MIXED).
-template <class R, class Src, int W = 1>
-__device__ __forceinline__ void pressure_force_body(const CaseDesc& cd, int i, const NList& nl, int li,
-                                                    const Src src, int lane = 0) {
+// KERNEL_pressureforce3D, functions_PPE.cuh:482-647
+__device__ __forceinline__ bool pressure_row(const PView& S, int i) {
+    return S.i_type[i] <= 2 && S.p_type[i] < 1000 && S.p_type[i] > 0 && S.buffer_type[i] == 0;
+}
+__global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force(Seg sg) {
+    SEG_PARTICLE_LIGHT(sg);
     const KConst kc = cd.kc;
     const sph_params pr = cd.pr;
     const PView S = cd.S;
     const QView Q = cd.Q;
-    if (S.i_type[i] > 2) return;
-    if (S.p_type[i] >= 1000) return;
-    if (S.p_type[i] <= 0) return;
-    if (S.buffer_type[i] != 0) return;
+    if (!pressure_row(S, i)) return;
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double hi_d = S.h[i];
-    double pi_d = S.pres[i] - S.pres0[i];
-    R pi = (R)pi_d, rhoi = (R)S.rho[i];
+    double hi = S.h[i];
+    double pi = S.pres[i] - S.pres0[i], rhoi = S.rho[i];
     double tmpx = 0, tmpy = 0, tmpz = 0;
     // the pair's kernel normalisation and derivative factor depend only on
     // h_ij: kept while consecutive pairs share it
-    R h_c = (R)-1, A_c = (R)0, f_c = (R)0;
-    const NLRow row = nl_row(nl, li);
-    if (sizeof(R) == 4 && src.ok()) {
-        // the same sums from the compact float records
-        for (int k = W > 1 ? lane : 0; k < row.cnt; k += W) {
-            unsigned e = NB_AT(row, k);
-            if (!(e & F_DM)) continue;
-            const float* C = src.at(e & NB_IDX);
-            const rec_f4 b = Src::f4(src.piece(C, 1));
-            if (__float_as_int(b.w) >= 1000) continue;
-            const rec_f4 a = Src::f4(C);
-            R dx = (R)(xi - (double)a.x), dy = (R)(yi - (double)a.y), dz = (R)(zi - (double)a.z);
-            R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-            R hij = (R)(0.5 * (hi_d + (double)b.z));
-            if (hij != h_c) { h_c = hij; A_c = calc_tmpA<R>(kc, hij); f_c = dw_factor<R>(kc, hij); }
-            R tdwij = kernel_dw_f<R>(kc, A_c, hij, f_c, tdist);
-            R tdwx = tdwij * dx / tdist;
-            R tdwy = tdwij * dy / tdist;
-            R tdwz = tdwij * dz / tdist;
-            R mj = (R)a.w, rhoj = (R)b.x, pj = (R)b.y;
-            if (pr.fp_solve) {
-                const R Pb = (R)0.0;
-                R C_p = (R)(-2.0) * mj / (rhoi * rhoj) * ((pi + Pb) * rhoj + (pj + Pb) * rhoi) / (rhoi + rhoj);
-                tmpx += (double)(C_p * tdwx); tmpy += (double)(C_p * tdwy); tmpz += (double)(C_p * tdwz);
-            }
-        }
-        if constexpr (W > 1) {
-            wave_fold(tmpx); wave_fold(tmpy); wave_fold(tmpz);
-            if (lane != 0) return;
-        }
-        Q.fpx[i] = tmpx; Q.fpy[i] = tmpy; Q.fpz[i] = tmpz;
-        return;
-    }
-    if constexpr (Src::lds) return;   // staged records are compact
-    for (int k = W > 1 ? lane : 0; k < row.cnt; k += W) {
+    double h_c = -1, A_c = 0, f_c = 0;
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = 0; k < row.cnt; k++) {
         unsigned e = NB_AT(row, k);
         if (!(e & F_DM)) continue;
         int j = e & NB_IDX;
         if (S.p_type[j] >= 1000) continue;
-        double hj, pqj, xj, yj, zj, mj_d, rhoj_d;
-        rec_pos(cd.rec, j, xj, yj, zj, mj_d, rhoj_d, pqj);
+        double hj, pj, xj, yj, zj, mj, rhoj;
+        rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pj);
         hj = ld_d2(rec_at(cd.rec, j, 4)).y;
-        R dx = (R)(xi - xj), dy = (R)(yi - yj), dz = (R)(zi - zj);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-        R hij = (R)(0.5 * (hi_d + hj));
-        if (hij != h_c) { h_c = hij; A_c = calc_tmpA<R>(kc, hij); f_c = dw_factor<R>(kc, hij); }
-        R tdwij = kernel_dw_f<R>(kc, A_c, hij, f_c, tdist);
-        R tdwx = tdwij * dx / tdist;
-        R tdwy = tdwij * dy / tdist;
-        R tdwz = tdwij * dz / tdist;
-        R mj = (R)mj_d, rhoj = (R)rhoj_d;
-        R pj = (R)pqj;
+        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
+        double hij = 0.5 * (hi + hj);
+        if (hij != h_c) { h_c = hij; A_c = calc_tmpA<double>(kc, hij); f_c = dw_factor<double>(kc, hij); }
+        double tdwij = kernel_dw_f<double>(kc, A_c, hij, f_c, tdist);
+        double tdwx = tdwij * dx / tdist;
+        double tdwy = tdwij * dy / tdist;
+        double tdwz = tdwij * dz / tdist;
         if (pr.fp_solve) {
-            const R Pb = (R)0.0;
-            R C_p = (R)(-2.0) * mj / (rhoi * rhoj) * ((pi + Pb) * rhoj + (pj + Pb) * rhoi) / (rhoi + rhoj);
-            tmpx += (double)(C_p * tdwx); tmpy += (double)(C_p * tdwy); tmpz += (double)(C_p * tdwz);
+            const double Pb = 0.0;
+            double C_p = -2.0 * mj / (rhoi * rhoj) * ((pi + Pb) * rhoj + (pj + Pb) * rhoi) / (rhoi + rhoj);
+            tmpx += C_p * tdwx; tmpy += C_p * tdwy; tmpz += C_p * tdwz;
         }
-    }
-    if constexpr (W > 1) {
-        wave_fold(tmpx); wave_fold(tmpy); wave_fold(tmpz);
-        if (lane != 0) return;
     }
     Q.fpx[i] = tmpx; Q.fpy[i] = tmpy; Q.fpz[i] = tmpz;
 }
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force(Seg sg) {
-    SEG_PARTICLE_LIGHT(sg);
-    pressure_force_body<R>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{sizeof(R) == 4 ? &cd.crec : nullptr});
+
+// MIXED (see prep_sums)
+template <bool REC, class Src, int W>
+__device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const NLRow row, const Src src, int g,
+                                              double& tmpx, double& tmpy, double& tmpz) {
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    const double* const rec = cd.rec;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i], hi_d = S.h[i];
+    const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
+    const float pi = (float)(S.pres[i] - S.pres0[i]), rhoi = (float)S.rho[i];
+    // the pair's kernel normalisation and derivative factor depend only on
+    // h_ij, its density terms on rho_j: kept while consecutive pairs share them
+    float h_c = -1.0f, A_c = 0.0f, f_c = 0.0f;
+    HScale hs(kc, 1.0f);
+    float rho_c = -1.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
+    for (int k = g; k < row.cnt; k += W) {
+        const unsigned e = NB_AT(row, k);
+        if (!(e & F_DM)) continue;
+        const int j = e & NB_IDX;
+        float dx, dy, dz, mj, rhoj, pj;
+        double hj;
+        if constexpr (REC) {
+            const float* C = src.at(j);
+            const rec_f4 b = Src::f4(src.piece(C, 1));
+            if (__float_as_int(b.w) >= 1000) continue;
+            const rec_f4 p = Src::f4(C);
+            dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
+            rhoj = b.x; pj = b.y; hj = b.z;
+        } else {
+            if (S.p_type[j] >= 1000) continue;
+            double xj, yj, zj, mj_d, rhoj_d, pqj;
+            rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, pqj);
+            hj = ld_d2(rec_at(rec, j, 4)).y;
+            dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
+            mj = (float)mj_d; rhoj = (float)rhoj_d; pj = (float)pqj;
+        }
+        const float hij = (float)(0.5 * (hi_d + hj));
+        if (hij != h_c) {
+            h_c = hij;
+            A_c = calc_tmpA<float>(kc, hij);
+            f_c = dw_factor<float>(kc, hij);
+            hs = HScale(kc, hij);
+        }
+        if (rhoj != rho_c) {
+            rho_c = rhoj;
+            rr = rhoi * rhoj; yrr = recip(rr);
+            rs = rhoi + rhoj; yrs = recip(rs);
+        }
+        const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+        const float dw = kernel_dw_t<float>(kc, A_c, f_c, hs.tR(d.r));
+        const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
+        const float C_p = quot(quot(-2.0f * mj, rr, yrr) * (pi * rhoj + pj * rhoi), rs, yrs);
+        tmpx += (double)(C_p * tx); tmpy += (double)(C_p * ty); tmpz += (double)(C_p * tz);
+    }
+}
+template <class Src, int W = 1>
+__device__ __forceinline__ void pressure_force_mixed(const CaseDesc& cd, int i, const NList& nl, int li,
+                                                     const Src src, int g = 0) {
+    if (!pressure_row(cd.S, i)) return;
+    double tx = 0, ty = 0, tz = 0;
+    const NLRow row = nl_row(nl, li);
+    if (cd.pr.fp_solve) {
+        if constexpr (Src::lds) {
+            pressure_sums<true, Src, W>(cd, i, row, src, g, tx, ty, tz);
+        } else {
+            if (src.ok()) pressure_sums<true, Src, W>(cd, i, row, src, g, tx, ty, tz);
+            else pressure_sums<false, Src, W>(cd, i, row, src, g, tx, ty, tz);
+        }
+    }
+    if constexpr (W > 1) {
+        group_fold<W>(tx); group_fold<W>(ty); group_fold<W>(tz);
+        if (g != 0) return;
+    }
+    const QView Q = cd.Q;
+    Q.fpx[i] = tx; Q.fpy[i] = ty; Q.fpz[i] = tz;
+}
+__global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force_mixed(Seg sg) {
+    SEG_GROUP_LIGHT(sg);
+    pressure_force_mixed<GSrc<CREC_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{&cd.crec}, g_);
 }
 __global__ void __launch_bounds__(WAVE_BLOCK) k_pressure_force_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    pressure_force_body<float, GSrc<CREC_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{&cd.crec}, lane_);
+    pressure_force_mixed<GSrc<CREC_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{&cd.crec}, lane_);
 }
-__global__ void __launch_bounds__(TILE_MAX) k_pressure_force_tile(Seg sg) {
-    TILE_PARTICLE(sg, cd.crec, CREC_FLOATS);
-    if (chunk_.y >= 0)
-        pressure_force_body<float>(cd, i, cd.tile.nl, lane_, LSrc<CREC_FLOATS>{(const float*)tile_lds_, chunk_.y,
-                                                     cd.tile.halo + chunk_.x,
-                                                      cd.tile.self[lane_]});
-    else pressure_force_body<float>(cd, i, cd.tile.nl, lane_, GSrc<CREC_FLOATS>{&cd.crec});
+__global__ void __launch_bounds__(TILE_THREADS) k_pressure_force_tile(Seg sg, int width) {
+    TILE_CHUNK(sg, width, cd.crec, CREC_FLOATS);
+    TILE_LANES(width) {
+        if (chunk_.y >= 0) pressure_force_mixed<LSrc<CREC_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_FLOATS), g_);
+        else pressure_force_mixed<GSrc<CREC_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, GSrc<CREC_FLOATS>{&cd.crec}, g_);
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -1393,8 +1686,8 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_wave(Seg sg) {
     const NList nl = cd.nl;
     const double dt = cd.dt;
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    float tmp_h = (float)(0.5 * S.h[i]);
-    float tmp_A = calc_tmpA<float>(kc, tmp_h);
+    const float tmp_h = (float)(0.5 * S.h[i]), tmp_A = calc_tmpA<float>(kc, tmp_h);
+    const HScale hs(kc, tmp_h);
     double t[4] = {0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
     for (int k = lane; k < row.cnt; k += 64) {
@@ -1403,13 +1696,12 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_wave(Seg sg) {
         int j = e & NB_IDX;
         if (S.i_type[j] == 4 || S.p_type[j] != 1) continue;
         float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
-        float tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20f;
-        float twij = kernel_w<float>(kc, tmp_A, tmp_h, tdist);
-        float tmprho = (float)S.m[j] / (float)S.rho[j];
-        t[0] += (double)(((float)S.ux[j]) * tmprho * twij);
-        t[1] += (double)(((float)S.uy[j]) * tmprho * twij);
-        t[2] += (double)(((float)S.uz[j]) * tmprho * twij);
-        t[3] += (double)(tmprho * twij);
+        const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
+        const float tmprho = (float)S.m[j] / (float)S.rho[j];
+        t[0] += (double)((float)S.ux[j] * tmprho * w);
+        t[1] += (double)((float)S.uy[j] * tmprho * w);
+        t[2] += (double)((float)S.uz[j] * tmprho * w);
+        t[3] += (double)(tmprho * w);
     }
     for (int off = 32; off > 0; off >>= 1)
         for (int q = 0; q < 4; q++) t[q] += __shfl_xor(t[q], off, 64);
@@ -1611,8 +1903,23 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
             const size_t lds_ = tile_lds_bytes(e, (recf));                                          \
             SPH_TRY(tile_lds_allow(e, (const void*)(kern), lds_));                                  \
             SPH_TRY(prof_begin(e, name, 0.0));                                                      \
-            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(e.tile_lanes), lds_, e.st, Seg{e.d_desc, sh_.tab}); \
+            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(TILE_THREADS), lds_, e.st, Seg{e.d_desc, sh_.tab}, e.tile_lanes); \
             SPH_TRY(launch_check(&e, name));                                                        \
+            SPH_TRY(prof_end(e));                                                                   \
+        }                                                                                           \
+    } while (0)
+// the same with GROUP lanes a particle
+#define SEGG(name, kid, kern, ...)                                                                   \
+    do {                                                                                            \
+        const int blk_ = tuned_block(e, (kid));                                                     \
+        Shape sh_;                                                                                  \
+        SPH_TRY(shape(e, 0, blk_ / GROUP, &sh_));                                                   \
+        if (sh_.grid > 0) {                                                                         \
+            SPH_TRY(prof_begin(e, name, 0.0));                                                      \
+            SPH_TRY(tune_begin(e, (kid), blk_));                                                    \
+            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(blk_), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
+            SPH_TRY(launch_check(&e, name));                                                        \
+            SPH_TRY(tune_end(e));                                                                   \
             SPH_TRY(prof_end(e));                                                                   \
         }                                                                                           \
     } while (0)
@@ -1879,15 +2186,15 @@ int step_physics_front(Eng& e) {
     bool any_gc = false;
     for (size_t k = 0; k < e.cs.size(); k++) any_gc |= !e.h_desc[k].gc_fresh;
     if (any_gc) {
-        if (mixed) SEGL("grad_corr", TK_GRAD_CORR, k_grad_corr<float>);
-        else SEGL("grad_corr", TK_GRAD_CORR, k_grad_corr<double>);
+        if (mixed) SEGG("grad_corr", TK_GRAD_CORR, k_grad_corr_mixed);
+        else SEGL("grad_corr", TK_GRAD_CORR, k_grad_corr);
     }
     SPH_TRY(pack_records(e, REC_PRE));   // compact records for the strain pass
     if (mixed && e.tile_lanes) TILEL("prep", k_prep_tile, CREC_ADV_FLOATS);
     else if (mixed) {
-        SEGL("prep", TK_PREP, k_prep<float>);
+        SEGG("prep", TK_PREP, k_prep_mixed);
         HEAVYL("prep_heavy", k_prep_heavy);
-    } else SEGL("prep", TK_PREP, k_prep<double>);
+    } else SEGL("prep", TK_PREP, k_prep);
     if (mixed) WAVEL("boundary3d", k_boundary3d_wave);
     else SEGL("boundary3d", TK_BOUNDARY, k_boundary3d<double>);
     SEGL("most_self", -1, k_most_self);
@@ -1901,15 +2208,15 @@ int step_physics_front(Eng& e) {
             if (scal) TILEL("advection", k_advection_tile<true>, CREC_ADV_FLOATS);
             else TILEL("advection", k_advection_tile<false>, CREC_ADV_FLOATS);
         } else if (scal) {
-            SEGL("advection", TK_ADVECTION, (k_advection<float, true>));
+            SEGG("advection", TK_ADVECTION, k_advection_mixed<true>);
             HEAVYL("advection_heavy", k_advection_heavy<true>);
         } else {
-            SEGL("advection", TK_ADVECTION, (k_advection<float, false>));
+            SEGG("advection", TK_ADVECTION, k_advection_mixed<false>);
             HEAVYL("advection_heavy", k_advection_heavy<false>);
         }
     } else {
-        if (scal) SEGL("advection", TK_ADVECTION, (k_advection<double, true>));
-        else SEGL("advection", TK_ADVECTION, (k_advection<double, false>));
+        if (scal) SEGL("advection", TK_ADVECTION, k_advection<true>);
+        else SEGL("advection", TK_ADVECTION, k_advection<false>);
     }
     SEGL("projection", -1, k_projection);
     SPH_TRY(run_periodic(e, 0));
@@ -1925,10 +2232,10 @@ int step_physics_back(Eng& e) {
     SPH_TRY(pack_records(e, REC_PQ));   // pressures after the solve and the boundary passes
     if (mixed && e.tile_lanes) TILEL("pressure_force", k_pressure_force_tile, CREC_FLOATS);
     else if (mixed) {
-        SEGL("pressure_force", TK_PRESSURE, k_pressure_force<float>);
+        SEGG("pressure_force", TK_PRESSURE, k_pressure_force_mixed);
         HEAVYL("pressure_force_heavy", k_pressure_force_heavy);
     }
-    else SEGL("pressure_force", TK_PRESSURE, k_pressure_force<double>);
+    else SEGL("pressure_force", TK_PRESSURE, k_pressure_force);
     if (mixed) WAVEL("ibm_force", k_ibm_force_wave);
     else SEGL("ibm_force", TK_IBM_FORCE, k_ibm_force<double>);
     if (mixed) SEGL("ibm_spread", TK_IBM_SPREAD, k_ibm_spread<float>);

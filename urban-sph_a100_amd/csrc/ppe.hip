@@ -669,135 +669,246 @@ __device__ __forceinline__ KSet<float> kset(const PPEView& v, float*) {
 // which no float or double sum of this operator can feel (its entries are
 // O(1 / dx^2)), and as zeros they can leave the stencil slices.  FP64 stores
 // every value as computed.
-template <class V, class R>
-__device__ __forceinline__ V stored_value(R cc) {
-    if constexpr (sizeof(V) == 4) {
-        const float v = (float)cc;
-        return fabsf(v) < 1e-30f ? 0.0f : v;
+__device__ __forceinline__ float stored_value(float c) { return fabsf(c) < 1e-30f ? 0.0f : c; }
+// The row's sums: b_i before the division by dt, sum_j c_ij, sum_j c_ij q_j
+// (Jacobi sweep), the known neighbours' share of the right-hand side.
+struct RowSums { double b = 0, A = 0, Ap = 0, kn = 0; };
+__device__ __forceinline__ void assemble_store(const CaseDesc& cd, int i, int r, const RowSums& a, bool write_diag,
+                                               int jacobi) {
+    const PPEView& pp = cd.ppe;
+    const PView S = cd.S;
+    const double bi = a.b / cd.dt;
+    if (jacobi) {
+        pp.pnew[r] = S.pres0[i] + (bi + a.Ap) / a.A;
     } else {
-        return (V)cc;
+        if (write_diag) {
+            pp.diag[r] = a.A;
+            if (pp.fdiag) pp.fdiag[r] = (float)a.A;
+        }
+        pp.rhs[r] = bi + a.kn;
+        pp.x[r] = S.pres[i] - S.pres0[i];
     }
 }
-template <class R, class V, class Src>
-__device__ __forceinline__ void assemble_body(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
-                                              int jacobi) {
+__global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble(Seg sg, int jacobi) {
+    SEG_ROW(sg);
+    if (row >= cd.n) return;
+    const int i = cd.porder ? cd.porder[row] : row;   // this thread's particle
     const PPEView pp = cd.ppe;
     const int r = pp.rowof[i];
     if (r < 0) return;
     const KConst kc = cd.kc;
     const PView S = cd.S;
     const QView Q = cd.Q;
-    const double dt = cd.dt;
     const int* rowof = pp.rowof;
-    R hi = (R)(1.0 * S.h[i]);
-    R tmp_A = calc_tmpA<R>(kc, hi);
+    double hi = 1.0 * S.h[i];
+    double tmp_A = calc_tmpA<double>(kc, hi);
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    R rhoi = (R)S.rho[i];
-    R gc11 = (R)Q.inv_xx[i], gc12 = (R)Q.inv_xy[i], gc22 = (R)Q.inv_yy[i];
-    R gc23 = (R)Q.inv_yz[i], gc31 = (R)Q.inv_zx[i], gc33 = (R)Q.inv_zz[i];
-    double bix = 0, biy = 0, biz = 0, Aij = 0, AijPij = 0, kn = 0;
-    const NLRow nr = nl_row(nl, li);
-    const int m = nr.cnt;
+    double rhoi = S.rho[i];
+    double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
+    double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
+    double bix = 0, biy = 0, biz = 0;
+    RowSums a;
+    const NLRow nr = nl_row(cd.nl, i);
     // with fixed particles the values of a search are written by its first
     // step only; later steps compute the right-hand side
-    V* out = (jacobi || cd.vals_fresh) ? nullptr : wvals_of(pp, (V*)nullptr) + prow(pp.sl_off, r);
+    double* out = (jacobi || cd.vals_fresh) ? nullptr : pp.vals64 + prow(pp.sl_off, r);
     const bool full = jacobi || out != nullptr;   // the coefficients of every pair are needed
-    const unsigned char* smap = pp.slotmap ? pp.slotmap + prow(pp.sl_off, r) : nullptr;
     int slot = 0;
-    // read once: the stores of the loop could alias the descriptor
-    const bool compact = Src::lds || (sizeof(R) == 4 && src.ok());
     const double* const rec = cd.rec;
-    for (int k = 0; k < m; k++) {
+    for (int k = 0; k < nr.cnt; k++) {
         unsigned e = NB_AT(nr, k);
         if (!(e & F_DP)) continue;
         int j = e & NB_IDX;
-        double xj, yj, zj, mj_d, rhoj_d, qj, uxj, uyj, uzj;
-        bool jrow;   // j is an unknown of the PPE
-        if (compact) {   // the compact record (positions float-exact)
-            const float* C = src.at(j);
-            const rec_f4 b = Src::f4(src.piece(C, 1));
-            if (crec_ptype(b.w) >= 1000 || crec_itype(b.w) == 4) continue;
-            jrow = crec_has_row(b.w);
-            const rec_f4 a = Src::f4(C);
-            const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
-            xj = a.x; yj = a.y; zj = a.z; mj_d = a.w; rhoj_d = b.x;
-            uxj = u.x; uyj = u.y; uzj = w.x; qj = w.y;
-        } else {
-            if constexpr (Src::lds) continue;   // staged records are compact
-            double vtj_, hj_;
-            int ptj, itj;
-            rec_aux(rec, j, vtj_, ptj, itj);
-            if (ptj >= 1000 || itj == 4) continue;
-            rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, qj);
-            rec_vel(rec, j, uxj, uyj, uzj, hj_);
-            jrow = rowof[j] >= 0;
-        }
-        R dx = (R)(xi - xj), dy = (R)(yi - yj), dz = (R)(zi - zj);
-        R rhoj = (R)rhoj_d, mj = (R)mj_d;
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) + (R)1e-20;
-        R tdwij = kernel_dwp<R>(kc, tmp_A, hi, tdist);
-        R tdwx = tdwij * dx / tdist;
-        R tdwy = tdwij * dy / tdist;
-        R tdwz = tdwij * dz / tdist;
-        R tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
-        R tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
-        R tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
-        R hm = (R)2.0 * rhoi * rhoj / (rhoi + rhoj);
-        bix += (double)(mj / rhoj * (R)(uxj - uxi) * tdwxc * hm);
-        biy += (double)(mj / rhoj * (R)(uyj - uyi) * tdwyc * hm);
-        biz += (double)(mj / rhoj * (R)(uzj - uzi) * tdwzc * hm);
-        auto coef = [&]() { return (R)2.0 * mj / rhoj * (dx * tdwxc + dy * tdwyc + dz * tdwzc) / tdist / tdist; };
+        double xj, yj, zj, mj, rhoj, qj, uxj, uyj, uzj, vtj_, hj_;
+        int ptj, itj;
+        rec_aux(rec, j, vtj_, ptj, itj);
+        if (ptj >= 1000 || itj == 4) continue;
+        rec_pos(rec, j, xj, yj, zj, mj, rhoj, qj);
+        rec_vel(rec, j, uxj, uyj, uzj, hj_);
+        const bool jrow = rowof[j] >= 0;   // j is an unknown of the PPE
+        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+        double tdwij = kernel_dwp<double>(kc, tmp_A, hi, tdist);
+        double tdwx = tdwij * dx / tdist;
+        double tdwy = tdwij * dy / tdist;
+        double tdwz = tdwij * dz / tdist;
+        double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
+        double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
+        double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
+        double hm = 2.0 * rhoi * rhoj / (rhoi + rhoj);
+        bix += mj / rhoj * (uxj - uxi) * tdwxc * hm;
+        biy += mj / rhoj * (uyj - uyi) * tdwyc * hm;
+        biz += mj / rhoj * (uzj - uzi) * tdwzc * hm;
+        auto coef = [&]() { return 2.0 * mj / rhoj * (dx * tdwxc + dy * tdwyc + dz * tdwzc) / tdist / tdist; };
         if (full) {
-            R cc = coef();
-            double ccd = (double)cc;
-            Aij += ccd;
-            if (jacobi) AijPij += ccd * qj;
-            if (!src.self(j, i)) {
+            double cc = coef();
+            a.A += cc;
+            if (jacobi) a.Ap += cc * qj;
+            if (j != i) {
                 if (jrow) {
-                    if (out) {
-                        const V v = stored_value<V>(cc);
-                        if (slot < LONG_ROW || !pp.ltail) out[pslot(smap ? smap[pslot(slot)] : slot)] = v;
-                        else pp.tail_vals[pp.tail_off[pp.ltail[r]] + (slot - LONG_ROW)] = (float)v;
-                    }
+                    if (out) out[pslot(slot)] = cc;
                     slot++;
                 } else {
-                    kn += ccd * qj;
+                    a.kn += cc * qj;
                 }
             }
-        } else if (!jrow && !src.self(j, i)) {
+        } else if (!jrow && j != i) {
             // values and diagonal kept from the search's first step: only the
             // known neighbours' share of the right-hand side needs the coefficient
-            kn += (double)coef() * qj;
+            a.kn += coef() * qj;
         }
     }
-    double bi = 1.0 * (bix + biy + biz + 0.0) / dt;
-    double q0 = S.pres[i] - S.pres0[i];
-    if (jacobi) {
-        pp.pnew[r] = S.pres0[i] + (bi + AijPij) / Aij;
+    a.b = 1.0 * (bix + biy + biz + 0.0);
+    assemble_store(cd, i, r, a, out != nullptr, jacobi);
+}
+
+// MIXED: GROUP lanes a particle, the pair arithmetic in float, the sums in
+// double.  REC: the pair's fields come from the compact records (float
+// positions, whose float difference is the rounded exact difference), else
+// from the 128-byte double records.  FULL writes the row's values (a
+// search's first step) or sums every coefficient (the Jacobi sweep); the slot
+// of a value is its rank among the row's entries, counted over the group.
+template <bool REC, bool FULL, class Src>
+__device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, const NLRow row, const Src src, int g,
+                                              float* out, int jacobi, double (&b)[3], RowSums& a) {
+    const KConst kc = cd.kc;
+    const PPEView& pp = cd.ppe;
+    const PView S = cd.S;
+    const QView Q = cd.Q;
+    const double* const rec = cd.rec;
+    const int* const rowof = pp.rowof;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const float rhoi = (float)S.rho[i];
+    const float gc11 = (float)Q.inv_xx[i], gc12 = (float)Q.inv_xy[i], gc22 = (float)Q.inv_yy[i];
+    const float gc23 = (float)Q.inv_yz[i], gc31 = (float)Q.inv_zx[i], gc33 = (float)Q.inv_zz[i];
+    const float hi = (float)S.h[i], tmp_A = calc_tmpA<float>(kc, hi), f = 1.0f / ((float)kc.kappa * hi);
+    const HScale hs(kc, hi);
+    const unsigned char* const smap = pp.slotmap ? pp.slotmap + prow(pp.sl_off, r) : nullptr;
+    const int* const ltail = pp.ltail;
+    const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);   // the group's first lane
+    int slot = 0;
+    // consecutive neighbours mostly share rho: what it enters is kept
+    float rho_c = -1.0f, yrho = 0.0f, hm = 0.0f;
+    for (int k0 = 0; k0 < row.cnt; k0 += GROUP) {
+        const int k = k0 + g;
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        bool pair = (e & F_DP) != 0, own = false;   // own: an entry of the row
+        const int j = e & NB_IDX;
+        float cc = 0.0f;
+        float dx = 0, dy = 0, dz = 0, mj = 0, rhoj = 0;
+        double qj = 0, uxj = 0, uyj = 0, uzj = 0;
+        bool jrow = false;   // j is an unknown of the PPE
+        if (pair) {
+            if constexpr (REC) {
+                const float* C = src.at(j);
+                const rec_f4 q = Src::f4(src.piece(C, 1));
+                pair = crec_ptype(q.w) < 1000 && crec_itype(q.w) != 4;
+                if (pair) {
+                    jrow = crec_has_row(q.w);
+                    const rec_f4 p = Src::f4(C);
+                    const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
+                    dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w; rhoj = q.x;
+                    uxj = u.x; uyj = u.y; uzj = w.x; qj = w.y;
+                }
+            } else {
+                double vtj_, hj_, xj, yj, zj, mj_d, rhoj_d;
+                int ptj, itj;
+                rec_aux(rec, j, vtj_, ptj, itj);
+                pair = ptj < 1000 && itj != 4;
+                if (pair) {
+                    rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, qj);
+                    rec_vel(rec, j, uxj, uyj, uzj, hj_);
+                    jrow = rowof[j] >= 0;
+                    dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
+                    mj = (float)mj_d; rhoj = (float)rhoj_d;
+                }
+            }
+        }
+        if (pair) {
+            if (rhoj != rho_c) {
+                rho_c = rhoj;
+                yrho = recip(rhoj);
+                hm = 2.0f * rhoi * rhoj / (rhoi + rhoj);
+            }
+            const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+            const float dw = kernel_dwp_t<float>(tmp_A, f, hs.tR(d.r));
+            const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
+            const float cx = gc11 * tx + gc12 * ty + gc31 * tz, cy = gc12 * tx + gc22 * ty + gc23 * tz,
+                        cz = gc31 * tx + gc23 * ty + gc33 * tz;
+            const float vj = quot(mj, rhoj, yrho);
+            b[0] += (double)(vj * (float)(uxj - uxi) * cx * hm);
+            b[1] += (double)(vj * (float)(uyj - uyi) * cy * hm);
+            b[2] += (double)(vj * (float)(uzj - uzi) * cz * hm);
+            const bool other = !src.self(j, i);
+            // (with the values kept from the search's first step, only the known
+            // neighbours' share of the right-hand side needs the coefficient)
+            if (FULL || (!jrow && other)) {
+                cc = quot(quot(quot(2.0f * mj, rhoj, yrho) * (dx * cx + dy * cy + dz * cz), d.r, d.y), d.r, d.y);
+                if (FULL) {
+                    a.A += (double)cc;
+                    if (jacobi) a.Ap += (double)cc * qj;
+                }
+                if (other && !jrow) a.kn += (double)cc * qj;
+                own = FULL && other && jrow;
+            }
+        }
+        if (FULL && out) {
+            const unsigned m = (unsigned)(__ballot(own) >> gbit) & ((1u << GROUP) - 1u);
+            if (own) {
+                const int s = slot + __popc(m & ((1u << g) - 1u));
+                const float v = stored_value(cc);
+                if (s < LONG_ROW || !ltail) out[pslot(smap ? smap[pslot(s)] : s)] = v;
+                else pp.tail_vals[pp.tail_off[ltail[r]] + (s - LONG_ROW)] = v;
+            }
+            slot += __popc(m);
+        }
+    }
+}
+template <class Src>
+__device__ __forceinline__ void assemble_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src, int g,
+                                               int jacobi) {
+    const PPEView& pp = cd.ppe;
+    const int r = pp.rowof[i];
+    if (r < 0) return;
+    float* out = (jacobi || cd.vals_fresh) ? nullptr : pp.vals32 + prow(pp.sl_off, r);
+    const NLRow row = nl_row(nl, li);
+    RowSums a;
+    double b[3] = {0.0, 0.0, 0.0};
+    const bool full = jacobi || out != nullptr;
+    if constexpr (Src::lds) {
+        if (full) assemble_sums<true, true>(cd, i, r, row, src, g, out, jacobi, b, a);
+        else assemble_sums<true, false>(cd, i, r, row, src, g, out, jacobi, b, a);
+    } else if (src.ok()) {
+        if (full) assemble_sums<true, true>(cd, i, r, row, src, g, out, jacobi, b, a);
+        else assemble_sums<true, false>(cd, i, r, row, src, g, out, jacobi, b, a);
     } else {
-        if (out) {
-            pp.diag[r] = Aij;
-            if (pp.fdiag) pp.fdiag[r] = (float)Aij;
-        }
-        pp.rhs[r] = bi + kn;
-        pp.x[r] = q0;
+        if (full) assemble_sums<false, true>(cd, i, r, row, src, g, out, jacobi, b, a);
+        else assemble_sums<false, false>(cd, i, r, row, src, g, out, jacobi, b, a);
     }
+    for (double& v : b) group_fold<GROUP>(v);
+    group_fold<GROUP>(a.A); group_fold<GROUP>(a.Ap); group_fold<GROUP>(a.kn);
+    if (g != 0) return;
+    a.b = 1.0 * (b[0] + b[1] + b[2] + 0.0);
+    assemble_store(cd, i, r, a, out != nullptr, jacobi);
 }
-template <class R, class V>
-__global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble(Seg sg, int jacobi) {
-    SEG_ROW(sg);
-    if (row >= cd.n) return;
-    const int i = cd.porder ? cd.porder[row] : row;   // this thread's particle
-    assemble_body<R, V>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{sizeof(R) == 4 ? &cd.crec_adv : nullptr}, jacobi);
+__global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble_mixed(Seg sg, int jacobi) {
+    int first_;
+    const int cid_ = seg_case(sg, first_);
+    const CaseDesc& cd = sg.cd[cid_];
+    const int t = first_ + (int)threadIdx.x / GROUP;
+    if (t >= cd.n) return;
+    const int i = cd.porder ? cd.porder[t] : t;   // this group's particle
+    assemble_mixed(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, (int)threadIdx.x % GROUP, jacobi);
 }
-__global__ void __launch_bounds__(TILE_MAX) k_ppe_assemble_tile(Seg sg, int jacobi) {
-    TILE_PARTICLE(sg, cd.crec_adv, CREC_ADV_FLOATS);
-    if (chunk_.y >= 0)
-        assemble_body<float, float>(cd, i, cd.tile.nl, lane_, LSrc<CREC_ADV_FLOATS>{(const float*)tile_lds_, chunk_.y,
-                                                     cd.tile.halo + chunk_.x,
-                                                        cd.tile.self[lane_]}, jacobi);
-    else assemble_body<float, float>(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, jacobi);
+__global__ void __launch_bounds__(TILE_THREADS) k_ppe_assemble_tile(Seg sg, int width, int jacobi) {
+    TILE_CHUNK(sg, width, cd.crec_adv, CREC_ADV_FLOATS);
+    TILE_LANES(width) {
+        if (chunk_.y >= 0) assemble_mixed(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_, jacobi);
+        else assemble_mixed(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_, jacobi);
+    }
 }
 
 // pressure <- Jacobi sweep output, or p0 + solved increment
@@ -1863,21 +1974,21 @@ int ppe_solve(Eng& e) {
         const size_t lds = tile_lds_bytes(e, CREC_ADV_FLOATS);
         SPH_TRY(tile_lds_allow(e, (const void*)k_ppe_assemble_tile, lds));
         SPH_TRY(prof_begin(e, "ppe_assemble", asm_bytes));
-        hipLaunchKernelGGL(k_ppe_assemble_tile, dim3(sh.grid), dim3(e.tile_lanes), lds, e.st, Seg{e.d_desc, sh.tab},
-                           jacobi ? 1 : 0);
+        hipLaunchKernelGGL(k_ppe_assemble_tile, dim3(sh.grid), dim3(TILE_THREADS), lds, e.st, Seg{e.d_desc, sh.tab},
+                           e.tile_lanes, jacobi ? 1 : 0);
         SPH_TRY(launch_check(&e, "ppe_assemble"));
         SPH_TRY(prof_end(e));
     } else {
         const int blk = tuned_block(e, TK_ASSEMBLE);
         Shape sh;
-        SPH_TRY(shape(e, 0, blk, &sh));   // over particles
+        SPH_TRY(shape(e, 0, mixed ? blk / GROUP : blk, &sh));   // over particles
         SPH_TRY(prof_begin(e, "ppe_assemble", asm_bytes));
         SPH_TRY(tune_begin(e, TK_ASSEMBLE, blk));
         if (mixed)
-            hipLaunchKernelGGL((k_ppe_assemble<float, float>), dim3(sh.grid), dim3(blk), 0, e.st, Seg{e.d_desc, sh.tab},
+            hipLaunchKernelGGL(k_ppe_assemble_mixed, dim3(sh.grid), dim3(blk), 0, e.st, Seg{e.d_desc, sh.tab},
                                jacobi ? 1 : 0);
         else
-            hipLaunchKernelGGL((k_ppe_assemble<double, double>), dim3(sh.grid), dim3(blk), 0, e.st,
+            hipLaunchKernelGGL(k_ppe_assemble, dim3(sh.grid), dim3(blk), 0, e.st,
                                Seg{e.d_desc, sh.tab}, jacobi ? 1 : 0);
         SPH_TRY(launch_check(&e, "ppe_assemble"));
         SPH_TRY(tune_end(e));

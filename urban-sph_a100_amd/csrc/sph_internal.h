@@ -60,7 +60,7 @@ __device__ __forceinline__ NLRow nl_row(const NList& nl, long long i) {
 
 // Cell tiles of the record-gathering passes (tiles.hip): chunks of at most
 // tile_particles particles of one block of cells, each with its halo.
-constexpr int TILE_MAX = 256;   // most lanes of a tile chunk (the tile passes' workgroup size)
+constexpr int TILE_MAX = 256;   // most lanes of a tile chunk
 struct TileView {
     const int* part;     // lane -> particle (chunk c: lanes c * cap ..), -1 on padding
     const int2* chunk;   // per chunk: first halo entry, halo size (-1: entries hold particle indices)
@@ -198,6 +198,24 @@ __device__ __forceinline__ void wave_fold(double& v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
 }
+// MIXED passes over the particles' lists: GROUP lanes a particle, lane g_
+// taking entries g_, g_ + GROUP, ... of its list, a fixed butterfly adding
+// the lanes' sums (so a case's results do not depend on the launch); the
+// table of the launch hands out blockDim / GROUP particles a block.  Lanes of
+// a group read neighbours that lie next to each other (the lists ascend in
+// cell order), so a gather touches fewer cache lines than 64 particles' k-th
+// neighbours do, and a small case has GROUP times the waves to hide its
+// gathers behind.  Advection, by lanes a particle (1 as it was before, 2, 4,
+// 8, 16): 2.39, 1.70, 1.53, 1.60, 1.80 ms on the 2.13 M canyon; 198, 76, 42, 29,
+// 25 us on 20,609 particles.  Prep, assembly and the pressure force alike; the
+// refined canyon's gradient correction, where a particle lists up to 5000
+// neighbours: 3.1, 1.76, 0.97, 0.64 ms.
+constexpr int GROUP = 8;
+template <int W>
+__device__ __forceinline__ void group_fold(double& v) {
+#pragma unroll
+    for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+}
 // Workgroups are dispatched to the 8 XCDs round-robin (block b runs on XCD
 // b mod 8).  Logical block order is remapped so that each XCD works on one
 // contiguous range of blocks: neighbouring rows, whose gathers touch the
@@ -331,10 +349,13 @@ struct LSrc {
     __device__ bool self(int j, int) const { return j == self_slot; }
 };
 
-// Cell-tile passes (tiles.hip): a workgroup per chunk, blockDim = the chunk
-// width.  Stages the chunk's halo records (RECF floats each, from RECS) in
-// LDS, then maps the thread to its lane (a row of cd.tile.nl) and the
-// lane's particle; padding lanes return after the barrier.
+// Cell-tile passes (tiles.hip): a workgroup of TILE_THREADS per chunk of
+// `width` lanes.  TILE_CHUNK stages the chunk's halo records (RECF floats
+// each, from RECS) in LDS; TILE_LANES runs its body for the lanes (rows of
+// cd.tile.nl) and their particles, GROUP threads a lane, as the per-particle
+// passes do; padding lanes are left out.
+constexpr int TILE_THREADS = 512;
+static_assert(TILE_THREADS % (SLICE * GROUP) == 0 || (SLICE * GROUP) % TILE_THREADS == 0, "a chunk is whole rounds of lanes");
 // A thread copies whole records (Q float4 pieces), TILE_U of them a round,
 // all loads of a round issued before its stores; piece q of record r goes
 // to float4 q * cnt + r.
@@ -364,17 +385,21 @@ __device__ __forceinline__ void tile_stage(float4* lds, const float* recs, const
     if (recf == 8) tile_stage_q<2>(lds, recs, halo, cnt);
     else tile_stage_q<4>(lds, recs, halo, cnt);
 }
-#define TILE_PARTICLE(sg, RECS, RECF)                                                            \
+#define TILE_CHUNK(sg, width, RECS, RECF)                                                       \
     extern __shared__ float4 tile_lds_[];                                                       \
-    int first_;                                                                                 \
-    const int cid_ = seg_case((sg), first_);                                                    \
-    const CaseDesc& cd = (sg).cd[cid_];                                                         \
-    const int2 chunk_ = cd.tile.chunk[first_ / (int)blockDim.x];                                \
+    const unsigned lb_ = xcd_block();                                                           \
+    const int2 te_ = (sg).tab ? (sg).tab[lb_] : make_int2(0, (int)(lb_ * (unsigned)(width)));   \
+    const CaseDesc& cd = (sg).cd[te_.x];                                                        \
+    const int2 chunk_ = cd.tile.chunk[te_.y / (width)];                                         \
     if (chunk_.y > 0) tile_stage(tile_lds_, (RECS), cd.tile.halo + chunk_.x, chunk_.y, (RECF)); \
     __syncthreads();                                                                            \
-    const int lane_ = first_ + (int)threadIdx.x;                                                \
-    const int i = cd.tile.part[lane_];                                                          \
-    if (i < 0) return;
+    const int g_ = (int)threadIdx.x % GROUP;
+#define TILE_LANES(width)                                                                       \
+    for (int l_ = (int)threadIdx.x / GROUP, lane_, i;                                           \
+         l_ < (width) && (lane_ = te_.y + l_, i = cd.tile.part[lane_], true); l_ += TILE_THREADS / GROUP) \
+        if (i >= 0)
+#define TILE_SRC(RECF) \
+    LSrc<RECF> { (const float*)tile_lds_, chunk_.y, cd.tile.halo + chunk_.x, cd.tile.self[lane_] }
 __device__ __forceinline__ int crec_ptype(float w) { return (int)(short)(__float_as_int(w) & 0xffff); }
 __device__ __forceinline__ int crec_itype(float w) { return (__float_as_int(w) >> 16) & 0x3fff; }
 __device__ __forceinline__ bool crec_has_row(float w) { return (__float_as_int(w) & CREC_ROW_BIT) != 0; }

@@ -33,10 +33,9 @@ __device__ __forceinline__ R calc_tmpA(const KConst& k, R tH) {
 }
 
 // calc_kernel_wij, functions_KNL.cuh:41-71 (3-D)
+// over tR = r / h / kappa
 template <class R>
-__device__ __forceinline__ R kernel_w(const KConst& k, R tA, R tH, R rr) {
-    const R kap = (R)k.kappa;
-    R tR = rr / tH / kap;
+__device__ __forceinline__ R kernel_w_t(const KConst& k, R tA, R tR) {
     const R one = (R)1;
     switch (k.type) {
     case SPH_GAUSSIAN: { R a = (R)2.0 * tR; return tA * exp(-(a * a)); }
@@ -61,6 +60,11 @@ __device__ __forceinline__ R kernel_w(const KConst& k, R tA, R tH, R rr) {
     return (R)0;
 }
 
+template <class R>
+__device__ __forceinline__ R kernel_w(const KConst& k, R tA, R tH, R rr) {
+    return kernel_w_t<R>(k, tA, rr / tH / (R)k.kappa);
+}
+
 // calc_kernel_dwij, functions_KNL.cuh:73-103 (3-D).  The leading factor
 // 1/h (Gaussian, quintic, quartic) or 1/(kappa h) (Wendland) depends on h
 // only: dw_factor computes it, kernel_dw_f takes it, so that a caller whose
@@ -73,9 +77,7 @@ __device__ __forceinline__ R dw_factor(const KConst& k, R tH) {
                                                                                        : one / ((R)k.kappa * tH);
 }
 template <class R>
-__device__ __forceinline__ R kernel_dw_f(const KConst& k, R tA, R tH, R f, R rr) {
-    const R kap = (R)k.kappa;
-    R tR = rr / tH / kap;
+__device__ __forceinline__ R kernel_dw_t(const KConst& k, R tA, R f, R tR) {
     const R one = (R)1;
     switch (k.type) {
     case SPH_GAUSSIAN: { R a = (R)2.0 * tR; return f * tA * (R)(-2.0) * (R)2.0 * tR * exp(-(a * a)); }
@@ -100,20 +102,64 @@ __device__ __forceinline__ R kernel_dw_f(const KConst& k, R tA, R tH, R f, R rr)
     return (R)0;
 }
 template <class R>
+__device__ __forceinline__ R kernel_dw_f(const KConst& k, R tA, R tH, R f, R rr) {
+    return kernel_dw_t<R>(k, tA, f, rr / tH / (R)k.kappa);
+}
+template <class R>
 __device__ __forceinline__ R kernel_dw(const KConst& k, R tA, R tH, R rr) {
     return kernel_dw_f(k, tA, tH, dw_factor(k, tH), rr);
 }
 
 // calc_kernel_dwij_pressure, functions_KNL.cuh:355-369: Wendland-6 shape,
 // caller's normalisation.
+// f = 1 / (kappa h)
 template <class R>
-__device__ __forceinline__ R kernel_dwp(const KConst& k, R tA, R tH, R rr) {
-    const R kap = (R)k.kappa;
-    R tR = rr / tH / kap;
+__device__ __forceinline__ R kernel_dwp_t(R tA, R f, R tR) {
     const R one = (R)1;
-    return (R)(tR < one) * (one / (kap * tH)) * tA *
+    return (R)(tR < one) * f * tA *
            ((R)(-22) * tR * (one - tR) * (one - tR) * (one - tR) * (one - tR) * (one - tR) * (one - tR) * (one - tR) * ((R)16 * tR * tR + (R)7 * tR + one));
 }
+
+template <class R>
+__device__ __forceinline__ R kernel_dwp(const KConst& k, R tA, R tH, R rr) {
+    return kernel_dwp_t<R>(tA, (R)1 / ((R)k.kappa * tH), rr / tH / (R)k.kappa);
+}
+
+// ------------------------------------------------------------------------
+// Division and square root of the float (MIXED) pair formulas.  A pair
+// divides several numerators by one denominator (its distance, its
+// neighbour's density, the particle's h), and the compiler's IEEE division
+// is ten instructions each; with the denominator's reciprocal refined once,
+// a quotient is three: the product with the reciprocal, the exact remainder,
+// the correction (Markstein, IBM J. Res. Dev. 34(1), 1990).  It is the
+// correctly rounded quotient of normal-range operands (none of 4e8 random pairs
+// differed on the CPU, reciprocal started one ulp off; the root differs in
+// one of 1.4 million), so the pair terms keep the accuracy and, but for those,
+// the bits of the IEEE operations.
+__device__ __forceinline__ float fma1(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ float recip(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return fma1(fma1(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float quot(float a, float b, float y) {   // a / b, y = recip(b)
+    const float q = a * y;
+    return fma1(fma1(-b, q, a), y, q);
+}
+// a distance and its reciprocal from its square; coinciding particles (and
+// the particle itself) get a distance of 1e-15 instead of the pair
+// formulas' + 1e-20
+struct Dist { float r, y; };
+__device__ __forceinline__ Dist dist_of(float r2) {
+    const float x = fmaxf(r2, 1e-30f), y = __builtin_amdgcn_rsqf(x), s = x * y;
+    const float r = fma1(fma1(-s, s, x), 0.5f * y, s);
+    return {r, fma1(fma1(-r, y, 1.0f), y, y)};
+}
+// r / h / kappa of pairs that share h
+struct HScale {
+    float h, yh, kap, yk;
+    __device__ HScale(const KConst& k, float h_) : h(h_), yh(recip(h_)), kap((float)k.kappa), yk(recip((float)k.kappa)) {}
+    __device__ float tR(float r) const { return quot(quot(r, h, yh), kap, yk); }
+};
 
 // Cell formulas (float arithmetic, as the reference computes them).
 // Binning: functions_NNPS.cuh:891-900.  Query: e.g. functions_PPE.cuh:52-57.
