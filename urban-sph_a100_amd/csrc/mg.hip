@@ -657,10 +657,14 @@ struct MGLv {
 };
 
 // sum_k (a_rk / d_r) x[col_k] over the compact level-0 operator, in entry
-// order, accumulated in double; four independent loads in flight per lane
+// order, accumulated in double (row_sum)
+struct HTerm { unsigned short h; float x; };
 __device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int r, const float* x,
                                            const int* wb) {
     const unsigned* ev = L.ev;
+    auto mac = [](double s, const HTerm& t) {
+        return s + (double)(float)__builtin_bit_cast(_Float16, t.h) * (double)t.x;
+    };
     const int w = L.hw ? __builtin_amdgcn_readfirstlane(L.hw[r >> 6]) : -1;
     if (w >= 0) {   // a stencil slice: the kept halves only, columns row + offset
         // the slice's first slot and offset, wave-uniform (scalar offset loads)
@@ -670,44 +674,17 @@ __device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int
         const gmem<unsigned short> hp = (gmem<unsigned short>)(L.eh + pslot(hb) + (r & 63));
         const cmem<int> off = (cmem<int>)(L.hoff + hq);
         const gmem<float> xr = (gmem<float>)(x + r);
-        auto hterm = [&](unsigned short u, int o) {
-            return (double)(float)__builtin_bit_cast(_Float16, u) * (double)xr[o];
-        };
-        double s = 0.0;
-        int k = 0;
-        for (; k + 4 <= w; k += 4) {
-            const unsigned short u0 = __builtin_nontemporal_load(hp + pslot(k + 0));
-            const unsigned short u1 = __builtin_nontemporal_load(hp + pslot(k + 1));
-            const unsigned short u2 = __builtin_nontemporal_load(hp + pslot(k + 2));
-            const unsigned short u3 = __builtin_nontemporal_load(hp + pslot(k + 3));
-            s += hterm(u0, off[k + 0]);
-            s += hterm(u1, off[k + 1]);
-            s += hterm(u2, off[k + 2]);
-            s += hterm(u3, off[k + 3]);
-        }
-        for (; k < w; k++) s += hterm(__builtin_nontemporal_load(hp + pslot(k)), off[k]);
-        return s;
+        return row_sum<HTerm, ROW_U>(
+            w, [&](int k) { return HTerm{__builtin_nontemporal_load(hp + pslot(k)), xr[off[k]]}; }, mac);
     }
     const unsigned* p = ev + prow(pp.sl_off, r);
-    const int m = pp.cnt[r];
-    auto term = [&](unsigned u) {
-        const _Float16 h = __builtin_bit_cast(_Float16, (unsigned short)(u >> 16));
-        return (double)(float)h * (double)x[ecol(wb, (int)(u & 0xffffu))];
-    };
-    double s = 0.0;
-    int k = 0;
-    for (; k + 4 <= m; k += 4) {
-        const unsigned u0 = __builtin_nontemporal_load(p + pslot(k + 0));
-        const unsigned u1 = __builtin_nontemporal_load(p + pslot(k + 1));
-        const unsigned u2 = __builtin_nontemporal_load(p + pslot(k + 2));
-        const unsigned u3 = __builtin_nontemporal_load(p + pslot(k + 3));
-        s += term(u0);
-        s += term(u1);
-        s += term(u2);
-        s += term(u3);
-    }
-    for (; k < m; k++) s += term(__builtin_nontemporal_load(p + pslot(k)));
-    return s;
+    return row_sum<HTerm, ROW_U>(
+        pp.cnt[r],
+        [&](int k) {
+            const unsigned u = __builtin_nontemporal_load(p + pslot(k));
+            return HTerm{(unsigned short)(u >> 16), x[ecol(wb, (int)(u & 0xffffu))]};
+        },
+        mac);
 }
 
 // block -> (case, first row of the level); the block returns when the

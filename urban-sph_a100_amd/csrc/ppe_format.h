@@ -26,30 +26,51 @@ __host__ __device__ __forceinline__ long long prow(const long long* sl_off, int 
 __host__ __device__ __forceinline__ long long pslot(int k) { return (long long)k * SLICE; }
 
 // Off-diagonal part of one row, sum_k vals[k] * x[col[k]], accumulated in
-// double in entry order.  Matrix entries stream through once: nontemporal
-// loads keep the caches for the x gathers; four independent loads in flight
-// per lane.
-template <class V, class X>
-__device__ __forceinline__ double offdiag_i32(const int* cp, const V* vp, int m, const X* x) {
+// double in entry order: ld(k) loads entry k's operands, mac(s, operands)
+// adds its term.  Matrix entries stream through once: nontemporal loads keep
+// the caches for the x gathers.  U entries' loads are issued before the
+// first of their terms is added, in the remainder too (entries past the
+// row's end reload the last one and add nothing): a small case has about
+// a wave a SIMD, and its product takes the number of such rounds times the
+// memory latency.  Measured with 4 (and a remainder entry by entry), 8, 16
+// and 24 entries a round, HIP events: float product 29.9, 21.4, 16.9, 16.0 us
+// on 20,609 particles and 137, 132, 131, 143 us on the 2.13 M canyon, whose
+// level-0 passes (half values) take 94, 83, 83, 104 us; double product (FP64,
+// 150 k canyon, bound by its bytes) 36.3, 36.9, 39.9, 43.5 us, 32^3 box 27.0,
+// 26.8, 25.5, 25.0 us.  Giving a row to four waves (an LDS sum) was slower from
+// 200 k particles on and no faster below.
+constexpr int ROW_U = 16;        // float and half values
+constexpr int ROW_U_F64 = 8;
+template <class T, int U, class LD, class MAC>
+__device__ __forceinline__ double row_sum(int m, LD&& ld, MAC&& mac) {
     double s = 0.0;
     int k = 0;
-    for (; k + 4 <= m; k += 4) {
-        const int c0 = __builtin_nontemporal_load(cp + pslot(k + 0));
-        const int c1 = __builtin_nontemporal_load(cp + pslot(k + 1));
-        const int c2 = __builtin_nontemporal_load(cp + pslot(k + 2));
-        const int c3 = __builtin_nontemporal_load(cp + pslot(k + 3));
-        const V v0 = __builtin_nontemporal_load(vp + pslot(k + 0));
-        const V v1 = __builtin_nontemporal_load(vp + pslot(k + 1));
-        const V v2 = __builtin_nontemporal_load(vp + pslot(k + 2));
-        const V v3 = __builtin_nontemporal_load(vp + pslot(k + 3));
-        const X x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
-        s += (double)v0 * (double)x0;
-        s += (double)v1 * (double)x1;
-        s += (double)v2 * (double)x2;
-        s += (double)v3 * (double)x3;
+    for (; k + U <= m; k += U) {
+        T t[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) t[u] = ld(k + u);
+#pragma unroll
+        for (int u = 0; u < U; u++) s = mac(s, t[u]);
     }
-    for (; k < m; k++) s += (double)__builtin_nontemporal_load(vp + pslot(k)) * (double)x[__builtin_nontemporal_load(cp + pslot(k))];
+    if (k < m) {
+        T t[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) t[u] = ld(min(k + u, m - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++) s = k + u < m ? mac(s, t[u]) : s;
+    }
     return s;
+}
+template <class V, class X> struct Term { V v; X x; };
+template <class V> constexpr int row_u() { return sizeof(V) == 8 ? ROW_U_F64 : ROW_U; }
+template <class V, class X>
+__device__ __forceinline__ double offdiag_i32(const int* cp, const V* vp, int m, const X* x) {
+    return row_sum<Term<V, X>, row_u<V>()>(
+        m,
+        [&](int k) {
+            return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)), x[__builtin_nontemporal_load(cp + pslot(k))]};
+        },
+        [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
 // The same over 16-bit columns: entry e = (group << EC_OFF_BITS) | offset,
 // column = wb[group] + offset, wb = the slice's group bases (in LDS).
@@ -57,26 +78,13 @@ __device__ __forceinline__ int ecol(const int* wb, int e) { return wb[e >> EC_OF
 template <class V, class X>
 __device__ __forceinline__ double offdiag_u16(const unsigned short* ep, const V* vp, int m, const int* wb,
                                               const X* x) {
-    double s = 0.0;
-    int k = 0;
-    for (; k + 4 <= m; k += 4) {
-        const int e0 = __builtin_nontemporal_load(ep + pslot(k + 0));
-        const int e1 = __builtin_nontemporal_load(ep + pslot(k + 1));
-        const int e2 = __builtin_nontemporal_load(ep + pslot(k + 2));
-        const int e3 = __builtin_nontemporal_load(ep + pslot(k + 3));
-        const V v0 = __builtin_nontemporal_load(vp + pslot(k + 0));
-        const V v1 = __builtin_nontemporal_load(vp + pslot(k + 1));
-        const V v2 = __builtin_nontemporal_load(vp + pslot(k + 2));
-        const V v3 = __builtin_nontemporal_load(vp + pslot(k + 3));
-        const X x0 = x[ecol(wb, e0)], x1 = x[ecol(wb, e1)], x2 = x[ecol(wb, e2)], x3 = x[ecol(wb, e3)];
-        s += (double)v0 * (double)x0;
-        s += (double)v1 * (double)x1;
-        s += (double)v2 * (double)x2;
-        s += (double)v3 * (double)x3;
-    }
-    for (; k < m; k++)
-        s += (double)__builtin_nontemporal_load(vp + pslot(k)) * (double)x[ecol(wb, __builtin_nontemporal_load(ep + pslot(k)))];
-    return s;
+    return row_sum<Term<V, X>, row_u<V>()>(
+        m,
+        [&](int k) {
+            return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)),
+                              x[ecol(wb, __builtin_nontemporal_load(ep + pslot(k)))]};
+        },
+        [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
 
 // The same over a stencil slice: column row + off[k], off the slice's
@@ -92,22 +100,9 @@ __device__ __forceinline__ double offdiag_stencil(const V* vals, int m, const in
     const gmem<V> vp = (gmem<V>)vals;
     const gmem<X> x = (gmem<X>)(xv + r);
     const cmem<int> off = (cmem<int>)offs;
-    double s = 0.0;
-    int k = 0;
-    for (; k + 4 <= m; k += 4) {
-        const int o0 = off[k + 0], o1 = off[k + 1], o2 = off[k + 2], o3 = off[k + 3];
-        const V v0 = __builtin_nontemporal_load(vp + pslot(k + 0));
-        const V v1 = __builtin_nontemporal_load(vp + pslot(k + 1));
-        const V v2 = __builtin_nontemporal_load(vp + pslot(k + 2));
-        const V v3 = __builtin_nontemporal_load(vp + pslot(k + 3));
-        const X x0 = x[o0], x1 = x[o1], x2 = x[o2], x3 = x[o3];
-        s += (double)v0 * (double)x0;
-        s += (double)v1 * (double)x1;
-        s += (double)v2 * (double)x2;
-        s += (double)v3 * (double)x3;
-    }
-    for (; k < m; k++) s += (double)__builtin_nontemporal_load(vp + pslot(k)) * (double)x[off[k]];
-    return s;
+    return row_sum<Term<V, X>, row_u<V>()>(
+        m, [&](int k) { return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)), x[off[k]]}; },
+        [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
 // Row r's slice: the first of its stencil offsets in pp.poff, or -1.  Every
 // active lane of the calling wave holds a row of the same slice (rows are
