@@ -54,14 +54,20 @@ void dfree(sph_ctx* c, void* p) {
     c->cache.emplace(it->second, p);
     c->live.erase(it);
 }
-// Returns the cached blocks to HIP (hipFree waits for the device first).
-void dcache_release(sph_ctx* c) {
-    for (auto& b : c->cache) {
-        (void)hipFree(b.second);
-        c->bytes -= (long long)b.first;
+// Returns cached blocks to HIP, the largest first, until the cache holds at
+// most `keep` bytes (hipFree waits for the device first).
+void dcache_trim(sph_ctx* c, size_t keep) {
+    size_t held = 0;
+    for (auto& b : c->cache) held += b.first;
+    while (held > keep) {
+        auto it = std::prev(c->cache.end());
+        (void)hipFree(it->second);
+        c->bytes -= (long long)it->first;
+        held -= it->first;
+        c->cache.erase(it);
     }
-    c->cache.clear();
 }
+void dcache_release(sph_ctx* c) { dcache_trim(c, 0); }
 
 // AoS (reference layout) -> SoA (same order)
 __global__ void __launch_bounds__(BLOCK) k_unpack(int n, const sph_part1* A, const sph_part2* B, const float* nrm,

@@ -587,6 +587,7 @@ int dmalloc(sph_ctx* c, void** p, size_t bytes);
 template <class T>
 int dalloc(sph_ctx* c, T** p, size_t count) { return dmalloc(c, (void**)p, count * sizeof(T)); }
 void dfree(sph_ctx* c, void* p);
+void dcache_trim(sph_ctx* c, size_t keep);
 void dcache_release(sph_ctx* c);
 
 // profiling around launches (the profile of the driving engine)
