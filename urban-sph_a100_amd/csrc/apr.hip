@@ -19,6 +19,8 @@
 // (apr_cond) in its particle record, but both are commented out of the
 // compiled record (class_Cuda_Particle_Array.cuh:37-43); here the target
 // level is a per-particle array of the context, inherited by the children.
+#include <climits>
+
 #include "flags.h"
 #include "sph_internal.h"
 #include "sph_math.h"
@@ -40,29 +42,36 @@ __device__ __forceinline__ double apr_cbrt(double v) {
     return ldexp(y, e / 3);
 }
 
-__global__ void __launch_bounds__(BLOCK) k_apr_pick(int ncells, const int* gstr, const int* gend, PView P,
-                                                    const double* target, int* flag, int* pick) {
+// The first particle of each cell (in cell order) that wants to split: a
+// thread per particle, the lowest index of a cell kept (a refined cell holds
+// hundreds of particles, which a thread per cell walked one by one: 205 us a pass of
+// the 226 k refined canyon).
+__global__ void __launch_bounds__(BLOCK) k_apr_first(int ncells, int* pick) {
+    const int cell = blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell < ncells) pick[cell] = INT_MAX;
+}
+__global__ void __launch_bounds__(BLOCK) k_apr_want(int n, int ncells, const int* keys, PView P, const double* target,
+                                                    int* pick) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const int cell = keys[j];
+    if (cell < 0 || cell >= ncells) return;   // a dummy
+    const double level = log(P.m_ref[j] / P.m[j]) / log(8.0);
+    if (target[j] - level >= 0.75) atomicMin(&pick[cell], j);
+}
+// the split loop passes over a non-fluid particle whose target exceeds 2, and
+// the condition marked only the cell's first one (functions_APR.cuh:423)
+__global__ void __launch_bounds__(BLOCK) k_apr_pick(int ncells, PView P, const double* target, const int* pick,
+                                                    int* flag) {
     const int cell = blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= ncells) return;
-    flag[cell] = 0;
-    pick[cell] = -1;
-    const int s = gstr[cell];
-    if (s == -1) return;
-    const int e = gend[cell];
-    const double l8 = log(8.0);
-    for (int j = s; j < e; j++) {
-        const double level = log(P.m_ref[j] / P.m[j]) / l8;
-        if (target[j] - level >= 0.75) {
-            // the split loop passes over a non-fluid particle whose target
-            // exceeds 2, and the condition marked only this one
-            // (functions_APR.cuh:423)
-            if (!(P.p_type[j] != 1 && target[j] > 2.0)) {
-                flag[cell] = 1;
-                pick[cell] = j;
-            }
-            return;
-        }
-    }
+    const int j = pick[cell];
+    flag[cell] = j != INT_MAX && !(P.p_type[j] != 1 && target[j] > 2.0) ? 1 : 0;
+}
+__global__ void __launch_bounds__(BLOCK) k_apr_list(int ncells, const int* flag, const int* rank, const int* pick,
+                                                    int* list) {
+    const int cell = blockIdx.x * blockDim.x + threadIdx.x;
+    if (cell < ncells && flag[cell]) list[rank[cell]] = pick[cell];
 }
 
 constexpr int APR_MAX_F64 = 64;
@@ -73,31 +82,32 @@ struct AprFields {
     double *x, *y, *z, *m, *vol, *h, *rho;
 };
 
-__global__ void __launch_bounds__(BLOCK) k_apr_split(int ncells, const int* flag, const int* rank, const int* pick,
-                                                     int n0, AprFields F, int h_change) {
-    const int cell = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= ncells || !flag[cell]) return;
-    const int j = pick[cell];
-    const int base = n0 + 8 * rank[cell];
+// A thread per child (the children of consecutive splits are consecutive, so
+// every field is written in whole lines).
+__global__ void __launch_bounds__(BLOCK) k_apr_split(int nsplit, const int* list, int n0, AprFields F, int h_change) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, k = t & 7;
+    if (t >= 8 * nsplit) return;
+    const int j = list[t >> 3], c = n0 + t;
     const double xm = F.x[j], ym = F.y[j], zm = F.z[j];
     const double a = 0.25 * apr_cbrt(F.m[j] / F.rho[j]);
-    for (int k = 0; k < 8; k++) {
-        const int c = base + k;
-        for (int f = 0; f < F.nf; f++) F.f[f][c] = F.f[f][j];
-        for (int f = 0; f < SPH_I_COUNT; f++) F.iv[f][c] = F.iv[f][j];
-        // child order of functions_APR.cuh:440-478: x +,+,+,+,-,-,-,-;
-        // y +,+,-,-,+,+,-,-; z +,-,+,-,+,-,+,-.  The reference stores the
-        // children's positions in its float records (functions_APR.cuh:
-        // 544-590): rounded to float here too, so a refined case's positions
-        // stay float values
-        F.x[c] = (double)(float)(k < 4 ? xm + a : xm - a);
-        F.y[c] = (double)(float)((k & 2) ? ym - a : ym + a);
-        F.z[c] = (double)(float)((k & 1) ? zm - a : zm + a);
-        F.m[c] = 0.125 * F.m[j];
-        F.vol[c] = 0.125 * F.vol[j];
-        if (h_change) F.h[c] = 0.5 * F.h[j];
-    }
-    F.iv[SPH_I_I_TYPE][j] = 3;
+    for (int f = 0; f < F.nf; f++) F.f[f][c] = F.f[f][j];
+    for (int f = 0; f < SPH_I_COUNT; f++) F.iv[f][c] = F.iv[f][j];
+    // child order of functions_APR.cuh:440-478: x +,+,+,+,-,-,-,-;
+    // y +,+,-,-,+,+,-,-; z +,-,+,-,+,-,+,-.  The reference stores the
+    // children's positions in its float records (functions_APR.cuh:
+    // 544-590): rounded to float here too, so a refined case's positions
+    // stay float values
+    F.x[c] = (double)(float)(k < 4 ? xm + a : xm - a);
+    F.y[c] = (double)(float)((k & 2) ? ym - a : ym + a);
+    F.z[c] = (double)(float)((k & 1) ? zm - a : zm + a);
+    F.m[c] = 0.125 * F.m[j];
+    F.vol[c] = 0.125 * F.vol[j];
+    if (h_change) F.h[c] = 0.5 * F.h[j];
+}
+// the parents become dummies once their children hold their fields
+__global__ void __launch_bounds__(BLOCK) k_apr_parents(int nsplit, const int* list, int* i_type) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nsplit) i_type[list[t]] = 3;
 }
 
 int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
@@ -108,15 +118,19 @@ int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
     }
     if (target)
         SPH_HIP(c, hipMemcpyAsync(c->apr_target, target, sizeof(double) * (size_t)c->n, hipMemcpyHostToDevice, c->stream));
-    int *flag = nullptr, *rank = nullptr, *pick = nullptr;
+    int *flag = nullptr, *rank = nullptr, *pick = nullptr, *list = nullptr;
+    SPH_TRY(dalloc(c, &list, ncells));
     SPH_TRY(dalloc(c, &flag, ncells));
     SPH_TRY(dalloc(c, &rank, ncells));
     SPH_TRY(dalloc(c, &pick, ncells));
     int rc = 0;
     bool split_any = false;
     for (int pass = 0; pass < max_passes && rc == 0; pass++) {
-        hipLaunchKernelGGL(k_apr_pick, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, (const int*)c->gstr,
-                           (const int*)c->gend, c->pview(), (const double*)c->apr_target, flag, pick);
+        hipLaunchKernelGGL(k_apr_first, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, pick);
+        hipLaunchKernelGGL(k_apr_want, dim3(grid1(c->n)), dim3(BLOCK), 0, c->stream, c->n, ncells, (const int*)c->keys,
+                           c->pview(), (const double*)c->apr_target, pick);
+        hipLaunchKernelGGL(k_apr_pick, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, c->pview(),
+                           (const double*)c->apr_target, (const int*)pick, flag);
         if ((rc = launch_check(c, "apr_pick"))) break;
         int nsplit = 0;
         if ((rc = exclusive_scan_i32(c, flag, rank, ncells, &nsplit))) break;
@@ -135,8 +149,12 @@ int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
         for (int f = 0; f < SPH_I_COUNT; f++) F.iv[f] = c->pi[f];
         F.x = c->pf[SPH_F_X]; F.y = c->pf[SPH_F_Y]; F.z = c->pf[SPH_F_Z]; F.m = c->pf[SPH_F_M];
         F.vol = c->pf[SPH_F_VOL]; F.h = c->pf[SPH_F_H]; F.rho = c->pf[SPH_F_RHO];
-        hipLaunchKernelGGL(k_apr_split, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, (const int*)flag,
-                           (const int*)rank, (const int*)pick, c->n, F, c->prm.apr_h_change);
+        hipLaunchKernelGGL(k_apr_list, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, (const int*)flag,
+                           (const int*)rank, (const int*)pick, list);
+        hipLaunchKernelGGL(k_apr_split, dim3(grid1(8LL * nsplit)), dim3(BLOCK), 0, c->stream, nsplit, (const int*)list,
+                           c->n, F, c->prm.apr_h_change);
+        hipLaunchKernelGGL(k_apr_parents, dim3(grid1(nsplit)), dim3(BLOCK), 0, c->stream, nsplit, (const int*)list,
+                           c->pi[SPH_I_I_TYPE]);
         if ((rc = launch_check(c, "apr_split"))) break;
         c->n += 8 * nsplit;   // the children's positions are float values like their parents'
         dfree(c, c->porder);   // the pass order covers the old count; the next list rebuilds it
@@ -148,10 +166,14 @@ int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
         rc = nnps_run(c, false);
         split_any = true;
     }
-    if (rc == 0 && split_any) rc = nnps_list(c);
+    if (split_any) {   // also after a failed pass: the lists match the particles there are
+        const int lrc = nnps_list(c);
+        if (rc == 0) rc = lrc;
+    }
     dfree(c, flag);
     dfree(c, rank);
     dfree(c, pick);
+    dfree(c, list);
     if (n_out) *n_out = c->n;
     return rc;
 }
