@@ -265,7 +265,9 @@ __global__ void __launch_bounds__(BLOCK) k_mg_link(int n, const int* key, const 
     if (t == n - 1) mstart[I + 1] = n;
 }
 
-// One coarse row per 64-thread block (one wave): its terms are the
+// One coarse row per block (one wave; the rows of more than MG_ENT_CAP terms
+// 1024 threads: one wave sorted 8192 keys in 4-6 ms while the device waited):
+// its terms are the
 // members' diagonals and entries mapped to aggregates, numbered in order
 // (members ascending, each member's diagonal first, then its entries in
 // storage order).  A bitonic sort in LDS of 32-bit keys (column - the row's
@@ -280,8 +282,9 @@ __global__ void __launch_bounds__(BLOCK) k_mg_link(int n, const int* key, const 
 // its run of sorted positions and sums each of them to its end.  err:
 // SPH_MG_TERMS (too many terms or members), SPH_MG_SPAN (columns too far
 // apart).
+template <int CAP> constexpr int rap_threads() { return CAP > MG_ENT_CAP ? 1024 : SLICE; }
 template <class OP, int CAP>
-__global__ void __launch_bounds__(SLICE) k_mg_rap(OP op, int n1, const int* agg, const int* mstart, const int* mem,
+__global__ void __launch_bounds__(rap_threads<CAP>()) k_mg_rap(OP op, int n1, const int* agg, const int* mstart, const int* mem,
                                                   const int* redo, int* cnt1, const long long* row_off, int* cols1,
                                                   float* vals1, float* diag1, int* err) {
     constexpr bool BIG = CAP > MG_ENT_CAP;
@@ -290,13 +293,15 @@ __global__ void __launch_bounds__(SLICE) k_mg_rap(OP op, int n1, const int* agg,
     __shared__ unsigned sk[CAP];                    // (column - jmin) << TB | term number
     __shared__ float sv[BIG ? 1 : CAP];             // term values by term number
     __shared__ int moff[BIG ? MG_BIG_MEMBERS + 1 : 1];   // first term of each member
+    constexpr int T = rap_threads<CAP>();
+    __shared__ int red[T / SLICE][2];
     const int I = blockIdx.x;
     const int lane = threadIdx.x;
     if (I >= n1 || !redo[I]) return;
     const int t0 = mstart[I], t1 = mstart[I + 1];
     int nterm = 0;
-    for (int t = t0 + lane; t < t1; t += SLICE) nterm += op.cnt(mem[t]) + 1;
-    nterm = wave_sum(nterm);
+    for (int t = t0 + (lane & 63); t < t1; t += SLICE) nterm += op.cnt(mem[t]) + 1;
+    nterm = wave_sum(nterm);   // (every wave forms it)
     if (BIG ? nterm <= MG_ENT_CAP : nterm > MG_ENT_CAP) return;   // the other kernel's row
     if (nterm > CAP || (BIG && t1 - t0 > MG_BIG_MEMBERS)) {
         if (lane == 0) err[0] = SPH_MG_TERMS;
@@ -309,7 +314,7 @@ __global__ void __launch_bounds__(SLICE) k_mg_rap(OP op, int n1, const int* agg,
         const int m = mem[t];
         const int c = op.cnt(m);
         if (BIG && lane == 0) moff[t - t0] = pos;
-        for (int k = lane - 1; k < c; k += SLICE) {
+        for (int k = lane - 1; k < c; k += T) {
             const int q = pos + k + 1;
             const float v = k < 0 ? op.dg(m) : -op.val(m, k);
             // a stored zero (a stencil slot the row lacks) joins the
@@ -325,17 +330,22 @@ __global__ void __launch_bounds__(SLICE) k_mg_rap(OP op, int n1, const int* agg,
     if (BIG && lane == 0) moff[t1 - t0] = pos;
     jmin = -wave_max(-jmin);
     jmax = wave_max(jmax);
+    if constexpr (T > SLICE) {
+        if ((lane & 63) == 0) { red[lane >> 6][0] = jmin; red[lane >> 6][1] = jmax; }
+        __syncthreads();
+        for (int w = 0; w < T / SLICE; w++) { jmin = min(jmin, red[w][0]); jmax = max(jmax, red[w][1]); }
+    }
     if (jmax - jmin >= (1 << (32 - TB)) - 1) {
         if (lane == 0) err[0] = SPH_MG_SPAN;
         return;
     }
     __syncthreads();
-    for (int p = lane; p < np2; p += SLICE)
+    for (int p = lane; p < np2; p += T)
         sk[p] = p < nterm ? ((sk[p] - (unsigned)jmin) << TB) | (unsigned)p : 0xffffffffu;
     __syncthreads();
     for (int k = 2; k <= np2; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = lane; i < np2; i += SLICE) {
+            for (int i = lane; i < np2; i += T) {
                 const int ixj = i ^ j;
                 if (ixj > i) {
                     const unsigned a = sk[i], b = sk[ixj];
@@ -350,14 +360,23 @@ __global__ void __launch_bounds__(SLICE) k_mg_rap(OP op, int n1, const int* agg,
     // those below the diagonal's column (the diagonal's slot)
     auto col_at = [&](int p) { return (int)(sk[p] >> TB) + jmin; };
     auto starts = [&](int p) { return p == 0 || col_at(p) != col_at(p - 1); };
-    const int per = (nterm + SLICE - 1) / SLICE;
+    const int per = (nterm + T - 1) / T;
     const int p0 = min(nterm, lane * per), p1 = min(nterm, p0 + per);
     int own = 0, below = 0;
     for (int p = p0; p < p1; p++)
         if (starts(p)) { own++; below += col_at(p) < I ? 1 : 0; }
-    const int at = wave_excl(own);
-    const int total = wave_sum(own);
-    const int sI = wave_sum(below);
+    int at = wave_excl(own), total = wave_sum(own), sI = wave_sum(below);
+    if constexpr (T > SLICE) {   // across the waves, in order
+        __syncthreads();
+        if ((lane & 63) == 0) { red[lane >> 6][0] = total; red[lane >> 6][1] = sI; }
+        __syncthreads();
+        total = sI = 0;
+        for (int w = 0; w < T / SLICE; w++) {
+            if (w < (lane >> 6)) at += red[w][0];
+            total += red[w][0];
+            sI += red[w][1];
+        }
+    }
     if (lane == 0) cnt1[I] = total - 1;
     // a term's value: from LDS, or (large rows) from its member's entry
     auto term_val = [&](int q) -> float {
@@ -496,15 +515,28 @@ __global__ void __launch_bounds__(SLICE) k_mg_rap_hash(OP op, int n1, const int*
         }
     }
 }
-// largest |entry| of an operator (the diagonal included), as float bits
+// largest |entry| of an operator (the diagonal included), as float bits;
+// GROUP lanes a row (a long row would hold its wave) and at most
+// MAXABS_BLOCKS blocks, one atomic each: an atomic a wave, all on one word,
+// took 1.2 ms for 1 M rows
+constexpr int MAXABS_BLOCKS = 2048;
 template <class OP>
 __global__ void __launch_bounds__(BLOCK) k_mg_maxabs(OP op, int n, unsigned* out) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    float m = fabsf(op.dg(r));
-    const int c = op.cnt(r);
-    for (int k = 0; k < c; k++) m = fmaxf(m, fabsf(op.val(r, k)));
-    if (m == m) atomicMax(out, __float_as_uint(m));
+    __shared__ float red[BLOCK / SLICE];
+    const int g = threadIdx.x % GROUP;
+    float m = 0.0f;
+    for (int r = blockIdx.x * (BLOCK / GROUP) + threadIdx.x / GROUP; r < n; r += gridDim.x * (BLOCK / GROUP)) {
+        m = fmaxf(m, fabsf(op.dg(r)));
+        const int c = op.cnt(r);
+        for (int k = g; k < c; k += GROUP) m = fmaxf(m, fabsf(op.val(r, k)));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int w = 1; w < BLOCK / SLICE; w++) m = fmaxf(m, red[w]);
+    if (m > 0.0f) atomicMax(out, __float_as_uint(m));
 }
 
 // room for each coarse row's columns: its terms (members' entries + 1)
@@ -1001,7 +1033,7 @@ static int mg_galerkin(sph_ctx* c, const OP& src, MGLevel& L1, const MGLevel& L0
     SPH_TRY(tmp.get(&redo, n1));
     SPH_TRY(tmp.get(&aux, 2));
     SPH_HIP(c, hipMemsetAsync(aux, 0, 2 * sizeof(int), c->stream));
-    MGK("mg_rap_scale", grid1(L0.n), BLOCK, k_mg_maxabs<OP>, src, L0.n, (unsigned*)aux);
+    MGK("mg_rap_scale", min(grid1((long long)L0.n * GROUP), MAXABS_BLOCKS), BLOCK, k_mg_maxabs<OP>, src, L0.n, (unsigned*)aux);
     int h_aux[2] = {0, 0};
     SPH_HIP(c, hipMemcpyAsync(h_aux, aux, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     SPH_HIP(c, hipStreamSynchronize(c->stream));
@@ -1017,7 +1049,7 @@ static int mg_galerkin(sph_ctx* c, const OP& src, MGLevel& L1, const MGLevel& L0
     if (h_aux[1] > 0) {
         MGK("mg_rap_sort", n1, SLICE, (k_mg_rap<OP, MG_ENT_CAP>), src, n1, (const int*)L0.agg, (const int*)L0.mstart,
             (const int*)L0.mem, (const int*)redo, L1.cnt, (const long long*)row_off, pc, pv, L1.diag, err);
-        MGK("mg_rap_sort", n1, SLICE, (k_mg_rap<OP, MG_BIG_CAP>), src, n1, (const int*)L0.agg, (const int*)L0.mstart,
+        MGK("mg_rap_sort", n1, (rap_threads<MG_BIG_CAP>()), (k_mg_rap<OP, MG_BIG_CAP>), src, n1, (const int*)L0.agg, (const int*)L0.mstart,
             (const int*)L0.mem, (const int*)redo, L1.cnt, (const long long*)row_off, pc, pv, L1.diag, err);
     }
     int h_err = 0;

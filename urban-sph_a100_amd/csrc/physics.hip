@@ -1726,37 +1726,8 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_wave(Seg sg) {
 }
 
 // IBM_spreading_interpolation3D, functions_IBM.cuh:492-613
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_ibm_spread(Seg sg) {
-    SEG_PARTICLE(sg);
-    const KConst kc = cd.kc;
-    const PView S = cd.S;
-    const NList nl = cd.nl;
-    if (S.p_type[i] != 1) return;
-    if (S.buffer_type[i] == 2) return;
-    if (cd.ibm_near && !cd.ibm_near[i]) {   // no marker in the list: what the sums below give
-        S.fbx[i] = 0.0; S.fby[i] = 0.0; S.fbz[i] = 0.0; S.concentration[i] = 0.0;
-        return;
-    }
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    R tmp_h = (R)(0.5 * S.h[i]);
-    R tmp_A = calc_tmpA<R>(kc, tmp_h);
-    double filt = 0, fb_x = 0, fb_y = 0, fb_z = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_BH)) continue;
-        int j = e & NB_IDX;
-        if (S.i_type[j] == 4 || S.p_type[j] != 1000) continue;
-        R dx = (R)(xi - S.x[j]), dy = (R)(yi - S.y[j]), dz = (R)(zi - S.z[j]);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) + (R)1e-20;
-        R twij = kernel_w<R>(kc, tmp_A, tmp_h, tdist);
-        R tmprho = (R)S.m[j] / (R)S.rho[j];
-        fb_x += (double)((R)S.fbx[j] * twij * tmprho);
-        fb_y += (double)((R)S.fby[j] * twij * tmprho);
-        fb_z += (double)((R)S.fbz[j] * twij * tmprho);
-        filt += (double)(tmprho * twij);
-    }
+__device__ __forceinline__ void ibm_spread_store(const PView& S, int i, double fb_x, double fb_y, double fb_z,
+                                                 double filt) {
     if (filt < 1e-12) {
         S.fbx[i] = 0.0; S.fby[i] = 0.0; S.fbz[i] = 0.0; S.concentration[i] = 0.0;
         return;
@@ -1765,6 +1736,71 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_ibm_spread(Seg sg) {
     S.fby[i] = fb_y / (filt + 1e-10);
     S.fbz[i] = fb_z / (filt + 1e-10);
     S.concentration[i] = filt;
+}
+__global__ void __launch_bounds__(MAX_BLOCK) k_ibm_spread(Seg sg) {
+    SEG_PARTICLE(sg);
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    const NList nl = cd.nl;
+    if (S.p_type[i] != 1) return;
+    if (S.buffer_type[i] == 2) return;
+    if (cd.ibm_near && !cd.ibm_near[i]) {   // no marker in the list: what the sums below give
+        ibm_spread_store(S, i, 0.0, 0.0, 0.0, 0.0);
+        return;
+    }
+    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    double tmp_h = 0.5 * S.h[i];
+    double tmp_A = calc_tmpA<double>(kc, tmp_h);
+    double filt = 0, fb_x = 0, fb_y = 0, fb_z = 0;
+    NLRow row = nl_row(nl, i);
+    for (int k = 0; k < row.cnt; k++) {
+        unsigned e = NB_AT(row, k);
+        if (!(e & F_BH)) continue;
+        int j = e & NB_IDX;
+        if (S.i_type[j] == 4 || S.p_type[j] != 1000) continue;
+        double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+        double twij = kernel_w<double>(kc, tmp_A, tmp_h, tdist);
+        double tmprho = S.m[j] / S.rho[j];
+        fb_x += S.fbx[j] * twij * tmprho;
+        fb_y += S.fby[j] * twij * tmprho;
+        fb_z += S.fbz[j] * twij * tmprho;
+        filt += tmprho * twij;
+    }
+    ibm_spread_store(S, i, fb_x, fb_y, fb_z, filt);
+}
+// MIXED: GROUP lanes a particle, the pair arithmetic in float, the sums in
+// double
+__global__ void __launch_bounds__(MAX_BLOCK) k_ibm_spread_mixed(Seg sg) {
+    SEG_GROUP(sg);
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    if (S.p_type[i] != 1) return;
+    if (S.buffer_type[i] == 2) return;
+    if (cd.ibm_near && !cd.ibm_near[i]) {   // no marker in the list: what the sums below give
+        if (g_ == 0) ibm_spread_store(S, i, 0.0, 0.0, 0.0, 0.0);
+        return;
+    }
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const float tmp_h = (float)(0.5 * S.h[i]), tmp_A = calc_tmpA<float>(kc, tmp_h);
+    const HScale hs(kc, tmp_h);
+    double filt = 0, fb_x = 0, fb_y = 0, fb_z = 0;
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = g_; k < row.cnt; k += GROUP) {
+        const unsigned e = NB_AT(row, k);
+        if (!(e & F_BH)) continue;
+        const int j = e & NB_IDX;
+        if (S.i_type[j] == 4 || S.p_type[j] != 1000) continue;
+        const float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
+        const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
+        const float tmprho = (float)S.m[j] / (float)S.rho[j];
+        fb_x += (double)((float)S.fbx[j] * w * tmprho);
+        fb_y += (double)((float)S.fby[j] * w * tmprho);
+        fb_z += (double)((float)S.fbz[j] * w * tmprho);
+        filt += (double)(tmprho * w);
+    }
+    group_fold<GROUP>(fb_x); group_fold<GROUP>(fb_y); group_fold<GROUP>(fb_z); group_fold<GROUP>(filt);
+    if (g_ == 0) ibm_spread_store(S, i, fb_x, fb_y, fb_z, filt);
 }
 
 // ------------------------------------------------------------------------
@@ -1946,22 +1982,25 @@ static bool mixed_of(const Eng& e) { return e.cs[0]->prm.precision == SPH_MIXED;
 // 1 for a particle whose spreading list (the F_BH entries) holds an IB
 // marker (p_type 1000): a superset of the particles the spreading sums
 // reach, whatever the types of i and the markers' i_type become in the step
+// (GROUP lanes a particle)
 __global__ void __launch_bounds__(BLOCK) k_ibm_near(int n, PView S, NList nl, unsigned char* out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / GROUP, g = t % GROUP;
     if (i >= n) return;
-    unsigned char hit = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt && !hit; k++) {
-        const unsigned e = NB_AT(row, k);
-        if (e & F_BH) hit = S.p_type[e & NB_IDX] == 1000;
+    const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);
+    bool hit = false;
+    const NLRow row = nl_row(nl, i);
+    for (int k0 = 0; k0 < row.cnt && !hit; k0 += GROUP) {
+        const unsigned e = k0 + g < row.cnt ? NB_AT(row, k0 + g) : 0u;
+        const bool h = (e & F_BH) && S.p_type[e & NB_IDX] == 1000;
+        hit = ((__ballot(h) >> gbit) & ((1u << GROUP) - 1u)) != 0;   // the group agrees
     }
-    out[i] = hit;
+    if (g == 0) out[i] = hit ? 1 : 0;
 }
 int ibm_near_build(sph_ctx* c) {
     if (c->ibm_near_gen == c->generation && c->ibm_near) return 0;
     if (!c->ibm_near) SPH_TRY(dalloc(c, &c->ibm_near, (size_t)c->cap));
     if (c->n > 0) {
-        hipLaunchKernelGGL(k_ibm_near, dim3(grid1(c->n)), dim3(BLOCK), 0, c->stream, c->n, c->sview(), c->nlist(),
+        hipLaunchKernelGGL(k_ibm_near, dim3(grid1((long long)c->n * GROUP)), dim3(BLOCK), 0, c->stream, c->n, c->sview(), c->nlist(),
                            c->ibm_near);
         SPH_TRY(launch_check(c, "ibm_near"));
     }
@@ -2238,8 +2277,8 @@ int step_physics_back(Eng& e) {
     else SEGL("pressure_force", TK_PRESSURE, k_pressure_force);
     if (mixed) WAVEL("ibm_force", k_ibm_force_wave);
     else SEGL("ibm_force", TK_IBM_FORCE, k_ibm_force<double>);
-    if (mixed) SEGL("ibm_spread", TK_IBM_SPREAD, k_ibm_spread<float>);
-    else SEGL("ibm_spread", TK_IBM_SPREAD, k_ibm_spread<double>);
+    if (mixed) SEGG("ibm_spread", TK_IBM_SPREAD, k_ibm_spread_mixed);
+    else SEGL("ibm_spread", TK_IBM_SPREAD, k_ibm_spread);
     SEGL("time_update", -1, k_time_update);
     SPH_TRY(run_neumann(e, 1, 0));
     SPH_TRY(run_outlet(e, 1));

@@ -193,32 +193,37 @@ __global__ void __launch_bounds__(BLOCK) k_ppe_rows(int n, const int* flag, cons
     if (flag[i]) { rowof[i] = scan[i]; rows[scan[i]] = i; }
     else rowof[i] = -1;
 }
+// Columns of each row in list order, GROUP lanes a row: a round of GROUP list
+// entries is compacted by a ballot over the group, so the slots are those a
+// serial walk gives.  A thread a row left a wave waiting on its longest row
+// (up to 5000 entries beside refined particles): count and fill 3.5 and 4.7 ms
+// on the 226 k refined canyon.
 template <bool FILL>
 __global__ void __launch_bounds__(BLOCK) k_ppe_struct(int nr, const int* rows, const int* rowof, PView S, NList nl,
                                                       int* cnt, const long long* sl_off, int* cols, const int* ltail,
                                                       const long long* tail_off, int* tail_cols) {
-    int r = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, r = t / GROUP, g = t % GROUP;
     if (r >= nr) return;
-    int i = rows[r];
+    const int i = rows[r];
     const unsigned* row = nl.ent + nl.slice_off[i >> 6] + (i & 63);
-    int m = nl.cnt[i];
+    const int m = nl.cnt[i];
+    const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);   // the group's first lane
     int slot = 0;
     int* out = FILL ? cols + prow(sl_off, r) : nullptr;
-    for (int k = 0; k < m; k++) {
-        unsigned e = row[(size_t)k * SLICE];
-        if (!(e & F_DP)) continue;
-        int j = e & NB_IDX;
-        if (S.p_type[j] >= 1000 || S.i_type[j] == 4) continue;
-        if (j == i) continue;
-        int rj = rowof[j];
-        if (rj < 0) continue;
-        if (FILL) {
-            if (slot < LONG_ROW || !ltail) out[pslot(slot)] = rj;
-            else tail_cols[tail_off[ltail[r]] + (slot - LONG_ROW)] = rj;
+    for (int k0 = 0; k0 < m; k0 += GROUP) {
+        const unsigned e = k0 + g < m ? row[(size_t)(k0 + g) * SLICE] : 0u;
+        const int j = e & NB_IDX;
+        int rj = -1;
+        if ((e & F_DP) && j != i && S.p_type[j] < 1000 && S.i_type[j] != 4) rj = rowof[j];
+        const unsigned hit = (unsigned)(__ballot(rj >= 0) >> gbit) & ((1u << GROUP) - 1u);
+        if (FILL && rj >= 0) {
+            const int s = slot + __popc(hit & ((1u << g) - 1u));
+            if (s < LONG_ROW || !ltail) out[pslot(s)] = rj;
+            else tail_cols[tail_off[ltail[r]] + (s - LONG_ROW)] = rj;
         }
-        slot++;
+        slot += __popc(hit);
     }
-    if (!FILL) cnt[r] = slot;
+    if (!FILL && g == 0) cnt[r] = slot;
 }
 __global__ void __launch_bounds__(BLOCK) k_row_slice_width(int nr, int nslices, const int* cnt, long long* w) {
     int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -295,7 +300,7 @@ __global__ void __launch_bounds__(BLOCK) k_rowof_from_rows(int nr, const int* ro
 // Columns of each row in ascending (lattice) order, and the slot each entry
 // takes, indexed by its position in the neighbour list (the order in which
 // the assembly visits it).  The fill pass has written every row's columns in
-// list order, a thread per row; this pass sorts them in place, one workgroup
+// list order; this pass sorts them in place, one workgroup
 // per 64-row slice.  The slice's columns are read slot by slot (whole lines)
 // into LDS; then one wave per row sorts the row's (column, position) keys,
 // held in registers, by a bitonic network over 64, 128 or 256 keys (the keys
@@ -1350,7 +1355,7 @@ static int lattice_order(sph_ctx* c, PPEState* P, bool* used) {
 static int ppe_count_and_slices(sph_ctx* c, PPEState* P, bool tails) {
     const int nr = P->nr;
     SPH_TRY(prof_begin(c, "ppe_count", 0));
-    hipLaunchKernelGGL(k_ppe_struct<false>, dim3(grid1(nr)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
+    hipLaunchKernelGGL(k_ppe_struct<false>, dim3(grid1((long long)nr * GROUP)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
                        (const int*)P->rowof, c->sview(), c->nlist(), P->cnt, (const long long*)nullptr, (int*)nullptr,
                        (const int*)nullptr, (const long long*)nullptr, (int*)nullptr);
     SPH_TRY(launch_check(c, "ppe_count"));
@@ -1596,9 +1601,9 @@ static int ppe_build_ordered(sph_ctx* c, bool allow_lattice) {
         SPH_TRY(dalloc(c, &P->slotmap, P->nnz_slots + 1));
         SPH_TRY(dalloc(c, &ovf, 1));
         hipLaunchKernelGGL(k_zero<int>, dim3(1), dim3(BLOCK), 0, c->stream, 1LL, ovf);
-        // the columns in list order, a thread per row, then sorted in place
+        // the columns in list order, then sorted in place
         SPH_TRY(prof_begin(c, "ppe_cols", 0));
-        hipLaunchKernelGGL(k_ppe_struct<true>, dim3(grid1(nr)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
+        hipLaunchKernelGGL(k_ppe_struct<true>, dim3(grid1((long long)nr * GROUP)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
                            (const int*)P->rowof, S, c->nlist(), P->cnt, (const long long*)P->sl_off, P->cols,
                            (const int*)P->ltail, (const long long*)P->tail_off, P->tail_cols);
         SPH_TRY(launch_check(c, "ppe_cols"));
@@ -1629,7 +1634,7 @@ static int ppe_build_ordered(sph_ctx* c, bool allow_lattice) {
         if (c->prm.ppe_stencil && !c->prm.ale_positions) SPH_TRY(stencil_slices(c, P));
     } else {
         SPH_TRY(prof_begin(c, "ppe_cols", 0));
-        hipLaunchKernelGGL(k_ppe_struct<true>, dim3(grid1(nr)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
+        hipLaunchKernelGGL(k_ppe_struct<true>, dim3(grid1((long long)nr * GROUP)), dim3(BLOCK), 0, c->stream, nr, (const int*)P->rows,
                            (const int*)P->rowof, S, c->nlist(), P->cnt, (const long long*)P->sl_off, P->cols,
                            (const int*)P->ltail, (const long long*)P->tail_off, P->tail_cols);
         SPH_TRY(launch_check(c, "ppe_cols"));
