@@ -291,124 +291,293 @@ __global__ void __launch_bounds__(BLOCK) k_cell_start(int ncs, const int* keys, 
 // Neighbour list: the union of the dcell-query window and the binning
 // window of particle i (both +-ncell), scanned in increasing cell index so
 // entries come out in ascending j, each tagged with the flags of flags.h.
-// One 64-lane wave per particle (particle = global thread index / 64).  The
-// window's x-rows are numbered z-major then y (lane k describes row k of a
-// batch of 64), their particle ranges are flattened into one candidate
-// order v, and each round of 64 candidates is compacted in order with a
-// ballot, so the list is the one a serial scan in cell order produces.
-template <bool FILL>
-__device__ __forceinline__ int nl_wave(int i, const Grid& g, const double* x, const double* y, const double* z,
-                                       const double* h, const int* ncell, double kappa, unsigned* out, int cap) {
+//
+// The flags compare the distance r = sqrt(r2) (+- 1e-20) with a radius k.
+// Both sides are monotone in r2, so each test is r2 < T with T the least
+// double whose root fails it: no root per pair.  T is found per particle
+// (k = kappa h, and half of it), and max(T_i, T_j) is the threshold of
+// max(h_i, h_j).
+struct NLForm {
+    int bits;                   // NL_TINY: dp, dm, b differ somewhere (k near 1e-4); NL_VARIES: dp varies
+    unsigned long long reach;   // the largest dm, as bits
+};
+struct NLThr {
+    const double *dp, *dm, *b, *bh;   // r + 1e-20 < k; r - 1e-20 < k; r < k; r + 1e-20 < k / 2 (k = kappa h)
+    const NLForm* form;
+};
+constexpr int NL_TINY = 1, NL_VARIES = 2;
+// least y >= 0 for which sqrt(y) + add < k does not hold (infinity if none)
+__device__ double root_threshold(double k, double add) {
+    auto holds = [&](unsigned long long u) { return sqrt(__longlong_as_double((long long)u)) + add < k; };
+    const unsigned long long top = 0x7ff0000000000000ull;   // infinity; doubles >= 0 ascend with their bits
+    const double y = k > 0.0 ? k * k : 0.0;                 // (NaN: nothing holds, 0)
+    unsigned long long u = (unsigned long long)__double_as_longlong(y), lo, hi;
+    if (holds(u)) {
+        lo = u;
+        for (unsigned long long s = 1;; s <<= 1) {
+            if (lo == top) return __longlong_as_double((long long)top);
+            hi = s < top - lo ? lo + s : top;
+            if (!holds(hi)) break;
+            lo = hi;
+        }
+    } else {
+        hi = u;
+        for (unsigned long long s = 1;; s <<= 1) {
+            if (hi == 0) return 0.0;
+            lo = hi > s ? hi - s : 0;
+            if (holds(lo)) break;
+            hi = lo;
+        }
+    }
+    while (hi - lo > 1) {
+        const unsigned long long m = lo + (hi - lo) / 2;
+        if (holds(m)) lo = m;
+        else hi = m;
+    }
+    return __longlong_as_double((long long)hi);
+}
+__global__ void __launch_bounds__(BLOCK) k_nl_thresholds(int n, const double* h, double kappa, double* dp, double* dm,
+                                                         double* b, double* bh, NLForm* form) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    int fm = 0;
+    unsigned long long far = 0;
+    if (i < n) {
+        const double k = kappa * h[i];
+        const double tp = root_threshold(k, 1e-20), tm = root_threshold(k, -1e-20), t0 = root_threshold(k, 0.0);
+        dp[i] = tp;
+        dm[i] = tm;
+        b[i] = t0;
+        bh[i] = root_threshold(kappa * (0.5 * h[i]), 1e-20);
+        far = (unsigned long long)__double_as_longlong(tm);
+        fm = (tp != tm || tp != t0 ? NL_TINY : 0) | (h[i] != h[0] ? NL_VARIES : 0);
+    }
+    for (int bit = 1; bit <= NL_VARIES; bit <<= 1)
+        if (__ballot(fm & bit) && (threadIdx.x & 63) == 0 && !(form->bits & bit)) atomicOr(&form->bits, bit);
+    for (int off = 32; off > 0; off >>= 1) far = max(far, (unsigned long long)__shfl_xor((long long)far, off, 64));
+    if ((threadIdx.x & 63) == 0 && far > form->reach) atomicMax(&form->reach, far);
+}
+// Where the particles of a cell can lie along an axis: its share of the
+// binning range, `pad` wider for the float arithmetic here and in the binning
+// (together below 1e-6 of the range and of a coordinate), and without end
+// beyond the first and the last cell, which take what lies outside.
+struct Axis {
+    float lo, w, inv, pad;
+    int N;
+    __device__ Axis(float mn, float mx, int n)
+        : lo(mn), w((mx - mn) / (float)n), inv(1.0f / w), pad(4e-6f * (fabsf(mn) + fabsf(mx))), N(n) {}
+    // distance of cell c to [a, b], never too large
+    __device__ float gap(int c, float a, float b) const {
+        const float below = c < N - 1 ? a - (lo + (float)(c + 1) * w + pad) : 0.0f;
+        const float above = c > 0 ? (lo + (float)c * w - pad) - b : 0.0f;
+        return fmaxf(fmaxf(below, above), 0.0f);
+    }
+    // the cell that holds v (a NaN, of an axis without extent: the first)
+    __device__ int cell(float v) const { return (int)fminf(fmaxf(floorf((v - lo) * inv), 0.0f), (float)(N - 1)); }
+};
+// One 64-lane wave lists NL_P consecutive particles, those of one window
+// together: the window's x-rows are numbered z-major then y (lane k describes
+// row k of a batch of 64), their particle ranges are flattened into one
+// candidate order v, each round of 64 candidates is loaded once for the
+// particles that share it, and compacted in order with a ballot per
+// particle, so the lists are the ones a serial scan in cell order produces.
+// Bound by vector instructions, in equal parts of a window's set-up and of
+// its candidates.  A wave a particle, with a root a pair, a six-step search
+// for each candidate's row and no row left out, took 1365 of them a particle
+// and 2.85 ms for 1 M particles of ~590 candidates and 99 entries; this takes
+// 1.43 ms (count alone 2.5 -> 1.1 ms).
+constexpr int NL_P = 4;
+static_assert(SLICE % NL_P == 0, "a wave's particles share a slice");
+// inclusive prefix sum over the wave's lanes
+__device__ __forceinline__ int wave_incl(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8: rows of 16 lanes
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2, 3
+    return v;
+}
+template <bool FILL, bool TINY, bool VARIES>
+__device__ __forceinline__ int nl_wave(int i0, int np, const Grid& g, const double* x, const double* y,
+                                        const double* z, const NLThr& t, const int* ncell, int* marks, unsigned* out,
+                                        int cap, int* cnt) {
     const int lane = threadIdx.x & 63;
+    int longest = 0;
     const sph_domain& d = g.d;
-    const double xi = x[i], yi = y[i], zi = z[i], hi = h[i];
-    const int nc = ncell[i];
-    const Cell q = query_cell(d, xi, yi, zi);
-    const Cell b = bin_cell(d, xi, yi, zi);
-    const int jlo = max(min(q.j, b.j) - nc, 0), jhi = min(max(q.j, b.j) + nc, d.NJ - 1);
-    const int klo = max(min(q.k, b.k) - nc, 0), khi = min(max(q.k, b.k) + nc, d.NK - 1);
-    const int nj = max(jhi - jlo + 1, 0), nk = max(khi - klo + 1, 0), nrows = nj * nk;
-    const double khi_r = kappa * hi, khalf = kappa * (0.5 * hi);
-    int cnt = 0;
-    for (int r0 = 0; r0 < nrows; r0 += 64) {
-        // lane k: row r0 + k of the union window
-        int rs = 0, rl = 0, base = 0, flags = 0;
-        const int rk = r0 + lane;
-        if (rk < nrows) {
-            const int ck = klo + rk / nj, cj = jlo + rk % nj;
-            const bool rowD = abs(cj - q.j) <= nc && abs(ck - q.k) <= nc;
-            const bool rowB = abs(cj - b.j) <= nc && abs(ck - b.k) <= nc;
-            int i0 = INT_MAX, i1 = INT_MIN;
-            if (rowD) { i0 = min(i0, q.i - nc); i1 = max(i1, q.i + nc); }
-            if (rowB) { i0 = min(i0, b.i - nc); i1 = max(i1, b.i + nc); }
-            i0 = max(i0, 0);
-            i1 = min(i1, d.NI - 1);
-            base = d.NI * cj + d.NI * d.NJ * ck;
-            flags = (rowD ? 1 : 0) | (rowB ? 2 : 0);
-            if ((rowD || rowB) && i0 <= i1) {
-                rs = g.cstart[base + i0];
-                rl = g.cstart[base + i1 + 1] - rs;
-            }
-        }
-        int incl = rl;
+    // lane p: the cells of particle i0 + p
+    const int ip = i0 + min(lane, np - 1);
+    const double xp = x[ip], yp = y[ip], zp = z[ip], dpp = t.dp[ip], bhp = t.bh[ip];
+    const Cell qp = query_cell(d, xp, yp, zp), bp = bin_cell(d, xp, yp, zp);
+    const int ncp = ncell[ip];
+    const double dmp = TINY ? t.dm[ip] : 0.0, tbp = TINY ? t.b[ip] : 0.0;
+    auto at64 = [](double v, int l) {   // lane l's value, wave-uniform
+        const long long u = __double_as_longlong(v);
+        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)u, l);
+        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(u >> 32), l);
+        return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    };
+    // no pair of r2 >= reach has a flag
+    const float reach = (float)__longlong_as_double((long long)t.form->reach);
+    const Axis ax(d.x_min, d.x_max, d.NI), ay(d.y_min, d.y_max, d.NJ), az(d.z_min, d.z_max, d.NK);
+    for (int a = 0; a < np;) {
+        auto at = [&](int v) { return __builtin_amdgcn_readlane(v, a); };
+        const Cell q{at(qp.i), at(qp.j), at(qp.k)}, b{at(bp.i), at(bp.j), at(bp.k)};
+        const int nc = at(ncp);
+        const unsigned long long same =
+            __ballot(qp.i == q.i && qp.j == q.j && qp.k == q.k && bp.i == b.i && bp.j == b.j && bp.k == b.k && ncp == nc);
+        int C = 1;   // particles a .. a + C - 1 share the window
+        while (a + C < np && ((same >> (a + C)) & 1ULL)) C++;
+        double xi[NL_P], yi[NL_P], zi[NL_P], dp[NL_P], dm[NL_P], tb[NL_P], th[NL_P];
+        int m[NL_P] = {};
+        float bx0 = 0, bx1 = 0, by0 = 0, by1 = 0, bz0 = 0, bz1 = 0;   // the particles' box
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(incl, off, 64);
-            if (lane >= off) incl += o;
+        for (int p = 0; p < NL_P; p++) {
+            if (p >= C) break;
+            const int l = a + p;
+            xi[p] = at64(xp, l); yi[p] = at64(yp, l); zi[p] = at64(zp, l);
+            dp[p] = at64(dpp, l); th[p] = at64(bhp, l);
+            dm[p] = TINY ? at64(dmp, l) : 0.0; tb[p] = TINY ? at64(tbp, l) : 0.0;
+            const float fx = (float)xi[p], fy = (float)yi[p], fz = (float)zi[p];
+            bx0 = p ? fminf(bx0, fx) : fx; bx1 = p ? fmaxf(bx1, fx) : fx;
+            by0 = p ? fminf(by0, fy) : fy; by1 = p ? fmaxf(by1, fy) : fy;
+            bz0 = p ? fminf(bz0, fz) : fz; bz1 = p ? fmaxf(bz1, fz) : fz;
         }
-        const int excl = incl - rl, total = __shfl(incl, 63, 64);
-        const int nr_b = min(64, nrows - r0);
-        for (int v0 = 0; v0 < total; v0 += 64) {
-            const int v = v0 + lane, vv = min(v, total - 1);
-            int lo = 0;   // the row holding vv: the last row whose prefix is <= vv
-#pragma unroll
-            for (int step = 32; step > 0; step >>= 1) {
-                const int cand = lo + step;
-                const int pe = __shfl(excl, min(cand, 63), 64);
-                if (cand < nr_b && pe <= vv) lo = cand;
-            }
-            const int start = __shfl(rs, lo, 64), pre = __shfl(excl, lo, 64);
-            const int rbase = __shfl(base, lo, 64), rflags = __shfl(flags, lo, 64);
-            unsigned f = 0;
-            int j = -1;
-            if (v < total) {
-                j = start + (vv - pre);
-                const int ci = g.keys[j] - rbase;
-                const bool inD = (rflags & 1) && abs(ci - q.i) <= nc;
-                const bool inB = (rflags & 2) && abs(ci - b.i) <= nc;
-                if (inD || inB) {
-                    double r = dist3<double>(xi, yi, zi, x[j], y[j], z[j]);
-                    double kmax = kappa * fmax(hi, h[j]);
-                    double tp = r + 1e-20, tm = r - 1e-20;
-                    if (inD) {
-                        if (tp < kmax) f |= F_DP;
-                        if (tm < kmax) f |= F_DM;
-                        if (tp < khi_r) f |= F_HP;
-                        if (tm < khi_r) f |= F_HM;
-                    }
-                    if (inB) {
-                        if (r > 0 && r < khi_r) f |= F_B;
-                        if (tp < khalf) f |= F_BH;
-                    }
+        const bool one = q.i == b.i && q.j == b.j && q.k == b.k;   // the two windows are one
+        const int jlo = max(min(q.j, b.j) - nc, 0), jhi = min(max(q.j, b.j) + nc, d.NJ - 1);
+        const int klo = max(min(q.k, b.k) - nc, 0), khi = min(max(q.k, b.k) + nc, d.NK - 1);
+        const int nj = max(jhi - jlo + 1, 0), nk = max(khi - klo + 1, 0), nrows = nj * nk;
+        for (int r0 = 0; r0 < nrows; r0 += 64) {
+            // lane k: row r0 + k of the union window
+            int rs = 0, rl = 0, base = 0, flags = 0;
+            const int rk = r0 + lane;
+            if (rk < nrows) {
+                const int ck = klo + rk / nj, cj = jlo + rk % nj;
+                const bool rowD = abs(cj - q.j) <= nc && abs(ck - q.k) <= nc;
+                const bool rowB = abs(cj - b.j) <= nc && abs(ck - b.k) <= nc;
+                int c0 = INT_MAX, c1 = INT_MIN;
+                if (rowD) { c0 = min(c0, q.i - nc); c1 = max(c1, q.i + nc); }
+                if (rowB) { c0 = min(c0, b.i - nc); c1 = max(c1, b.i + nc); }
+                const float gy = ay.gap(cj, by0, by1), gz = az.gap(ck, bz0, bz1), left = reach - gy * gy - gz * gz;
+                if (left < -1e-5f * reach) c1 = INT_MIN;   // the row is out of reach
+                const float half = sqrtf(fmaxf(left, 0.0f) + 2e-5f * reach);
+                c0 = max(max(c0, 0), ax.cell(bx0 - half - ax.pad));
+                c1 = min(min(c1, d.NI - 1), ax.cell(bx1 + half + ax.pad));
+                base = d.NI * cj + d.NI * d.NJ * ck;
+                flags = (rowD ? 1 : 0) | (rowB ? 2 : 0);
+                if ((rowD || rowB) && c0 <= c1) {
+                    rs = g.cstart[base + c0];
+                    rl = g.cstart[base + c1 + 1] - rs;
                 }
             }
-            const unsigned long long m = __ballot(f != 0);
-            if (FILL && f) {
-                const int below = __popcll(m & ((1ULL << lane) - 1ULL));
-                if (cnt + below < cap) out[(size_t)(cnt + below) * SLICE] = (unsigned)j | f;
+            const int incl = wave_incl(rl);
+            const int excl = incl - rl, total = __builtin_amdgcn_readlane(incl, 63), first = rs - excl;
+            int held = 0;   // the row that holds the last candidate of the round before
+            for (int v0 = 0; v0 < total; v0 += 64) {
+                // the row of candidate v: each row that starts in the round marks its first candidate
+                marks[lane] = -1;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (rl > 0 && excl >= v0 && excl < v0 + 64) marks[excl - v0] = lane;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                const int mk = marks[lane];
+                const unsigned long long M = __ballot(mk >= 0), upto = M & (~0ULL >> (63 - lane));
+                const int near = __shfl(mk, upto ? 63 - __clzll((long long)upto) : 0, 64);
+                const int row = upto ? near : held;
+                if (M) held = __builtin_amdgcn_readlane(mk, 63 - __clzll((long long)M));
+                const int v = min(v0 + lane, total - 1);
+                const int rowv = v0 + lane < total ? row : held;
+                const int j = __shfl(first, rowv, 64) + v;
+                bool inD = v0 + lane < total, inB = inD;
+                if (!one) {
+                    const int rflags = __shfl(flags, rowv, 64);
+                    inD = inD && (rflags & 1);
+                    inB = inB && (rflags & 2);
+                    if (q.i != b.i) {
+                        const int ci = g.keys[j] - __shfl(base, rowv, 64);
+                        inD = inD && abs(ci - q.i) <= nc;
+                        inB = inB && abs(ci - b.i) <= nc;
+                    }
+                }
+                const double xj = x[j], yj = y[j], zj = z[j];
+                const double dpj = VARIES ? t.dp[j] : 0.0, dmj = VARIES && TINY ? t.dm[j] : 0.0;
+#pragma unroll
+                for (int p = 0; p < NL_P; p++) {
+                    if (p >= C) break;
+                    const double r2 =
+                        (xi[p] - xj) * (xi[p] - xj) + (yi[p] - yj) * (yi[p] - yj) + (zi[p] - zj) * (zi[p] - zj);
+                    const double kd = VARIES ? fmax(dp[p], dpj) : dp[p];
+                    unsigned f = 0;
+                    if (TINY) {
+                        const double km = VARIES ? fmax(dm[p], dmj) : dm[p];
+                        if (inD)
+                            f = (r2 < kd ? F_DP : 0u) | (r2 < km ? F_DM : 0u) | (r2 < dp[p] ? F_HP : 0u) |
+                                (r2 < dm[p] ? F_HM : 0u);
+                        if (inB) f |= (r2 > 0.0 && r2 < tb[p] ? F_B : 0u) | (r2 < th[p] ? F_BH : 0u);
+                    } else {
+                        const bool own = r2 < dp[p];
+                        if (inD) f = (r2 < kd ? F_DP | F_DM : 0u) | (own ? F_HP | F_HM : 0u);
+                        if (inB) f |= (r2 > 0.0 && own ? F_B : 0u) | (r2 < th[p] ? F_BH : 0u);
+                    }
+                    const unsigned long long hit = __ballot(f != 0);
+                    if (FILL && f) {
+                        const int slot = m[p] + (int)__builtin_amdgcn_mbcnt_hi(
+                                                    (unsigned)(hit >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((unsigned)hit, 0u));
+                        if (slot < cap) out[(size_t)slot * SLICE + a + p] = (unsigned)j | f;
+                    }
+                    m[p] += __popcll(hit);
+                }
             }
-            cnt += __popcll(m);
         }
+        if (lane < C) {
+            int v = 0;
+#pragma unroll
+            for (int p = 0; p < NL_P; p++) v = lane == p ? m[p] : v;
+            cnt[a + lane] = v;
+        }
+#pragma unroll
+        for (int p = 0; p < NL_P; p++) longest = max(longest, m[p]);
+        a += C;
     }
-    return cnt;
+    return longest;
+}
+// the first particle of this wave.  xcd_block: a list slice's 64 particles on
+// one XCD, so their interleaved entries fill whole lines in one L2
+__device__ __forceinline__ int nl_first() {
+    return __builtin_amdgcn_readfirstlane(
+        (int)((((long long)xcd_block() * blockDim.x + threadIdx.x) >> 6) * NL_P));
+}
+template <bool FILL>
+__device__ __forceinline__ int nl_lists(int i0, int np, const Grid& g, const double* x, const double* y,
+                                        const double* z, const NLThr& t, const int* ncell, int* marks, unsigned* out,
+                                        int cap, int* cnt) {
+    const int form = __builtin_amdgcn_readfirstlane(t.form->bits);
+    if (form & NL_TINY) return nl_wave<FILL, true, true>(i0, np, g, x, y, z, t, ncell, marks, out, cap, cnt);
+    if (form & NL_VARIES) return nl_wave<FILL, false, true>(i0, np, g, x, y, z, t, ncell, marks, out, cap, cnt);
+    return nl_wave<FILL, false, false>(i0, np, g, x, y, z, t, ncell, marks, out, cap, cnt);
 }
 __global__ void __launch_bounds__(BLOCK) k_nl_count(int n, Grid g, const double* x, const double* y, const double* z,
-                                                    const double* h, const int* ncell, double kappa, int* cnt) {
-    // xcd_block: a list slice's 64 particles on one XCD, so their
-    // interleaved entries fill whole lines in one L2
-    const int i = (int)(((long long)xcd_block() * blockDim.x + threadIdx.x) >> 6);
-    if (i >= n) return;   // whole waves
-    const int m = nl_wave<false>(i, g, x, y, z, h, ncell, kappa, nullptr, 0);
-    if ((threadIdx.x & 63) == 0) cnt[i] = m;
+                                                    NLThr t, const int* ncell, int* cnt) {
+    __shared__ int marks[BLOCK];
+    const int i0 = nl_first();
+    if (i0 >= n) return;   // whole waves
+    nl_lists<false>(i0, min(NL_P, n - i0), g, x, y, z, t, ncell, marks + (threadIdx.x & ~63), nullptr, 0, cnt + i0);
 }
-// fill pass; with cnt (a fill without a count pass) into the room of each
-// slice, writing the counts and over = 1 when a list does not fit
+// fill pass; with over (a fill without a count pass) into the room of each
+// slice, over = 1 when a list does not fit
 __global__ void __launch_bounds__(BLOCK) k_nl_fill(int n, Grid g, const double* x, const double* y, const double* z,
-                                                   const double* h, const int* ncell, double kappa,
-                                                   const long long* slice_off, long long total, unsigned* ent, int* cnt,
-                                                   int* over) {
-    // xcd_block: a list slice's 64 particles on one XCD, so their
-    // interleaved entries fill whole lines in one L2
-    const int i = (int)(((long long)xcd_block() * blockDim.x + threadIdx.x) >> 6);
-    if (i >= n) return;   // whole waves
-    const int s = i >> 6;
+                                                   NLThr t, const int* ncell, const long long* slice_off,
+                                                   long long total, unsigned* ent, int* cnt, int* over) {
+    __shared__ int marks[BLOCK];
+    const int i0 = nl_first();
+    if (i0 >= n) return;   // whole waves
+    const int s = i0 >> 6, np = min(NL_P, n - i0);
     const long long end = s + 1 < (n + SLICE - 1) / SLICE ? slice_off[s + 1] : total;
-    const int cap = cnt ? (int)((end - slice_off[s]) / SLICE) : INT_MAX;
-    const int m = nl_wave<true>(i, g, x, y, z, h, ncell, kappa, ent + slice_off[s] + (i & 63), cap);
-    if (cnt && (threadIdx.x & 63) == 0) {
-        cnt[i] = m;
-        if (m > cap) over[0] = 1;
-    }
+    const int cap = (int)((end - slice_off[s]) / SLICE);
+    const int longest = nl_lists<true>(i0, np, g, x, y, z, t, ncell, marks + (threadIdx.x & ~63),
+                                      ent + slice_off[s] + (i0 & 63), cap, cnt + i0);
+    if (over && longest > cap) over[0] = 1;
 }
 // room of each slice for a fill without a count pass
 __global__ void __launch_bounds__(BLOCK) k_slice_spare(int nslices, const long long* prev, long long spare,
@@ -508,7 +677,7 @@ static int build_porder(sph_ctx* c) {
     return 0;
 }
 
-// The list of a search: one wave per particle.  When the previous search
+// The list of a search.  When the previous search
 // had as many slices (the particles keep their cell order, and move little
 // between searches), the fill runs at once into each slice's previous
 // width plus NL_SPARE entries; if a list does not fit, the search counts
@@ -525,7 +694,18 @@ static int build_neighbor_list(sph_ctx* c) {
     SPH_TRY(dalloc(c, &c->nl_slice_off, nslices + 1));
     Grid g = c->grid();
     const double *x = c->pf[SPH_F_X], *y = c->pf[SPH_F_Y], *z = c->pf[SPH_F_Z], *h = c->pf[SPH_F_H];
-    const unsigned nlgrid = (unsigned)(((long long)n * 64 + BLOCK - 1) / BLOCK);
+    const unsigned nlgrid = (unsigned)grid1(((long long)n + NL_P - 1) / NL_P * 64);
+    double* thr[4] = {};
+    for (auto& a : thr) SPH_TRY(dalloc(c, &a, c->cap));
+    NLForm* form = nullptr;
+    SPH_TRY(dalloc(c, &form, 1));
+    SPH_HIP(c, hipMemsetAsync(form, 0, sizeof(NLForm), c->stream));
+    const NLThr t{thr[0], thr[1], thr[2], thr[3], form};
+    SPH_TRY(prof_begin(c, "nl_thresholds", 40.0 * n));
+    hipLaunchKernelGGL(k_nl_thresholds, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, n, h, c->prm.kappa, thr[0], thr[1],
+                       thr[2], thr[3], form);
+    SPH_TRY(launch_check(c, "nl_thresholds"));
+    SPH_TRY(prof_end(c));
     long long* w = nullptr;
     SPH_TRY(dalloc(c, &w, nslices + 1));
     long long total = 0;
@@ -539,8 +719,8 @@ static int build_neighbor_list(sph_ctx* c) {
         SPH_TRY(exclusive_scan_i64(c, w, c->nl_slice_off, nslices, &total));
         SPH_TRY(dalloc(c, &c->nl_ent, (size_t)total + 1));
         SPH_TRY(prof_begin(c, "nl_fill", 0));
-        hipLaunchKernelGGL(k_nl_fill, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, h,
-                           (const int*)c->pi[SPH_I_NCELL], c->prm.kappa, (const long long*)c->nl_slice_off, total,
+        hipLaunchKernelGGL(k_nl_fill, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, t,
+                           (const int*)c->pi[SPH_I_NCELL], (const long long*)c->nl_slice_off, total,
                            c->nl_ent, c->nl_cnt, over);
         SPH_TRY(launch_check(c, "nl_fill"));
         SPH_TRY(prof_end(c));
@@ -555,14 +735,16 @@ static int build_neighbor_list(sph_ctx* c) {
             SPH_TRY(launch_check(c, "slice_width"));
             c->nl_total = total;
             dfree(c, w);
+            for (auto a : thr) dfree(c, a);
+            dfree(c, form);
             return build_porder(c);
         }
         dfree(c, c->nl_ent);
         c->nl_ent = nullptr;
     }
     SPH_TRY(prof_begin(c, "nl_count", 0));
-    hipLaunchKernelGGL(k_nl_count, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, h,
-                       (const int*)c->pi[SPH_I_NCELL], c->prm.kappa, c->nl_cnt);
+    hipLaunchKernelGGL(k_nl_count, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, t,
+                       (const int*)c->pi[SPH_I_NCELL], c->nl_cnt);
     SPH_TRY(launch_check(c, "nl_count"));
     SPH_TRY(prof_end(c));
     hipLaunchKernelGGL(k_slice_width, dim3(grid1(nslices)), dim3(BLOCK), 0, c->stream, n, nslices,
@@ -580,11 +762,13 @@ static int build_neighbor_list(sph_ctx* c) {
     c->nl_total = total;
     SPH_TRY(dalloc(c, &c->nl_ent, (size_t)total + 1));
     SPH_TRY(prof_begin(c, "nl_fill", 0));
-    hipLaunchKernelGGL(k_nl_fill, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, h,
-                       (const int*)c->pi[SPH_I_NCELL], c->prm.kappa, (const long long*)c->nl_slice_off, total,
-                       c->nl_ent, (int*)nullptr, (int*)nullptr);
+    hipLaunchKernelGGL(k_nl_fill, dim3(nlgrid), dim3(BLOCK), 0, c->stream, n, g, x, y, z, t,
+                       (const int*)c->pi[SPH_I_NCELL], (const long long*)c->nl_slice_off, total, c->nl_ent,
+                       c->nl_cnt, (int*)nullptr);
     SPH_TRY(launch_check(c, "nl_fill"));
     SPH_TRY(prof_end(c));
+    for (auto a : thr) dfree(c, a);
+    dfree(c, form);
     return build_porder(c);
 }
 
