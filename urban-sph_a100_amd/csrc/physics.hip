@@ -30,16 +30,20 @@ namespace sph {
     const CaseDesc& cd = (sg).cd[cid_];           \
     const int i = first_ + (int)threadIdx.x;      \
     if (i >= cd.n) return;
-// prep, advection and the pressure force: the particles of short lists, a
-// thread each in the pass order; in MIXED the last cd.n_heavy of that order
-// (the heavy lists) are left to a wave each (SEG_HEAVY)
-#define SEG_PARTICLE_LIGHT(sg)                            \
-    int first_;                                           \
-    const int cid_ = seg_case((sg), first_);              \
-    const CaseDesc& cd = (sg).cd[cid_];                   \
-    const int t_ = first_ + (int)threadIdx.x;             \
-    if (t_ >= cd.n - cd.n_heavy) return;                  \
-    const int i = cd.porder ? cd.porder[t_] : t_;
+// BLANES lanes (lane: this one) per particle of the case's boundary list
+// (every p_type but fluid): wall, lid and marker passes, which leave most of
+// that list at once, so a wave of its own for each particle mostly waits on
+// the loads that lead to its p_type (free slip, 2.13 M canyon: 222 us, with 16
+// lanes 131; FP64, 1 M: 380 and 186 us, a thread each 190; 20 k: 13, 14, 65).
+constexpr int BLANES = 16;
+#define SEG_BOUNDARY(sg)                                               \
+    int first_;                                                        \
+    const int cid_ = seg_case(sg, first_);                             \
+    const CaseDesc& cd = sg.cd[cid_];                                  \
+    if ((sg).tab == nullptr) first_ *= 64 / BLANES;   /* blocks of blockDim * 64 / BLANES */ \
+    const int u_ = first_ / 64 + (int)threadIdx.x / BLANES, lane = (int)threadIdx.x % BLANES; \
+    if (u_ >= cd.nm_count) return;                                     \
+    const int i = cd.nm_list[u_];
 // GROUP lanes a particle (g_: the lane in its group)
 #define SEG_GROUP(sg)                                     \
     int first_;                                           \
@@ -47,6 +51,9 @@ namespace sph {
     const CaseDesc& cd = (sg).cd[cid_];                   \
     const int i = first_ + (int)threadIdx.x / GROUP, g_ = (int)threadIdx.x % GROUP; \
     if (i >= cd.n) return;
+// prep, advection and the pressure force: the particles of short lists in the
+// pass order; in MIXED the last cd.n_heavy of that order (the heavy lists) are
+// left to a wave each (SEG_HEAVY)
 #define SEG_GROUP_LIGHT(sg)                               \
     int first_;                                           \
     const int cid_ = seg_case((sg), first_);              \
@@ -62,16 +69,10 @@ namespace sph {
     const int lane_ = threadIdx.x & 63;                       \
     if (u_ >= cd.n_heavy) return;                             \
     const int i = cd.porder[cd.n - cd.n_heavy + u_];
-// The same through the case's pass order when it has one (long neighbour
-// lists last): for the record-gathering passes, where it measured faster.
-#define SEG_PARTICLE_ORDERED(sg)                          \
-    int first_;                                           \
-    const int cid_ = seg_case((sg), first_);              \
-    const CaseDesc& cd = (sg).cd[cid_];                   \
-    const int t_ = first_ + (int)threadIdx.x;             \
-    if (t_ >= cd.n) return;                               \
-    const int i = cd.porder ? cd.porder[t_] : t_;
-
+// FP64: dynamic LDS of ordered sums, this wave's part
+#define ORDERED_LDS(nt, n2)            \
+    extern __shared__ double ord_lds_[]; \
+    double* const wlds_ = ord_lds_ + (threadIdx.x >> 6) * ord_doubles((nt), (n2));
 
 // Particles of the cells (i0..i1, cj, ck) that lie inside the grid, as one
 // range [rg.x, rg.y) of the sorted order; false when the row is outside the
@@ -173,40 +174,41 @@ __device__ __forceinline__ void grad_corr_store(const QView& Q, int i, int ptype
     }
 }
 
+constexpr int GC_SUMS = 6;
 __global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr(Seg sg) {
-    SEG_PARTICLE(sg);
+    ORDERED_LDS(GC_SUMS, 0);
+    SEG_GROUP(sg);
     if (cd.gc_fresh) return;   // unchanged since the last step of this search
     const KConst kc = cd.kc;
     const PView S = cd.S;
-    const QView Q = cd.Q;
-    const NList nl = cd.nl;
-    int ptype_i = S.p_type[i];
-    double hi = (double)S.h[i];
-    double tmp_A = calc_tmpA<double>(kc, hi);
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double tmpxx = 0, tmpyy = 0, tmpzz = 0, tmpxy = 0, tmpyz = 0, tmpzx = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_B)) continue;
-        int j = e & NB_IDX;
-        double dx = (double)(xi - S.x[j]), dy = (double)(yi - S.y[j]), dz = (double)(zi - S.z[j]);
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz);
-        double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
-        double mj = (double)S.m[j], rhoj = (double)S.rho[j];
-        double mtd = mj * tdwij;
-        double rtd = (double)1.0 / (rhoj * tdist);
-        double txx = -mtd * dx * dx; txx *= rtd;
-        double txy = -mtd * dy * dx; txy *= rtd;
-        double tyy = -mtd * dy * dy; tyy *= rtd;
-        double tzx = -mtd * dx * dz; tzx *= rtd;
-        double tyz = -mtd * dy * dz; tyz *= rtd;
-        double tzz = -mtd * dz * dz; tzz *= rtd;
-        double f = (double)(S.p_type[j] == 1);
-        tmpxx += txx * f; tmpxy += txy * f; tmpyy += tyy * f;
-        tmpzx += tzx * f; tmpyz += tyz * f; tmpzz += tzz * f;
+    const double hi = S.h[i], tmp_A = calc_tmpA<double>(kc, hi);
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    OrderedSums<GC_SUMS, GROUP> sums(wlds_);   // xx, yy, zz, xy, yz, zx
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = g_; k - g_ < row.cnt; k += GROUP) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const bool pair = (e & F_B) != 0;
+        if (!__any(pair)) continue;
+        double v[GC_SUMS] = {};
+        if (pair) {
+            const int j = e & NB_IDX;
+            const double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz);
+            const double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+            const double mj = S.m[j], rhoj = S.rho[j];
+            const double mtd = mj * tdwij, rtd = 1.0 / (rhoj * tdist), f = (double)(S.p_type[j] == 1);
+            v[0] = -mtd * dx * dx * rtd * f;
+            v[1] = -mtd * dy * dy * rtd * f;
+            v[2] = -mtd * dz * dz * rtd * f;
+            v[3] = -mtd * dy * dx * rtd * f;
+            v[4] = -mtd * dy * dz * rtd * f;
+            v[5] = -mtd * dx * dz * rtd * f;
+        }
+        sums.add(v);
     }
-    grad_corr_store(Q, i, ptype_i, tmpxx, tmpyy, tmpzz, tmpxy, tmpyz, tmpzx);
+    double t[GC_SUMS];
+    for (int a = 0; a < GC_SUMS; a++) t[a] = sums.sum(a);
+    if (g_ == 0) grad_corr_store(cd.Q, i, S.p_type[i], t[0], t[1], t[2], t[3], t[4], t[5]);
 }
 // MIXED: GROUP lanes a particle (SEG_GROUP), the pair arithmetic in float,
 // the sums in double
@@ -312,57 +314,64 @@ __device__ __forceinline__ void prep_store(const CaseDesc& cd, int i, bool les, 
     if (cd.count == 0) S2.rho_ref[i] = S.rho[i];
     if (filt) S.flt_s[i] = tmp_flt;
 }
+constexpr int PREP_SUMS = 8;
 __global__ void __launch_bounds__(MAX_BLOCK) k_prep(Seg sg) {
-    SEG_PARTICLE_LIGHT(sg);
+    ORDERED_LDS(PREP_SUMS, 0);
+    SEG_GROUP_LIGHT(sg);
     const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
+    const sph_params& pr = cd.pr;
     const PView S = cd.S;
     const QView Q = cd.Q;
     if (S.i_type[i] > 2) return;
     if (S.p_type[i] >= 1000) return;
     if (S.p_type[i] <= 0) return;
     const double ki = fmax(S.k_turb[i], 0.0), nui = S.vis_t[i];
-    double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
-    double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    double hi = S.h[i];
-    double tmp_A = calc_tmpA<double>(kc, hi);
-    double tmp_flt = 0.0, tmp_sigma = 0.0;
-    double st11 = 0, st12 = 0, st22 = 0, st23 = 0, st31 = 0, st33 = 0;
+    const double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
+    const double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const double hi = S.h[i], tmp_A = calc_tmpA<double>(kc, hi);
     const bool filt = (cd.count % pr.freq_filt) == 0;
     const bool les = (pr.fv_solve != 0) && (pr.turbulence_model != SPH_LAMINAR);
+    OrderedSums<PREP_SUMS, GROUP> sums(wlds_);   // st11, 12, 22, 23, 31, 33, filter, sigma
     const NLRow row = nl_row(cd.nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_HP)) continue;
-        int j = e & NB_IDX;
-        double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
-        double mj = S.m[j], rhoj = S.rho[j];
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-        double tmp_wij = kernel_w<double>(kc, tmp_A, hi, tdist);
-        double tmp_dwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
-        double tdwx = tmp_dwij * dx / tdist;
-        double tdwy = tmp_dwij * dy / tdist;
-        double tdwz = tmp_dwij * dz / tdist;
-        if (filt) tmp_flt += mj / rhoj * tmp_wij;
-        if (les) {
-            tmp_sigma += tdist * tdist * tmp_wij * mj / rhoj;
-            if (S.p_type[j] == 1) {
-                double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
-                double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
-                double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
-                double dux = S.ux[j] - uxi, duy = S.uy[j] - uyi, duz = S.uz[j] - uzi;
-                st11 += mj / rhoj * dux * tdwxc;
-                st12 += 0.5 * mj / rhoj * (dux * tdwyc + duy * tdwxc);
-                st22 += mj / rhoj * duy * tdwyc;
-                st23 += 0.5 * mj / rhoj * (duy * tdwzc + duz * tdwyc);
-                st31 += 0.5 * mj / rhoj * (dux * tdwzc + duz * tdwxc);
-                st33 += mj / rhoj * duz * tdwzc;
+    for (int k = g_; k - g_ < row.cnt; k += GROUP) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const bool pair = (e & F_HP) != 0;
+        if (!__any(pair)) continue;
+        double v[PREP_SUMS] = {};
+        if (pair) {
+            const int j = e & NB_IDX;
+            const double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+            const double mj = S.m[j], rhoj = S.rho[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+            const double tmp_wij = kernel_w<double>(kc, tmp_A, hi, tdist);
+            if (filt) v[6] = mj / rhoj * tmp_wij;
+            if (les) {
+                v[7] = tdist * tdist * tmp_wij * mj / rhoj;
+                if (S.p_type[j] == 1) {
+                    const double tmp_dwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+                    const double tdwx = tmp_dwij * dx / tdist;
+                    const double tdwy = tmp_dwij * dy / tdist;
+                    const double tdwz = tmp_dwij * dz / tdist;
+                    const double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
+                    const double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
+                    const double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
+                    const double dux = S.ux[j] - uxi, duy = S.uy[j] - uyi, duz = S.uz[j] - uzi;
+                    v[0] = mj / rhoj * dux * tdwxc;
+                    v[1] = 0.5 * mj / rhoj * (dux * tdwyc + duy * tdwxc);
+                    v[2] = mj / rhoj * duy * tdwyc;
+                    v[3] = 0.5 * mj / rhoj * (duy * tdwzc + duz * tdwyc);
+                    v[4] = 0.5 * mj / rhoj * (dux * tdwzc + duz * tdwxc);
+                    v[5] = mj / rhoj * duz * tdwzc;
+                }
             }
         }
+        sums.add(v);
     }
-    prep_store(cd, i, les, filt, ki, nui, hi, tmp_flt, tmp_sigma, st11, st12, st22, st23, st31, st33);
+    double t[PREP_SUMS];
+    for (int a = 0; a < PREP_SUMS; a++) t[a] = sums.sum(a);
+    if (g_ == 0) prep_store(cd, i, les, filt, ki, nui, hi, t[6], t[7], t[0], t[1], t[2], t[3], t[4], t[5]);
 }
 
 // MIXED passes over the neighbours of particle i: the pair arithmetic in
@@ -477,61 +486,56 @@ __global__ void __launch_bounds__(TILE_THREADS) k_prep_tile(Seg sg, int width) {
 
 // ------------------------------------------------------------------------
 // KERNEL_boundary3D, functions_BC.cuh:100-190 (wall velocity)
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_boundary3d(Seg sg) {
-    SEG_PARTICLE(sg);
-    const sph_params pr = cd.pr;
+constexpr int BD_SUMS = 4;
+__global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d(Seg sg) {
+    __shared__ double lds[WAVE_BLOCK / 64][ord_doubles(BD_SUMS)];
+    SEG_BOUNDARY(sg);
+    const sph_params& pr = cd.pr;
     if (pr.noslip_bc != 1) return;   // ISPH_Calc.cuh:83
-    const KConst kc = cd.kc;
     const PView S = cd.S;
-    const NList nl = cd.nl;
     if (S.i_type[i] > 2) return;
-    int p_type_i = S.p_type[i];
-    if (p_type_i > 0) return;
-    R hi = (R)S.h[i];
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    double tmpx = 0.0, tmpy = 0.0, tmpz = 0.0, flt = 1.0e-10;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_HM)) continue;
-        int j = e & NB_IDX;
-        R dx = (R)(xi - S.x[j]), dy = (R)(yi - S.y[j]), dz = (R)(zi - S.z[j]);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-        R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-        int p_type_j = S.p_type[j];
-        if (pr.noslip_bc == 1) {
+    if (S.p_type[i] != 0) return;
+    const KConst kc = cd.kc;
+    const double hi = S.h[i], tmp_A = calc_tmpA<double>(kc, hi);
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    OrderedSums<BD_SUMS, BLANES> sums(lds[threadIdx.x >> 6]);
+    if (lane == 3) sums.acc = 1.0e-10;   // the weights' sum
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = lane; k - lane < row.cnt; k += BLANES) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        double v[BD_SUMS] = {};
+        if (e & F_HM) {
+            const int p_type_j = S.p_type[j];
             if ((p_type_j > 0) && (p_type_j != 9)) {
-                tmpx += (double)((R)S.ux[j] * twij);
-                tmpy += (double)((R)S.uy[j] * twij);
-                tmpz += (double)((R)S.uz[j] * twij);
-                flt += (double)twij;
+                const double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+                const double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
+                const double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
+                v[0] = S.ux[j] * twij;
+                v[1] = S.uy[j] * twij;
+                v[2] = S.uz[j] * twij;
+                v[3] = twij;
             }
         }
+        sums.add(v);
     }
-    if (pr.noslip_bc == 1 && (p_type_i == 0 || p_type_i == 9)) {
-        S.ux[i] = 2 * uxi * (p_type_i == 9) - tmpx / flt;
-        S.uy[i] = 2 * uyi * (p_type_i == 9) - tmpy / flt;
-        S.uz[i] = 2 * uzi * (p_type_i == 9) - tmpz / flt;
-    }
+    double t[BD_SUMS];
+    for (int a = 0; a < BD_SUMS; a++) t[a] = sums.sum(a);
+    if (lane != 0) return;
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    S.ux[i] = 2 * uxi * 0 - t[0] / t[3];
+    S.uy[i] = 2 * uyi * 0 - t[1] / t[3];
+    S.uz[i] = 2 * uzi * 0 - t[2] / t[3];
 }
 
-// The same in MIXED, a 64-lane wave per boundary particle (walls are a few
-// per cent of the case): lane sums over entries lane, lane + 64, ..., then
-// a fixed butterfly; only the particles the serial kernel writes (p_type 0
-// and 9) are visited.
-__global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_wave(Seg sg) {
-    int first_;
-    const int cid_ = seg_case(sg, first_);
-    const CaseDesc& cd = sg.cd[cid_];
-    const int u = (first_ + (int)threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (u >= cd.nm_count) return;
+// The same in MIXED: lane sums over entries lane, lane + BLANES, ..., then a
+// fixed butterfly, so a case gives the same bits alone and in a batch; only
+// the particles the reference's kernel writes (p_type 0 and 9) are visited.
+__global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_mixed(Seg sg) {
+    SEG_BOUNDARY(sg);
     const sph_params pr = cd.pr;
     if (pr.noslip_bc != 1) return;   // ISPH_Calc.cuh:83
     const PView S = cd.S;
-    const int i = cd.nm_list[u];
     if (S.i_type[i] > 2) return;
     const int p_type_i = S.p_type[i];
     if (p_type_i != 0 && p_type_i != 9) return;
@@ -542,7 +546,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_wave(Seg sg) {
     double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     double t[4] = {0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
-    for (int k = lane; k < row.cnt; k += 64) {
+    for (int k = lane; k < row.cnt; k += BLANES) {
         unsigned e = NB_AT(row, k);
         if (!(e & F_HM)) continue;
         int j = e & NB_IDX;
@@ -555,8 +559,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_boundary3d_wave(Seg sg) {
         t[2] += (double)((float)S.uz[j] * twij);
         t[3] += (double)twij;
     }
-    for (int off = 32; off > 0; off >>= 1)
-        for (int q = 0; q < 4; q++) t[q] += __shfl_xor(t[q], off, 64);
+    for (double& v : t) group_fold<BLANES>(v);
     if (lane != 0) return;
     const double flt = 1.0e-10 + t[3];
     const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
@@ -877,48 +880,42 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
         return;
     }
     // FP64: each lane forms the terms of one candidate exactly as the serial
-    // scan does; lanes 0..7 then add term k of every contributing candidate
-    // in candidate order, so every sum is bit for bit the serial one.
-    __shared__ double term[8][64];
-    __shared__ int use[64];
-    double acc = 0.0;   // lane k < 8 holds sum k
+    // scan does, and the sums are added in candidate order (OrderedSums).
+    // (Each lane adding the terms that a flag marked, one LDS read after
+    // another, took half of the pass: 268 us on a 150 k canyon.)
+    __shared__ double terms[ord_doubles(8)];
+    OrderedSums<8, 64> sums(terms);
     const bool listed = cd.nmp_off != nullptr;
     // one chunk of candidates v0 .. v0 + 63 of the window's flattened order:
     // lane l holds candidate v0 + l (particle j, or j < 0 for none)
-    auto chunk = [&](int j, int count) {
-        int ok = 0;
+    auto chunk = [&](int j, int) {
+        double v[8] = {};
         // only fluid, non-buffer neighbours carry weight (the reference
         // multiplies the others by 0; skipping those exact zeros leaves every
         // sum bit for bit the same); the pair list holds only those
         if (j >= 0 && (listed || (A.p_type[j] == 1 && A.buffer_type[j] == 0))) {
-            R dx = (R)(xg - A.x[j]), dy = (R)(yg - A.y[j]), dz = (R)(zg - A.z[j]);
-            R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
+            const R dx = (R)(xg - A.x[j]), dy = (R)(yg - A.y[j]), dz = (R)(zg - A.z[j]);
+            const R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
             if (tdist < search_range) {
-                ok = 1;
-                R mj = (R)A.m[j], rhoj = (R)A.rho[j];
-                double presj = pold[j];
-                R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-                term[0][lane] = (double)(mj / rhoj * (R)presj * twij);
-                term[1][lane] = (double)(mj / rhoj * (R)A.ux[j] * twij);
-                term[2][lane] = (double)(mj / rhoj * (R)A.uy[j] * twij);
-                term[3][lane] = (double)(mj / rhoj * (R)A.uz[j] * twij);
-                term[4][lane] = (double)(mj / rhoj * twij);
+                const R mj = (R)A.m[j], rhoj = (R)A.rho[j];
+                const double presj = pold[j];
+                const R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
+                v[0] = (double)(mj / rhoj * (R)presj * twij);
+                v[1] = (double)(mj / rhoj * (R)A.ux[j] * twij);
+                v[2] = (double)(mj / rhoj * (R)A.uy[j] * twij);
+                v[3] = (double)(mj / rhoj * (R)A.uz[j] * twij);
+                v[4] = (double)(mj / rhoj * twij);
                 if (inlet) {
-                    R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-                    R tdwx = dx / tdist * tdwij, tdwy = dy / tdist * tdwij, tdwz = dz / tdist * tdwij;
-                    R dp = (R)(presj - pres_g);
-                    term[5][lane] = (double)(mj / rhoj * dp * tdwx);
-                    term[6][lane] = (double)(mj / rhoj * dp * tdwy);
-                    term[7][lane] = (double)(mj / rhoj * dp * tdwz);
+                    const R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
+                    const R tdwx = dx / tdist * tdwij, tdwy = dy / tdist * tdwij, tdwz = dz / tdist * tdwij;
+                    const R dp = (R)(presj - pres_g);
+                    v[5] = (double)(mj / rhoj * dp * tdwx);
+                    v[6] = (double)(mj / rhoj * dp * tdwy);
+                    v[7] = (double)(mj / rhoj * dp * tdwz);
                 }
             }
         }
-        use[lane] = ok;
-        __syncthreads();   // one wave per block: a wave barrier
-        if (lane < nt)
-            for (int q = 0; q < count; q++)
-                if (use[q]) acc += term[lane][q];
-        __syncthreads();
+        sums.add(v);
     };
     if (cd.nmp_off) {
         // the pairs of this search (the window's weighted candidates, scan order)
@@ -930,9 +927,8 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
     } else {
         neumann_window(g, c, A.ncell[i], lane, chunk);
     }
-    const double tpres = __shfl(acc, 0, 64), tux = __shfl(acc, 1, 64), tuy = __shfl(acc, 2, 64);
-    const double tuz = __shfl(acc, 3, 64), tflt_s = __shfl(acc, 4, 64);
-    const double grad_px = __shfl(acc, 5, 64), grad_py = __shfl(acc, 6, 64), grad_pz = __shfl(acc, 7, 64);
+    const double tpres = sums.sum(0), tux = sums.sum(1), tuy = sums.sum(2), tuz = sums.sum(3), tflt_s = sums.sum(4);
+    const double grad_px = sums.sum(5), grad_py = sums.sum(6), grad_pz = sums.sum(7);
     if (lane != 0) return;
     if (tflt_s < 1e-6) {
         A.pres[i] = 0.0;
@@ -967,121 +963,148 @@ __device__ __forceinline__ void advection_store(const CaseDesc& cd, int i, const
     Q.ftotal[i] = sqrt(a.tx * a.tx + a.ty * a.ty + tz * tz);
     if (concn_solve) Q.dconcn[i] = a.rd;
 }
+// sums tx, ty, tz (a second term each with the artificial viscosity), cx, cy,
+// cz and, with SCAL, rc, ct; then rd (two terms), temp, flt
+template <bool SCAL> constexpr int adv_sums() { return SCAL ? 8 : 6; }
+constexpr int ADV_SECOND = 3, ADV_SUMS2 = 3;
 template <bool SCAL>
-__global__ void __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(SCAL ? 1 : 4))) k_advection(Seg sg) {
-    SEG_PARTICLE_LIGHT(sg);
+__global__ void __launch_bounds__(MAX_BLOCK) k_advection(Seg sg) {
+    ORDERED_LDS(adv_sums<SCAL>(), ADV_SECOND);
+    SEG_GROUP_LIGHT(sg);
+    constexpr int NT = adv_sums<SCAL>();
     const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
+    const sph_params& pr = cd.pr;
     const bool con_solve = SCAL && pr.con_solve, concn_solve = SCAL && pr.concn_solve;
     const bool boussinesq_solve = SCAL && pr.boussinesq_solve;
     const PView S = cd.S;
     if (S.i_type[i] > 2) return;
-    int ptypei = S.p_type[i];
+    const int ptypei = S.p_type[i];
     if (ptypei == 1000) return;
     if (ptypei <= 0) return;
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    double tempi = SCAL ? S.temp[i] : 0.0;
-    double hi = S.h[i], mi = S.m[i], rhoi = S.rho[i];
-    double eli = S.eli[i];
-    double tmp_A = calc_tmpA<double>(kc, hi);
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const double tempi = SCAL ? S.temp[i] : 0.0;
+    const double hi = S.h[i], mi = S.m[i], rhoi = S.rho[i];
+    const double eli = S.eli[i];
+    const double tmp_A = calc_tmpA<double>(kc, hi);
     double kci = 0, cpi = 1, concni = 0, diffi = 0;
     if (con_solve) {
         kci = pr.solid_k * (ptypei == 0 || ptypei == 1000) + pr.air_k * (ptypei == 1 || ptypei == -1);
         cpi = pr.solid_cp * (ptypei == 0 || ptypei == 1000) + pr.air_cp * (ptypei == 1 || ptypei == -1);
     }
     if (concn_solve) { concni = S.concn[i]; diffi = pr.diff_coef; }
-    double visi = viscosity2(pr, ptypei) + S.vis_t[i] * S.rho[i];
-    AdvSums a;
+    const double visi = viscosity2(pr, ptypei) + S.vis_t[i] * S.rho[i];
     const double Alpha = pr.av_alpha, Beta = pr.av_beta, soundspeed = pr.av_c;
     const double ome = 1 - eli;
+    const int fv = pr.fv_solve;
+    const bool art = pr.artificial_viscosity != 0;
+    OrderedSums<NT, GROUP> sums(wlds_);
+    OrderedSums<ADV_SUMS2, GROUP> sums2(wlds_);
     const NLRow row = nl_row(cd.nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_DP)) continue;
-        int j = e & NB_IDX;
+    for (int k = g_; k - g_ < row.cnt; k += GROUP) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        bool pair = (e & F_DP) != 0;
         double hj, vis_tj, xj, yj, zj, mj, uxj, uyj, uzj, rhoj, pqj_;
-        int ptypej, itj_;
-        rec_aux(cd.rec, j, vis_tj, ptypej, itj_);
-        if (ptypej >= 1000) continue;
-        rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pqj_);
-        rec_vel(cd.rec, j, uxj, uyj, uzj, hj);
-        double visj = viscosity2(pr, ptypej) + vis_tj * rhoj;
-        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-        double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
-        double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
-        double tdwx = tdwij * dx / tdist;
-        double tdwy = tdwij * dy / tdist;
-        double tdwz = tdwij * dz / tdist;
-        double dux = uxi - uxj, duy = uyi - uyj, duz = uzi - uzj;   // u_i - u_j
-        double tempj = 0.0, concnj = 0.0;
-        if (con_solve || concn_solve || boussinesq_solve) rec_scalar(cd.rec, j, tempj, concnj);
-        if (pr.fv_solve == SPH_FV_CLEARY) {
-            double C_v = dx * tdwx + dy * tdwy + dz * tdwz;
-            C_v *= (visi * visj) / (visi + visj);
-            C_v *= 4.0 * (mj / (rhoi * rhoj));
-            C_v /= tdist;
-            C_v /= tdist;
-            a.tx += C_v * dux; a.ty += C_v * duy; a.tz += C_v * duz;
-        } else if (pr.fv_solve == SPH_FV_MONAGHAN) {
-            double uij_xij = dux * dx + duy * dy + duz * dz;
-            double phi_ij = uij_xij;
-            phi_ij /= (tdist * tdist + 0.01 * hi * hi);
-            double P_ij = -2.0 * (3 + 2.0) * phi_ij * mj / rhoj;
-            double C_v = 2.0 * (visi * visj) / (visi + visj - 1e-20);
-            double nui = C_v / rhoi;
-            P_ij *= nui;
-            if (ptypei <= 0 || ptypei >= 1000) P_ij = 0;
-            if (ptypej <= 0 || ptypei >= 1000) P_ij = 0;
-            a.tx += -(P_ij)*tdwx; a.ty += -(P_ij)*tdwy; a.tz += -(P_ij)*tdwz;
+        int ptypej = 0, itj_;
+        if (pair) {
+            rec_aux(cd.rec, j, vis_tj, ptypej, itj_);
+            pair = ptypej < 1000;
         }
-        if (eli < 1.0) {
-            double vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
-            a.cx += (uxi * vx * tdwx + uyi * vx * tdwy + uzi * vx * tdwz) * mj / rhoj * ome;
-            a.cy += (uxi * vy * tdwx + uyi * vy * tdwy + uzi * vy * tdwz) * mj / rhoj * ome;
-            a.cz += (uxi * vz * tdwx + uyi * vz * tdwy + uzi * vz * tdwz) * mj / rhoj * ome;
-            if (con_solve)
-                a.ct -= 2.0 * mj / (rhoi + rhoj) * (tempj - tempi) * (dux * tdwx + duy * tdwy + duz * tdwz) * ome;
-            if (concn_solve) {
-                double dc = concnj - concni;
-                a.rd -= (uxi * dc * tdwx + uyi * dc * tdwy + uzi * dc * tdwz) * mj / rhoj * ome;
+        if (!__any(pair)) continue;
+        double v[NT] = {}, v2[ADV_SECOND] = {}, w[ADV_SUMS2] = {}, w2[1] = {};
+        if (pair) {
+            rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pqj_);
+            rec_vel(cd.rec, j, uxj, uyj, uzj, hj);
+            const double visj = viscosity2(pr, ptypej) + vis_tj * rhoj;
+            const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+            const double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+            const double tdwx = tdwij * dx / tdist;
+            const double tdwy = tdwij * dy / tdist;
+            const double tdwz = tdwij * dz / tdist;
+            const double dux = uxi - uxj, duy = uyi - uyj, duz = uzi - uzj;   // u_i - u_j
+            double tempj = 0.0, concnj = 0.0;
+            if (con_solve || concn_solve || boussinesq_solve) rec_scalar(cd.rec, j, tempj, concnj);
+            if (fv == SPH_FV_CLEARY) {
+                double C_v = dx * tdwx + dy * tdwy + dz * tdwz;
+                C_v *= (visi * visj) / (visi + visj);
+                C_v *= 4.0 * (mj / (rhoi * rhoj));
+                C_v /= tdist;
+                C_v /= tdist;
+                v[0] = C_v * dux; v[1] = C_v * duy; v[2] = C_v * duz;
+            } else if (fv == SPH_FV_MONAGHAN) {
+                double uij_xij = dux * dx + duy * dy + duz * dz;
+                double phi_ij = uij_xij;
+                phi_ij /= (tdist * tdist + 0.01 * hi * hi);
+                double P_ij = -2.0 * (3 + 2.0) * phi_ij * mj / rhoj;
+                double C_v = 2.0 * (visi * visj) / (visi + visj - 1e-20);
+                double nui = C_v / rhoi;
+                P_ij *= nui;
+                if (ptypei <= 0 || ptypei >= 1000) P_ij = 0;
+                if (ptypej <= 0 || ptypei >= 1000) P_ij = 0;
+                v[0] = -(P_ij)*tdwx; v[1] = -(P_ij)*tdwy; v[2] = -(P_ij)*tdwz;
+            }
+            if (eli < 1.0) {
+                const double vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
+                v[3] = (uxi * vx * tdwx + uyi * vx * tdwy + uzi * vx * tdwz) * mj / rhoj * ome;
+                v[4] = (uxi * vy * tdwx + uyi * vy * tdwy + uzi * vy * tdwz) * mj / rhoj * ome;
+                v[5] = (uxi * vz * tdwx + uyi * vz * tdwy + uzi * vz * tdwz) * mj / rhoj * ome;
+                if constexpr (SCAL) {
+                    if (con_solve)
+                        v[7] = -(2.0 * mj / (rhoi + rhoj) * (tempj - tempi) * (dux * tdwx + duy * tdwy + duz * tdwz) * ome);
+                    if (concn_solve) {
+                        const double dc = concnj - concni;
+                        w[0] = -((uxi * dc * tdwx + uyi * dc * tdwy + uzi * dc * tdwz) * mj / rhoj * ome);
+                    }
+                }
+            }
+            if constexpr (SCAL) {
+                if (con_solve) {
+                    double kcj = pr.solid_k * (ptypej == 0 || ptypej == 1000) + pr.air_k * (ptypej == 1 || ptypej == -1);
+                    double rhoj_temp = (ptypej == 1 || ptypej == -1) ? rhoj : pr.solid_rho;
+                    double mj_temp = mj * rhoj_temp / rhoj;
+                    double sum_con_H = 4.0 * mj_temp * kcj * kci * (tempi - tempj) * tdwij;
+                    sum_con_H /= (tdist + 1e-10) * rhoi * rhoj_temp * (kci + kcj);
+                    v[6] = sum_con_H;
+                }
+                if (concn_solve) {
+                    double diffj = pr.diff_coef;
+                    double tmprd = mi * (diffi * rhoi + diffj * rhoj);
+                    tmprd *= (dx * tdwx + dy * tdwy + dz * tdwz);
+                    tmprd /= (rhoi * rhoj * (tdist * tdist + 0.01 * hi * hi));
+                    w2[0] = tmprd * (concni - concnj) * (double)(ptypei == ptypej);
+                }
+                if (boussinesq_solve) {
+                    const double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
+                    w[1] = (mj / rhoj) * tempj * twij;
+                    w[2] = (mj / rhoj) * twij;
+                }
+            }
+            if (art) {
+                double uij_xij = dux * dx + duy * dy + duz * dz;
+                if (uij_xij < 0) {
+                    double h_ij = (hi + hj) * 0.5;
+                    double phi_ij = h_ij * uij_xij;
+                    phi_ij /= (tdist * tdist + 0.01 * h_ij * h_ij);
+                    double P_ij = mi * phi_ij * (-Alpha * soundspeed + Beta * phi_ij);
+                    P_ij /= (rhoi + rhoj);
+                    P_ij *= 0.5;
+                    v2[0] = -(P_ij)*tdwx; v2[1] = -(P_ij)*tdwy; v2[2] = -(P_ij)*tdwz;
+                }
             }
         }
-        if (con_solve) {
-            double kcj = pr.solid_k * (ptypej == 0 || ptypej == 1000) + pr.air_k * (ptypej == 1 || ptypej == -1);
-            double rhoj_temp = (ptypej == 1 || ptypej == -1) ? rhoj : pr.solid_rho;
-            double mj_temp = mj * rhoj_temp / rhoj;
-            double sum_con_H = 4.0 * mj_temp * kcj * kci * (tempi - tempj) * tdwij;
-            sum_con_H /= (tdist + 1e-10) * rhoi * rhoj_temp * (kci + kcj);
-            a.rc += sum_con_H;
-        }
-        if (concn_solve) {
-            double diffj = pr.diff_coef;
-            double tmprd = mi * (diffi * rhoi + diffj * rhoj);
-            tmprd *= (dx * tdwx + dy * tdwy + dz * tdwz);
-            tmprd /= (rhoi * rhoj * (tdist * tdist + 0.01 * hi * hi));
-            double tmprd1 = tmprd * (concni - concnj) * (double)(ptypei == ptypej);
-            a.rd += tmprd1;
-        }
-        if (boussinesq_solve) {
-            a.temp += (mj / rhoj) * tempj * twij;
-            a.flt += (mj / rhoj) * twij;
-        }
-        if (pr.artificial_viscosity) {
-            double uij_xij = dux * dx + duy * dy + duz * dz;
-            if (uij_xij < 0) {
-                double h_ij = (hi + hj) * 0.5;
-                double phi_ij = h_ij * uij_xij;
-                phi_ij /= (tdist * tdist + 0.01 * h_ij * h_ij);
-                double P_ij = mi * phi_ij * (-Alpha * soundspeed + Beta * phi_ij);
-                P_ij /= (rhoi + rhoj);
-                P_ij *= 0.5;
-                a.tx += -(P_ij)*tdwx; a.ty += -(P_ij)*tdwy; a.tz += -(P_ij)*tdwz;
-            }
-        }
+        sums.template add<ADV_SECOND>(v, v2, art);
+        if (SCAL && (concn_solve || boussinesq_solve)) sums2.template add<1>(w, w2, true);
     }
-    advection_store(cd, i, a, con_solve, concn_solve, boussinesq_solve, cpi);
+    AdvSums a;
+    a.tx = sums.sum(0); a.ty = sums.sum(1); a.tz = sums.sum(2);
+    a.cx = sums.sum(3); a.cy = sums.sum(4); a.cz = sums.sum(5);
+    if constexpr (SCAL) {
+        a.rc = sums.sum(6); a.ct = sums.sum(7);
+        a.rd = sums2.sum(0); a.temp = sums2.sum(1); a.flt = sums2.sum(2);
+    }
+    if (g_ == 0) advection_store(cd, i, a, con_solve, concn_solve, boussinesq_solve, cpi);
 }
 
 // MIXED (see prep_sums)
@@ -1357,55 +1380,50 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_periodic(Seg sg, int which) {
 
 // ------------------------------------------------------------------------
 // KERNEL_freeslip_boundary3D, functions_BC.cuh:1156-1271
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_freeslip(Seg sg, int which) {
-    SEG_PARTICLE(sg);
+constexpr int FS_SUMS = 6;
+__global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip(Seg sg, int which) {
+    __shared__ double lds[WAVE_BLOCK / 64][ord_doubles(FS_SUMS)];
+    SEG_BOUNDARY(sg);
     const KConst kc = cd.kc;
     const PView A = which ? cd.P : cd.S;
-    const NList nl = cd.nl;
     if (A.p_type[i] != -1) return;
-    R hi = (R)A.h[i];
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    double xg = A.x[i], yg = A.y[i], zg = A.z[i];
-    double tux = 0, tuy = 0, tuz = 0, tpres = 0, ttemp = 0, tflt_s = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_HM)) continue;
-        int j = e & NB_IDX;
+    const double hi = A.h[i], tmp_A = calc_tmpA<double>(kc, hi);
+    const double xg = A.x[i], yg = A.y[i], zg = A.z[i];
+    OrderedSums<FS_SUMS, BLANES> sums(lds[threadIdx.x >> 6]);
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = lane; k - lane < row.cnt; k += BLANES) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        double v[FS_SUMS] = {};
         // fluid neighbours only (the reference weights the others by an
         // exact 0, which leaves the sums unchanged)
-        if (A.p_type[j] != 1) continue;
-        R dx = (R)(xg - A.x[j]), dy = (R)(yg - A.y[j]), dz = (R)(zg - A.z[j]);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-        R mj = (R)A.m[j], rhoj = (R)A.rho[j];
-        R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-        tux += (double)((R)A.ux[j] * (mj / rhoj) * twij);
-        tuy += (double)((R)A.uy[j] * (mj / rhoj) * twij);
-        tuz += (double)((R)A.uz[j] * (mj / rhoj) * twij);
-        tpres += (double)((R)A.pres[j] * (mj / rhoj) * twij);
-        ttemp += (double)((R)A.temp[j] * (mj / rhoj) * twij);
-        tflt_s += (double)((mj / rhoj) * twij);
+        if ((e & F_HM) && A.p_type[j] == 1) {
+            const double dx = xg - A.x[j], dy = yg - A.y[j], dz = zg - A.z[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
+            const double mj = A.m[j], rhoj = A.rho[j];
+            const double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
+            v[0] = A.ux[j] * (mj / rhoj) * twij;
+            v[1] = A.uy[j] * (mj / rhoj) * twij;
+            v[2] = A.uz[j] * (mj / rhoj) * twij;
+            v[3] = A.pres[j] * (mj / rhoj) * twij;
+            v[4] = A.temp[j] * (mj / rhoj) * twij;
+            v[5] = (mj / rhoj) * twij;
+        }
+        sums.add(v);
     }
-    if (tflt_s > 1e-5) {
-        A.ux[i] = tux / tflt_s; A.uy[i] = tuy / tflt_s; A.uz[i] = tuz / tflt_s;
-        A.pres[i] = tpres / tflt_s; A.temp[i] = ttemp / tflt_s;
+    double t[FS_SUMS];
+    for (int a = 0; a < FS_SUMS; a++) t[a] = sums.sum(a);
+    if (lane != 0) return;
+    if (t[5] > 1e-5) {
+        A.ux[i] = t[0] / t[5]; A.uy[i] = t[1] / t[5]; A.uz[i] = t[2] / t[5];
+        A.pres[i] = t[3] / t[5]; A.temp[i] = t[4] / t[5];
     }
 }
 
-// The same sums in MIXED with a 64-lane wave per boundary particle (the
-// lid's particles are a few per cent of the case, one thread each left
-// the device nearly idle): lane l adds entries l, l + 64, ... of the list,
-// then a fixed butterfly adds the lane sums, so a case gives the same bits
-// alone and in a batch.
-__global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_wave(Seg sg, int which) {
-    int first_;
-    const int cid_ = seg_case(sg, first_);
-    const CaseDesc& cd = sg.cd[cid_];
-    const int u = (first_ + (int)threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (u >= cd.nm_count) return;
+// The same sums in MIXED (see k_boundary3d_mixed)
+__global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_mixed(Seg sg, int which) {
+    SEG_BOUNDARY(sg);
     const PView A = which ? cd.P : cd.S;
-    const int i = cd.nm_list[u];
     if (A.p_type[i] != -1) return;
     const KConst kc = cd.kc;
     const NList nl = cd.nl;
@@ -1415,7 +1433,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_wave(Seg sg, int which)
     double xg = A.x[i], yg = A.y[i], zg = A.z[i];
     double t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
-    for (int k = lane; k < row.cnt; k += 64) {
+    for (int k = lane; k < row.cnt; k += BLANES) {
         unsigned e = NB_AT(row, k);
         if (!(e & F_HM)) continue;
         int j = e & NB_IDX;
@@ -1432,8 +1450,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_wave(Seg sg, int which)
         t[4] += (double)((float)A.temp[j] * vj * w);
         t[5] += (double)(vj * w);
     }
-    for (int off = 32; off > 0; off >>= 1)
-        for (int q = 0; q < 6; q++) t[q] += __shfl_xor(t[q], off, 64);
+    for (double& v : t) group_fold<BLANES>(v);
     if (lane != 0) return;
     if (t[5] > 1e-5) {
         A.ux[i] = t[0] / t[5]; A.uy[i] = t[1] / t[5]; A.uz[i] = t[2] / t[5];
@@ -1487,44 +1504,48 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_outlet(Seg sg, int which) {
 __device__ __forceinline__ bool pressure_row(const PView& S, int i) {
     return S.i_type[i] <= 2 && S.p_type[i] < 1000 && S.p_type[i] > 0 && S.buffer_type[i] == 0;
 }
+constexpr int PF_SUMS = 3;
 __global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force(Seg sg) {
-    SEG_PARTICLE_LIGHT(sg);
+    ORDERED_LDS(PF_SUMS, 0);
+    SEG_GROUP_LIGHT(sg);
     const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
     const PView S = cd.S;
     const QView Q = cd.Q;
     if (!pressure_row(S, i)) return;
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double hi = S.h[i];
-    double pi = S.pres[i] - S.pres0[i], rhoi = S.rho[i];
-    double tmpx = 0, tmpy = 0, tmpz = 0;
+    const bool on = cd.pr.fp_solve != 0;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double hi = S.h[i];
+    const double pi = S.pres[i] - S.pres0[i], rhoi = S.rho[i];
     // the pair's kernel normalisation and derivative factor depend only on
-    // h_ij: kept while consecutive pairs share it
+    // h_ij: kept while a lane's consecutive pairs share it
     double h_c = -1, A_c = 0, f_c = 0;
+    OrderedSums<PF_SUMS, GROUP> sums(wlds_);
     const NLRow row = nl_row(cd.nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_DM)) continue;
-        int j = e & NB_IDX;
-        if (S.p_type[j] >= 1000) continue;
-        double hj, pj, xj, yj, zj, mj, rhoj;
-        rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pj);
-        hj = ld_d2(rec_at(cd.rec, j, 4)).y;
-        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
-        double hij = 0.5 * (hi + hj);
-        if (hij != h_c) { h_c = hij; A_c = calc_tmpA<double>(kc, hij); f_c = dw_factor<double>(kc, hij); }
-        double tdwij = kernel_dw_f<double>(kc, A_c, hij, f_c, tdist);
-        double tdwx = tdwij * dx / tdist;
-        double tdwy = tdwij * dy / tdist;
-        double tdwz = tdwij * dz / tdist;
-        if (pr.fp_solve) {
+    for (int k = g_; k - g_ < row.cnt && on; k += GROUP) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        const bool pair = (e & F_DM) && S.p_type[j] < 1000;
+        if (!__any(pair)) continue;
+        double v[PF_SUMS] = {};
+        if (pair) {
+            double hj, pj, xj, yj, zj, mj, rhoj;
+            rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pj);
+            hj = ld_d2(rec_at(cd.rec, j, 4)).y;
+            const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
+            const double hij = 0.5 * (hi + hj);
+            if (hij != h_c) { h_c = hij; A_c = calc_tmpA<double>(kc, hij); f_c = dw_factor<double>(kc, hij); }
+            const double tdwij = kernel_dw_f<double>(kc, A_c, hij, f_c, tdist);
             const double Pb = 0.0;
-            double C_p = -2.0 * mj / (rhoi * rhoj) * ((pi + Pb) * rhoj + (pj + Pb) * rhoi) / (rhoi + rhoj);
-            tmpx += C_p * tdwx; tmpy += C_p * tdwy; tmpz += C_p * tdwz;
+            const double C_p = -2.0 * mj / (rhoi * rhoj) * ((pi + Pb) * rhoj + (pj + Pb) * rhoi) / (rhoi + rhoj);
+            v[0] = C_p * (tdwij * dx / tdist);
+            v[1] = C_p * (tdwij * dy / tdist);
+            v[2] = C_p * (tdwij * dz / tdist);
         }
+        sums.add(v);
     }
-    Q.fpx[i] = tmpx; Q.fpy[i] = tmpy; Q.fpz[i] = tmpz;
+    const double tx = sums.sum(0), ty = sums.sum(1), tz = sums.sum(2);
+    if (g_ == 0) { Q.fpx[i] = tx; Q.fpy[i] = ty; Q.fpz[i] = tz; }
 }
 
 // MIXED (see prep_sums)
@@ -1621,92 +1642,12 @@ __global__ void __launch_bounds__(TILE_THREADS) k_pressure_force_tile(Seg sg, in
 
 // ------------------------------------------------------------------------
 // IBM_force_interpolation3D, functions_IBM.cuh:342-490
-template <class R>
-__global__ void __launch_bounds__(MAX_BLOCK) k_ibm_force(Seg sg) {
-    SEG_PARTICLE(sg);
-    const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
+// the force from the interpolated velocity's sums
+__device__ __forceinline__ void ibm_force_store(const CaseDesc& cd, int i, const double (&t)[4]) {
+    const sph_params& pr = cd.pr;
     const PView S = cd.S;
     const QView Q = cd.Q;
-    const NList nl = cd.nl;
-    const double dt = cd.dt;
-    if (S.p_type[i] < 1000) return;
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    R tmp_h = (R)(0.5 * S.h[i]);
-    R tmp_A = calc_tmpA<R>(kc, tmp_h);
-    double tmpux = 0, tmpuy = 0, tmpuz = 0, filt = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_BH)) continue;
-        int j = e & NB_IDX;
-        if (S.i_type[j] == 4 || S.p_type[j] != 1) continue;
-        R dx = (R)(xi - S.x[j]), dy = (R)(yi - S.y[j]), dz = (R)(zi - S.z[j]);
-        R tdist = sqrt(dx * dx + dy * dy + dz * dz) + (R)1e-20;
-        R twij = kernel_w<R>(kc, tmp_A, tmp_h, tdist);
-        R tmprho = (R)S.m[j] / (R)S.rho[j];
-        tmpux += (double)(((R)S.ux[j]) * tmprho * twij);
-        tmpuy += (double)(((R)S.uy[j]) * tmprho * twij);
-        tmpuz += (double)(((R)S.uz[j]) * tmprho * twij);
-        filt += (double)(tmprho * twij);
-    }
-    S.concentration[i] = filt;
-    double ufx = tmpux / (filt + 1e-10), ufy = tmpuy / (filt + 1e-10), ufz = tmpuz / (filt + 1e-10);
-    double nx = Q.nx[i], ny = Q.ny[i], nz = Q.nz[i];
-    double nmag = sqrt(nx * nx + ny * ny + nz * nz) + 1e-20;
-    nx = nx / nmag; ny = ny / nmag; nz = nz / nmag;
-    double un = ufx * nx + ufy * ny + ufz * nz;
-    double utx = ufx - un * nx, uty = ufy - un * ny, utz = ufz - un * nz;
-    double Ubtx = pr.ibm_ut_factor * interp_ux_caseH(zi, 1.0);
-    double Ubty = 0.0, Ubtz = 0.0;
-    double beta_t = 1.0;
-    double corrx = (-un) * nx + beta_t * (Ubtx - utx);
-    double corry = (-un) * ny + beta_t * (Ubty - uty);
-    double corrz = (-un) * nz + beta_t * (Ubtz - utz);
-    S.fbx[i] = pr.rho_air * corrx / dt;
-    S.fby[i] = pr.rho_air * corry / dt;
-    S.fbz[i] = pr.rho_air * corrz / dt;
-}
-
-// The marker force in MIXED, a 64-lane wave per marker (markers are in the
-// boundary list): lane sums over entries lane, lane + 64, ..., then a fixed
-// butterfly; lane 0 forms the force from the sums as the serial kernel does.
-__global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_wave(Seg sg) {
-    int first_;
-    const int cid_ = seg_case(sg, first_);
-    const CaseDesc& cd = sg.cd[cid_];
-    const int u = (first_ + (int)threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (u >= cd.nm_count) return;
-    const PView S = cd.S;
-    const int i = cd.nm_list[u];
-    if (S.p_type[i] < 1000) return;
-    const KConst kc = cd.kc;
-    const sph_params pr = cd.pr;
-    const QView Q = cd.Q;
-    const NList nl = cd.nl;
-    const double dt = cd.dt;
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    const float tmp_h = (float)(0.5 * S.h[i]), tmp_A = calc_tmpA<float>(kc, tmp_h);
-    const HScale hs(kc, tmp_h);
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    const NLRow row = nl_row(nl, i);
-    for (int k = lane; k < row.cnt; k += 64) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_BH)) continue;
-        int j = e & NB_IDX;
-        if (S.i_type[j] == 4 || S.p_type[j] != 1) continue;
-        float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
-        const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
-        const float tmprho = (float)S.m[j] / (float)S.rho[j];
-        t[0] += (double)((float)S.ux[j] * tmprho * w);
-        t[1] += (double)((float)S.uy[j] * tmprho * w);
-        t[2] += (double)((float)S.uz[j] * tmprho * w);
-        t[3] += (double)(tmprho * w);
-    }
-    for (int off = 32; off > 0; off >>= 1)
-        for (int q = 0; q < 4; q++) t[q] += __shfl_xor(t[q], off, 64);
-    if (lane != 0) return;
-    const double filt = t[3];
+    const double dt = cd.dt, zi = S.z[i], filt = t[3];
     S.concentration[i] = filt;
     double ufx = t[0] / (filt + 1e-10), ufy = t[1] / (filt + 1e-10), ufz = t[2] / (filt + 1e-10);
     double nx = Q.nx[i], ny = Q.ny[i], nz = Q.nz[i];
@@ -1724,6 +1665,65 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_wave(Seg sg) {
     S.fby[i] = pr.rho_air * corry / dt;
     S.fbz[i] = pr.rho_air * corrz / dt;
 }
+__global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force(Seg sg) {
+    __shared__ double lds[WAVE_BLOCK / 64][ord_doubles(4)];
+    SEG_BOUNDARY(sg);
+    const KConst kc = cd.kc;
+    const PView S = cd.S;
+    if (S.p_type[i] < 1000) return;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double tmp_h = 0.5 * S.h[i], tmp_A = calc_tmpA<double>(kc, tmp_h);
+    OrderedSums<4, BLANES> sums(lds[threadIdx.x >> 6]);
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = lane; k - lane < row.cnt; k += BLANES) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        double v[4] = {};
+        if ((e & F_BH) && S.i_type[j] != 4 && S.p_type[j] == 1) {
+            const double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+            const double twij = kernel_w<double>(kc, tmp_A, tmp_h, tdist);
+            const double tmprho = S.m[j] / S.rho[j];
+            v[0] = S.ux[j] * tmprho * twij;
+            v[1] = S.uy[j] * tmprho * twij;
+            v[2] = S.uz[j] * tmprho * twij;
+            v[3] = tmprho * twij;
+        }
+        sums.add(v);
+    }
+    double t[4];
+    for (int a = 0; a < 4; a++) t[a] = sums.sum(a);
+    if (lane == 0) ibm_force_store(cd, i, t);
+}
+
+// The marker force in MIXED (see k_boundary3d_mixed)
+__global__ void __launch_bounds__(WAVE_BLOCK) k_ibm_force_mixed(Seg sg) {
+    SEG_BOUNDARY(sg);
+    const PView S = cd.S;
+    if (S.p_type[i] < 1000) return;
+    const KConst kc = cd.kc;
+    const NList nl = cd.nl;
+    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const float tmp_h = (float)(0.5 * S.h[i]), tmp_A = calc_tmpA<float>(kc, tmp_h);
+    const HScale hs(kc, tmp_h);
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    const NLRow row = nl_row(nl, i);
+    for (int k = lane; k < row.cnt; k += BLANES) {
+        unsigned e = NB_AT(row, k);
+        if (!(e & F_BH)) continue;
+        int j = e & NB_IDX;
+        if (S.i_type[j] == 4 || S.p_type[j] != 1) continue;
+        float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
+        const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
+        const float tmprho = (float)S.m[j] / (float)S.rho[j];
+        t[0] += (double)((float)S.ux[j] * tmprho * w);
+        t[1] += (double)((float)S.uy[j] * tmprho * w);
+        t[2] += (double)((float)S.uz[j] * tmprho * w);
+        t[3] += (double)(tmprho * w);
+    }
+    for (double& v : t) group_fold<BLANES>(v);
+    if (lane == 0) ibm_force_store(cd, i, t);
+}
 
 // IBM_spreading_interpolation3D, functions_IBM.cuh:492-613
 __device__ __forceinline__ void ibm_spread_store(const PView& S, int i, double fb_x, double fb_y, double fb_z,
@@ -1738,36 +1738,40 @@ __device__ __forceinline__ void ibm_spread_store(const PView& S, int i, double f
     S.concentration[i] = filt;
 }
 __global__ void __launch_bounds__(MAX_BLOCK) k_ibm_spread(Seg sg) {
-    SEG_PARTICLE(sg);
+    ORDERED_LDS(4, 0);
+    SEG_GROUP(sg);
     const KConst kc = cd.kc;
     const PView S = cd.S;
-    const NList nl = cd.nl;
     if (S.p_type[i] != 1) return;
     if (S.buffer_type[i] == 2) return;
     if (cd.ibm_near && !cd.ibm_near[i]) {   // no marker in the list: what the sums below give
-        ibm_spread_store(S, i, 0.0, 0.0, 0.0, 0.0);
+        if (g_ == 0) ibm_spread_store(S, i, 0.0, 0.0, 0.0, 0.0);
         return;
     }
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double tmp_h = 0.5 * S.h[i];
-    double tmp_A = calc_tmpA<double>(kc, tmp_h);
-    double filt = 0, fb_x = 0, fb_y = 0, fb_z = 0;
-    NLRow row = nl_row(nl, i);
-    for (int k = 0; k < row.cnt; k++) {
-        unsigned e = NB_AT(row, k);
-        if (!(e & F_BH)) continue;
-        int j = e & NB_IDX;
-        if (S.i_type[j] == 4 || S.p_type[j] != 1000) continue;
-        double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-        double twij = kernel_w<double>(kc, tmp_A, tmp_h, tdist);
-        double tmprho = S.m[j] / S.rho[j];
-        fb_x += S.fbx[j] * twij * tmprho;
-        fb_y += S.fby[j] * twij * tmprho;
-        fb_z += S.fbz[j] * twij * tmprho;
-        filt += tmprho * twij;
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double tmp_h = 0.5 * S.h[i], tmp_A = calc_tmpA<double>(kc, tmp_h);
+    OrderedSums<4, GROUP> sums(wlds_);
+    const NLRow row = nl_row(cd.nl, i);
+    for (int k = g_; k - g_ < row.cnt; k += GROUP) {
+        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+        const int j = e & NB_IDX;
+        const bool pair = (e & F_BH) && S.i_type[j] != 4 && S.p_type[j] == 1000;
+        if (!__any(pair)) continue;
+        double v[4] = {};
+        if (pair) {
+            const double dx = xi - S.x[j], dy = yi - S.y[j], dz = zi - S.z[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+            const double twij = kernel_w<double>(kc, tmp_A, tmp_h, tdist);
+            const double tmprho = S.m[j] / S.rho[j];
+            v[0] = S.fbx[j] * twij * tmprho;
+            v[1] = S.fby[j] * twij * tmprho;
+            v[2] = S.fbz[j] * twij * tmprho;
+            v[3] = tmprho * twij;
+        }
+        sums.add(v);
     }
-    ibm_spread_store(S, i, fb_x, fb_y, fb_z, filt);
+    const double fx = sums.sum(0), fy = sums.sum(1), fz = sums.sum(2), filt = sums.sum(3);
+    if (g_ == 0) ibm_spread_store(S, i, fx, fy, fz, filt);
 }
 // MIXED: GROUP lanes a particle, the pair arithmetic in float, the sums in
 // double
@@ -1906,10 +1910,10 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
 // launch over the particles of every case; tunable passes (kid >= 0) run at
 // the workgroup size the autotuner picked for this batch size
 // a boundary pass with a 64-lane wave per boundary particle of each case
-#define WAVEL(name, kern, ...)                                                                        \
+#define BOUNDL(name, kern, ...)                                                                        \
     do {                                                                                            \
         Shape sh_;                                                                                  \
-        SPH_TRY(shape(e, 3, WAVE_BLOCK, &sh_));                                                     \
+        SPH_TRY(shape(e, 3, WAVE_BLOCK * (64 / BLANES), &sh_));                                                     \
         if (sh_.grid > 0) {                                                                         \
             SPH_TRY(prof_begin(e, name, 0.0));                                                      \
             hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(WAVE_BLOCK), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
@@ -1945,7 +1949,9 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
         }                                                                                           \
     } while (0)
 // the same with GROUP lanes a particle
-#define SEGG(name, kid, kern, ...)                                                                   \
+// (SEGO: FP64, with the LDS of nd doubles a wave for ordered sums)
+#define SEGG(name, kid, kern, ...) SEGO(name, kid, 0, kern, ##__VA_ARGS__)
+#define SEGO(name, kid, nd, kern, ...)                                                                   \
     do {                                                                                            \
         const int blk_ = tuned_block(e, (kid));                                                     \
         Shape sh_;                                                                                  \
@@ -1953,7 +1959,7 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
         if (sh_.grid > 0) {                                                                         \
             SPH_TRY(prof_begin(e, name, 0.0));                                                      \
             SPH_TRY(tune_begin(e, (kid), blk_));                                                    \
-            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(blk_), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
+            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(blk_), (size_t)(blk_ / 64) * (nd) * sizeof(double), e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
             SPH_TRY(launch_check(&e, name));                                                        \
             SPH_TRY(tune_end(e));                                                                   \
             SPH_TRY(prof_end(e));                                                                   \
@@ -2133,8 +2139,8 @@ static int run_periodic(Eng& e, int which) {
     return 0;
 }
 static int run_freeslip(Eng& e, int which) {
-    if (mixed_of(e)) WAVEL("freeslip", k_freeslip_wave, which);   // the lid's particles among the boundary ones
-    else SEGL("freeslip", TK_FREESLIP, k_freeslip<double>, which);
+    if (mixed_of(e)) BOUNDL("freeslip", k_freeslip_mixed, which);   // the lid's particles among the boundary ones
+    else BOUNDL("freeslip", k_freeslip, which);
     return 0;
 }
 
@@ -2226,16 +2232,16 @@ int step_physics_front(Eng& e) {
     for (size_t k = 0; k < e.cs.size(); k++) any_gc |= !e.h_desc[k].gc_fresh;
     if (any_gc) {
         if (mixed) SEGG("grad_corr", TK_GRAD_CORR, k_grad_corr_mixed);
-        else SEGL("grad_corr", TK_GRAD_CORR, k_grad_corr);
+        else SEGO("grad_corr", TK_GRAD_CORR, ord_doubles(GC_SUMS), k_grad_corr);
     }
     SPH_TRY(pack_records(e, REC_PRE));   // compact records for the strain pass
     if (mixed && e.tile_lanes) TILEL("prep", k_prep_tile, CREC_ADV_FLOATS);
     else if (mixed) {
         SEGG("prep", TK_PREP, k_prep_mixed);
         HEAVYL("prep_heavy", k_prep_heavy);
-    } else SEGL("prep", TK_PREP, k_prep);
-    if (mixed) WAVEL("boundary3d", k_boundary3d_wave);
-    else SEGL("boundary3d", TK_BOUNDARY, k_boundary3d<double>);
+    } else SEGO("prep", TK_PREP, ord_doubles(PREP_SUMS), k_prep);
+    if (mixed) BOUNDL("boundary3d", k_boundary3d_mixed);
+    else BOUNDL("boundary3d", k_boundary3d);
     SEGL("most_self", -1, k_most_self);
     SEGL("most_deposit", -1, k_most_deposit);
     if (any_count0) SPH_TRY(run_neumann(e, 0, 1));
@@ -2254,8 +2260,8 @@ int step_physics_front(Eng& e) {
             HEAVYL("advection_heavy", k_advection_heavy<false>);
         }
     } else {
-        if (scal) SEGL("advection", TK_ADVECTION, k_advection<true>);
-        else SEGL("advection", TK_ADVECTION, k_advection<false>);
+        if (scal) SEGO("advection", TK_ADVECTION, ord_doubles(adv_sums<true>(), ADV_SECOND), k_advection<true>);
+        else SEGO("advection", TK_ADVECTION, ord_doubles(adv_sums<false>(), ADV_SECOND), k_advection<false>);
     }
     SEGL("projection", -1, k_projection);
     SPH_TRY(run_periodic(e, 0));
@@ -2274,11 +2280,11 @@ int step_physics_back(Eng& e) {
         SEGG("pressure_force", TK_PRESSURE, k_pressure_force_mixed);
         HEAVYL("pressure_force_heavy", k_pressure_force_heavy);
     }
-    else SEGL("pressure_force", TK_PRESSURE, k_pressure_force);
-    if (mixed) WAVEL("ibm_force", k_ibm_force_wave);
-    else SEGL("ibm_force", TK_IBM_FORCE, k_ibm_force<double>);
+    else SEGO("pressure_force", TK_PRESSURE, ord_doubles(PF_SUMS), k_pressure_force);
+    if (mixed) BOUNDL("ibm_force", k_ibm_force_mixed);
+    else BOUNDL("ibm_force", k_ibm_force);
     if (mixed) SEGG("ibm_spread", TK_IBM_SPREAD, k_ibm_spread_mixed);
-    else SEGL("ibm_spread", TK_IBM_SPREAD, k_ibm_spread);
+    else SEGO("ibm_spread", TK_IBM_SPREAD, ord_doubles(4), k_ibm_spread);
     SEGL("time_update", -1, k_time_update);
     SPH_TRY(run_neumann(e, 1, 0));
     SPH_TRY(run_outlet(e, 1));

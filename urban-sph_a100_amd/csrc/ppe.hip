@@ -694,78 +694,93 @@ __device__ __forceinline__ void assemble_store(const CaseDesc& cd, int i, int r,
         pp.x[r] = S.pres[i] - S.pres0[i];
     }
 }
+// FP64: GROUP lanes a particle, the sums in list order; the slot of a value is
+// its rank among the row's entries, counted over the group.
+constexpr int ASM_SUMS = 6;   // b_x, b_y, b_z, A, Ap, kn
 __global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble(Seg sg, int jacobi) {
-    SEG_ROW(sg);
+    extern __shared__ double asm_lds[];
+    int first_;
+    const int cid_ = seg_case(sg, first_);
+    const CaseDesc& cd = sg.cd[cid_];
+    const int row = first_ + (int)threadIdx.x / GROUP, g = (int)threadIdx.x % GROUP;
     if (row >= cd.n) return;
-    const int i = cd.porder ? cd.porder[row] : row;   // this thread's particle
-    const PPEView pp = cd.ppe;
+    const int i = cd.porder ? cd.porder[row] : row;
+    const PPEView& pp = cd.ppe;
     const int r = pp.rowof[i];
     if (r < 0) return;
     const KConst kc = cd.kc;
     const PView S = cd.S;
     const QView Q = cd.Q;
-    const int* rowof = pp.rowof;
-    double hi = 1.0 * S.h[i];
-    double tmp_A = calc_tmpA<double>(kc, hi);
-    double xi = S.x[i], yi = S.y[i], zi = S.z[i];
-    double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
-    double rhoi = S.rho[i];
-    double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
-    double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
-    double bix = 0, biy = 0, biz = 0;
-    RowSums a;
+    const int* const rowof = pp.rowof;
+    const double hi = 1.0 * S.h[i], tmp_A = calc_tmpA<double>(kc, hi);
+    const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
+    const double uxi = S.ux[i], uyi = S.uy[i], uzi = S.uz[i];
+    const double rhoi = S.rho[i];
+    const double gc11 = Q.inv_xx[i], gc12 = Q.inv_xy[i], gc22 = Q.inv_yy[i];
+    const double gc23 = Q.inv_yz[i], gc31 = Q.inv_zx[i], gc33 = Q.inv_zz[i];
     const NLRow nr = nl_row(cd.nl, i);
     // with fixed particles the values of a search are written by its first
     // step only; later steps compute the right-hand side
-    double* out = (jacobi || cd.vals_fresh) ? nullptr : pp.vals64 + prow(pp.sl_off, r);
+    double* const out = (jacobi || cd.vals_fresh) ? nullptr : pp.vals64 + prow(pp.sl_off, r);
     const bool full = jacobi || out != nullptr;   // the coefficients of every pair are needed
+    const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);   // the group's first lane
     int slot = 0;
     const double* const rec = cd.rec;
-    for (int k = 0; k < nr.cnt; k++) {
-        unsigned e = NB_AT(nr, k);
-        if (!(e & F_DP)) continue;
-        int j = e & NB_IDX;
-        double xj, yj, zj, mj, rhoj, qj, uxj, uyj, uzj, vtj_, hj_;
+    OrderedSums<ASM_SUMS, GROUP> sums(asm_lds + (threadIdx.x >> 6) * ord_doubles(ASM_SUMS));
+    for (int k = g; k - g < nr.cnt; k += GROUP) {
+        const unsigned e = k < nr.cnt ? NB_AT(nr, k) : 0u;
+        const int j = e & NB_IDX;
+        bool pair = (e & F_DP) != 0, own = false;   // own: an entry of the row
+        double vtj_, hj_;
         int ptj, itj;
-        rec_aux(rec, j, vtj_, ptj, itj);
-        if (ptj >= 1000 || itj == 4) continue;
-        rec_pos(rec, j, xj, yj, zj, mj, rhoj, qj);
-        rec_vel(rec, j, uxj, uyj, uzj, hj_);
-        const bool jrow = rowof[j] >= 0;   // j is an unknown of the PPE
-        double dx = xi - xj, dy = yi - yj, dz = zi - zj;
-        double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
-        double tdwij = kernel_dwp<double>(kc, tmp_A, hi, tdist);
-        double tdwx = tdwij * dx / tdist;
-        double tdwy = tdwij * dy / tdist;
-        double tdwz = tdwij * dz / tdist;
-        double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
-        double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
-        double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
-        double hm = 2.0 * rhoi * rhoj / (rhoi + rhoj);
-        bix += mj / rhoj * (uxj - uxi) * tdwxc * hm;
-        biy += mj / rhoj * (uyj - uyi) * tdwyc * hm;
-        biz += mj / rhoj * (uzj - uzi) * tdwzc * hm;
-        auto coef = [&]() { return 2.0 * mj / rhoj * (dx * tdwxc + dy * tdwyc + dz * tdwzc) / tdist / tdist; };
-        if (full) {
-            double cc = coef();
-            a.A += cc;
-            if (jacobi) a.Ap += cc * qj;
-            if (j != i) {
-                if (jrow) {
-                    if (out) out[pslot(slot)] = cc;
-                    slot++;
-                } else {
-                    a.kn += cc * qj;
-                }
-            }
-        } else if (!jrow && j != i) {
-            // values and diagonal kept from the search's first step: only the
-            // known neighbours' share of the right-hand side needs the coefficient
-            a.kn += coef() * qj;
+        if (pair) {
+            rec_aux(rec, j, vtj_, ptj, itj);
+            pair = !(ptj >= 1000 || itj == 4);
         }
+        if (!__any(pair)) continue;
+        double v[ASM_SUMS] = {}, cc = 0.0;
+        if (pair) {
+            double xj, yj, zj, mj, rhoj, qj, uxj, uyj, uzj;
+            rec_pos(rec, j, xj, yj, zj, mj, rhoj, qj);
+            rec_vel(rec, j, uxj, uyj, uzj, hj_);
+            const bool jrow = rowof[j] >= 0;   // j is an unknown of the PPE
+            const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
+            const double tdwij = kernel_dwp<double>(kc, tmp_A, hi, tdist);
+            const double tdwx = tdwij * dx / tdist;
+            const double tdwy = tdwij * dy / tdist;
+            const double tdwz = tdwij * dz / tdist;
+            const double tdwxc = gc11 * tdwx + gc12 * tdwy + gc31 * tdwz;
+            const double tdwyc = gc12 * tdwx + gc22 * tdwy + gc23 * tdwz;
+            const double tdwzc = gc31 * tdwx + gc23 * tdwy + gc33 * tdwz;
+            const double hm = 2.0 * rhoi * rhoj / (rhoi + rhoj);
+            v[0] = mj / rhoj * (uxj - uxi) * tdwxc * hm;
+            v[1] = mj / rhoj * (uyj - uyi) * tdwyc * hm;
+            v[2] = mj / rhoj * (uzj - uzi) * tdwzc * hm;
+            // (values and diagonal kept from the search's first step: only the
+            // known neighbours' share of the right-hand side needs the coefficient)
+            if (full || (!jrow && j != i)) {
+                cc = 2.0 * mj / rhoj * (dx * tdwxc + dy * tdwyc + dz * tdwzc) / tdist / tdist;
+                if (full) {
+                    v[3] = cc;
+                    if (jacobi) v[4] = cc * qj;
+                }
+                if (j != i && !jrow) v[5] = cc * qj;
+                own = j != i && jrow;
+            }
+        }
+        if (out) {
+            const unsigned m = (unsigned)(__ballot(own) >> gbit) & ((1u << GROUP) - 1u);
+            if (own) out[pslot(slot + __popc(m & ((1u << g) - 1u)))] = cc;
+            slot += __popc(m);
+        }
+        sums.add(v);
     }
-    a.b = 1.0 * (bix + biy + biz + 0.0);
-    assemble_store(cd, i, r, a, out != nullptr, jacobi);
+    const double bx = sums.sum(0), by = sums.sum(1), bz = sums.sum(2);
+    RowSums a;
+    a.A = sums.sum(3); a.Ap = sums.sum(4); a.kn = sums.sum(5);
+    a.b = 1.0 * (bx + by + bz + 0.0);
+    if (g == 0) assemble_store(cd, i, r, a, out != nullptr, jacobi);
 }
 
 // MIXED: GROUP lanes a particle, the pair arithmetic in float, the sums in
@@ -1989,14 +2004,15 @@ int ppe_solve(Eng& e) {
     } else {
         const int blk = tuned_block(e, TK_ASSEMBLE);
         Shape sh;
-        SPH_TRY(shape(e, 0, mixed ? blk / GROUP : blk, &sh));   // over particles
+        SPH_TRY(shape(e, 0, blk / GROUP, &sh));   // over particles
         SPH_TRY(prof_begin(e, "ppe_assemble", asm_bytes));
         SPH_TRY(tune_begin(e, TK_ASSEMBLE, blk));
         if (mixed)
             hipLaunchKernelGGL(k_ppe_assemble_mixed, dim3(sh.grid), dim3(blk), 0, e.st, Seg{e.d_desc, sh.tab},
                                jacobi ? 1 : 0);
         else
-            hipLaunchKernelGGL(k_ppe_assemble, dim3(sh.grid), dim3(blk), 0, e.st,
+            hipLaunchKernelGGL(k_ppe_assemble, dim3(sh.grid), dim3(blk),
+                               (size_t)(blk / 64) * ord_doubles(ASM_SUMS) * sizeof(double), e.st,
                                Seg{e.d_desc, sh.tab}, jacobi ? 1 : 0);
         SPH_TRY(launch_check(&e, "ppe_assemble"));
         SPH_TRY(tune_end(e));

@@ -192,12 +192,6 @@ struct Seg {
 // The passes that give a boundary particle or a heavy list a 64-lane wave
 // run four waves (four particles) to a workgroup.  The waves share nothing.
 constexpr int WAVE_BLOCK = 256;
-// The lane sums of a wave added by a fixed butterfly (every lane gets the
-// total), so a particle's sums do not depend on the launch.
-__device__ __forceinline__ void wave_fold(double& v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-}
 // MIXED passes over the particles' lists: GROUP lanes a particle, lane g_
 // taking entries g_, g_ + GROUP, ... of its list, a fixed butterfly adding
 // the lanes' sums (so a case's results do not depend on the launch); the
@@ -216,6 +210,53 @@ __device__ __forceinline__ void group_fold(double& v) {
 #pragma unroll
     for (int o = W / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
 }
+// FP64 passes: W lanes a particle form the terms of W list entries at a time,
+// and lane a of the group then adds sum a's terms in list order, through LDS,
+// so every sum is bit for bit the one a serial walk of the list gives (a left
+// out entry adds +0.0, which changes no sum that began at a number other than
+// -0.0).  A thread a particle left small cases waiting on one serial chain of
+// gathers a particle.  Advection 216 -> 54 us on 20 k particles, 320 -> 220 on
+// 150 k, the same 1.43 ms on 1 M; assembly 165 -> 41, 249 -> 185, 1479 -> 1230.
+constexpr int ORD_PITCH = SLICE + 1;   // doubles from one sum's terms to the next: lanes read distinct banks
+// LDS doubles of a wave that adds NT sums, the first N2 of them two terms an entry
+constexpr int ord_doubles(int nt, int n2 = 0) { return (nt + n2) * ORD_PITCH; }
+template <int NT, int W>
+struct OrderedSums {
+    static_assert(NT <= W && SLICE % W == 0, "a lane a sum");
+    double* const t;   // this wave's terms
+    const int lane, first, g;
+    double acc;        // lane g < NT of the group: sum g
+    __device__ OrderedSums(double* wave_lds)
+        : t(wave_lds), lane((int)threadIdx.x & 63), first(lane & ~(W - 1)), g(lane & (W - 1)), acc(0.0) {}
+    // entry terms v (then, for the sums below N2 when two, v2) of this lane's entry
+    template <int N2 = 0>
+    __device__ __forceinline__ void add(const double (&v)[NT], const double* v2 = nullptr, bool two = false) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int a = 0; a < NT; a++) t[a * ORD_PITCH + lane] = v[a];
+        if (N2 && two) {
+#pragma unroll
+            for (int a = 0; a < N2; a++) t[(NT + a) * ORD_PITCH + lane] = v2[a];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (g < NT) {
+            const double* const r = t + g * ORD_PITCH + first;
+            if (N2 && two && g < N2) {
+#pragma unroll 8
+                for (int q = 0; q < W; q++) {
+                    acc += r[q];
+                    acc += r[q + NT * ORD_PITCH];
+                }
+            } else {
+#pragma unroll 16
+                for (int q = 0; q < W; q++) acc += r[q];
+            }
+        }
+    }
+    __device__ double sum(int a) const { return __shfl(acc, first + a, 64); }
+};
 // Workgroups are dispatched to the 8 XCDs round-robin (block b runs on XCD
 // b mod 8).  Logical block order is remapped so that each XCD works on one
 // contiguous range of blocks: neighbouring rows, whose gathers touch the
