@@ -601,6 +601,7 @@ static int step_body(Eng& e, sph_ctx* const* cases, int nc, const int* count, co
     // descriptors
     SPH_HIP(&e, hipEventSynchronize(e.up_ev));
     for (int k = 0; k < nc; k++) fill_desc(e, k, cases[k], count[k], dt[k], time[k]);
+    ppe_streams(e);
     SPH_HIP(&e, hipMemcpyAsync(e.d_desc, e.h_desc, sizeof(CaseDesc) * nc, hipMemcpyHostToDevice, e.st));
     SPH_HIP(&e, hipEventRecord(e.up_ev, e.st));
     // cell tiles: every case of the step has them, with one chunk width

@@ -736,8 +736,9 @@ struct MGLv {
 // sum_k (a_rk / d_r) x[col_k] over the compact level-0 operator, in entry
 // order, accumulated in double (row_sum)
 struct HTerm { unsigned short h; float x; };
-__device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int r, const float* x,
-                                           const int* wb) {
+template <bool NT>
+__device__ __forceinline__ double mg_row16_ld(const PPEView& pp, const MGLv& L, int r, const float* x,
+                                              const int* wb) {
     const unsigned* ev = L.ev;
     auto mac = [](double s, const HTerm& t) {
         return s + (double)(float)__builtin_bit_cast(_Float16, t.h) * (double)t.x;
@@ -752,16 +753,20 @@ __device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int
         const cmem<int> off = (cmem<int>)(L.hoff + hq);
         const gmem<float> xr = (gmem<float>)(x + r);
         return row_sum<HTerm, ROW_U>(
-            w, [&](int k) { return HTerm{__builtin_nontemporal_load(hp + pslot(k)), xr[off[k]]}; }, mac);
+            w, [&](int k) { return HTerm{ld_matrix<NT>(hp + pslot(k)), xr[off[k]]}; }, mac);
     }
     const unsigned* p = ev + prow(pp.sl_off, r);
     return row_sum<HTerm, ROW_U>(
         pp.cnt[r],
         [&](int k) {
-            const unsigned u = __builtin_nontemporal_load(p + pslot(k));
+            const unsigned u = ld_matrix<NT>(p + pslot(k));
             return HTerm{(unsigned short)(u >> 16), x[ecol(wb, (int)(u & 0xffffu))]};
         },
         mac);
+}
+__device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int r, const float* x,
+                                           const int* wb) {
+    return (pp.stream & STREAM_MG) ? mg_row16_ld<true>(pp, L, r, x, wb) : mg_row16_ld<false>(pp, L, r, x, wb);
 }
 
 // block -> (case, first row of the level); the block returns when the

@@ -1741,6 +1741,20 @@ PPEView ppe_view(const sph_ctx* c) {
     return v;
 }
 
+// Which operators of the step's cases are read past the caches (STREAM_*).
+void ppe_streams(Eng& e) {
+    double krylov = 0.0, mg = 0.0;
+    for (const sph_ctx* c : e.cs) {
+        const PPEState* P = c->ppe;
+        if (!P) continue;
+        const double cols = (double)(P->nnz - P->nnz_stencil);   // entries of a stored column
+        krylov += (double)P->nnz_slots * (c->prm.precision == SPH_MIXED ? 4.0 : 8.0) + cols * (P->ecols ? 2.0 : 4.0);
+        mg += (double)P->nnz_slots * 2.0 + cols * 2.0;
+    }
+    const int stream = (krylov > STREAM_BYTES ? STREAM_KRYLOV : 0) | (mg > STREAM_BYTES ? STREAM_MG : 0);
+    for (size_t k = 0; k < e.cs.size(); k++) e.h_desc[k].ppe.stream = stream;
+}
+
 static int nr_of(const sph_ctx* c) { return c->ppe ? c->ppe->nr : 0; }
 
 static int read_scalars(Eng& e) {
@@ -2036,6 +2050,7 @@ int ppe_solve(Eng& e) {
         if (any) {
             SPH_HIP(&e, hipEventSynchronize(e.up_ev));
             for (int k = 0; k < nc; k++) e.h_desc[k].ppe = ppe_view(e.cs[k]);
+            ppe_streams(e);
             SPH_HIP(&e, hipMemcpyAsync(e.d_desc, e.h_desc, sizeof(CaseDesc) * nc, hipMemcpyHostToDevice, e.st));
             SPH_HIP(&e, hipEventRecord(e.up_ev, e.st));
         }

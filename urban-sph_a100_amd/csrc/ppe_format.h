@@ -27,18 +27,18 @@ __host__ __device__ __forceinline__ long long pslot(int k) { return (long long)k
 
 // Off-diagonal part of one row, sum_k vals[k] * x[col[k]], accumulated in
 // double in entry order: ld(k) loads entry k's operands, mac(s, operands)
-// adds its term.  Matrix entries stream through once: nontemporal loads keep
-// the caches for the x gathers.  U entries' loads are issued before the
+// adds its term.  U entries' loads are issued before the
 // first of their terms is added, in the remainder too (entries past the
 // row's end reload the last one and add nothing): a small case has about
 // a wave a SIMD, and its product takes the number of such rounds times the
 // memory latency.  Measured with 4 (and a remainder entry by entry), 8, 16
-// and 24 entries a round, HIP events: float product 29.9, 21.4, 16.9, 16.0 us
-// on 20,609 particles and 137, 132, 131, 143 us on the 2.13 M canyon, whose
-// level-0 passes (half values) take 94, 83, 83, 104 us; double product (FP64,
-// 150 k canyon, bound by its bytes) 36.3, 36.9, 39.9, 43.5 us, 32^3 box 27.0,
-// 26.8, 25.5, 25.0 us.  Giving a row to four waves (an LDS sum) was slower from
-// 200 k particles on and no faster below.
+// and 24 entries a round, HIP events, operators read past the caches: float
+// product 29.9, 21.4, 16.9, 16.0 us on 20,609 particles and 137, 132, 131,
+// 143 us on the 2.13 M canyon, whose level-0 passes (half values) take 94, 83,
+// 83, 104 us; double product (150 k canyon) 36.3, 36.9, 39.9, 43.5 us, through
+// the caches with 8 and 16: 27.9, 30.9, and 21.3, 20.8 us on the 32^3 box.
+// Giving a row to four waves (an LDS sum) was slower from 200 k particles on
+// and no faster below.
 constexpr int ROW_U = 16;        // float and half values
 constexpr int ROW_U_F64 = 8;
 template <class T, int U, class LD, class MAC>
@@ -63,26 +63,26 @@ __device__ __forceinline__ double row_sum(int m, LD&& ld, MAC&& mac) {
 }
 template <class V, class X> struct Term { V v; X x; };
 template <class V> constexpr int row_u() { return sizeof(V) == 8 ? ROW_U_F64 : ROW_U; }
-template <class V, class X>
+template <class V, class X, bool NT>
 __device__ __forceinline__ double offdiag_i32(const int* cp, const V* vp, int m, const X* x) {
     return row_sum<Term<V, X>, row_u<V>()>(
         m,
         [&](int k) {
-            return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)), x[__builtin_nontemporal_load(cp + pslot(k))]};
+            return Term<V, X>{ld_matrix<NT>(vp + pslot(k)), x[ld_matrix<NT>(cp + pslot(k))]};
         },
         [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
 // The same over 16-bit columns: entry e = (group << EC_OFF_BITS) | offset,
 // column = wb[group] + offset, wb = the slice's group bases (in LDS).
 __device__ __forceinline__ int ecol(const int* wb, int e) { return wb[e >> EC_OFF_BITS] + (e & EC_OFF_MASK); }
-template <class V, class X>
+template <class V, class X, bool NT>
 __device__ __forceinline__ double offdiag_u16(const unsigned short* ep, const V* vp, int m, const int* wb,
                                               const X* x) {
     return row_sum<Term<V, X>, row_u<V>()>(
         m,
         [&](int k) {
-            return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)),
-                              x[ecol(wb, __builtin_nontemporal_load(ep + pslot(k)))]};
+            return Term<V, X>{ld_matrix<NT>(vp + pslot(k)),
+                              x[ecol(wb, ld_matrix<NT>(ep + pslot(k)))]};
         },
         [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
@@ -95,13 +95,13 @@ __device__ __forceinline__ double offdiag_u16(const unsigned short* ep, const V*
 // global address space.
 template <class T> using gmem = const __attribute__((address_space(1))) T*;
 template <class T> using cmem = const __attribute__((address_space(4))) T*;
-template <class V, class X>
+template <class V, class X, bool NT>
 __device__ __forceinline__ double offdiag_stencil(const V* vals, int m, const int* offs, int r, const X* xv) {
     const gmem<V> vp = (gmem<V>)vals;
     const gmem<X> x = (gmem<X>)(xv + r);
     const cmem<int> off = (cmem<int>)offs;
     return row_sum<Term<V, X>, row_u<V>()>(
-        m, [&](int k) { return Term<V, X>{__builtin_nontemporal_load(vp + pslot(k)), x[off[k]]}; },
+        m, [&](int k) { return Term<V, X>{ld_matrix<NT>(vp + pslot(k)), x[off[k]]}; },
         [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
 }
 // Row r's slice: the first of its stencil offsets in pp.poff, or -1.  Every
@@ -153,21 +153,24 @@ __device__ __forceinline__ void load_group_bases(const PPEView& pp, int first, i
 }
 
 // y_r = diag_r x_r - offdiag_r(x); dg = the diagonal of this operator
-template <class V, class X, class DG>
-__device__ __forceinline__ double spmv_row(const PPEView& pp, int r, const V* vals, const DG* dg, const X* x,
-                                           const int* wbase) {
+template <bool NT, class V, class X>
+__device__ __forceinline__ double offdiag_row(const PPEView& pp, int r, const V* vals, const X* x, const int* wbase) {
     const long long base = prow(pp.sl_off, r);
     const int st = stencil_of(pp, r);
-    double s;
     if (st >= 0) {
         // a stencil slice's rows all hold its offsets: a uniform count
         const int m = __builtin_amdgcn_readfirstlane(pp.cnt[r]);
-        s = offdiag_stencil<V, X>(vals + base, m, pp.poff + st, r, x);
-    } else {
-        const int m = pp.cnt[r];
-        if (pp.ecols) s = offdiag_u16<V, X>(pp.ecols + base, vals + base, m, wbase + (threadIdx.x & ~63), x);
-        else s = offdiag_i32<V, X>(pp.cols + base, vals + base, m, x);
+        return offdiag_stencil<V, X, NT>(vals + base, m, pp.poff + st, r, x);
     }
+    const int m = pp.cnt[r];
+    if (pp.ecols) return offdiag_u16<V, X, NT>(pp.ecols + base, vals + base, m, wbase + (threadIdx.x & ~63), x);
+    return offdiag_i32<V, X, NT>(pp.cols + base, vals + base, m, x);
+}
+template <class V, class X, class DG>
+__device__ __forceinline__ double spmv_row(const PPEView& pp, int r, const V* vals, const DG* dg, const X* x,
+                                           const int* wbase) {
+    double s = (pp.stream & STREAM_KRYLOV) ? offdiag_row<true>(pp, r, vals, x, wbase)
+                                           : offdiag_row<false>(pp, r, vals, x, wbase);
     if (pp.ltail) {
         const int u = pp.ltail[r];
         if (u >= 0) s += pp.lsum[u];

@@ -130,8 +130,26 @@ struct PPEView {
     float* tail_vals;
     int nlong;
     double* lsum;                 // long-row index -> tail sum for the next product
+    int stream;                   // STREAM_*: operators read past the caches (ppe_streams)
 };
 constexpr int LONG_ROW = 256;
+// The Krylov product's operator (STREAM_KRYLOV), the multigrid's compact
+// finest one (STREAM_MG): read with nontemporal loads when the step's cases
+// together hold more of it than the 256 MB Infinity Cache takes beside the
+// vectors, so that it does not push the gathered vectors out; a smaller one
+// stays in the caches from one product to the next.  With plain loads: FP64
+// product 26.3 -> 16.7 us (20 k particles, 16 MB), 36.8 -> 27.9 (150 k, 115 MB),
+// 65.8 -> 50.7 (300 k, 232 MB), 99.8 -> 102.6 (500 k, 393 MB); float 17.4 -> 13.5
+// (60 k, 16 MB), 26.7 -> 24.3 (400 k, 104 MB), 55.2 -> 61.0 (1 M, 264 MB), 130 -> 144
+// (2.13 M); the finest level's passes 15.4 -> 12.0 (20 k), 52.7 -> 49.2 (1.5 M,
+// 198 MB), 83 -> 88 (2.13 M, 270 MB).
+constexpr int STREAM_KRYLOV = 1, STREAM_MG = 2;
+constexpr double STREAM_BYTES = 240e6;
+template <bool NT, class P>
+__device__ __forceinline__ auto ld_matrix(P p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
 
 // Everything a pass needs to know about one case.  The engine keeps one per
 // case of a step in device memory; kernels find theirs through the segment
@@ -683,6 +701,7 @@ int stats_run_noalloc(sph_ctx* c, float* umax, float* drho, float* fmax);
 // ppe.hip
 int ppe_build(sph_ctx* c);
 PPEView ppe_view(const sph_ctx* c);
+void ppe_streams(Eng& e);
 int ppe_nlong(const sph_ctx* c);   // rows with tails of the case's PPE
 // neighbour records from the working state (physics.hip): REC_ALL, or only
 // the pairs that hold velocities and pressures (REC_VEL_PQ) or pressures (REC_PQ)
