@@ -393,8 +393,9 @@ int eng_init(Eng& e, hipStream_t st) {
 }
 
 static void drop_graphs(Eng& e) {
-    for (auto& g : e.iter_graph)
-        if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
+    for (auto& pair : e.iter_graph)
+        for (auto& g : pair)
+            if (g) { (void)hipGraphExecDestroy(g); g = nullptr; }
     for (auto& g : e.step_graph) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         g = Eng::StepGraph{};

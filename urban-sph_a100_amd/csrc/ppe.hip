@@ -1862,28 +1862,32 @@ static int kr_iteration(Eng& e, double spmv_bytes, bool mg) {
     return 0;
 }
 
-// The iteration as a HIP graph, captured once per composition of the step
-// (its launches read everything else from the device descriptors).
+// The iteration (run: KR_RUN of them) as a HIP graph, captured once per
+// composition of the step (its launches read everything else from the device
+// descriptors).  A graph's first kernel starts about 9 us after the last of the
+// graph before it, a kernel within it about 1 us after its predecessor.
 template <class V, class X>
-static int kr_graph(Eng& e, int gi, double spmv_bytes, bool mg, hipGraphExec_t* out) {
-    if (!e.iter_graph[gi]) {
+static int kr_graph(Eng& e, int gi, bool run, double spmv_bytes, bool mg, hipGraphExec_t* out) {
+    hipGraphExec_t& exec = e.iter_graph[gi][run ? 1 : 0];
+    if (!exec) {
         Shape sh;
         SPH_TRY(shape(e, 1, BLOCK, &sh));   // segment table exists before the capture
         hipGraph_t g = nullptr;
         SPH_HIP(&e, hipStreamBeginCapture(e.st, hipStreamCaptureModeThreadLocal));
-        int rc = kr_iteration<V, X>(e, spmv_bytes, mg);
+        int rc = 0;
+        for (int b = 0; b < (run ? Eng::KR_RUN : 1) && rc == 0; b++) rc = kr_iteration<V, X>(e, spmv_bytes, mg);
         hipError_t er = hipStreamEndCapture(e.st, &g);
         if (rc) {
             if (er == hipSuccess && g) (void)hipGraphDestroy(g);
             return rc;
         }
         SPH_HIP(&e, er);
-        er = hipGraphInstantiate(&e.iter_graph[gi], g, nullptr, nullptr, 0);
+        er = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
-        if (er != hipSuccess) e.iter_graph[gi] = nullptr;
+        if (er != hipSuccess) exec = nullptr;
         SPH_HIP(&e, er);
     }
-    *out = e.iter_graph[gi];
+    *out = exec;
     return 0;
 }
 
@@ -1923,7 +1927,6 @@ static int bicgstab(Eng& e, int gi, int pred_slot, std::vector<int>& iters, bool
     }
     KF(FIN_INIT);
     RL("kr_zerox", 0, k_kr_zerox<X>);
-    SPH_TRY(read_scalars(e));
     auto all_done = [&]() {
         for (int k = 0; k < nc; k++)
             if (e.h_ctl[k * CTL_COUNT + CTL_SKIP] == 0.0 && e.h_sc[k * SC_COUNT + SC_DONE] == 0.0) return false;
@@ -1931,20 +1934,31 @@ static int bicgstab(Eng& e, int gi, int pred_slot, std::vector<int>& iters, bool
     };
     const bool graphs = e.use_graphs && !e.prof.on;
     int& pred = e.pred_iters[gi][std::min(pred_slot, Eng::PRED_SLOTS - 1)];
+    // A look at the scalars costs a stop of the device of about 25 us, an
+    // iteration past the end a few us a launch: with a prediction the solve
+    // runs straight to it (a long one to just before it), then looks often;
+    // without one the batches grow geometrically.
+    const bool brief = pred > 0 && pred <= 8;
+    if (pred == 0 || e.prof.on) SPH_TRY(read_scalars(e));
     int launched = 0;
-    while (!all_done() && launched < maxit) {
-        // run straight to just before the expected end, then poll often;
-        // without a prediction grow the batches geometrically
+    for (bool first = pred > 0 && !e.prof.on; (first || !all_done()) && launched < maxit; first = false) {
         int batch;
-        if (pred > 0) batch = launched + 4 < (pred * 9) / 10 ? (pred * 9) / 10 - launched : 2;
+        if (brief) batch = launched == 0 ? pred : 1;
+        else if (pred > 0) batch = launched + 4 < (pred * 9) / 10 ? (pred * 9) / 10 - launched : 2;
         else batch = std::max(4, launched / 2);
         batch = std::min(batch, maxit - launched);
-        if (graphs) {
-            hipGraphExec_t g = nullptr;
-            SPH_TRY((kr_graph<V, X>(e, gi, spmv_bytes, mg, &g)));
-            for (int b = 0; b < batch; b++) SPH_HIP(&e, hipGraphLaunch(g, e.st));
-        } else {
-            for (int b = 0; b < batch; b++) SPH_TRY((kr_iteration<V, X>(e, spmv_bytes, mg)));
+        for (int b = 0; b < batch;) {
+            if (graphs) {
+                // (a solve expected to be long: the larger graph's capture pays)
+                const bool run = batch - b >= Eng::KR_RUN && (pred > 0 ? !brief : launched >= 16);
+                hipGraphExec_t g = nullptr;
+                SPH_TRY((kr_graph<V, X>(e, gi, run, spmv_bytes, mg, &g)));
+                SPH_HIP(&e, hipGraphLaunch(g, e.st));
+                b += run ? Eng::KR_RUN : 1;
+            } else {
+                SPH_TRY((kr_iteration<V, X>(e, spmv_bytes, mg)));
+                b++;
+            }
         }
         launched += batch;
         SPH_TRY(read_scalars(e));
@@ -1957,7 +1971,7 @@ static int bicgstab(Eng& e, int gi, int pred_slot, std::vector<int>& iters, bool
         iters[k] = sc[SC_DONE] != 0.0 ? (int)sc[SC_ITERS] : (int)e.h_ctl[k * CTL_COUNT + CTL_MAXIT];
         most = std::max(most, iters[k]);
     }
-    if (launched > 0) pred = std::max(4, most);
+    if (launched > 0) pred = std::max(1, most);
     return 0;
 }
 
@@ -2107,10 +2121,11 @@ int ppe_solve(Eng& e) {
         bool changed = false;
         SPH_TRY(mg_prepare(e, mgs, SC_DONE, &changed));
         for (int gi : {2, 3})
-            if (changed && e.iter_graph[gi]) {   // its launches hold the old tables
-                (void)hipGraphExecDestroy(e.iter_graph[gi]);
-                e.iter_graph[gi] = nullptr;
-            }
+            for (hipGraphExec_t& g : e.iter_graph[gi])
+                if (changed && g) {   // its launches hold the old tables
+                    (void)hipGraphExecDestroy(g);
+                    g = nullptr;
+                }
         return 0;
     };
     if (any_mg) SPH_TRY(mg_tables());

@@ -502,10 +502,12 @@ struct Eng {
     bool use_graphs = true;
     // FP64, float, float with multigrid, FP64 with multigrid
     static constexpr int NGRAPH = 4;
-    hipGraphExec_t iter_graph[NGRAPH] = {nullptr, nullptr, nullptr, nullptr};
+    // [0]: one iteration; [1]: KR_RUN of them (long solves)
+    hipGraphExec_t iter_graph[NGRAPH][2] = {};
     // Krylov iterations of the last solves (per vector precision and
     // refinement pass): the host polls for convergence only near them
     static constexpr int PRED_SLOTS = 4;
+    static constexpr int KR_RUN = 4;
     int pred_iters[NGRAPH][PRED_SLOTS] = {};
     // the physics before (0) and after (1) the pressure solve as graphs, for
     // the composition of the step and the variant of its launch sequence
