@@ -736,6 +736,16 @@ struct MGLv {
 // sum_k (a_rk / d_r) x[col_k] over the compact level-0 operator, in entry
 // order, accumulated in double (row_sum)
 struct HTerm { unsigned short h; float x; };
+// A level's passes of fewer threads than this run in 64-thread blocks, which
+// put a wave on each CU where 256-thread blocks would fill a fraction of them
+// (20 k particles: finest level 11.6 -> 10.9 us a pass, coarse 6.6 -> 6.3; at
+// 200 k and more particles nothing or 0.4 us lost on the finest level).
+constexpr long long SPREAD_THREADS = 131072;
+// Coarse levels: a lane's entries (members, for the restriction) loaded at a
+// time (row_sum).  One after another, each was a chain of two loads: on the
+// 226 k refined canyon long rows 34 -> 12.7 us, residual 18 -> 9.7, restriction
+// 9.8 -> 7.3 us, on 2.13 M 12.4 -> 10.5, 8.8 -> 7.0 us (HIP events).
+constexpr int COARSE_U = 8;
 template <bool NT>
 __device__ __forceinline__ double mg_row16_ld(const PPEView& pp, const MGLv& L, int r, const float* x,
                                               const int* wb) {
@@ -769,10 +779,10 @@ __device__ __forceinline__ double mg_row16(const PPEView& pp, const MGLv& L, int
     return (pp.stream & STREAM_MG) ? mg_row16_ld<true>(pp, L, r, x, wb) : mg_row16_ld<false>(pp, L, r, x, wb);
 }
 
-// block -> (case, first row of the level); the block returns when the
-// case's solve is done
+// block -> (case, first row of the level), in an order that keeps neighbouring
+// rows on one XCD; the block returns when the case's solve is done
 #define MG_HEAD(tab, lvl)                                      \
-    const int2 te_ = (tab)[blockIdx.x];                        \
+    const int2 te_ = (tab)[xcd_block()];                       \
     const CaseDesc& cd = cds[te_.x];                           \
     if (cd.sc[sc_done] != 0.0) return;                         \
     const MGLv& L = lv[te_.x * MG_MAX_LEVELS + (lvl)];         \
@@ -836,20 +846,30 @@ __global__ void __launch_bounds__(BLOCK) k_mg_post(const CaseDesc* cds, const MG
 // group's sums, so the result does not depend on the launch.  A long row's
 // product comes from k_mg_clong.  tab: BLOCK / MG_G rows per block; every
 // lane of a group has the same row, so a group returns or stays whole.
+// sum of entries k0, k0 + step, ... < m of a coarse row, in that order
+__device__ __forceinline__ double coarse_sum(const MGLv& L, long long base, int k0, int m, int step) {
+    return row_sum<Term<float, float>, COARSE_U>(
+        (m - k0 + step - 1) / step,
+        [&](int q) {
+            const long long e = base + pslot(k0 + q * step);
+            return Term<float, float>{L.vals[e], L.x[L.cols[e]]};
+        },
+        [](double s, const Term<float, float>& t) { return s + (double)t.v * (double)t.x; });
+}
 __device__ __forceinline__ double coarse_ax_g(const MGLv& L, int row, int g) {
     const int u = L.lidx ? L.lidx[row] : -1;
     double s = 0.0;
     if (u < 0) {
         const long long base = prow(L.sl_off, row);
         const int m = L.cnt[row];
-        for (int k = g; k < m; k += MG_G) s += (double)L.vals[base + pslot(k)] * (double)L.x[L.cols[base + pslot(k)]];
+        s = coarse_sum(L, base, g, m, MG_G);
     }
 #pragma unroll
     for (int off = MG_G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     return (double)L.diag[row] * (double)L.x[row] - (u >= 0 ? L.lsum[u] : s);
 }
 #define MG_HEAD_G(tab, lvl)                                    \
-    const int2 te_ = (tab)[blockIdx.x];                        \
+    const int2 te_ = (tab)[xcd_block()];                       \
     const CaseDesc& cd = cds[te_.x];                           \
     if (cd.sc[sc_done] != 0.0) return;                         \
     const MGLv& L = lv[te_.x * MG_MAX_LEVELS + (lvl)];         \
@@ -885,8 +905,9 @@ __global__ void __launch_bounds__(BLOCK) k_mg_restrict(const CaseDesc* cds, cons
     MG_HEAD(tab, l);
     const MGLv& N = lv[te_.x * MG_MAX_LEVELS + l + 1];
     if (row >= N.n) return;
-    double s = 0.0;
-    for (int t = L.mstart[row]; t < L.mstart[row + 1]; t++) s += (double)L.r[L.mem[t]];
+    const int t0 = L.mstart[row];
+    const double s = row_sum<float, COARSE_U>(
+        L.mstart[row + 1] - t0, [&](int t) { return L.r[L.mem[t0 + t]]; }, [](double a, float r) { return a + (double)r; });
     const float b = (float)s;
     N.b[row] = b;
     // the next level's pre-smoothing, x = w b / diag, when it has a level below
@@ -905,9 +926,15 @@ __global__ void __launch_bounds__(BLOCK) k_mg_long(const CaseDesc* cds, const MG
     const int u = te_.y + (int)(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (u >= pp.nlong) return;
-    double s = 0.0;
-    for (long long e = pp.tail_off[u] + lane; e < pp.tail_off[u + 1]; e += SLICE)
-        s += (double)pp.tail_vals[e] * (double)L.x[pp.tail_cols[e]];
+    const long long e0 = pp.tail_off[u] + lane, e1 = pp.tail_off[u + 1];
+    double s = e0 < e1 ? row_sum<Term<float, float>, COARSE_U>(
+                             (int)((e1 - e0 + SLICE - 1) / SLICE),
+                             [&](int q) {
+                                 const long long e = e0 + (long long)q * SLICE;
+                                 return Term<float, float>{pp.tail_vals[e], L.x[pp.tail_cols[e]]};
+                             },
+                             [](double a, const Term<float, float>& t) { return a + (double)t.v * (double)t.x; })
+                       : 0.0;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane == 0) L.lsum[u] = s;
@@ -926,9 +953,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_clong(const CaseDesc* cds, const M
     if (u >= L.nlong) return;
     const int row = L.lrows[u];
     const long long base = prow(L.sl_off, row);
-    double s = 0.0;
-    for (int k = lane; k < L.cnt[row]; k += SLICE)
-        s += (double)L.vals[base + pslot(k)] * (double)L.x[L.cols[base + pslot(k)]];
+    double s = coarse_sum(L, base, lane, L.cnt[row], SLICE);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane == 0) L.lsum[u] = s;
@@ -958,8 +983,10 @@ __global__ void __launch_bounds__(BLOCK) k_mg_dense(const CaseDesc* cds, const M
     if (row >= C.n) return;
     const int n = C.n;
     const float* a = C.ainv + (long long)row * n;
-    double s = 0.0;
-    for (int j = lane; j < n; j += SLICE) s += (double)a[j] * (double)C.b[j];
+    double s = row_sum<Term<float, float>, COARSE_U>(
+        (n - lane + SLICE - 1) / SLICE,
+        [&](int q) { return Term<float, float>{a[lane + q * SLICE], C.b[lane + q * SLICE]}; },
+        [](double t, const Term<float, float>& e) { return t + (double)e.v * (double)e.x; });
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane != 0) return;
@@ -1352,23 +1379,24 @@ int mg_prepare(Eng& e, const std::vector<const MGState*>& mgs, int sc_done, bool
             D.lidx = S.lidx;
         }
     }
-    auto rows_table = [&](int l, bool below, int* off, int* cnt) {
+    auto rows_table = [&](int l, bool below, int* off, int* cnt, int* blk) {
         // the coarse levels' residual and post-smoothing passes run MG_G
         // lanes per row
-        const int per = (below && l > 0) ? BLOCK / MG_G : BLOCK;
+        const int lanes = (below && l > 0) ? MG_G : 1;
+        auto has = [&](const MGState* mg) { return mg && (below ? l < mg->nlev - 1 : l <= mg->nlev - 1); };
+        long long threads = 0;
+        for (int k = 0; k < nc; k++)
+            if (has(mgs[k])) threads += (long long)mgs[k]->L[l].n * lanes;
+        *blk = threads < SPREAD_THREADS ? SLICE : BLOCK;
         *off = (int)tab.size();
-        for (int k = 0; k < nc; k++) {
-            const MGState* mg = mgs[k];
-            if (!mg) continue;
-            const int lc = mg->nlev - 1;
-            if (below ? !(l < lc) : !(l <= lc)) continue;
-            for (int f = 0; f < mg->L[l].n; f += per) tab.push_back(make_int2(k, f));
-        }
+        for (int k = 0; k < nc; k++)
+            if (has(mgs[k]))
+                for (int f = 0; f < mgs[k]->L[l].n; f += *blk / lanes) tab.push_back(make_int2(k, f));
         *cnt = (int)tab.size() - *off;
     };
     for (int l = 0; l < P.lmax; l++) {
-        rows_table(l, true, &P.down_off[l], &P.down_cnt[l]);
-        rows_table(l, false, &P.lvl_off[l], &P.lvl_cnt[l]);
+        rows_table(l, true, &P.down_off[l], &P.down_cnt[l], &P.down_blk[l]);
+        rows_table(l, false, &P.lvl_off[l], &P.lvl_cnt[l], &P.lvl_blk[l]);
     }
     P.dense_off = (int)tab.size();
     for (int k = 0; k < nc; k++) {
@@ -1423,11 +1451,12 @@ int mg_apply(Eng& e, int which, int sc_done) {
     const CaseDesc* cds = e.d_desc;
     const MGLv* lv = (const MGLv*)e.mg_lv;
     const int2* T = e.mg_tab;
-#define MGE(name, bytes, tab_off, cnt, kern, ...)                                                    \
+#define MGE(name, bytes, tab_off, cnt, kern, ...) MGB(name, bytes, tab_off, cnt, BLOCK, kern, ##__VA_ARGS__)
+#define MGB(name, bytes, tab_off, cnt, blk, kern, ...)                                                    \
     do {                                                                                             \
         if ((cnt) > 0) {                                                                             \
             SPH_TRY(prof_begin(e, name, (double)(bytes)));                                           \
-            hipLaunchKernelGGL(kern, dim3(cnt), dim3(BLOCK), 0, e.st, cds, lv, T + (tab_off), ##__VA_ARGS__); \
+            hipLaunchKernelGGL(kern, dim3(cnt), dim3(blk), 0, e.st, cds, lv, T + (tab_off), ##__VA_ARGS__); \
             SPH_TRY(launch_check(&e, name));                                                         \
             SPH_TRY(prof_end(e));                                                                    \
         }                                                                                            \
@@ -1440,17 +1469,18 @@ int mg_apply(Eng& e, int which, int sc_done) {
     for (int l = 0; l + 1 < P.lmax; l++) {
         if (l == 0) MGE("mg_long", 0, P.long_off, P.long_cnt, k_mg_long, sc_done);
         else MGE("mg_clong", 0, P.clong_off[l], P.clong_cnt[l], k_mg_clong, l, sc_done);
-        if (l == 0) MGE("mg_res0", P.spmv_bytes0, P.down_off[l], P.down_cnt[l], k_mg_res, l, which, sc_done);
-        else MGE("mg_res", 0, P.down_off[l], P.down_cnt[l], k_mg_res_g, l, sc_done);
-        MGE("mg_restrict", 0, P.lvl_off[l + 1], P.lvl_cnt[l + 1], k_mg_restrict, l, sc_done);
+        if (l == 0) MGB("mg_res0", P.spmv_bytes0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_res, l, which, sc_done);
+        else MGB("mg_res", 0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_res_g, l, sc_done);
+        MGB("mg_restrict", 0, P.lvl_off[l + 1], P.lvl_cnt[l + 1], P.lvl_blk[l + 1], k_mg_restrict, l, sc_done);
     }
     MGE("mg_dense", 0, P.dense_off, P.dense_cnt, k_mg_dense, sc_done);
     for (int l = P.lmax - 2; l >= 0; l--) {
         if (l == 0) MGE("mg_long", 0, P.long_off, P.long_cnt, k_mg_long, sc_done);
         else MGE("mg_clong", 0, P.clong_off[l], P.clong_cnt[l], k_mg_clong, l, sc_done);
-        if (l == 0) MGE("mg_post0", P.spmv_bytes0, P.down_off[l], P.down_cnt[l], k_mg_post, l, which, sc_done);
-        else MGE("mg_post", 0, P.down_off[l], P.down_cnt[l], k_mg_post_g, l, sc_done);
+        if (l == 0) MGB("mg_post0", P.spmv_bytes0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_post, l, which, sc_done);
+        else MGB("mg_post", 0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_post_g, l, sc_done);
     }
+#undef MGB
 #undef MGE
     return 0;
 }

@@ -965,13 +965,17 @@ __global__ void __launch_bounds__(BLOCK) k_kr_long(Seg sg) {
     const int lane = t & 63, u = t >> 6;
     const KSet<X> K = kset(pp, (X*)nullptr);
     const X* x = WHICH == 0 ? K.x : WHICH == 1 ? K.phat : K.shat;
-    const long long e1 = pp.tail_off[u + 1];
+    const long long e0 = pp.tail_off[u] + lane, e1 = pp.tail_off[u + 1];
     double s = 0.0;
-    for (long long e = pp.tail_off[u] + lane; e < e1; e += 64) {
-        const int c = pp.tail_cols[e];
-        const double xv = WHICH == 3 ? pp.x[c] : (double)x[c];
-        s += (double)pp.tail_vals[e] * xv;
-    }
+    if (e0 < e1)
+        s = row_sum<Term<float, double>, 8>(
+            (int)((e1 - e0 + 63) / 64),
+            [&](int q) {
+                const long long e = e0 + 64LL * q;
+                const int c = pp.tail_cols[e];
+                return Term<float, double>{pp.tail_vals[e], WHICH == 3 ? pp.x[c] : (double)x[c]};
+            },
+            [](double a, const Term<float, double>& t) { return a + (double)t.v * t.x; });
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane == 0) pp.lsum[u] = s;
