@@ -144,10 +144,11 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_snapshot(Seg sg, int which, int n
     cd.snap[3][i] = A.pres[i]; cd.snap[4][i] = A.temp[i];
     if (nm_pack && cd.nm_rec && i < cd.nm_nset) {   // the Neumann pass's records, from the same state
         const int j = cd.nm_set[i];
-        float4* r = (float4*)(cd.nm_rec + (size_t)i * NMREC_FLOATS);
+        const size_t n = (size_t)cd.nm_nset;
+        float4* r = (float4*)cd.nm_rec + i;
         r[0] = make_float4((float)A.x[j], (float)A.y[j], (float)A.z[j], (float)A.m[j]);
-        r[1] = make_float4((float)A.rho[j], (float)A.ux[j], (float)A.uy[j], (float)A.uz[j]);
-        *(double2*)(r + 2) = make_double2(A.pres[j], 0.0);
+        r[n] = make_float4((float)A.rho[j], (float)A.ux[j], (float)A.uy[j], (float)A.uz[j]);
+        *(double2*)(r + 2 * n) = make_double2(A.pres[j], 0.0);
     }
 }
 
@@ -249,38 +250,39 @@ template <int WHICH>
 __global__ void __launch_bounds__(BLOCK) k_pack_records(Seg sg) {
     SEG_PARTICLE(sg);
     const PView S = cd.S;
+    const size_t n = (size_t)cd.n;   // piece q of particle i: element q * n + i
     if (cd.crec) {   // the gathering passes of this case read the compact records
         if (WHICH == REC_PQ) {
-            float4* c = (float4*)(cd.crec + (size_t)i * CREC_FLOATS);
+            float4* c = (float4*)cd.crec + i;
             c[0] = make_float4((float)S.x[i], (float)S.y[i], (float)S.z[i], (float)S.m[i]);
-            c[1] = make_float4((float)S.rho[i], (float)(S.pres[i] - S.pres0[i]), (float)S.h[i],
+            c[n] = make_float4((float)S.rho[i], (float)(S.pres[i] - S.pres0[i]), (float)S.h[i],
                                __int_as_float(S.p_type[i]));
             return;
         }
-        float4* c = (float4*)(cd.crec_adv + (size_t)i * CREC_ADV_FLOATS);
-        double2* d = (double2*)(c + 2);
+        float4* c = (float4*)cd.crec_adv + i;
+        double2* d = (double2*)(c + 2 * n);
         d[0] = make_double2(S.ux[i], S.uy[i]);
-        d[1] = make_double2(S.uz[i], S.pres[i] - S.pres0[i]);
+        d[n] = make_double2(S.uz[i], S.pres[i] - S.pres0[i]);
         if (WHICH == REC_VEL_PQ) return;
         const int t = (S.p_type[i] & 0xffff) | (S.i_type[i] << 16) |
                       (cd.ppe.rowof && cd.ppe.rowof[i] >= 0 ? CREC_ROW_BIT : 0);
         if (WHICH == REC_PRE) c[0] = make_float4((float)S.x[i], (float)S.y[i], (float)S.z[i], (float)S.m[i]);
-        c[1] = make_float4((float)S.rho[i], (float)S.h[i],
+        c[n] = make_float4((float)S.rho[i], (float)S.h[i],
                            (float)(viscosity2(cd.pr, S.p_type[i]) + S.vis_t[i] * S.rho[i]), __int_as_float(t));
         return;
     }
     if (WHICH == REC_PRE) return;
-    double2* r = (double2*)(cd.rec + (size_t)i * REC_DOUBLES);
-    r[2] = make_double2(S.rho[i], S.pres[i] - S.pres0[i]);
+    double2* r = (double2*)cd.rec + i;
+    r[2 * n] = make_double2(S.rho[i], S.pres[i] - S.pres0[i]);
     if (WHICH == REC_PQ) return;
-    r[3] = make_double2(S.ux[i], S.uy[i]);
-    r[4] = make_double2(S.uz[i], S.h[i]);
+    r[3 * n] = make_double2(S.ux[i], S.uy[i]);
+    r[4 * n] = make_double2(S.uz[i], S.h[i]);
     if (WHICH == REC_VEL_PQ) return;
     const long long t = (long long)(unsigned)S.p_type[i] | ((long long)S.i_type[i] << 32);
     r[0] = make_double2(S.x[i], S.y[i]);
-    r[1] = make_double2(S.z[i], S.m[i]);
-    r[5] = make_double2(S.vis_t[i], __longlong_as_double(t));
-    r[6] = make_double2(S.temp[i], S.concn[i]);
+    r[n] = make_double2(S.z[i], S.m[i]);
+    r[5 * n] = make_double2(S.vis_t[i], __longlong_as_double(t));
+    r[6 * n] = make_double2(S.temp[i], S.concn[i]);
 }
 
 // A particle's strain rate and eddy viscosity from its sums.
@@ -378,7 +380,7 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_prep(Seg sg) {
 // float, the sums in double.  REC: the pair's fields come from the compact
 // records (float positions, whose float difference is the rounded exact
 // difference), else from the field arrays (prep, which runs before the
-// 128-byte double records are packed) or those records.
+// double records are packed) or those records.
 template <bool REC, class Src, int W>
 __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow row, const Src src, int g, bool filt,
                                           bool les, double& flt, double& sigma, double (&st)[6]) {
@@ -400,10 +402,9 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
         const int j = e & NB_IDX;
         float dx, dy, dz, mj, rhoj;
         int ptj;
-        const float* C = nullptr;
+        const auto C = src.at(j);
         if constexpr (REC) {
-            C = src.at(j);
-            const rec_f4 a = Src::f4(C), b = Src::f4(src.piece(C, 1));
+            const rec_f4 a = Src::f4(src.piece(C, 0)), b = Src::f4(src.piece(C, 1));
             dx = xf - a.x; dy = yf - a.y; dz = zf - a.z; mj = a.w; rhoj = b.x;
             ptj = crec_ptype(b.w);
         } else {
@@ -470,17 +471,17 @@ __device__ __forceinline__ void prep_mixed(const CaseDesc& cd, int i, const NLis
 }
 __global__ void __launch_bounds__(MAX_BLOCK) k_prep_mixed(Seg sg) {
     SEG_GROUP_LIGHT(sg);
-    prep_mixed<GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+    prep_mixed<GSrc, GROUP>(cd, i, cd.nl, i, GSrc{&cd.crec_adv, (size_t)cd.n}, g_);
 }
 __global__ void __launch_bounds__(WAVE_BLOCK) k_prep_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    prep_mixed<GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
+    prep_mixed<GSrc, 64>(cd, i, cd.nl, i, GSrc{&cd.crec_adv, (size_t)cd.n}, lane_);
 }
 __global__ void __launch_bounds__(TILE_THREADS) k_prep_tile(Seg sg, int width) {
     TILE_CHUNK(sg, width, cd.crec_adv, CREC_ADV_FLOATS);
     TILE_LANES(width) {
         if (chunk_.y >= 0) prep_mixed<LSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_);
-        else prep_mixed<GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+        else prep_mixed<GSrc, GROUP>(cd, i, cd.tile.nl, lane_, GSrc{&cd.crec_adv, (size_t)cd.n}, g_);
     }
 }
 
@@ -834,14 +835,15 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
         double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         const long long e0 = cd.nmp_off[u], e1 = cd.nmp_off[u + 1];
         const float* const nrec = cd.nm_rec;   // the same values, packed (float-exact positions)
+        const size_t nn = (size_t)cd.nm_nset;
         for (long long e = e0 + lane; e < e1; e += 64) {
             double xj, yj, zj, presj;
             float mj, rhoj, uxj, uyj, uzj;
             if (nrec) {
-                const float* C = nrec + (size_t)cd.nmp_cent[e] * NMREC_FLOATS;
-                const rec_f4 a = ld_f4(C), b = ld_f4(C + 4);
+                const unsigned C = (unsigned)cd.nmp_cent[e] * 16u;
+                const rec_f4 a = ld_f4(nrec, C), b = ld_f4(nrec + 4 * nn, C);
                 xj = a.x; yj = a.y; zj = a.z; mj = a.w; rhoj = b.x; uxj = b.y; uyj = b.z; uzj = b.w;
-                presj = ld_d2(C + 8).x;
+                presj = ld_d2(nrec + 8 * nn, C).x;
             } else {
                 const int j = cd.nmp_ent[e];
                 xj = A.x[j]; yj = A.y[j]; zj = A.z[j]; mj = (float)A.m[j]; rhoj = (float)A.rho[j];
@@ -1008,14 +1010,14 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_advection(Seg sg) {
         double hj, vis_tj, xj, yj, zj, mj, uxj, uyj, uzj, rhoj, pqj_;
         int ptypej = 0, itj_;
         if (pair) {
-            rec_aux(cd.rec, j, vis_tj, ptypej, itj_);
+            rec_aux(Rec(cd), j, vis_tj, ptypej, itj_);
             pair = ptypej < 1000;
         }
         if (!__any(pair)) continue;
         double v[NT] = {}, v2[ADV_SECOND] = {}, w[ADV_SUMS2] = {}, w2[1] = {};
         if (pair) {
-            rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pqj_);
-            rec_vel(cd.rec, j, uxj, uyj, uzj, hj);
+            rec_pos(Rec(cd), j, xj, yj, zj, mj, rhoj, pqj_);
+            rec_vel(Rec(cd), j, uxj, uyj, uzj, hj);
             const double visj = viscosity2(pr, ptypej) + vis_tj * rhoj;
             const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
             const double tdist = sqrt(dx * dx + dy * dy + dz * dz) + 1e-20;
@@ -1025,7 +1027,7 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_advection(Seg sg) {
             const double tdwz = tdwij * dz / tdist;
             const double dux = uxi - uxj, duy = uyi - uyj, duz = uzi - uzj;   // u_i - u_j
             double tempj = 0.0, concnj = 0.0;
-            if (con_solve || concn_solve || boussinesq_solve) rec_scalar(cd.rec, j, tempj, concnj);
+            if (con_solve || concn_solve || boussinesq_solve) rec_scalar(Rec(cd), j, tempj, concnj);
             if (fv == SPH_FV_CLEARY) {
                 double C_v = dx * tdwx + dy * tdwy + dz * tdwz;
                 C_v *= (visi * visj) / (visi + visj);
@@ -1114,7 +1116,7 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
     const KConst kc = cd.kc;
     const sph_params& pr = cd.pr;
     const PView S = cd.S;
-    const double* const rec = cd.rec;
+    const Rec rec(cd);
     const int ptypei = S.p_type[i];
     const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
@@ -1142,11 +1144,11 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
         double uxj, uyj, uzj, hj_d;
         int ptypej;
         if constexpr (REC) {
-            const float* C = src.at(j);
+            const auto C = src.at(j);
             const rec_f4 b = Src::f4(src.piece(C, 1));
             ptypej = crec_ptype(b.w);
             if (ptypej >= 1000) continue;
-            const rec_f4 p = Src::f4(C);
+            const rec_f4 p = Src::f4(src.piece(C, 0));
             const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
             dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
             rhoj = b.x; hj_d = b.y; visj = b.z;
@@ -1269,12 +1271,12 @@ __device__ __forceinline__ void advection_mixed(const CaseDesc& cd, int i, const
 template <bool SCAL>
 __global__ void __launch_bounds__(MAX_BLOCK) k_advection_mixed(Seg sg) {
     SEG_GROUP_LIGHT(sg);
-    advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+    advection_mixed<SCAL, GSrc, GROUP>(cd, i, cd.nl, i, GSrc{&cd.crec_adv, (size_t)cd.n}, g_);
 }
 template <bool SCAL>
 __global__ void __launch_bounds__(WAVE_BLOCK) k_advection_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, lane_);
+    advection_mixed<SCAL, GSrc, 64>(cd, i, cd.nl, i, GSrc{&cd.crec_adv, (size_t)cd.n}, lane_);
 }
 template <bool SCAL>
 __global__ void __launch_bounds__(TILE_THREADS) k_advection_tile(Seg sg, int width) {
@@ -1283,8 +1285,8 @@ __global__ void __launch_bounds__(TILE_THREADS) k_advection_tile(Seg sg, int wid
         if (chunk_.y >= 0)
             advection_mixed<SCAL, LSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_);
         else
-            advection_mixed<SCAL, GSrc<CREC_ADV_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_,
-                                                                GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_);
+            advection_mixed<SCAL, GSrc, GROUP>(cd, i, cd.tile.nl, lane_,
+                                                                GSrc{&cd.crec_adv, (size_t)cd.n}, g_);
     }
 }
 
@@ -1529,8 +1531,8 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force(Seg sg) {
         double v[PF_SUMS] = {};
         if (pair) {
             double hj, pj, xj, yj, zj, mj, rhoj;
-            rec_pos(cd.rec, j, xj, yj, zj, mj, rhoj, pj);
-            hj = ld_d2(rec_at(cd.rec, j, 4)).y;
+            rec_pos(Rec(cd), j, xj, yj, zj, mj, rhoj, pj);
+            hj = Rec(cd).piece(j, 4).y;
             const double dx = xi - xj, dy = yi - yj, dz = zi - zj;
             const double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
             const double hij = 0.5 * (hi + hj);
@@ -1554,7 +1556,7 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
                                               double& tmpx, double& tmpy, double& tmpz) {
     const KConst kc = cd.kc;
     const PView S = cd.S;
-    const double* const rec = cd.rec;
+    const Rec rec(cd);
     const double xi = S.x[i], yi = S.y[i], zi = S.z[i], hi_d = S.h[i];
     const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
     const float pi = (float)(S.pres[i] - S.pres0[i]), rhoi = (float)S.rho[i];
@@ -1570,17 +1572,17 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
         float dx, dy, dz, mj, rhoj, pj;
         double hj;
         if constexpr (REC) {
-            const float* C = src.at(j);
+            const auto C = src.at(j);
             const rec_f4 b = Src::f4(src.piece(C, 1));
             if (__float_as_int(b.w) >= 1000) continue;
-            const rec_f4 p = Src::f4(C);
+            const rec_f4 p = Src::f4(src.piece(C, 0));
             dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
             rhoj = b.x; pj = b.y; hj = b.z;
         } else {
             if (S.p_type[j] >= 1000) continue;
             double xj, yj, zj, mj_d, rhoj_d, pqj;
             rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, pqj);
-            hj = ld_d2(rec_at(rec, j, 4)).y;
+            hj = rec.piece(j, 4).y;
             dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
             mj = (float)mj_d; rhoj = (float)rhoj_d; pj = (float)pqj;
         }
@@ -1626,17 +1628,17 @@ __device__ __forceinline__ void pressure_force_mixed(const CaseDesc& cd, int i, 
 }
 __global__ void __launch_bounds__(MAX_BLOCK) k_pressure_force_mixed(Seg sg) {
     SEG_GROUP_LIGHT(sg);
-    pressure_force_mixed<GSrc<CREC_FLOATS>, GROUP>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{&cd.crec}, g_);
+    pressure_force_mixed<GSrc, GROUP>(cd, i, cd.nl, i, GSrc{&cd.crec, (size_t)cd.n}, g_);
 }
 __global__ void __launch_bounds__(WAVE_BLOCK) k_pressure_force_heavy(Seg sg) {
     SEG_HEAVY(sg);
-    pressure_force_mixed<GSrc<CREC_FLOATS>, 64>(cd, i, cd.nl, i, GSrc<CREC_FLOATS>{&cd.crec}, lane_);
+    pressure_force_mixed<GSrc, 64>(cd, i, cd.nl, i, GSrc{&cd.crec, (size_t)cd.n}, lane_);
 }
 __global__ void __launch_bounds__(TILE_THREADS) k_pressure_force_tile(Seg sg, int width) {
     TILE_CHUNK(sg, width, cd.crec, CREC_FLOATS);
     TILE_LANES(width) {
         if (chunk_.y >= 0) pressure_force_mixed<LSrc<CREC_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_FLOATS), g_);
-        else pressure_force_mixed<GSrc<CREC_FLOATS>, GROUP>(cd, i, cd.tile.nl, lane_, GSrc<CREC_FLOATS>{&cd.crec}, g_);
+        else pressure_force_mixed<GSrc, GROUP>(cd, i, cd.tile.nl, lane_, GSrc{&cd.crec, (size_t)cd.n}, g_);
     }
 }
 

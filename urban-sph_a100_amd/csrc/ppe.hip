@@ -725,7 +725,7 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble(Seg sg, int jacobi) 
     const bool full = jacobi || out != nullptr;   // the coefficients of every pair are needed
     const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);   // the group's first lane
     int slot = 0;
-    const double* const rec = cd.rec;
+    const Rec rec(cd);
     OrderedSums<ASM_SUMS, GROUP> sums(asm_lds + (threadIdx.x >> 6) * ord_doubles(ASM_SUMS));
     for (int k = g; k - g < nr.cnt; k += GROUP) {
         const unsigned e = k < nr.cnt ? NB_AT(nr, k) : 0u;
@@ -786,7 +786,7 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble(Seg sg, int jacobi) 
 // MIXED: GROUP lanes a particle, the pair arithmetic in float, the sums in
 // double.  REC: the pair's fields come from the compact records (float
 // positions, whose float difference is the rounded exact difference), else
-// from the 128-byte double records.  FULL writes the row's values (a
+// from the double records.  FULL writes the row's values (a
 // search's first step) or sums every coefficient (the Jacobi sweep); the slot
 // of a value is its rank among the row's entries, counted over the group.
 template <bool REC, bool FULL, class Src>
@@ -796,7 +796,7 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
     const PPEView& pp = cd.ppe;
     const PView S = cd.S;
     const QView Q = cd.Q;
-    const double* const rec = cd.rec;
+    const Rec rec(cd);
     const int* const rowof = pp.rowof;
     const double xi = S.x[i], yi = S.y[i], zi = S.z[i];
     const float xf = (float)xi, yf = (float)yi, zf = (float)zi;
@@ -823,12 +823,12 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
         bool jrow = false;   // j is an unknown of the PPE
         if (pair) {
             if constexpr (REC) {
-                const float* C = src.at(j);
+                const auto C = src.at(j);
                 const rec_f4 q = Src::f4(src.piece(C, 1));
                 pair = crec_ptype(q.w) < 1000 && crec_itype(q.w) != 4;
                 if (pair) {
                     jrow = crec_has_row(q.w);
-                    const rec_f4 p = Src::f4(C);
+                    const rec_f4 p = Src::f4(src.piece(C, 0));
                     const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
                     dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w; rhoj = q.x;
                     uxj = u.x; uyj = u.y; uzj = w.x; qj = w.y;
@@ -921,13 +921,13 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_ppe_assemble_mixed(Seg sg, int ja
     const int t = first_ + (int)threadIdx.x / GROUP;
     if (t >= cd.n) return;
     const int i = cd.porder ? cd.porder[t] : t;   // this group's particle
-    assemble_mixed(cd, i, cd.nl, i, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, (int)threadIdx.x % GROUP, jacobi);
+    assemble_mixed(cd, i, cd.nl, i, GSrc{&cd.crec_adv, (size_t)cd.n}, (int)threadIdx.x % GROUP, jacobi);
 }
 __global__ void __launch_bounds__(TILE_THREADS) k_ppe_assemble_tile(Seg sg, int width, int jacobi) {
     TILE_CHUNK(sg, width, cd.crec_adv, CREC_ADV_FLOATS);
     TILE_LANES(width) {
         if (chunk_.y >= 0) assemble_mixed(cd, i, cd.tile.nl, lane_, TILE_SRC(CREC_ADV_FLOATS), g_, jacobi);
-        else assemble_mixed(cd, i, cd.tile.nl, lane_, GSrc<CREC_ADV_FLOATS>{&cd.crec_adv}, g_, jacobi);
+        else assemble_mixed(cd, i, cd.tile.nl, lane_, GSrc{&cd.crec_adv, (size_t)cd.n}, g_, jacobi);
     }
 }
 

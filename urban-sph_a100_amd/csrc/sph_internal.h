@@ -304,15 +304,25 @@ constexpr int TUNE_CANDIDATES = 4;           // 64, 128, 256, 512 threads
 constexpr int TUNE_BLOCKS[TUNE_CANDIDATES] = {64, 128, 256, 512};
 constexpr int MAX_BLOCK = 512;
 
-// Neighbour record: the fields a gathering pass reads of its neighbour j,
-// one 128-byte line per particle, so a pair costs one line from L2 instead
-// of one line per field array (advection, PPE assembly and pressure force;
-// the strain pass reads fewer fields and is faster from the field arrays).  Pairs of doubles: 0 (x, y), 1 (z, m),
-// 2 (rho, pres - pres0), 3 (ux, uy), 4 (uz, h), 5 (vis_t, p_type | i_type << 32),
-// 6 (temp, concn).  The values are copies of the working state taken just
-// before the pass (k_pack_records), so every pass computes with exactly the
-// values it read from the field arrays before.
-constexpr int REC_DOUBLES = 16;
+// Neighbour record: the fields a gathering pass reads of its neighbour j
+// (advection, PPE assembly and pressure force; the strain pass reads fewer
+// fields and is faster from the field arrays).  Pairs of doubles: 0 (x, y),
+// 1 (z, m), 2 (rho, pres - pres0), 3 (ux, uy), 4 (uz, h), 5 (vis_t, p_type |
+// i_type << 32), 6 (temp, concn).  The values are copies of the working state
+// taken just before the pass (k_pack_records), so every pass computes with
+// exactly the values it read from the field arrays before.
+//
+// All records here are piece-major: 16-byte piece q of particle j at
+// (q * n + j) * 16 bytes.  The lanes of a group read neighbours that lie next
+// to each other, so a piece's load covers 16 consecutive bytes a lane where
+// whole records put every lane on its own half line: the gathering passes are
+// bound by those cache accesses as much as by their arithmetic (cache accesses
+// a load of the 2.13 M canyon's advection: 35 with whole records, 25 so).  Whole
+// records and pieces: advection 1608, 1546 us, assembly 1562, 1460, strain
+// 1461, 1349, packing 93, 52 us; with double records (moving 300 k canyon) advection
+// 329, 192 us, assembly 466, 342, pressure force 208, 135 us; FP64 150 k 224, 212,
+// 190, 150, 128, 106 us.
+constexpr int REC_DOUBLES = 14;
 // 16-byte loads of record pieces: explicit vector types in the global
 // address space, so each piece is one global_load_dwordx4 (a double2 read
 // through a generic pointer becomes two 8-byte flat loads)
@@ -324,31 +334,41 @@ __device__ __forceinline__ rec_d2 ld_d2(const void* p) {
 __device__ __forceinline__ rec_f4 ld_f4(const void* p) {
     return *(const __attribute__((address_space(1))) rec_f4*)p;
 }
-__device__ __forceinline__ const double* rec_at(const double* rec, int j, int piece) {
-    return rec + (size_t)j * REC_DOUBLES + 2 * piece;
+// at a byte offset of a wave-uniform base
+__device__ __forceinline__ rec_d2 ld_d2(const void* base, unsigned off) {
+    return *(const __attribute__((address_space(1))) rec_d2*)((const __attribute__((address_space(1))) char*)base + off);
 }
+__device__ __forceinline__ rec_f4 ld_f4(const void* base, unsigned off) {
+    return *(const __attribute__((address_space(1))) rec_f4*)((const __attribute__((address_space(1))) char*)base + off);
+}
+struct Rec {
+    const double* p;
+    size_t n;
+    __device__ explicit Rec(const CaseDesc& cd) : p(cd.rec), n((size_t)cd.n) {}
+    __device__ rec_d2 piece(int j, int q) const { return ld_d2(p + 2 * q * n, (unsigned)j * 16u); }
+};
 // x y z m rho pq
-__device__ __forceinline__ void rec_pos(const double* rec, int j, double& x, double& y, double& z, double& m,
+__device__ __forceinline__ void rec_pos(const Rec& rec, int j, double& x, double& y, double& z, double& m,
                                         double& rho, double& pq) {
-    const rec_d2 a = ld_d2(rec_at(rec, j, 0)), b = ld_d2(rec_at(rec, j, 1)), c = ld_d2(rec_at(rec, j, 2));
+    const rec_d2 a = rec.piece(j, 0), b = rec.piece(j, 1), c = rec.piece(j, 2);
     x = a.x; y = a.y; z = b.x; m = b.y; rho = c.x; pq = c.y;
 }
 // ux uy uz h
-__device__ __forceinline__ void rec_vel(const double* rec, int j, double& ux, double& uy, double& uz, double& h) {
-    const rec_d2 a = ld_d2(rec_at(rec, j, 3)), b = ld_d2(rec_at(rec, j, 4));
+__device__ __forceinline__ void rec_vel(const Rec& rec, int j, double& ux, double& uy, double& uz, double& h) {
+    const rec_d2 a = rec.piece(j, 3), b = rec.piece(j, 4);
     ux = a.x; uy = a.y; uz = b.x; h = b.y;
 }
 // vis_t p_type i_type
-__device__ __forceinline__ void rec_aux(const double* rec, int j, double& vis_t, int& p_type, int& i_type) {
-    const rec_d2 a = ld_d2(rec_at(rec, j, 5));
+__device__ __forceinline__ void rec_aux(const Rec& rec, int j, double& vis_t, int& p_type, int& i_type) {
+    const rec_d2 a = rec.piece(j, 5);
     vis_t = a.x;
     const long long t = __double_as_longlong(a.y);
     p_type = (int)(unsigned)(t & 0xffffffffLL);
     i_type = (int)(t >> 32);
 }
 // temp concn
-__device__ __forceinline__ void rec_scalar(const double* rec, int j, double& temp, double& concn) {
-    const rec_d2 a = ld_d2(rec_at(rec, j, 6));
+__device__ __forceinline__ void rec_scalar(const Rec& rec, int j, double& temp, double& concn) {
+    const rec_d2 a = rec.piece(j, 6);
     temp = a.x; concn = a.y;
 }
 
@@ -359,7 +379,7 @@ __device__ __forceinline__ void rec_scalar(const double* rec, int j, double& tem
 // and p - p0 enter the pressure force rounded to float; h is float-exact; the
 // neighbour's viscosity is stored as the float the kernels round it to;
 // velocities and the assembly's p - p0 stay double), so the results are bit
-// for bit those of the 128-byte double records.
+// for bit those of the double records.
 // Pressure force, 32 bytes: float4 (x, y, z, m), float4 (rho, pres - pres0, h,
 // p_type as bits).
 constexpr int CREC_FLOATS = 8;
@@ -377,15 +397,16 @@ constexpr int NMREC_FLOATS = 12;
 // Where a gathering pass reads its neighbour records: in memory, indexed by
 // particle (base null: the FP64 field arrays), or staged in LDS by a tile,
 // indexed by halo slot.
-template <int STRIDE>   // floats per record
 struct GSrc {
     static constexpr bool lds = false;
     float* const* ref;   // the descriptor's record pointer (read where the loop starts), or null
+    size_t n;            // particles (the stride between pieces, in 16-byte units)
+    struct Piece { const float* base; unsigned off; };
     __device__ bool ok() const { return ref && *ref; }
-    __device__ const float* at(int j) const { return *ref + (size_t)j * STRIDE; }
-    __device__ const float* piece(const float* rec, int q) const { return rec + 4 * q; }   // 16-byte piece q
-    __device__ static rec_f4 f4(const float* p) { return ld_f4(p); }
-    __device__ static rec_d2 d2(const float* p) { return ld_d2(p); }
+    __device__ unsigned at(int j) const { return (unsigned)j * 16u; }
+    __device__ Piece piece(unsigned rec, int q) const { return {*ref + 4 * q * n, rec}; }   // 16-byte piece q
+    __device__ static rec_f4 f4(const Piece& p) { return ld_f4(p.base, p.off); }
+    __device__ static rec_d2 d2(const Piece& p) { return ld_d2(p.base, p.off); }
     __device__ int gidx(int j) const { return j; }           // particle of an entry
     __device__ bool self(int j, int i) const { return j == i; }
 };
@@ -420,7 +441,7 @@ static_assert(TILE_THREADS % (SLICE * GROUP) == 0 || (SLICE * GROUP) % TILE_THRE
 // to float4 q * cnt + r.
 constexpr int TILE_U = 4;
 template <int Q>
-__device__ __forceinline__ void tile_stage_q(float4* lds, const float* recs, const int* halo, int cnt) {
+__device__ __forceinline__ void tile_stage_q(float4* lds, const float* recs, size_t n, const int* halo, int cnt) {
     const int B = blockDim.x;
     for (int r0 = threadIdx.x; r0 < cnt; r0 += TILE_U * B) {
         int idx[TILE_U];
@@ -431,7 +452,7 @@ __device__ __forceinline__ void tile_stage_q(float4* lds, const float* recs, con
         for (int u = 0; u < TILE_U; u++)
             if (idx[u] >= 0)
 #pragma unroll
-                for (int q = 0; q < Q; q++) v[u][q] = ld_f4(recs + ((size_t)idx[u] * Q + q) * 4);
+                for (int q = 0; q < Q; q++) v[u][q] = ld_f4(recs + 4 * q * n, (unsigned)idx[u] * 16u);
 #pragma unroll
         for (int u = 0; u < TILE_U; u++)
             if (idx[u] >= 0)
@@ -440,9 +461,10 @@ __device__ __forceinline__ void tile_stage_q(float4* lds, const float* recs, con
                     lds[q * cnt + r0 + u * B] = make_float4(v[u][q].x, v[u][q].y, v[u][q].z, v[u][q].w);
     }
 }
-__device__ __forceinline__ void tile_stage(float4* lds, const float* recs, const int* halo, int cnt, int recf) {
-    if (recf == 8) tile_stage_q<2>(lds, recs, halo, cnt);
-    else tile_stage_q<4>(lds, recs, halo, cnt);
+__device__ __forceinline__ void tile_stage(float4* lds, const float* recs, size_t n, const int* halo, int cnt,
+                                           int recf) {
+    if (recf == 8) tile_stage_q<2>(lds, recs, n, halo, cnt);
+    else tile_stage_q<4>(lds, recs, n, halo, cnt);
 }
 #define TILE_CHUNK(sg, width, RECS, RECF)                                                       \
     extern __shared__ float4 tile_lds_[];                                                       \
@@ -450,7 +472,7 @@ __device__ __forceinline__ void tile_stage(float4* lds, const float* recs, const
     const int2 te_ = (sg).tab ? (sg).tab[lb_] : make_int2(0, (int)(lb_ * (unsigned)(width)));   \
     const CaseDesc& cd = (sg).cd[te_.x];                                                        \
     const int2 chunk_ = cd.tile.chunk[te_.y / (width)];                                         \
-    if (chunk_.y > 0) tile_stage(tile_lds_, (RECS), cd.tile.halo + chunk_.x, chunk_.y, (RECF)); \
+    if (chunk_.y > 0) tile_stage(tile_lds_, (RECS), (size_t)cd.n, cd.tile.halo + chunk_.x, chunk_.y, (RECF)); \
     __syncthreads();                                                                            \
     const int g_ = (int)threadIdx.x % GROUP;
 #define TILE_LANES(width)                                                                       \
