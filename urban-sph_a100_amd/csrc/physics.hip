@@ -396,15 +396,16 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
     const HScale hs(kc, hi);
     // consecutive neighbours mostly share rho: its reciprocal is kept
     float rho_c = -1.0f, yrho = 0.0f;
-    for (int k = g; k < row.cnt; k += W) {
-        const unsigned e = NB_AT(row, k);
-        if (!(e & F_HP)) continue;
+    walk_row<REC, 2, 2, W>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
+        if (!(e & F_HP)) return;
         const int j = e & NB_IDX;
-        float dx, dy, dz, mj, rhoj;
+        float dx, dy, dz, mj, rhoj, dux, duy, duz;
         int ptj;
-        const auto C = src.at(j);
         if constexpr (REC) {
-            const rec_f4 a = Src::f4(src.piece(C, 0)), b = Src::f4(src.piece(C, 1));
+            // (every piece is read here: see walk_row)
+            const rec_f4 a = rec_.f[0], b = rec_.f[1];
+            const rec_d2 p = rec_.d[0], q = rec_.d[1];
+            dux = (float)(p.x - uxi); duy = (float)(p.y - uyi); duz = (float)(q.x - uzi);
             dx = xf - a.x; dy = yf - a.y; dz = zf - a.z; mj = a.w; rhoj = b.x;
             ptj = crec_ptype(b.w);
         } else {
@@ -421,18 +422,13 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
         if (les) {
             sigma += (double)quot(d.r * d.r * wij * mj, rhoj, yrho);
             if (ptj == 1) {
-                double uxj, uyj, uzj;
-                if constexpr (REC) {
-                    const rec_d2 p = Src::d2(src.piece(C, 2)), q = Src::d2(src.piece(C, 3));
-                    uxj = p.x; uyj = p.y; uzj = q.x;
-                } else {
-                    uxj = S.ux[j]; uyj = S.uy[j]; uzj = S.uz[j];
+                if constexpr (!REC) {
+                    dux = (float)(S.ux[j] - uxi); duy = (float)(S.uy[j] - uyi); duz = (float)(S.uz[j] - uzi);
                 }
                 const float dw = kernel_dw_t<float>(kc, tmp_A, f, tR);
                 const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
                 const float cx = gc11 * tx + gc12 * ty + gc31 * tz, cy = gc12 * tx + gc22 * ty + gc23 * tz,
                             cz = gc31 * tx + gc23 * ty + gc33 * tz;
-                const float dux = (float)(uxj - uxi), duy = (float)(uyj - uyi), duz = (float)(uzj - uzi);
                 st[0] += (double)(vj * dux * cx);
                 st[1] += (double)(0.5f * vj * (dux * cy + duy * cx));
                 st[2] += (double)(vj * duy * cy);
@@ -441,7 +437,7 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
                 st[5] += (double)(vj * duz * cz);
             }
         }
-    }
+    });
 }
 template <class Src, int W = 1>
 __device__ __forceinline__ void prep_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
@@ -1136,33 +1132,32 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
     const float Alpha = (float)pr.av_alpha, Beta = (float)pr.av_beta, soundspeed = (float)pr.av_c;
     // consecutive neighbours mostly share rho: the reciprocals it enters are kept
     float rho_c = -1.0f, yrho = 0.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
-    for (int k = g; k < row.cnt; k += W) {
-        const unsigned e = NB_AT(row, k);
-        if (!(e & F_DP)) continue;
+    walk_row<REC, 2, 2, W>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
+        if (!(e & F_DP)) return;
         const int j = e & NB_IDX;
         float dx, dy, dz, mj, rhoj, visj;
-        double uxj, uyj, uzj, hj_d;
+        float dux, duy, duz;   // u_i - u_j
+        double hj_d;
         int ptypej;
-        if constexpr (REC) {
-            const auto C = src.at(j);
-            const rec_f4 b = Src::f4(src.piece(C, 1));
+        if constexpr (REC) {   // (every piece is read here: see walk_row)
+            const rec_f4 p = rec_.f[0], b = rec_.f[1];
+            const rec_d2 u = rec_.d[0], w = rec_.d[1];
             ptypej = crec_ptype(b.w);
-            if (ptypej >= 1000) continue;
-            const rec_f4 p = Src::f4(src.piece(C, 0));
-            const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
             dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
             rhoj = b.x; hj_d = b.y; visj = b.z;
-            uxj = u.x; uyj = u.y; uzj = w.x;
+            dux = (float)(uxi - u.x); duy = (float)(uyi - u.y); duz = (float)(uzi - w.x);
+            if (ptypej >= 1000) return;
         } else {
-            double vis_tj, xj, yj, zj, mj_d, rhoj_d, pqj_;
+            double vis_tj, xj, yj, zj, mj_d, rhoj_d, pqj_, uxj, uyj, uzj;
             int itj_;
             rec_aux(rec, j, vis_tj, ptypej, itj_);
-            if (ptypej >= 1000) continue;
+            if (ptypej >= 1000) return;
             rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, pqj_);
             rec_vel(rec, j, uxj, uyj, uzj, hj_d);
             dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
             mj = (float)mj_d; rhoj = (float)rhoj_d;
             visj = (float)(viscosity2(pr, ptypej) + vis_tj * rhoj_d);
+            dux = (float)(uxi - uxj); duy = (float)(uyi - uyj); duz = (float)(uzi - uzj);
         }
         if (rhoj != rho_c) {
             rho_c = rhoj;
@@ -1173,7 +1168,6 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
         const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
         const float tR = hs.tR(d.r), dw = kernel_dw_t<float>(kc, tmp_A, f, tR);
         const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
-        const float dux = (float)(uxi - uxj), duy = (float)(uyi - uyj), duz = (float)(uzi - uzj);   // u_i - u_j
         if (fv == SPH_FV_CLEARY) {
             float C_v = dx * tx + dy * ty + dz * tz;
             const float vs = visi + visj;
@@ -1236,7 +1230,7 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
                 a.tx += (double)(-P * tx); a.ty += (double)(-P * ty); a.tz += (double)(-P * tz);
             }
         }
-    }
+    });
 }
 template <bool SCAL, class Src, int W = 1>
 __device__ __forceinline__ void advection_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src,
@@ -1565,21 +1559,18 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
     float h_c = -1.0f, A_c = 0.0f, f_c = 0.0f;
     HScale hs(kc, 1.0f);
     float rho_c = -1.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
-    for (int k = g; k < row.cnt; k += W) {
-        const unsigned e = NB_AT(row, k);
-        if (!(e & F_DM)) continue;
+    walk_row<REC, 2, 0, W>(row, src, g, [&](unsigned e, const Pieces<2, 0>& rec_) {
+        if (!(e & F_DM)) return;
         const int j = e & NB_IDX;
         float dx, dy, dz, mj, rhoj, pj;
         double hj;
         if constexpr (REC) {
-            const auto C = src.at(j);
-            const rec_f4 b = Src::f4(src.piece(C, 1));
-            if (__float_as_int(b.w) >= 1000) continue;
-            const rec_f4 p = Src::f4(src.piece(C, 0));
+            const rec_f4 p = rec_.f[0], b = rec_.f[1];
+            if (__float_as_int(b.w) >= 1000) return;
             dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w;
             rhoj = b.x; pj = b.y; hj = b.z;
         } else {
-            if (S.p_type[j] >= 1000) continue;
+            if (S.p_type[j] >= 1000) return;
             double xj, yj, zj, mj_d, rhoj_d, pqj;
             rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, pqj);
             hj = rec.piece(j, 4).y;
@@ -1603,7 +1594,7 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
         const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
         const float C_p = quot(quot(-2.0f * mj, rr, yrr) * (pi * rhoj + pj * rhoi), rs, yrs);
         tmpx += (double)(C_p * tx); tmpy += (double)(C_p * ty); tmpz += (double)(C_p * tz);
-    }
+    });
 }
 template <class Src, int W = 1>
 __device__ __forceinline__ void pressure_force_mixed(const CaseDesc& cd, int i, const NList& nl, int li,

@@ -812,39 +812,34 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
     int slot = 0;
     // consecutive neighbours mostly share rho: what it enters is kept
     float rho_c = -1.0f, yrho = 0.0f, hm = 0.0f;
-    for (int k0 = 0; k0 < row.cnt; k0 += GROUP) {
-        const int k = k0 + g;
-        const unsigned e = k < row.cnt ? NB_AT(row, k) : 0u;
+    walk_row<REC, 2, 2, GROUP>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
         bool pair = (e & F_DP) != 0, own = false;   // own: an entry of the row
         const int j = e & NB_IDX;
         float cc = 0.0f;
         float dx = 0, dy = 0, dz = 0, mj = 0, rhoj = 0;
-        double qj = 0, uxj = 0, uyj = 0, uzj = 0;
+        float dux = 0, duy = 0, duz = 0;   // u_j - u_i
+        double qj = 0;
         bool jrow = false;   // j is an unknown of the PPE
-        if (pair) {
-            if constexpr (REC) {
-                const auto C = src.at(j);
-                const rec_f4 q = Src::f4(src.piece(C, 1));
-                pair = crec_ptype(q.w) < 1000 && crec_itype(q.w) != 4;
-                if (pair) {
-                    jrow = crec_has_row(q.w);
-                    const rec_f4 p = Src::f4(src.piece(C, 0));
-                    const rec_d2 u = Src::d2(src.piece(C, 2)), w = Src::d2(src.piece(C, 3));
-                    dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w; rhoj = q.x;
-                    uxj = u.x; uyj = u.y; uzj = w.x; qj = w.y;
-                }
-            } else {
-                double vtj_, hj_, xj, yj, zj, mj_d, rhoj_d;
-                int ptj, itj;
-                rec_aux(rec, j, vtj_, ptj, itj);
-                pair = ptj < 1000 && itj != 4;
-                if (pair) {
-                    rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, qj);
-                    rec_vel(rec, j, uxj, uyj, uzj, hj_);
-                    jrow = rowof[j] >= 0;
-                    dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
-                    mj = (float)mj_d; rhoj = (float)rhoj_d;
-                }
+        if constexpr (REC) {   // (every piece is read here: see walk_row)
+            const rec_f4 p = rec_.f[0], q = rec_.f[1];
+            const rec_d2 u = rec_.d[0], w = rec_.d[1];
+            pair = pair && crec_ptype(q.w) < 1000 && crec_itype(q.w) != 4;
+            jrow = crec_has_row(q.w);
+            dx = xf - p.x; dy = yf - p.y; dz = zf - p.z; mj = p.w; rhoj = q.x;
+            dux = (float)(u.x - uxi); duy = (float)(u.y - uyi); duz = (float)(w.x - uzi);
+            qj = w.y;
+        } else if (pair) {
+            double vtj_, hj_, xj, yj, zj, mj_d, rhoj_d, uxj, uyj, uzj;
+            int ptj, itj;
+            rec_aux(rec, j, vtj_, ptj, itj);
+            pair = ptj < 1000 && itj != 4;
+            if (pair) {
+                rec_pos(rec, j, xj, yj, zj, mj_d, rhoj_d, qj);
+                rec_vel(rec, j, uxj, uyj, uzj, hj_);
+                jrow = rowof[j] >= 0;
+                dx = (float)(xi - xj); dy = (float)(yi - yj); dz = (float)(zi - zj);
+                mj = (float)mj_d; rhoj = (float)rhoj_d;
+                dux = (float)(uxj - uxi); duy = (float)(uyj - uyi); duz = (float)(uzj - uzi);
             }
         }
         if (pair) {
@@ -859,9 +854,9 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
             const float cx = gc11 * tx + gc12 * ty + gc31 * tz, cy = gc12 * tx + gc22 * ty + gc23 * tz,
                         cz = gc31 * tx + gc23 * ty + gc33 * tz;
             const float vj = quot(mj, rhoj, yrho);
-            b[0] += (double)(vj * (float)(uxj - uxi) * cx * hm);
-            b[1] += (double)(vj * (float)(uyj - uyi) * cy * hm);
-            b[2] += (double)(vj * (float)(uzj - uzi) * cz * hm);
+            b[0] += (double)(vj * dux * cx * hm);
+            b[1] += (double)(vj * duy * cy * hm);
+            b[2] += (double)(vj * duz * cz * hm);
             const bool other = !src.self(j, i);
             // (with the values kept from the search's first step, only the known
             // neighbours' share of the right-hand side needs the coefficient)
@@ -885,7 +880,7 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
             }
             slot += __popc(m);
         }
-    }
+    });
 }
 template <class Src>
 __device__ __forceinline__ void assemble_mixed(const CaseDesc& cd, int i, const NList& nl, int li, const Src src, int g,

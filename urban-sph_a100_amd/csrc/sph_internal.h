@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/urbansph.h"
+#include "flags.h"
 
 namespace sph {
 
@@ -52,9 +53,10 @@ struct NList {
     const unsigned* ent;          // j | selection flags (flags.h)
 };
 // one particle's (or tile lane's) entries: entry k at p[k * SLICE]
-struct NLRow { const unsigned* p; int cnt; };
+typedef const __attribute__((address_space(1))) unsigned nl_entry;   // (a generic pointer's loads are flat ones)
+struct NLRow { nl_entry* p; int cnt; };
 __device__ __forceinline__ NLRow nl_row(const NList& nl, long long i) {
-    return {nl.ent + nl.slice_off[i >> 6] + (i & 63), nl.cnt[i]};
+    return {(nl_entry*)(nl.ent + nl.slice_off[i >> 6] + (i & 63)), nl.cnt[i]};
 }
 #define NB_AT(row, k) ((row).p[(size_t)(k) * SLICE])
 
@@ -428,6 +430,53 @@ struct LSrc {
     __device__ int gidx(int j) const { return halo[j]; }
     __device__ bool self(int j, int) const { return j == self_slot; }
 };
+
+// The record pieces of one entry's neighbour: NF float pieces, then ND pairs
+// of doubles.
+template <int NF, int ND>
+struct Pieces {
+    rec_f4 f[NF];
+    rec_d2 d[ND > 0 ? ND : 1];
+    template <class Src>
+    __device__ __forceinline__ void load(const Src& src, unsigned e) {
+        const auto C = src.at((int)(e & NB_IDX));
+#pragma unroll
+        for (int q = 0; q < NF; q++) f[q] = Src::f4(src.piece(C, q));
+#pragma unroll
+        for (int q = 0; q < ND; q++) d[q] = Src::d2(src.piece(C, NF + q));
+    }
+};
+// A lane's walk over entries g, g + W, ... of a row: body(entry, pieces) for
+// each (entry 0, without flags, where a lane of the group has none left).
+// While it works on one entry, the next one's record (REC: compact records) and
+// the entry after that are on their way; two sets of pieces take turns, since a
+// copy would wait for the loads, and the body reads every piece at its start:
+// read behind a branch, a piece is waited for together with the loads issued
+// after it.  Loaded when needed, the entry and its record cost a round two
+// memory latencies, with four or five waves a SIMD to hide them.  2.13 M canyon:
+// advection 1536 -> 1337 us, assembly 1460 -> 1219, strain 1349 -> 1228, pressure
+// force 892 -> 681; 20 k: 30 -> 24, 24 -> 20, 27 -> 22, 23 -> 15 us.  The double
+// records' six pieces, twice, cost more waves than they gain.
+template <bool REC, int NF, int ND, int W, class Src, class Body>
+__device__ __forceinline__ void walk_row(const NLRow& row, const Src& src, int g, Body&& body) {
+    const int last = row.cnt - 1;
+    if (last < 0) return;
+    Pieces<NF, ND> A, B;
+    // (beyond the end: the last entry again, dropped when its turn comes)
+    unsigned ea = NB_AT(row, min(g, last)), eb = NB_AT(row, min(g + W, last));
+    if constexpr (REC) A.load(src, ea);
+    for (int k = g; k - g < row.cnt; k += 2 * W) {
+        if constexpr (REC) B.load(src, eb);
+        const unsigned ec = NB_AT(row, min(k + 2 * W, last));
+        body(k < row.cnt ? ea : 0u, A);
+        if (k - g + W >= row.cnt) break;
+        if constexpr (REC) A.load(src, ec);
+        const unsigned ed = NB_AT(row, min(k + 3 * W, last));
+        body(k + W < row.cnt ? eb : 0u, B);
+        ea = ec;
+        eb = ed;
+    }
+}
 
 // Cell-tile passes (tiles.hip): a workgroup of TILE_THREADS per chunk of
 // `width` lanes.  TILE_CHUNK stages the chunk's halo records (RECF floats
