@@ -120,6 +120,9 @@ struct PPEView {
     float *fr, *frhat, *fp, *fphat, *fv, *fs, *fshat, *ft, *fx, *frhs;
     float* mgx0;                  // the multigrid V-cycle's finest-level x (allocated with the PPE when the
                                   // multigrid may run), or null: k_kr_p / k_kr_s write its pre-smoothing
+    // chunk partials of the reductions, three sets of nb: the products' (and the
+    // set-up's), s.s, and the iteration's last ones (a kernel that adds up one
+    // set itself writes another)
     double *partA, *partB;
     // MIXED: a row of more than LONG_ROW entries (a coarse row beside
     // refined particles) keeps its first LONG_ROW entries in the SELL slices
