@@ -36,12 +36,13 @@ namespace sph {
 // the loads that lead to its p_type (free slip, 2.13 M canyon: 222 us, with 16
 // lanes 131; FP64, 1 M: 380 and 186 us, a thread each 190; 20 k: 13, 14, 65).
 constexpr int BLANES = 16;
-#define SEG_BOUNDARY(sg)                                               \
+#define SEG_BOUNDARY(sg) SEG_BOUNDARY_LANES(sg, BLANES)
+#define SEG_BOUNDARY_LANES(sg, lanes)                                  \
     int first_;                                                        \
     const int cid_ = seg_case(sg, first_);                             \
     const CaseDesc& cd = sg.cd[cid_];                                  \
-    if ((sg).tab == nullptr) first_ *= 64 / BLANES;   /* blocks of blockDim * 64 / BLANES */ \
-    const int u_ = first_ / 64 + (int)threadIdx.x / BLANES, lane = (int)threadIdx.x % BLANES; \
+    if ((sg).tab == nullptr) first_ *= 64 / (lanes);   /* blocks of blockDim * 64 / lanes */ \
+    const int u_ = first_ / 64 + (int)threadIdx.x / (lanes), lane = (int)threadIdx.x % (lanes); \
     if (u_ >= cd.nm_count) return;                                     \
     const int i = cd.nm_list[u_];
 // GROUP lanes a particle (g_: the lane in its group)
@@ -140,8 +141,11 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_commit_positions(Seg sg) {
 __global__ void __launch_bounds__(MAX_BLOCK) k_snapshot(Seg sg, int which, int nm_pack) {
     SEG_PARTICLE(sg);
     const PView A = which ? cd.P : cd.S;
-    cd.snap[0][i] = A.ux[i]; cd.snap[1][i] = A.uy[i]; cd.snap[2][i] = A.uz[i];
-    cd.snap[3][i] = A.pres[i]; cd.snap[4][i] = A.temp[i];
+    cd.snap[3][i] = A.pres[i];
+    if (!nm_pack) {   // (the Neumann pass reads the pressures only)
+        cd.snap[0][i] = A.ux[i]; cd.snap[1][i] = A.uy[i]; cd.snap[2][i] = A.uz[i];
+        cd.snap[4][i] = A.temp[i];
+    }
     if (nm_pack && cd.nm_rec && i < cd.nm_nset) {   // the Neumann pass's records, from the same state
         const int j = cd.nm_set[i];
         const size_t n = (size_t)cd.nm_nset;
@@ -779,6 +783,7 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
     const int u = first_ >> 6, lane = threadIdx.x;
     if (u >= cd.nm_count) return;
     if (only_count0 && cd.count != 0) return;   // the extra pre-advection call, ISPH_Calc.cuh:88-90
+    if (sizeof(R) == 4 && cd.nmp_off) return;   // k_neumann_mixed
     const KConst kc = cd.kc;
     const sph_params pr = cd.pr;
     const PView A = which ? cd.P : cd.S;
@@ -819,64 +824,6 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
                 if (m) pres_g = __shfl(pj, 63 - __clzll(m), 64);
             }
         }
-    const int nt = inlet ? 8 : 5;
-    if (sizeof(R) == 4 && cd.nmp_off) {
-        // MIXED: each lane adds the terms of its share of the listed pairs
-        // (pairs lane, lane + 64, ... in list order), then a fixed butterfly
-        // adds the 64 lane sums; lane 0's total is used, so the sums are the
-        // same on every call, alone or in a batch
-        const HScale hs(kc, (float)hi);
-        const float dwf = dw_factor<float>(kc, (float)hi);
-        float rho_c = -1.0f, yrho = 0.0f;
-        double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        const long long e0 = cd.nmp_off[u], e1 = cd.nmp_off[u + 1];
-        const float* const nrec = cd.nm_rec;   // the same values, packed (float-exact positions)
-        const size_t nn = (size_t)cd.nm_nset;
-        for (long long e = e0 + lane; e < e1; e += 64) {
-            double xj, yj, zj, presj;
-            float mj, rhoj, uxj, uyj, uzj;
-            if (nrec) {
-                const unsigned C = (unsigned)cd.nmp_cent[e] * 16u;
-                const rec_f4 a = ld_f4(nrec, C), b = ld_f4(nrec + 4 * nn, C);
-                xj = a.x; yj = a.y; zj = a.z; mj = a.w; rhoj = b.x; uxj = b.y; uyj = b.z; uzj = b.w;
-                presj = ld_d2(nrec + 8 * nn, C).x;
-            } else {
-                const int j = cd.nmp_ent[e];
-                xj = A.x[j]; yj = A.y[j]; zj = A.z[j]; mj = (float)A.m[j]; rhoj = (float)A.rho[j];
-                uxj = (float)A.ux[j]; uyj = (float)A.uy[j]; uzj = (float)A.uz[j];
-                presj = pold[j];
-            }
-            if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
-            // (the list holds exactly the pairs inside the search range)
-            const float dx = (float)(xg - xj), dy = (float)(yg - yj), dz = (float)(zg - zj);
-            const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
-            const float tR = hs.tR(d.r), w = kernel_w_t<float>(kc, (float)tmp_A, tR), vj = quot(mj, rhoj, yrho);
-            s[0] += (double)(vj * (float)presj * w);
-            s[1] += (double)(vj * uxj * w);
-            s[2] += (double)(vj * uyj * w);
-            s[3] += (double)(vj * uzj * w);
-            s[4] += (double)(vj * w);
-            if (inlet) {
-                const float dw = kernel_dw_t<float>(kc, (float)tmp_A, dwf, tR), dp = vj * (float)(presj - pres_g);
-                s[5] += (double)(dp * (quot(dx, d.r, d.y) * dw));
-                s[6] += (double)(dp * (quot(dy, d.r, d.y) * dw));
-                s[7] += (double)(dp * (quot(dz, d.r, d.y) * dw));
-            }
-        }
-        for (int off = 32; off > 0; off >>= 1)
-            for (int q = 0; q < 8; q++)
-                if (q < nt) s[q] += __shfl_xor(s[q], off, 64);
-        if (lane != 0) return;
-        const double tflt = s[4];
-        if (tflt < 1e-6) {
-            A.pres[i] = 0.0;
-        } else {
-            A.pres[i] = s[0] / tflt;
-            if (A.p_type[i] == -1) { A.ux[i] = s[1] / tflt; A.uy[i] = s[2] / tflt; A.uz[i] = s[3] / tflt; }
-            if (inlet) A.pres[i] = pres_g + (xi - xg) * s[5] + (yi - yg) * s[6] + (zi - zg) * s[7];
-        }
-        return;
-    }
     // FP64: each lane forms the terms of one candidate exactly as the serial
     // scan does, and the sums are added in candidate order (OrderedSums).
     // (Each lane adding the terms that a flag marked, one LDS read after
@@ -934,6 +881,111 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
         A.pres[i] = tpres / tflt_s;
         if (A.p_type[i] == -1) { A.ux[i] = tux / tflt_s; A.uy[i] = tuy / tflt_s; A.uz[i] = tuz / tflt_s; }
         if (bt == 1 || bt == -1) A.pres[i] = pres_g + (xi - xg) * grad_px + (yi - yg) * grad_py + (zi - zg) * grad_pz;
+    }
+}
+
+// The listed pairs of one boundary particle (nm_cent or particle numbers) as
+// a row of entries for walk_row; every entry counts.
+struct NMRow {
+    const int* p;
+    int cnt;
+    __device__ unsigned at(int k) const {
+        return (unsigned)((const __attribute__((address_space(1))) int*)p)[k] | F_DP;
+    }
+};
+// MIXED with listed pairs: NM_LANES lanes a boundary particle, each adding the
+// terms of pairs lane, lane + NM_LANES, ... in list order, then a fixed butterfly
+// (so the sums are the same on every call, alone or in a batch).  A wave a
+// particle spent most of its time on the loads before its few rounds.  By lanes
+// (64 without the pipelined walk, 32, 16): 374, 273, 238 us on the 2.13 M canyon,
+// 91, 67, 63 on 200 k, 20.6, 19.3, 24.3 on 20 k, 171, 198, 355 on a refined canyon,
+// whose 329 markers have thousands of pairs.
+constexpr int NM_LANES = 32;
+__global__ void __launch_bounds__(WAVE_BLOCK) k_neumann_mixed(Seg sg, int which, int only_count0) {
+    SEG_BOUNDARY_LANES(sg, NM_LANES);
+    if (only_count0 && cd.count != 0) return;   // the extra pre-advection call, ISPH_Calc.cuh:88-90
+    if (!cd.nmp_off) return;                    // k_neumann
+    const KConst kc = cd.kc;
+    const sph_params& pr = cd.pr;
+    const PView A = which ? cd.P : cd.S;
+    const Grid g = cd.g;
+    const double* const pold = cd.snap[3];
+    const float hi = (float)(2.0 * A.h[i]), tmp_A = calc_tmpA<float>(kc, hi);
+    const double xi = A.x[i], yi = A.y[i], zi = A.z[i];
+    const int bt = A.buffer_type[i];
+    const bool inlet = (bt == 1 || bt == -1);
+    const double xg = inlet ? 2.0 * pr.L2 - xi : xi;
+    double pres_g = 0;
+    if (inlet) {   // the ghost pressure: see k_neumann
+        const Cell c = query_cell(g.d, xg, yi, zi);
+        const int first = (int)(threadIdx.x & 63) & ~(NM_LANES - 1);
+        for (int z = -1; z <= 1; z++)
+            for (int y = -1; y <= 1; y++) {
+                int2 rg;
+                if (!row_range(g, c.i - 1, c.i + 1, c.j + y, c.k + z, rg)) continue;
+                for (int b = rg.x; b < rg.y; b += NM_LANES) {
+                    const int j = b + lane;
+                    bool hit = false;
+                    double pj = 0.0;
+                    if (j < rg.y) {
+                        const float dx = (float)(xg - A.x[j]), dy = (float)(yi - A.y[j]), dz = (float)(zi - A.z[j]);
+                        const float dist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20f;
+                        hit = dist < (float)pr.neumann_ghost_r;
+                        pj = pold[j];
+                    }
+                    const unsigned m = (unsigned)(__ballot(hit) >> first) & ((unsigned)(~0ULL >> (64 - NM_LANES)));
+                    if (m) pres_g = __shfl(pj, first + 31 - __clz((int)m), 64);
+                }
+            }
+    }
+    const HScale hs(kc, hi);
+    const float dwf = dw_factor<float>(kc, hi);
+    float rho_c = -1.0f, yrho = 0.0f;
+    double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    auto add = [&](float dx, float dy, float dz, float mj, float rhoj, float uxj, float uyj, float uzj, double presj) {
+        if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
+        // (the list holds exactly the pairs inside the search range)
+        const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
+        const float tR = hs.tR(d.r), w = kernel_w_t<float>(kc, tmp_A, tR), vj = quot(mj, rhoj, yrho);
+        s[0] += (double)(vj * (float)presj * w);
+        s[1] += (double)(vj * uxj * w);
+        s[2] += (double)(vj * uyj * w);
+        s[3] += (double)(vj * uzj * w);
+        s[4] += (double)(vj * w);
+        if (inlet) {
+            const float dw = kernel_dw_t<float>(kc, tmp_A, dwf, tR), dp = vj * (float)(presj - pres_g);
+            s[5] += (double)(dp * (quot(dx, d.r, d.y) * dw));
+            s[6] += (double)(dp * (quot(dy, d.r, d.y) * dw));
+            s[7] += (double)(dp * (quot(dz, d.r, d.y) * dw));
+        }
+    };
+    const long long e0 = cd.nmp_off[u_];
+    const int cnt = (int)(cd.nmp_off[u_ + 1] - e0);
+    if (cd.nm_rec) {   // packed, with float-exact positions (see walk_row)
+        const GSrc src{&cd.nm_rec, (size_t)cd.nm_nset};
+        walk_row<true, 2, 1, NM_LANES>(NMRow{cd.nmp_cent + e0, cnt}, src, lane, [&](unsigned e, const Pieces<2, 1>& r) {
+            const rec_f4 a = r.f[0], b = r.f[1];
+            const float dx = (float)(xg - (double)a.x), dy = (float)(yi - (double)a.y), dz = (float)(zi - (double)a.z);
+            const double presj = r.d[0].x;
+            if (e) add(dx, dy, dz, a.w, b.x, b.y, b.z, b.w, presj);
+        });
+    } else {
+        walk_row<false, 1, 0, NM_LANES>(NMRow{cd.nmp_ent + e0, cnt}, 0, lane, [&](unsigned e, const Pieces<1, 0>&) {
+            if (!e) return;
+            const int j = (int)(e & NB_IDX);
+            add((float)(xg - A.x[j]), (float)(yi - A.y[j]), (float)(zi - A.z[j]), (float)A.m[j], (float)A.rho[j],
+                (float)A.ux[j], (float)A.uy[j], (float)A.uz[j], pold[j]);
+        });
+    }
+    for (double& v : s) group_fold<NM_LANES>(v);
+    if (lane != 0) return;
+    const double tflt = s[4];
+    if (tflt < 1e-6) {
+        A.pres[i] = 0.0;
+    } else {
+        A.pres[i] = s[0] / tflt;
+        if (A.p_type[i] == -1) { A.ux[i] = s[1] / tflt; A.uy[i] = s[2] / tflt; A.uz[i] = s[3] / tflt; }
+        if (inlet) A.pres[i] = pres_g + (xi - xg) * s[5] + 0.0 * s[6] + 0.0 * s[7];
     }
 }
 
@@ -1903,10 +1955,11 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
 // launch over the particles of every case; tunable passes (kid >= 0) run at
 // the workgroup size the autotuner picked for this batch size
 // a boundary pass with a 64-lane wave per boundary particle of each case
-#define BOUNDL(name, kern, ...)                                                                        \
+#define BOUNDL(name, kern, ...) BOUNDW(name, BLANES, kern, ##__VA_ARGS__)
+#define BOUNDW(name, lanes, kern, ...)                                                                        \
     do {                                                                                            \
         Shape sh_;                                                                                  \
-        SPH_TRY(shape(e, 3, WAVE_BLOCK * (64 / BLANES), &sh_));                                                     \
+        SPH_TRY(shape(e, 3, WAVE_BLOCK * (64 / (lanes)), &sh_));                                                     \
         if (sh_.grid > 0) {                                                                         \
             SPH_TRY(prof_begin(e, name, 0.0));                                                      \
             hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(WAVE_BLOCK), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
@@ -2105,10 +2158,14 @@ int neumann_pairs(sph_ctx* c) {
 
 static int run_neumann(Eng& e, int which, int only_count0) {
     SEGL("snapshot", -1, k_snapshot, which, 1);
+    bool listed = false, general = !mixed_of(e);   // MIXED cases with and without listed pairs
+    for (size_t k = 0; k < e.cs.size() && mixed_of(e); k++)
+        (e.h_desc[k].nmp_off ? listed : general) = true;
+    if (listed) BOUNDW("neumann", NM_LANES, k_neumann_mixed, which, only_count0);
     // one 64-thread block (one wave) per boundary particle of each case
     Shape sh;
     SPH_TRY(shape(e, 3, 64, &sh));
-    if (sh.grid > 0) {
+    if (general && sh.grid > 0) {
         SPH_TRY(prof_begin(e, "neumann", 0.0));
         if (mixed_of(e))
             hipLaunchKernelGGL(k_neumann<float>, dim3(sh.grid), dim3(64), 0, e.st, Seg{e.d_desc, sh.tab}, which,

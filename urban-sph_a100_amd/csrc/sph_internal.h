@@ -54,11 +54,15 @@ struct NList {
 };
 // one particle's (or tile lane's) entries: entry k at p[k * SLICE]
 typedef const __attribute__((address_space(1))) unsigned nl_entry;   // (a generic pointer's loads are flat ones)
-struct NLRow { nl_entry* p; int cnt; };
+struct NLRow {
+    nl_entry* p;
+    int cnt;
+    __device__ unsigned at(int k) const { return p[(size_t)k * SLICE]; }
+};
 __device__ __forceinline__ NLRow nl_row(const NList& nl, long long i) {
     return {(nl_entry*)(nl.ent + nl.slice_off[i >> 6] + (i & 63)), nl.cnt[i]};
 }
-#define NB_AT(row, k) ((row).p[(size_t)(k) * SLICE])
+#define NB_AT(row, k) ((row).at(k))
 
 // Cell tiles of the record-gathering passes (tiles.hip): chunks of at most
 // tile_particles particles of one block of cells, each with its halo.
@@ -460,21 +464,21 @@ struct Pieces {
 // advection 1536 -> 1337 us, assembly 1460 -> 1219, strain 1349 -> 1228, pressure
 // force 892 -> 681; 20 k: 30 -> 24, 24 -> 20, 27 -> 22, 23 -> 15 us.  The double
 // records' six pieces, twice, cost more waves than they gain.
-template <bool REC, int NF, int ND, int W, class Src, class Body>
-__device__ __forceinline__ void walk_row(const NLRow& row, const Src& src, int g, Body&& body) {
+template <bool REC, int NF, int ND, int W, class Row, class Src, class Body>
+__device__ __forceinline__ void walk_row(const Row& row, const Src& src, int g, Body&& body) {
     const int last = row.cnt - 1;
     if (last < 0) return;
     Pieces<NF, ND> A, B;
     // (beyond the end: the last entry again, dropped when its turn comes)
-    unsigned ea = NB_AT(row, min(g, last)), eb = NB_AT(row, min(g + W, last));
+    unsigned ea = row.at(min(g, last)), eb = row.at(min(g + W, last));
     if constexpr (REC) A.load(src, ea);
     for (int k = g; k - g < row.cnt; k += 2 * W) {
         if constexpr (REC) B.load(src, eb);
-        const unsigned ec = NB_AT(row, min(k + 2 * W, last));
+        const unsigned ec = row.at(min(k + 2 * W, last));
         body(k < row.cnt ? ea : 0u, A);
         if (k - g + W >= row.cnt) break;
         if constexpr (REC) A.load(src, ec);
-        const unsigned ed = NB_AT(row, min(k + 3 * W, last));
+        const unsigned ed = row.at(min(k + 3 * W, last));
         body(k + W < row.cnt ? eb : 0u, B);
         ea = ec;
         eb = ed;
