@@ -1002,21 +1002,20 @@ __global__ void __launch_bounds__(BLOCK) k_kr_long(Seg sg) {
     if (lane == 0) pp.lsum[u] = s;
 }
 
-// r = rhs - A x ; rhat = r ; partials rhs.rhs (A) and r.r (B).  ZERO: x is
-// zero (the inner solves of the mixed mode start from it), so r = rhs and
-// the product is not formed
-template <class V, class X, bool ZERO>
+// r = rhs - A x ; rhat = r ; partials rhs.rhs (A) and r.r (B).  (The inner
+// solves of the mixed mode start from x = 0: k_outer_res sets them up.)
+template <class V, class X>
 __global__ void __launch_bounds__(BLOCK) k_kr_init(Seg sg) {
     __shared__ double sh[2 * BLOCK];
     __shared__ int wbase[BLOCK];
     SEG_ROW(sg);
     if (SKIPPED(cd)) return;
     const PPEView pp = cd.ppe;
-    if (!ZERO) load_group_bases(pp, first_, wbase);
+    load_group_bases(pp, first_, wbase);
     const KSet<X> K = kset(pp, (X*)nullptr);
     double a = 0.0, b = 0.0;
     if (row < pp.nr) {
-        double y = ZERO ? 0.0 : spmv_row(pp, row, vals_of(pp, (V*)nullptr), kdiag(pp, (X*)nullptr), K.x, wbase);
+        double y = spmv_row(pp, row, vals_of(pp, (V*)nullptr), kdiag(pp, (X*)nullptr), K.x, wbase);
         X rr = (X)((double)K.rhs[row] - y);
         K.r[row] = rr;
         K.rhat[row] = rr;
@@ -1186,7 +1185,8 @@ __global__ void __launch_bounds__(BLOCK) k_kr_xr(Seg sg) {
 // One block per case: reduce the case's chunk partials canonically and
 // advance its scalars.
 // FIN_RS: FIN_S and FIN_R, of an iteration whose other steps were folded.
-enum FinOp { FIN_INIT, FIN_ALPHA, FIN_S, FIN_OMEGA, FIN_R, FIN_RS, FIN_NORM };
+// FIN_INIT0: FIN_INIT of a solve that starts from x = 0 (k_outer_res).
+enum FinOp { FIN_INIT, FIN_INIT0, FIN_ALPHA, FIN_S, FIN_OMEGA, FIN_R, FIN_RS, FIN_NORM };
 constexpr int FIN_BLOCK = 1024;
 __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int op) {
     __shared__ double lvl[256];
@@ -1194,7 +1194,7 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int o
     double* sc = cd.sc;
     const double* ctl = cd.ctl;
     if (ctl[CTL_SKIP] != 0.0) {
-        if (op == FIN_INIT && threadIdx.x == 0) {
+        if ((op == FIN_INIT || op == FIN_INIT0) && threadIdx.x == 0) {
             sc[SC_DONE] = 1.0; sc[SC_HALF] = 0.0; sc[SC_CONV] = 0.0; sc[SC_ITERS] = 0.0; sc[SC_ZEROX] = 0.0;
         }
         return;
@@ -1202,7 +1202,7 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int o
     const bool half = sc[SC_HALF] == 1.0;
     if (op == FIN_R) {
         if (sc[SC_DONE] != 0.0 && !half) return;
-    } else if (op != FIN_INIT && op != FIN_NORM) {
+    } else if (op != FIN_INIT && op != FIN_INIT0 && op != FIN_NORM) {
         if (sc[SC_DONE] != 0.0) return;
     }
     if (op == FIN_R && half) {
@@ -1211,7 +1211,7 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int o
     }
     const long long nb = cd.ppe.nb;
     const bool last = op == FIN_R || op == FIN_RS;
-    const long long set = last ? 2 * nb : op == FIN_S ? nb : 0;
+    const long long set = last ? 2 * nb : op == FIN_S || op == FIN_INIT0 ? nb : 0;
     double A = canon_partials(cd.ppe.partA + set, nb, lvl);
     double B = 0.0, ss = 0.0;
     if (op == FIN_INIT || op == FIN_OMEGA || last || op == FIN_NORM) B = canon_partials(cd.ppe.partB + set, nb, lvl);
@@ -1219,6 +1219,7 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int o
     if (threadIdx.x != 0) return;
     const double tol = ctl[CTL_TOL];
     switch (op) {
+    case FIN_INIT0: B = A; [[fallthrough]];   // r = rhs
     case FIN_INIT: {
         double bnorm = sqrt(A), rnorm = sqrt(B);
         sc[SC_BNORM] = bnorm; sc[SC_RNORM] = rnorm;
@@ -1273,7 +1274,10 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_kr_fin(const CaseDesc* cds, int o
 }
 
 // outer residual of the mixed solve: r = rhs - A x (double x, float values,
-// double accumulation); partials r.r (A) and rhs.rhs (B); float copy of r
+// double accumulation); partials r.r (A) and rhs.rhs (B).  And the start of the
+// inner solve for the correction, in case one follows: its right-hand side
+// and residual are the float copy of r, its x is zero; partials f.f (the second
+// set).  (As kernels of their own these were three launches a refinement.)
 __global__ void __launch_bounds__(BLOCK) k_outer_res(Seg sg) {
     __shared__ double sh[2 * BLOCK];
     __shared__ int wbase[BLOCK];
@@ -1281,29 +1285,30 @@ __global__ void __launch_bounds__(BLOCK) k_outer_res(Seg sg) {
     if (SKIPPED(cd)) return;
     const PPEView pp = cd.ppe;
     load_group_bases(pp, first_, wbase);
-    double a = 0.0, b = 0.0;
+    double a = 0.0, b = 0.0, f2 = 0.0;
     if (row < pp.nr) {
         double y = spmv_row(pp, row, (const float*)pp.vals32, (const double*)pp.diag, (const double*)pp.x, wbase);
         double rr = pp.rhs[row] - y;
-        pp.frhs[row] = (float)rr;
+        const float f = (float)rr;
+        pp.frhs[row] = f;
+        pp.fr[row] = f;
+        pp.frhat[row] = f;
+        pp.fx[row] = 0.0f;
         a = rr * rr;
         b = pp.rhs[row] * pp.rhs[row];
+        f2 = (double)f * (double)f;
     }
     const Pair t2 = block_canon2(a, b, sh);
     if (threadIdx.x == 0) pp.partA[chunk] = t2.a;
     if (threadIdx.x == 64) pp.partB[chunk] = t2.b;
+    const double tf = block_canon(f2, sh);
+    if (threadIdx.x == 0) pp.partA[pp.nb + chunk] = tf;
 }
 __global__ void __launch_bounds__(BLOCK) k_add_correction(Seg sg) {
     SEG_ROW(sg);
     if (SKIPPED(cd)) return;
     const PPEView pp = cd.ppe;
     if (row < pp.nr) pp.x[row] = pp.x[row] + (double)pp.fx[row];
-}
-__global__ void __launch_bounds__(BLOCK) k_zero_fx(Seg sg) {
-    SEG_ROW(sg);
-    if (SKIPPED(cd)) return;
-    const PPEView pp = cd.ppe;
-    if (row < pp.nr) pp.fx[row] = 0.0f;
 }
 template <class T>
 __global__ void __launch_bounds__(BLOCK) k_zero(long long n, T* a) {
@@ -1996,14 +2001,14 @@ static int bicgstab(Eng& e, int gi, int pred_slot, std::vector<int>& iters, bool
         maxit = std::max(maxit, (int)e.h_ctl[k * CTL_COUNT + CTL_MAXIT]);
     }
     if (mg) e.mg_plan.spmv_bytes0 = spmv_bytes0;
-    if (x_zero) {
-        RL("kr_init", 0, (k_kr_init<V, X, true>));
+    if (x_zero) {   // set up by k_outer_res
+        KF(FIN_INIT0);
     } else {
         RLONG(V, X, 0);
-        RL("kr_init", spmv_bytes, (k_kr_init<V, X, false>));
+        RL("kr_init", spmv_bytes, (k_kr_init<V, X>));
+        KF(FIN_INIT);
+        RL("kr_zerox", 0, k_kr_zerox<X>);
     }
-    KF(FIN_INIT);
-    RL("kr_zerox", 0, k_kr_zerox<X>);
     auto all_done = [&]() {
         for (int k = 0; k < nc; k++)
             if (e.h_ctl[k * CTL_COUNT + CTL_SKIP] == 0.0 && e.h_sc[k * SC_COUNT + SC_DONE] == 0.0) return false;
@@ -2304,7 +2309,6 @@ int ppe_solve(Eng& e) {
             }
             SPH_TRY(ctl_upload(e));
             if (!any) break;
-            RL("zero_fx", 0, k_zero_fx);
             SPH_TRY((bicgstab<float, float>(e, any_mg ? 2 : 1, outer, iters, any_mg, true)));
             bool stalled = false;
             for (int k = 0; k < nc; k++) {
