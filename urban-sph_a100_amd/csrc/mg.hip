@@ -913,6 +913,41 @@ __global__ void __launch_bounds__(BLOCK) k_mg_restrict(const CaseDesc* cds, cons
     // the next level's pre-smoothing, x = w b / diag, when it has a level below
     if (l + 1 < L.lc) N.x[row] = (float)(MG_OMEGA * (double)b / (double)N.diag[row]);
 }
+// The residual of coarse level l and its restriction in one pass, for levels
+// of few rows, whose passes cost their launch and a chain of loads: RR_LANES
+// lanes an aggregate of level l + 1, MG_G a member's row, the members' residuals
+// added in member order (the same bits as the two passes).
+constexpr int RR_LANES = 32;
+// (rows of the step's cases on the level: the 200 k request's 30 launches fewer
+// an iteration pair are 51.4 -> 50.2 ms; a level of 240 k rows loses 9 us by its
+// scattered rows what the launch gains)
+constexpr long long RR_ROWS = 40000;
+__global__ void __launch_bounds__(BLOCK) k_mg_res_restrict(const CaseDesc* cds, const MGLv* lv, const int2* tab, int l,
+                                                           int sc_done) {
+    const int2 te_ = tab[xcd_block()];
+    const CaseDesc& cd = cds[te_.x];
+    if (cd.sc[sc_done] != 0.0) return;
+    const MGLv& L = lv[te_.x * MG_MAX_LEVELS + l];
+    const MGLv& N = lv[te_.x * MG_MAX_LEVELS + l + 1];
+    const int row = te_.y + (int)threadIdx.x / RR_LANES, g = (int)threadIdx.x % RR_LANES;
+    if (row >= N.n) return;
+    const int first = (int)(threadIdx.x & 63) & ~(RR_LANES - 1);
+    const int t0 = L.mstart[row], cnt = L.mstart[row + 1] - t0;
+    constexpr int M = RR_LANES / MG_G;   // members a round
+    double s = 0.0;
+    for (int c = 0; c < cnt; c += M) {
+        float r = 0.0f;
+        if (c + g / MG_G < cnt) {
+            const int m = L.mem[t0 + c + g / MG_G];
+            r = (float)((double)L.b[m] - coarse_ax_g(L, m, g % MG_G));
+        }
+        for (int t = 0; t < min(M, cnt - c); t++) s += (double)__shfl(r, first + t * MG_G, 64);
+    }
+    if (g != 0) return;
+    const float b = (float)s;
+    N.b[row] = b;
+    if (l + 1 < L.lc) N.x[row] = (float)(MG_OMEGA * (double)b / (double)N.diag[row]);
+}
 // level 0: the tail sums of the long rows over the current x, one wave per
 // long row, lanes over its contiguous tail, fixed shuffle tree (tab: four
 // long rows per block)
@@ -1379,10 +1414,7 @@ int mg_prepare(Eng& e, const std::vector<const MGState*>& mgs, int sc_done, bool
             D.lidx = S.lidx;
         }
     }
-    auto rows_table = [&](int l, bool below, int* off, int* cnt, int* blk) {
-        // the coarse levels' residual and post-smoothing passes run MG_G
-        // lanes per row
-        const int lanes = (below && l > 0) ? MG_G : 1;
+    auto rows_table = [&](int l, bool below, int lanes, int* off, int* cnt, int* blk) {
         auto has = [&](const MGState* mg) { return mg && (below ? l < mg->nlev - 1 : l <= mg->nlev - 1); };
         long long threads = 0;
         for (int k = 0; k < nc; k++)
@@ -1395,8 +1427,15 @@ int mg_prepare(Eng& e, const std::vector<const MGState*>& mgs, int sc_done, bool
         *cnt = (int)tab.size() - *off;
     };
     for (int l = 0; l < P.lmax; l++) {
-        rows_table(l, true, &P.down_off[l], &P.down_cnt[l], &P.down_blk[l]);
-        rows_table(l, false, &P.lvl_off[l], &P.lvl_cnt[l], &P.lvl_blk[l]);
+        // (the coarse levels' residual and post-smoothing passes: MG_G lanes a row)
+        rows_table(l, true, l > 0 ? MG_G : 1, &P.down_off[l], &P.down_cnt[l], &P.down_blk[l]);
+        rows_table(l, false, 1, &P.lvl_off[l], &P.lvl_cnt[l], &P.lvl_blk[l]);
+        long long rows = 0;
+        for (int k = 0; k < nc; k++)
+            if (mgs[k] && l < mgs[k]->nlev - 1) rows += mgs[k]->L[l].n;
+        P.rr_cnt[l] = 0;
+        if (l > 0 && l + 1 < P.lmax && rows <= RR_ROWS)
+            rows_table(l + 1, false, RR_LANES, &P.rr_off[l], &P.rr_cnt[l], &P.rr_blk[l]);
     }
     P.dense_off = (int)tab.size();
     for (int k = 0; k < nc; k++) {
@@ -1469,6 +1508,10 @@ int mg_apply(Eng& e, int which, int sc_done) {
     for (int l = 0; l + 1 < P.lmax; l++) {
         if (l == 0) MGE("mg_long", 0, P.long_off, P.long_cnt, k_mg_long, sc_done);
         else MGE("mg_clong", 0, P.clong_off[l], P.clong_cnt[l], k_mg_clong, l, sc_done);
+        if (P.rr_cnt[l] > 0) {
+            MGB("mg_res", 0, P.rr_off[l], P.rr_cnt[l], P.rr_blk[l], k_mg_res_restrict, l, sc_done);
+            continue;
+        }
         if (l == 0) MGB("mg_res0", P.spmv_bytes0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_res, l, which, sc_done);
         else MGB("mg_res", 0, P.down_off[l], P.down_cnt[l], P.down_blk[l], k_mg_res_g, l, sc_done);
         MGB("mg_restrict", 0, P.lvl_off[l + 1], P.lvl_cnt[l + 1], P.lvl_blk[l + 1], k_mg_restrict, l, sc_done);

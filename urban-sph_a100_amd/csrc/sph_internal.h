@@ -607,6 +607,7 @@ struct Eng {
         int down_off[16], down_cnt[16];   // rows of level l, cases with a level below l
         int lvl_off[16], lvl_cnt[16];     // rows of level l, cases that have level l
         int down_blk[16], lvl_blk[16];    // threads of their blocks
+        int rr_off[16], rr_cnt[16], rr_blk[16];   // level l's residual with its restriction (cnt 0: apart)
         int dense_off = 0, dense_cnt = 0; // coarsest rows, four per block
         int long_off = 0, long_cnt = 0;   // level-0 long rows, four per block
         int clong_off[16], clong_cnt[16]; // coarse level l's long rows, four per block
