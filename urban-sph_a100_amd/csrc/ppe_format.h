@@ -63,14 +63,52 @@ __device__ __forceinline__ double row_sum(int m, LD&& ld, MAC&& mac) {
 }
 template <class V, class X> struct Term { V v; X x; };
 template <class V> constexpr int row_u() { return sizeof(V) == 8 ? ROW_U_F64 : ROW_U; }
+// The same for double entries with stored columns: while a round's x values
+// are gathered, the next round's entries are on their way, so a round costs one
+// memory latency, not two.  32^3 box 21.3 -> 18.8 us a product, 4 k 15.9 -> 15.3,
+// 150 k canyon the same 27; the float products, 16 entries a round, lose more
+// waves to the registers than they gain (35 -> 40 us on 300 k, 130 -> 148 on
+// 2.13 M).  ld(k): entry k; x_of(entry): its x; val(entry): its value.
+template <class E, class X, int U, class LD, class XOF, class VAL>
+__device__ __forceinline__ double row_sum_cols(int m, LD&& ld, XOF&& x_of, VAL&& val) {
+    double s = 0.0;
+    if (m <= 0) return s;
+    E a[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) a[u] = ld(min(u, m - 1));
+    int k = 0;
+    for (; k + U < m; k += U) {
+        X x[U];
+        E b[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = x_of(a[u]);
+#pragma unroll
+        for (int u = 0; u < U; u++) b[u] = ld(min(k + U + u, m - 1));
+#pragma unroll
+        for (int u = 0; u < U; u++) s += (double)val(a[u]) * (double)x[u];
+#pragma unroll
+        for (int u = 0; u < U; u++) a[u] = b[u];
+    }
+    X x[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) x[u] = x_of(a[u]);
+#pragma unroll
+    for (int u = 0; u < U; u++) s = k + u < m ? s + (double)val(a[u]) * (double)x[u] : s;
+    return s;
+}
+template <class V, class C> struct Entry { V v; C c; };
 template <class V, class X, bool NT>
 __device__ __forceinline__ double offdiag_i32(const int* cp, const V* vp, int m, const X* x) {
-    return row_sum<Term<V, X>, row_u<V>()>(
-        m,
-        [&](int k) {
-            return Term<V, X>{ld_matrix<NT>(vp + pslot(k)), x[ld_matrix<NT>(cp + pslot(k))]};
-        },
-        [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
+    if constexpr (sizeof(V) == 8) {
+        typedef Entry<V, int> E;
+        return row_sum_cols<E, X, row_u<V>()>(
+            m, [&](int k) { return E{ld_matrix<NT>(vp + pslot(k)), ld_matrix<NT>(cp + pslot(k))}; },
+            [&](const E& e) { return x[e.c]; }, [](const E& e) { return e.v; });
+    } else {
+        return row_sum<Term<V, X>, row_u<V>()>(
+            m, [&](int k) { return Term<V, X>{ld_matrix<NT>(vp + pslot(k)), x[ld_matrix<NT>(cp + pslot(k))]}; },
+            [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
+    }
 }
 // The same over 16-bit columns: entry e = (group << EC_OFF_BITS) | offset,
 // column = wb[group] + offset, wb = the slice's group bases (in LDS).
@@ -78,13 +116,16 @@ __device__ __forceinline__ int ecol(const int* wb, int e) { return wb[e >> EC_OF
 template <class V, class X, bool NT>
 __device__ __forceinline__ double offdiag_u16(const unsigned short* ep, const V* vp, int m, const int* wb,
                                               const X* x) {
-    return row_sum<Term<V, X>, row_u<V>()>(
-        m,
-        [&](int k) {
-            return Term<V, X>{ld_matrix<NT>(vp + pslot(k)),
-                              x[ecol(wb, ld_matrix<NT>(ep + pslot(k)))]};
-        },
-        [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
+    if constexpr (sizeof(V) == 8) {
+        typedef Entry<V, unsigned short> E;
+        return row_sum_cols<E, X, row_u<V>()>(
+            m, [&](int k) { return E{ld_matrix<NT>(vp + pslot(k)), ld_matrix<NT>(ep + pslot(k))}; },
+            [&](const E& e) { return x[ecol(wb, e.c)]; }, [](const E& e) { return e.v; });
+    } else {
+        return row_sum<Term<V, X>, row_u<V>()>(
+            m, [&](int k) { return Term<V, X>{ld_matrix<NT>(vp + pslot(k)), x[ecol(wb, ld_matrix<NT>(ep + pslot(k)))]}; },
+            [](double s, const Term<V, X>& t) { return s + (double)t.v * (double)t.x; });
+    }
 }
 
 // The same over a stencil slice: column row + off[k], off the slice's
