@@ -48,8 +48,6 @@ __global__ void __launch_bounds__(BLOCK) k_hash(int n, sph_domain d, const int* 
 
 // ------------------------------------------------------------------------
 // radix sort
-constexpr int RS_ITEMS = 8;
-constexpr int RS_TILE = BLOCK * RS_ITEMS;
 
 __global__ void __launch_bounds__(BLOCK) k_rs_hist(const int* keys, int n, int shift, int ntiles, int* hist) {
     __shared__ int h[256];
@@ -65,14 +63,36 @@ __global__ void __launch_bounds__(BLOCK) k_rs_hist(const int* keys, int n, int s
     hist[threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
+// offs: the histogram's prefixes within its scan tiles, sums: the tiles' sums
+// (nsums of them).  Each block adds the sums of the tiles before its entries:
+// thread t scans the t-th of 256 runs of sums, and a digit's base is the runs
+// before its tile's and the rest of that run.  As launches of their own the scan
+// of the sums and the addition were two of five a digit, of 2-3 us each with the
+// host's 6-15 us between them where a refinement pass searches 150 k particles.
 __global__ void __launch_bounds__(BLOCK) k_rs_scatter(const int* kin, const int* vin, int* kout, int* vout, int n,
-                                                      int shift, int ntiles, const int* offs) {
+                                                      int shift, int ntiles, const int* offs, const int* sums,
+                                                      int nsums) {
     __shared__ int cnt[256];
     __shared__ int wc[BLOCK / 64][256];
     __shared__ int boff[256];
+    __shared__ int run[BLOCK];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     cnt[tid] = 0;
-    boff[tid] = offs[tid * ntiles + blockIdx.x];
+    const int entry = tid * ntiles + blockIdx.x, tile = entry / RS_TILE, per = (nsums + BLOCK - 1) / BLOCK;
+    int base_d = offs[entry];
+    int s = 0;
+    for (int q = tid * per; q < min(nsums, (tid + 1) * per); q++) s += sums[q];
+    run[tid] = s;
+    __syncthreads();
+    for (int off = 1; off < BLOCK; off <<= 1) {
+        const int a = tid >= off ? run[tid - off] : 0;
+        __syncthreads();
+        run[tid] += a;
+        __syncthreads();
+    }
+    if (tile >= per) base_d += run[tile / per - 1];
+    for (int q = tile / per * per; q < tile; q++) base_d += sums[q];
+    boff[tid] = base_d;
 #pragma unroll
     for (int q = 0; q < BLOCK / 64; q++) wc[q][tid] = 0;
     __syncthreads();
@@ -193,8 +213,11 @@ int radix_sort_pairs(sph_ctx* c, int** keys, int** vals, int** ktmp, int** vtmp,
     int hist_n = 256 * ntiles;
     int* hist = nullptr;
     int* offs = nullptr;
+    int* sums = nullptr;
+    const int nsums = (hist_n + RS_TILE - 1) / RS_TILE;
     SPH_TRY(dalloc(c, &hist, hist_n));
     SPH_TRY(dalloc(c, &offs, hist_n));
+    SPH_TRY(dalloc(c, &sums, nsums));
     int *kin = *keys, *vin = *vals, *kout = *ktmp, *vout = *vtmp;
     for (int p = 0; p < passes; p++) {
         int shift = 8 * p;
@@ -202,10 +225,12 @@ int radix_sort_pairs(sph_ctx* c, int** keys, int** vals, int** ktmp, int** vtmp,
         hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(BLOCK), 0, c->stream, (const int*)kin, n, shift, ntiles, hist);
         SPH_TRY(launch_check(c, "radix_hist"));
         SPH_TRY(prof_end(c));
-        SPH_TRY(exclusive_scan_i32(c, hist, offs, hist_n, nullptr));
+        hipLaunchKernelGGL(k_scan_block<int>, dim3(nsums), dim3(BLOCK), 0, c->stream, (const int*)hist, offs,
+                           (long long)hist_n, sums);
+        SPH_TRY(launch_check(c, "scan_block"));
         SPH_TRY(prof_begin(c, "radix_scatter", 16.0 * n));
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(BLOCK), 0, c->stream, (const int*)kin, (const int*)vin,
-                           kout, vout, n, shift, ntiles, (const int*)offs);
+                           kout, vout, n, shift, ntiles, (const int*)offs, (const int*)sums, nsums);
         SPH_TRY(launch_check(c, "radix_scatter"));
         SPH_TRY(prof_end(c));
         std::swap(kin, kout);
@@ -217,6 +242,7 @@ int radix_sort_pairs(sph_ctx* c, int** keys, int** vals, int** ktmp, int** vtmp,
     }
     dfree(c, hist);
     dfree(c, offs);
+    dfree(c, sums);
     return 0;
 }
 static int radix_sort(sph_ctx* c, int max_key) {
@@ -224,20 +250,33 @@ static int radix_sort(sph_ctx* c, int max_key) {
 }
 
 // ------------------------------------------------------------------------
-// cell start / end, KERNEL_reorder functions_NNPS.cuh:825-838
-__global__ void __launch_bounds__(BLOCK) k_fill_i32(int* a, long long n, int v) {
-    long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = v;
-}
-__global__ void __launch_bounds__(BLOCK) k_cell_bounds(int n, const int* keys, int* gstr, int* gend) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int h = keys[i];
-    if (i == 0 || h != keys[i - 1]) {
-        gstr[h] = i;
-        if (i > 0) gend[keys[i - 1]] = i;
+// cell start / end, KERNEL_reorder functions_NNPS.cuh:825-838.
+// First particle of the sorted order whose key is >= cell, for every cell
+// and one past the last: the particles of consecutive cells a..b are
+// [cstart[a], cstart[b + 1]), in the order the cells hold them.  A cell's own
+// start and end (-1 and 0 where it is empty) are its and the next cell's: a
+// block searches CELLS + 1 cells and writes CELLS.  (Two fills, a pass over the
+// particles for the bounds and this one took four launches a
+// search, 13 us and as much between them; one takes 6.)
+constexpr int CELLS = BLOCK - 1;
+__global__ void __launch_bounds__(BLOCK) k_cells(int num_cells, const int* keys, int n, int* cstart, int* gstr,
+                                                 int* gend) {
+    __shared__ int first[BLOCK];
+    const int cell = blockIdx.x * CELLS + threadIdx.x;   // 0 .. num_cells + 1
+    int lo = 0, hi = cell <= num_cells + 1 ? n : 0;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (keys[mid] < cell) lo = mid + 1;
+        else hi = mid;
     }
-    if (i == n - 1) gend[h] = i + 1;
+    first[threadIdx.x] = lo;
+    __syncthreads();
+    if (threadIdx.x >= CELLS || cell > num_cells + 1) return;
+    cstart[cell] = lo;
+    if (cell > num_cells) return;
+    const int next = first[threadIdx.x + 1];
+    gstr[cell] = next > lo ? lo : -1;
+    gend[cell] = next > lo ? next : 0;
 }
 
 // gather arrays through the permutation, out[f][i] = in[f][perm[i]]: GATHER_N
@@ -270,21 +309,6 @@ __global__ void __launch_bounds__(BLOCK) k_gather(int n, const int* perm, Gather
 #pragma unroll
     for (int f = 0; f < GATHER_N; f++)
         if (f < nd) G.out[f][i] = v[f];
-}
-
-// First particle of the sorted order whose key is >= cell, for every cell
-// and one past the last: the particles of consecutive cells a..b are
-// [cstart[a], cstart[b + 1]), in the order the cells hold them.
-__global__ void __launch_bounds__(BLOCK) k_cell_start(int ncs, const int* keys, int n, int* cstart) {
-    const int cell = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cell >= ncs) return;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (keys[mid] < cell) lo = mid + 1;
-        else hi = mid;
-    }
-    cstart[cell] = lo;
 }
 
 // ------------------------------------------------------------------------
@@ -835,16 +859,9 @@ int nnps_run(sph_ctx* c, bool build_list) {
     SPH_TRY(prof_end(c));
     SPH_TRY(radix_sort(c, d.num_cells));
     SPH_TRY(prof_begin(c, "cell_bounds", 4.0 * n + 8.0 * (d.num_cells + 1)));
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid1((long long)d.num_cells + 1)), dim3(BLOCK), 0, c->stream, c->gstr,
-                       (long long)d.num_cells + 1, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid1((long long)d.num_cells + 1)), dim3(BLOCK), 0, c->stream, c->gend,
-                       (long long)d.num_cells + 1, 0);
-    hipLaunchKernelGGL(k_cell_bounds, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, n, (const int*)c->keys, c->gstr,
-                       c->gend);
-    SPH_TRY(launch_check(c, "cell_bounds"));
-    hipLaunchKernelGGL(k_cell_start, dim3(grid1((long long)d.num_cells + 2)), dim3(BLOCK), 0, c->stream,
-                       d.num_cells + 2, (const int*)c->keys, n, c->cstart);
-    SPH_TRY(launch_check(c, "cell_start"));
+    hipLaunchKernelGGL(k_cells, dim3((unsigned)(((long long)d.num_cells + 2 + CELLS - 1) / CELLS)), dim3(BLOCK), 0,
+                       c->stream, d.num_cells, (const int*)c->keys, n, c->cstart, c->gstr, c->gend);
+    SPH_TRY(launch_check(c, "cells"));
     SPH_TRY(prof_end(c));
     SPH_TRY(permute_state(c));
     if (build_list) SPH_TRY(nnps_list(c));

@@ -750,6 +750,8 @@ inline unsigned grid1(long long n, int block = BLOCK) { return (unsigned)((n + b
 // nnps.hip
 int nnps_run(sph_ctx* c, bool build_list = true);
 int nnps_list(sph_ctx* c);
+// entries a block of the sort's passes and of the scans takes
+constexpr int RS_ITEMS = 8, RS_TILE = BLOCK * RS_ITEMS;
 int radix_sort_pairs(sph_ctx* c, int** keys, int** vals, int** ktmp, int** vtmp, int n, int max_key);
 int set_ncell_run(sph_ctx* c);
 int exclusive_scan_i32(sph_ctx* c, const int* in, int* out, long long n, int* total_out);
