@@ -65,3 +65,31 @@ def test_refinement_list_over_several_tiles_of_cells(shift):
         np.testing.assert_array_equal(fg[f], fo[f], err_msg=f)
     for a, b in zip(sg, so):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1728, 2048, 2049, 8191, 8192, 8193])
+@pytest.mark.parametrize("shift", [0.0, 5.0])
+def test_sort_of_few_particles(n, shift):
+    """One workgroup up to 8192 particles; one digit of cells and three."""
+    B, _ = cases.box(nf=6, walls=3)
+    B["z"][B["z"] > 0.055] += shift
+    B["y"][B["y"] > 0.055] += shift
+    r = np.random.RandomState(n)
+    P = np.zeros(n, dtype=B.dtype)
+    P[:] = B[:1]
+    P["i_type"] = 3
+    P[r.choice(n, len(B), replace=False)] = B
+    prm = cases.box_params(urbansph.default_params())
+    prm.update(ppe_solver=abi.PPE_REF_JACOBI)
+    g = urbansph.Case(prm, n)
+    g.upload(P)
+    g.step(0, 1e-9)
+    keys, perm, start, end = g.nnps()
+    cells = len(start)
+    assert cells > (1 << 16) if shift else cells < 1 << 12
+    up = np.empty(n, keys.dtype)
+    up[perm] = keys
+    np.testing.assert_array_equal(np.sort(perm), np.arange(n))
+    np.testing.assert_array_equal(perm, np.argsort(up, kind="stable"))
+    np.testing.assert_array_equal(keys == cells, P["i_type"][perm] == 3)
+    np.testing.assert_array_equal(g.field("X"), P["x"][perm].astype(np.float64))

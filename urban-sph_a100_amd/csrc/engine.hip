@@ -223,7 +223,10 @@ static int shape_device(Eng& e, int block, long long total, const U& units, Eng:
         hipLaunchKernelGGL(k_block_morton, dim3(grid1(nb)), dim3(256), 0, e.st, (const int*)c->keys, nb, block,
                            c->dom.NI, c->dom.NJ, code, first);
         SPH_TRY(launch_check(&e, "block_morton"));
-        SPH_TRY(radix_sort_pairs(c, &code, &first, &ct, &ft, nb, (1 << 30) - 1));
+        // the codes' bits: three times those of the longest axis (fewer digits)
+        int bits = 1;
+        while ((1 << bits) < std::max({c->dom.NI, c->dom.NJ, c->dom.NK + 1})) bits++;
+        SPH_TRY(radix_sort_pairs(c, &code, &first, &ct, &ft, nb, (1 << 3 * bits) - 1));
         hipLaunchKernelGGL(k_block_table, dim3(grid1(nb)), dim3(256), 0, e.st, (const int*)first, nb, k, t->d + off);
         SPH_TRY(launch_check(&e, "block_table"));
         dfree(c, code);
