@@ -635,6 +635,7 @@ void sph_destroy(sph_ctx* c) {
     for (auto p : rest) dfree(c, p);
     dcache_release(c);
     for (auto& b : c->live) (void)hipFree(b.first);   // none expected: every buffer is freed above
+    if (c->back) (void)hipHostFree(c->back);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
 }

@@ -183,12 +183,13 @@ int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
     }
     if (target)
         SPH_HIP(c, hipMemcpyAsync(c->apr_target, target, sizeof(double) * (size_t)c->n, hipMemcpyHostToDevice, c->stream));
-    int *rank = nullptr, *pick = nullptr, *list = nullptr, *sums = nullptr;   // sums: and the total behind them
+    int *rank = nullptr, *pick = nullptr, *list = nullptr, *sums = nullptr;
     const int ntiles = (ncells + RS_TILE - 1) / RS_TILE;
     SPH_TRY(dalloc(c, &list, ncells));
     SPH_TRY(dalloc(c, &rank, ncells));
     SPH_TRY(dalloc(c, &pick, ncells));
-    SPH_TRY(dalloc(c, &sums, ntiles + 1));
+    SPH_TRY(dalloc(c, &sums, ntiles));
+    SPH_TRY(back_slot(c));
     hipLaunchKernelGGL(k_apr_first, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, pick);
     int rc = launch_check(c, "apr_first");
     bool split_any = false;
@@ -198,12 +199,12 @@ int apr_refine(sph_ctx* c, const double* target, int max_passes, int* n_out) {
         hipLaunchKernelGGL(k_apr_pick, dim3(ntiles), dim3(BLOCK), 0, c->stream, ncells, c->pview(),
                            (const double*)c->apr_target, (const int*)pick, rank, sums);
         hipLaunchKernelGGL(k_apr_list, dim3(grid1(ncells)), dim3(BLOCK), 0, c->stream, ncells, ntiles, (const int*)rank,
-                           (const int*)sums, pick, list, sums + ntiles);
+                           (const int*)sums, pick, list, (int*)c->back);
         if ((rc = launch_check(c, "apr_pick"))) break;
         int nsplit = 0;
-        hipError_t he = hipMemcpyAsync(&nsplit, sums + ntiles, sizeof(int), hipMemcpyDeviceToHost, c->stream);
-        if (he == hipSuccess) he = hipStreamSynchronize(c->stream);
+        const hipError_t he = hipStreamSynchronize(c->stream);
         if (he != hipSuccess) { rc = fail(c, SPH_E_HIP, hipGetErrorString(he)); break; }
+        nsplit = *(const int*)c->back;
         if (nsplit == 0) break;
         if ((long long)c->n + 8LL * nsplit > c->cap) {
             rc = fail(c, SPH_E_NOMEM, "APR needs room for " + std::to_string(c->n + 8LL * nsplit) +

@@ -1148,16 +1148,14 @@ static int mg_galerkin(sph_ctx* c, const OP& src, MGLevel& L1, const MGLevel& L0
     SPH_HIP(c, hipMemsetAsync(aux, 0, 2 * sizeof(int), c->stream));
     MGK("mg_rap_scale", min(grid1((long long)L0.n * GROUP), MAXABS_BLOCKS), BLOCK, k_mg_maxabs<OP>, src, L0.n, (unsigned*)aux);
     int h_aux[2] = {0, 0};
-    SPH_HIP(c, hipMemcpyAsync(h_aux, aux, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(c, hipStreamSynchronize(c->stream));
+    SPH_TRY(read_back(c, h_aux, aux, sizeof(int)));
     float amax = 0.0f;
     std::memcpy(&amax, &h_aux[0], sizeof(float));
     if (!(amax > 0.0f) || !std::isfinite(amax)) amax = 1.0f;
     const double scale = std::ldexp(1.0, 49 - (std::ilogb((double)amax) + 1));
     MGK("mg_rap_fill", n1, SLICE, k_mg_rap_hash<OP>, src, n1, (const int*)L0.agg, (const int*)L0.mstart,
         (const int*)L0.mem, scale, redo, aux + 1, L1.cnt, (const long long*)row_off, pc, pv, L1.diag, err, force_sort);
-    SPH_HIP(c, hipMemcpyAsync(h_aux + 1, aux + 1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(c, hipStreamSynchronize(c->stream));
+    SPH_TRY(read_back(c, h_aux + 1, aux + 1, sizeof(int)));
     *nsorted += h_aux[1];
     if (h_aux[1] > 0) {
         MGK("mg_rap_sort", n1, SLICE, (k_mg_rap<OP, MG_ENT_CAP>), src, n1, (const int*)L0.agg, (const int*)L0.mstart,
@@ -1166,8 +1164,7 @@ static int mg_galerkin(sph_ctx* c, const OP& src, MGLevel& L1, const MGLevel& L0
             (const int*)L0.mem, (const int*)redo, L1.cnt, (const long long*)row_off, pc, pv, L1.diag, err);
     }
     int h_err = 0;
-    SPH_HIP(c, hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(c, hipStreamSynchronize(c->stream));
+    SPH_TRY(read_back(c, &h_err, err, sizeof(int)));
     if (h_err) {
         *ok = 0;
         *why = h_err;
@@ -1295,8 +1292,7 @@ int mg_build(sph_ctx* c, const PPEView& pp, long long slots, double q, MGState**
         hipLaunchKernelGGL(k_mg_coord0, dim3(grid1(L0.n)), dim3(BLOCK), 0, c->stream, L0.n, pp.rows, c->sview(), x0,
                            y0, z0, q, L0.nx, L0.ny, L0.nz, L0.cx, L0.cy, L0.cz, L0.ex, err);
         MGTRY(launch_check(c, "mg_coord"));
-        MGTRY(hipc(hipMemcpyAsync(&rmax, err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "mg: lattice"));
-        MGTRY(hipc(hipStreamSynchronize(c->stream), "mg: lattice"));
+        MGTRY(read_back(c, &rmax, err, sizeof(int)));
         // every level's keys are 32-bit
         if (mg_key_count(L0, rmax + MG_MAX_LEVELS) > 2000000000LL) return fail_out(0);
     }
@@ -1352,8 +1348,7 @@ int mg_build(sph_ctx* c, const PPEView& pp, long long slots, double q, MGState**
         hipLaunchKernelGGL(k_mg_tofloat, dim3(grid1(nn)), dim3(BLOCK), 0, c->stream, nn, (const double*)a, mg->ainv);
         MGTRY(launch_check(c, "mg_tofloat"));
         int h_err = 0;
-        MGTRY(hipc(hipMemcpyAsync(&h_err, err, sizeof(int), hipMemcpyDeviceToHost, c->stream), "mg: coarsest level"));
-        MGTRY(hipc(hipStreamSynchronize(c->stream), "mg: coarsest level"));
+        MGTRY(read_back(c, &h_err, err, sizeof(int)));
         dfree(c, a);
         dfree(c, rowk);
         dfree(c, colk);

@@ -14,6 +14,7 @@
 #include "flags.h"
 #include <algorithm>
 #include <climits>
+#include <cstring>
 #include <utility>
 
 #include "sph_internal.h"
@@ -238,7 +239,7 @@ __global__ void __launch_bounds__(SMALL_T) k_sort_small(int* keys, int* vals, in
 // ------------------------------------------------------------------------
 // exclusive scans (device-wide), 2048 elements per 256-thread block
 template <class T>
-__global__ void __launch_bounds__(BLOCK) k_scan_block(const T* in, T* out, long long n, T* sums) {
+__global__ void __launch_bounds__(BLOCK) k_scan_block(const T* in, T* out, long long n, T* sums, T* total) {
     __shared__ T sh[BLOCK];
     const int t = threadIdx.x;
     long long base = (long long)blockIdx.x * RS_TILE + (long long)t * RS_ITEMS;
@@ -265,7 +266,10 @@ __global__ void __launch_bounds__(BLOCK) k_scan_block(const T* in, T* out, long 
         if (idx < n) out[idx] = run;
         run += v[k];
     }
-    if (t == BLOCK - 1) sums[blockIdx.x] = sh[t];
+    if (t == BLOCK - 1) {
+        sums[blockIdx.x] = sh[t];
+        if (total) *total = sh[t];
+    }
 }
 template <class T>
 __global__ void __launch_bounds__(BLOCK) k_scan_add(T* out, long long n, const T* offs) {
@@ -273,29 +277,54 @@ __global__ void __launch_bounds__(BLOCK) k_scan_add(T* out, long long n, const T
     if (idx < n) out[idx] += offs[idx / RS_TILE];
 }
 
+int back_slot(sph_ctx* c) {
+    if (!c->back) SPH_HIP(c, hipHostMalloc(&c->back, BACK_BYTES, hipHostMallocDefault));
+    return 0;
+}
+__global__ void k_read_back(const unsigned char* src, unsigned char* dst, int bytes) {
+    if ((int)threadIdx.x < bytes) dst[threadIdx.x] = src[threadIdx.x];
+}
+int read_back(sph_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes > BACK_BYTES) return fail(c, SPH_E_ARG, "read_back: too many bytes");
+    SPH_TRY(back_slot(c));
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(BACK_BYTES), 0, c->stream, (const unsigned char*)src,
+                       (unsigned char*)c->back, (int)bytes);
+    SPH_TRY(launch_check(c, "read_back"));
+    SPH_HIP(c, hipStreamSynchronize(c->stream));
+    std::memcpy(dst, c->back, bytes);
+    return 0;
+}
+
+// total: where the last block of sums leaves the total (or null)
 template <class T>
-static int exclusive_scan(sph_ctx* c, const T* in, T* out, long long n, T* total_out) {
+static int scan_launches(sph_ctx* c, const T* in, T* out, long long n, T* total) {
     long long nb = (n + RS_TILE - 1) / RS_TILE;
     if (nb < 1) nb = 1;
     T* sums = nullptr;
     T* sums_scan = nullptr;
     SPH_TRY(dalloc(c, &sums, nb + 1));
-    hipLaunchKernelGGL(k_scan_block<T>, dim3((unsigned)nb), dim3(BLOCK), 0, c->stream, in, out, n, sums);
+    hipLaunchKernelGGL(k_scan_block<T>, dim3((unsigned)nb), dim3(BLOCK), 0, c->stream, in, out, n, sums,
+                       nb > 1 ? nullptr : total);
     SPH_TRY(launch_check(c, "scan_block"));
-    T total = 0;
-    // the total goes to the host (a wait for the stream) only when asked for
     if (nb > 1) {
         SPH_TRY(dalloc(c, &sums_scan, nb + 1));
-        SPH_TRY(exclusive_scan<T>(c, sums, sums_scan, nb, total_out ? &total : nullptr));
+        SPH_TRY(scan_launches<T>(c, sums, sums_scan, nb, total));
         hipLaunchKernelGGL(k_scan_add<T>, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, out, n, (const T*)sums_scan);
         SPH_TRY(launch_check(c, "scan_add"));
         dfree(c, sums_scan);
-    } else if (total_out) {
-        SPH_HIP(c, hipMemcpyAsync(&total, sums, sizeof(T), hipMemcpyDeviceToHost, c->stream));
-        SPH_HIP(c, hipStreamSynchronize(c->stream));
     }
     dfree(c, sums);
-    if (total_out) *total_out = total;
+    return 0;
+}
+// the total goes to the host (a wait for the stream) only when asked for
+template <class T>
+static int exclusive_scan(sph_ctx* c, const T* in, T* out, long long n, T* total_out) {
+    if (total_out) SPH_TRY(back_slot(c));
+    SPH_TRY(scan_launches<T>(c, in, out, n, total_out ? (T*)c->back : nullptr));
+    if (total_out) {
+        SPH_HIP(c, hipStreamSynchronize(c->stream));
+        *total_out = *(const T*)c->back;
+    }
     return 0;
 }
 int exclusive_scan_i32(sph_ctx* c, const int* in, int* out, long long n, int* total) {
@@ -336,7 +365,7 @@ int radix_sort_pairs(sph_ctx* c, int** keys, int** vals, int** ktmp, int** vtmp,
         SPH_TRY(launch_check(c, "radix_hist"));
         SPH_TRY(prof_end(c));
         hipLaunchKernelGGL(k_scan_block<int>, dim3(nsums), dim3(BLOCK), 0, c->stream, (const int*)hist, offs,
-                           (long long)hist_n, sums);
+                           (long long)hist_n, sums, (int*)nullptr);
         SPH_TRY(launch_check(c, "scan_block"));
         SPH_TRY(prof_begin(c, "radix_scatter", 16.0 * n));
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(BLOCK), 0, c->stream, (const int*)kin, (const int*)vin,
@@ -859,8 +888,7 @@ static int build_neighbor_list(sph_ctx* c) {
         SPH_TRY(launch_check(c, "nl_fill"));
         SPH_TRY(prof_end(c));
         int h_over = 0;
-        SPH_HIP(c, hipMemcpyAsync(&h_over, over, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        SPH_HIP(c, hipStreamSynchronize(c->stream));
+        SPH_TRY(read_back(c, &h_over, over, sizeof(int)));
         dfree(c, over);
         if (!h_over) {
             // exact widths of this search: the next one's guess

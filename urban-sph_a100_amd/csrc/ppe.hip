@@ -1339,10 +1339,8 @@ void ppe_free(sph_ctx* c) {
 static int lattice_spacing(sph_ctx* c, const PPEState* P, double* q) {
     int r0 = 0;
     double h0 = 0.0;
-    SPH_HIP(c, hipMemcpyAsync(&r0, P->rows, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(c, hipStreamSynchronize(c->stream));
-    SPH_HIP(c, hipMemcpyAsync(&h0, c->sview().h + r0, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    SPH_HIP(c, hipStreamSynchronize(c->stream));
+    SPH_TRY(read_back(c, &r0, P->rows, sizeof(int)));
+    SPH_TRY(read_back(c, &h0, c->sview().h + r0, sizeof(double)));
     *q = h0 / 1.5;
     return 0;
 }
@@ -1707,8 +1705,7 @@ static int ppe_build_ordered(sph_ctx* c, bool allow_lattice) {
         SPH_TRY(launch_check(c, "ppe_cols_sorted"));
         SPH_TRY(prof_end(c));
         int hovf = 0;
-        SPH_HIP(c, hipMemcpyAsync(&hovf, ovf, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        SPH_HIP(c, hipStreamSynchronize(c->stream));
+        SPH_TRY(read_back(c, &hovf, ovf, sizeof(int)));
         dfree(c, ovf);
         if (hovf) {
             // a row with more entries than the in-block sort holds (refined
@@ -1743,8 +1740,7 @@ static int ppe_build_ordered(sph_ctx* c, bool allow_lattice) {
         SPH_TRY(launch_check(c, "ecols_build"));
         SPH_TRY(prof_end(c));
         int hovf = 0;
-        SPH_HIP(c, hipMemcpyAsync(&hovf, ovf, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        SPH_HIP(c, hipStreamSynchronize(c->stream));
+        SPH_TRY(read_back(c, &hovf, ovf, sizeof(int)));
         dfree(c, ovf);
         if (hovf) {
             dfree(c, P->ecols); P->ecols = nullptr;
