@@ -249,7 +249,8 @@ int shape(Eng& e, int kind, int block, Shape* out) {
     auto units = [&](int k) -> long long {
         const sph_ctx* c = e.cs[k];
         // kind 0: particles; 1: PPE rows; 2: one 64-lane wave per long PPE row;
-        // 3: one 64-lane wave per boundary particle of the Neumann pass;
+        // 3: 64 units per boundary particle (block: those of the particles a
+        // workgroup's groups of lanes take);
         // 4: the lanes of the cell-tile chunks (a block per chunk); 5: one
         // 64-lane wave per particle of a heavy neighbour list
         return kind == 0 ? c->n : kind == 1 ? ppe_view(c).nr : kind == 2 ? 64LL * ppe_view(c).nlong

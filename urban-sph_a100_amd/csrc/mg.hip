@@ -964,9 +964,9 @@ __global__ void __launch_bounds__(BLOCK) k_mg_restrict(const CaseDesc* cds, cons
 // lanes an aggregate of level l + 1, MG_G a member's row, the members' residuals
 // added in member order (the same bits as the two passes).
 constexpr int RR_LANES = 32;
-// (rows of the step's cases on the level: the 200 k request's 30 launches fewer
-// an iteration pair are 51.4 -> 50.2 ms; a level of 240 k rows loses 9 us by its
-// scattered rows what the launch gains)
+// The limit counts the rows of all the step's cases on the level.  Below it a
+// launch saved is worth more than coalesced rows (200 k request 51.4 -> 50.2 ms);
+// a level of 240 k rows is 9 us slower in one pass, its members' rows scattered.
 constexpr long long RR_ROWS = 40000;
 __global__ void __launch_bounds__(BLOCK) k_mg_res_restrict(const CaseDesc* cds, const MGLv* lv, const int2* tab, int l,
                                                            int sc_done) {

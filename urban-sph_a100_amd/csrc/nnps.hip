@@ -1,7 +1,7 @@
 // Neighbour search of the count==0 step on MI355X (ISPH_Calc.cuh:23-52):
 //   KERNEL_index_particle_to_cell  functions_NNPS.cuh:879-907  -> k_hash
 //   cub::DeviceRadixSort::SortPairs ISPH_Calc.cuh:33           -> radix_sort
-//   KERNEL_reorder (start/end)     functions_NNPS.cuh:813-838  -> k_cell_bounds
+//   KERNEL_reorder (start/end)     functions_NNPS.cuh:813-838  -> k_cells
 //   KERNEL_reorder (gather)        functions_NNPS.cuh:840-843  -> permute
 // plus the per-particle neighbour list that the per-step passes walk
 // (the reference rescans the cell window in every pass).

@@ -1954,7 +1954,7 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
 
 // launch over the particles of every case; tunable passes (kid >= 0) run at
 // the workgroup size the autotuner picked for this batch size
-// a boundary pass with a 64-lane wave per boundary particle of each case
+// a boundary pass with `lanes` lanes per boundary particle of each case
 #define BOUNDL(name, kern, ...) BOUNDW(name, BLANES, kern, ##__VA_ARGS__)
 #define BOUNDW(name, lanes, kern, ...)                                                                        \
     do {                                                                                            \
