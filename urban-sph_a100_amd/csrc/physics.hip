@@ -399,7 +399,7 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
     const float hi = (float)S.h[i], tmp_A = calc_tmpA<float>(kc, hi), f = dw_factor<float>(kc, hi);
     const HScale hs(kc, hi);
     // consecutive neighbours mostly share rho: its reciprocal is kept
-    float rho_c = -1.0f, yrho = 0.0f;
+    float rho_c = NO_VALUE, yrho = 0.0f;
     walk_row<REC, 2, 2, W>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
         if (!(e & F_HP)) return;
         const int j = e & NB_IDX;
@@ -940,7 +940,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_neumann_mixed(Seg sg, int which,
     }
     const HScale hs(kc, hi);
     const float dwf = dw_factor<float>(kc, hi);
-    float rho_c = -1.0f, yrho = 0.0f;
+    float rho_c = NO_VALUE, yrho = 0.0f;
     double s[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     auto add = [&](float dx, float dy, float dz, float mj, float rhoj, float uxj, float uyj, float uzj, double presj) {
         if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
@@ -1183,7 +1183,7 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
     const int fv = pr.fv_solve;
     const float Alpha = (float)pr.av_alpha, Beta = (float)pr.av_beta, soundspeed = (float)pr.av_c;
     // consecutive neighbours mostly share rho: the reciprocals it enters are kept
-    float rho_c = -1.0f, yrho = 0.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
+    float rho_c = NO_VALUE, yrho = 0.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
     walk_row<REC, 2, 2, W>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
         if (!(e & F_DP)) return;
         const int j = e & NB_IDX;
@@ -1477,7 +1477,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_mixed(Seg sg, int which
     const NList nl = cd.nl;
     const float hi = (float)A.h[i], tmp_A = calc_tmpA<float>(kc, hi);
     const HScale hs(kc, hi);
-    float rho_c = -1.0f, yrho = 0.0f;
+    float rho_c = NO_VALUE, yrho = 0.0f;
     double xg = A.x[i], yg = A.y[i], zg = A.z[i];
     double t[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const NLRow row = nl_row(nl, i);
@@ -1610,7 +1610,7 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
     // h_ij, its density terms on rho_j: kept while consecutive pairs share them
     float h_c = -1.0f, A_c = 0.0f, f_c = 0.0f;
     HScale hs(kc, 1.0f);
-    float rho_c = -1.0f, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
+    float rho_c = NO_VALUE, rr = 0.0f, yrr = 0.0f, rs = 0.0f, yrs = 0.0f;
     walk_row<REC, 2, 0, W>(row, src, g, [&](unsigned e, const Pieces<2, 0>& rec_) {
         if (!(e & F_DM)) return;
         const int j = e & NB_IDX;

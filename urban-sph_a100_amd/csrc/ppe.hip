@@ -837,7 +837,7 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
     const int gbit = (int)(threadIdx.x & 63) & ~(GROUP - 1);   // the group's first lane
     int slot = 0;
     // consecutive neighbours mostly share rho: what it enters is kept
-    float rho_c = -1.0f, yrho = 0.0f, hm = 0.0f;
+    float rho_c = NO_VALUE, yrho = 0.0f, hm = 0.0f;
     walk_row<REC, 2, 2, GROUP>(row, src, g, [&](unsigned e, const Pieces<2, 2>& rec_) {
         bool pair = (e & F_DP) != 0, own = false;   // own: an entry of the row
         const int j = e & NB_IDX;

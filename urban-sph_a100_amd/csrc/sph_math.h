@@ -145,6 +145,11 @@ __device__ __forceinline__ float quot(float a, float b, float y) {   // a / b, y
     const float q = a * y;
     return fma1(fma1(-b, q, a), y, q);
 }
+// What a pass that keeps the last neighbour's reciprocals starts from: it equals
+// no density, so the first neighbour's are formed.  (A number would not do: the
+// deck's densities are not checked, and from -1 a case of that density got zeros
+// for its sums.)
+constexpr float NO_VALUE = __builtin_nanf("");
 // a distance and its reciprocal from its square; coinciding particles (and
 // the particle itself) get a distance of 1e-15 instead of the pair
 // formulas' + 1e-20
