@@ -40,3 +40,29 @@ def test_mixed_passes_at_any_density(rho, compact, tiles):
         scale = np.abs(ref[f]).max()
         assert np.isfinite(scale) and scale > 0.0, f
         assert np.abs(got[f] - ref[f]).max() <= 1e-4 * scale, f
+
+
+@pytest.mark.parametrize("field,value,which", [("rho", 0.0, "wall"), ("rho", np.inf, "one"), ("m", np.inf, "one"),
+                                               ("m", 0.0, "wall"), ("rho", np.nan, "one")])
+def test_mixed_divides_by_what_the_deck_holds(field, value, which):
+    """Masses and densities are not checked: where the pair formulas divide by
+    a zero density or an infinite one, the MIXED passes give the zeros,
+    infinities and NaN of the division, as the FP64 mode does."""
+    P, _ = cases.box(nf=8, walls=3)
+    fluid = np.flatnonzero(P["p_type"] == 1)
+    P[field][np.flatnonzero(P["p_type"] == 0) if which == "wall" else fluid[3]] = value
+    got = {}
+    for precision in (abi.FP64, abi.MIXED):
+        prm = cases.box_params(urbansph.default_params(), precision=precision)
+        prm.update(ppe_solver=abi.PPE_REF_JACOBI)
+        c = urbansph.Case(prm, len(P))
+        c.upload(P)
+        c.step(0, 1e-4)
+        got[precision] = {f: c.field(f) for f in ("FLT_S", "INV_CM_XX", "INV_CM_XY", "INV_CM_ZZ")}
+        c.close()
+    for f, ref in got[abi.FP64].items():
+        g = got[abi.MIXED][f]
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(ref), err_msg=f)
+        odd = ~np.isfinite(ref)
+        np.testing.assert_array_equal(g[odd], ref[odd], err_msg=f)
+        assert np.abs(g[~odd] - ref[~odd]).max() <= 1e-4 * np.abs(ref[~odd]).max(), f

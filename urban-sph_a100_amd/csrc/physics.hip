@@ -231,13 +231,13 @@ __global__ void __launch_bounds__(MAX_BLOCK) k_grad_corr_mixed(Seg sg) {
         const unsigned e = NB_AT(row, k);
         if (!(e & F_B)) continue;
         const int j = e & NB_IDX;
-        if (S.p_type[j] != 1) continue;
         const float dx = (float)(xi - S.x[j]), dy = (float)(yi - S.y[j]), dz = (float)(zi - S.z[j]);
         const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
         const float w = -((float)S.m[j] * kernel_dw_t<float>(kc, tmp_A, f, hs.tR(d.r)));
-        const float rtd = recip((float)S.rho[j] * d.r);
-        txx += (double)(w * dx * dx * rtd); txy += (double)(w * dy * dx * rtd); tyy += (double)(w * dy * dy * rtd);
-        tzx += (double)(w * dx * dz * rtd); tyz += (double)(w * dy * dz * rtd); tzz += (double)(w * dz * dz * rtd);
+        const float rtd = 1.0f / ((float)S.rho[j] * d.r), fl = (float)(S.p_type[j] == 1);
+        txx += (double)(w * dx * dx * rtd * fl); txy += (double)(w * dy * dx * rtd * fl);
+        tyy += (double)(w * dy * dy * rtd * fl); tzx += (double)(w * dx * dz * rtd * fl);
+        tyz += (double)(w * dy * dz * rtd * fl); tzz += (double)(w * dz * dz * rtd * fl);
     }
     group_fold<GROUP>(txx); group_fold<GROUP>(tyy); group_fold<GROUP>(tzz);
     group_fold<GROUP>(txy); group_fold<GROUP>(tyz); group_fold<GROUP>(tzx);
@@ -421,10 +421,10 @@ __device__ __forceinline__ void prep_sums(const CaseDesc& cd, int i, const NLRow
         const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
         const float tR = hs.tR(d.r);
         const float wij = kernel_w_t<float>(kc, tmp_A, tR);
-        const float vj = quot(mj, rhoj, yrho);
+        const float vj = quot_any(mj, rhoj, yrho);
         if (filt) flt += (double)(vj * wij);
         if (les) {
-            sigma += (double)quot(d.r * d.r * wij * mj, rhoj, yrho);
+            sigma += (double)quot_any(d.r * d.r * wij * mj, rhoj, yrho);
             if (ptj == 1) {
                 if constexpr (!REC) {
                     dux = (float)(S.ux[j] - uxi); duy = (float)(S.uy[j] - uyi); duz = (float)(S.uz[j] - uzi);
@@ -946,7 +946,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_neumann_mixed(Seg sg, int which,
         if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
         // (the list holds exactly the pairs inside the search range)
         const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
-        const float tR = hs.tR(d.r), w = kernel_w_t<float>(kc, tmp_A, tR), vj = quot(mj, rhoj, yrho);
+        const float tR = hs.tR(d.r), w = kernel_w_t<float>(kc, tmp_A, tR), vj = quot_any(mj, rhoj, yrho);
         s[0] += (double)(vj * (float)presj * w);
         s[1] += (double)(vj * uxj * w);
         s[2] += (double)(vj * uyj * w);
@@ -1224,7 +1224,7 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
             float C_v = dx * tx + dy * ty + dz * tz;
             const float vs = visi + visj;
             C_v *= quot(visi * visj, vs, recip(vs));
-            C_v *= 4.0f * quot(mj, rr, yrr);
+            C_v *= 4.0f * quot_any(mj, rr, yrr);
             C_v = quot(quot(C_v, d.r, d.y), d.r, d.y);
             a.tx += (double)(C_v * dux); a.ty += (double)(C_v * duy); a.tz += (double)(C_v * duz);
         } else if (fv == SPH_FV_MONAGHAN) {
@@ -1237,9 +1237,9 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
         }
         if (conv) {
             const float vx = -dux, vy = -duy, vz = -duz;   // u_j - u_i
-            a.cx += (double)(quot((fux * vx * tx + fuy * vx * ty + fuz * vx * tz) * mj, rhoj, yrho) * ome);
-            a.cy += (double)(quot((fux * vy * tx + fuy * vy * ty + fuz * vy * tz) * mj, rhoj, yrho) * ome);
-            a.cz += (double)(quot((fux * vz * tx + fuy * vz * ty + fuz * vz * tz) * mj, rhoj, yrho) * ome);
+            a.cx += (double)(quot_any((fux * vx * tx + fuy * vx * ty + fuz * vx * tz) * mj, rhoj, yrho) * ome);
+            a.cy += (double)(quot_any((fux * vy * tx + fuy * vy * ty + fuz * vy * tz) * mj, rhoj, yrho) * ome);
+            a.cz += (double)(quot_any((fux * vz * tx + fuy * vz * ty + fuz * vz * tz) * mj, rhoj, yrho) * ome);
         }
         if (SCAL && (con_solve || concn_solve || boussinesq_solve)) {
             double tempj, concnj_d;
@@ -1278,7 +1278,7 @@ __device__ __forceinline__ void advection_sums(const CaseDesc& cd, int i, const 
                 const float h_ij = (float)((hi_d + hj_d) * 0.5);
                 const float den = d.r * d.r + 0.01f * h_ij * h_ij;
                 const float phi = quot(h_ij * ud, den, recip(den));
-                const float P = quot(mi * phi * (-Alpha * soundspeed + Beta * phi), rs, yrs) * 0.5f;
+                const float P = quot_any(mi * phi * (-Alpha * soundspeed + Beta * phi), rs, yrs) * 0.5f;
                 a.tx += (double)(-P * tx); a.ty += (double)(-P * ty); a.tz += (double)(-P * tz);
             }
         }
@@ -1489,7 +1489,7 @@ __global__ void __launch_bounds__(WAVE_BLOCK) k_freeslip_mixed(Seg sg, int which
         float dx = (float)(xg - A.x[j]), dy = (float)(yg - A.y[j]), dz = (float)(zg - A.z[j]);
         const float rhoj = (float)A.rho[j];
         if (rhoj != rho_c) { rho_c = rhoj; yrho = recip(rhoj); }
-        const float vj = quot((float)A.m[j], rhoj, yrho);
+        const float vj = quot_any((float)A.m[j], rhoj, yrho);
         const float w = kernel_w_t<float>(kc, tmp_A, hs.tR(dist_of(dx * dx + dy * dy + dz * dz).r));
         t[0] += (double)((float)A.ux[j] * vj * w);
         t[1] += (double)((float)A.uy[j] * vj * w);
@@ -1644,7 +1644,7 @@ __device__ __forceinline__ void pressure_sums(const CaseDesc& cd, int i, const N
         const Dist d = dist_of(dx * dx + dy * dy + dz * dz);
         const float dw = kernel_dw_t<float>(kc, A_c, f_c, hs.tR(d.r));
         const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
-        const float C_p = quot(quot(-2.0f * mj, rr, yrr) * (pi * rhoj + pj * rhoi), rs, yrs);
+        const float C_p = quot_any(quot_any(-2.0f * mj, rr, yrr) * (pi * rhoj + pj * rhoi), rs, yrs);
         tmpx += (double)(C_p * tx); tmpy += (double)(C_p * ty); tmpz += (double)(C_p * tz);
     });
 }

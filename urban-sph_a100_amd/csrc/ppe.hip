@@ -879,7 +879,7 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
             const float tx = quot(dw * dx, d.r, d.y), ty = quot(dw * dy, d.r, d.y), tz = quot(dw * dz, d.r, d.y);
             const float cx = gc11 * tx + gc12 * ty + gc31 * tz, cy = gc12 * tx + gc22 * ty + gc23 * tz,
                         cz = gc31 * tx + gc23 * ty + gc33 * tz;
-            const float vj = quot(mj, rhoj, yrho);
+            const float vj = quot_any(mj, rhoj, yrho);
             b[0] += (double)(vj * dux * cx * hm);
             b[1] += (double)(vj * duy * cy * hm);
             b[2] += (double)(vj * duz * cz * hm);
@@ -887,7 +887,7 @@ __device__ __forceinline__ void assemble_sums(const CaseDesc& cd, int i, int r, 
             // (with the values kept from the search's first step, only the known
             // neighbours' share of the right-hand side needs the coefficient)
             if (FULL || (!jrow && other)) {
-                cc = quot(quot(quot(2.0f * mj, rhoj, yrho) * (dx * cx + dy * cy + dz * cz), d.r, d.y), d.r, d.y);
+                cc = quot(quot(quot_any(2.0f * mj, rhoj, yrho) * (dx * cx + dy * cy + dz * cz), d.r, d.y), d.r, d.y);
                 if (FULL) {
                     a.A += (double)cc;
                     if (jacobi) a.Ap += (double)cc * qj;

@@ -145,6 +145,12 @@ __device__ __forceinline__ float quot(float a, float b, float y) {   // a / b, y
     const float q = a * y;
     return fma1(fma1(-b, q, a), y, q);
 }
+// The same where a mass or a density of the deck, which is not checked, is an
+// operand: zero, infinite and NaN ones give what the division gives (quot makes
+// NaN of them), by the instruction the compiler's division ends with.
+__device__ __forceinline__ float quot_any(float a, float b, float y) {
+    return __builtin_amdgcn_div_fixupf(quot(a, b, y), b, a);
+}
 // What a pass that keeps the last neighbour's reciprocals starts from: it equals
 // no density, so the first neighbour's are formed.  (A number would not do: the
 // deck's densities are not checked, and from -1 a case of that density got zeros
