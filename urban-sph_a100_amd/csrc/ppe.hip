@@ -43,6 +43,7 @@
 #include "sph_internal.h"
 #include "sph_math.h"
 #include "ppe_format.h"
+#include "solve_plan.h"
 
 namespace sph {
 
@@ -1953,7 +1954,7 @@ static int kr_graph(Eng& e, int gi, bool run, double spmv_bytes, bool mg, hipGra
         hipGraph_t g = nullptr;
         SPH_HIP(&e, hipStreamBeginCapture(e.st, hipStreamCaptureModeThreadLocal));
         int rc = 0;
-        for (int b = 0; b < (run ? Eng::KR_RUN : 1) && rc == 0; b++) rc = kr_iteration<V, X>(e, spmv_bytes, mg);
+        for (int b = 0; b < (run ? KR_RUN : 1) && rc == 0; b++) rc = kr_iteration<V, X>(e, spmv_bytes, mg);
         hipError_t er = hipStreamEndCapture(e.st, &g);
         if (rc) {
             if (er == hipSuccess && g) (void)hipGraphDestroy(g);
@@ -2012,27 +2013,18 @@ static int bicgstab(Eng& e, int gi, int pred_slot, std::vector<int>& iters, bool
     };
     const bool graphs = e.use_graphs && !e.prof.on;
     int& pred = e.pred_iters[gi][std::min(pred_slot, Eng::PRED_SLOTS - 1)];
-    // A look at the scalars costs a stop of the device of about 25 us, an
-    // iteration past the end a few us a launch: with a prediction the solve
-    // runs straight to it (a long one to just before it), then looks often;
-    // without one the batches grow geometrically.
-    const bool brief = pred > 0 && pred <= 8;
+    const SolvePlan plan{pred, maxit};
     if (pred == 0 || e.prof.on) SPH_TRY(read_scalars(e));
     int launched = 0;
     for (bool first = pred > 0 && !e.prof.on; (first || !all_done()) && launched < maxit; first = false) {
-        int batch;
-        if (brief) batch = launched == 0 ? pred : 1;
-        else if (pred > 0) batch = launched + 4 < (pred * 9) / 10 ? (pred * 9) / 10 - launched : 2;
-        else batch = std::max(4, launched / 2);
-        batch = std::min(batch, maxit - launched);
+        const int batch = plan.batch(launched);
         for (int b = 0; b < batch;) {
             if (graphs) {
-                // (a solve expected to be long: the larger graph's capture pays)
-                const bool run = batch - b >= Eng::KR_RUN && (pred > 0 ? !brief : launched >= 16);
+                const bool run = plan.run_graph(launched, batch - b);
                 hipGraphExec_t g = nullptr;
                 SPH_TRY((kr_graph<V, X>(e, gi, run, spmv_bytes, mg, &g)));
                 SPH_HIP(&e, hipGraphLaunch(g, e.st));
-                b += run ? Eng::KR_RUN : 1;
+                b += run ? KR_RUN : 1;
             } else {
                 SPH_TRY((kr_iteration<V, X>(e, spmv_bytes, mg)));
                 b++;

@@ -585,7 +585,6 @@ struct Eng {
     // Krylov iterations of the last solves (per vector precision and
     // refinement pass): the host polls for convergence only near them
     static constexpr int PRED_SLOTS = 4;
-    static constexpr int KR_RUN = 4;
     int pred_iters[NGRAPH][PRED_SLOTS] = {};
     // the physics before (0) and after (1) the pressure solve as graphs, for
     // the composition of the step and the variant of its launch sequence
