@@ -517,7 +517,7 @@ static void fill_desc(Eng& e, int k, sph_ctx* c, int count, double dt, double ti
     d.nm_count = c->nm_count;
     d.nmp_off = c->nmp_off;
     d.nmp_ent = c->nmp_ent;
-    const bool nmrec = c->prm.precision == SPH_MIXED && c->pos_f32 && !c->prm.ale_positions && c->prm.compact_records &&
+    const bool nmrec = c->compact() &&
                        c->nm_rec;
     d.nmp_cent = nmrec ? c->nmp_cent : nullptr;
     d.nm_set = nmrec ? c->nm_set : nullptr;
@@ -541,7 +541,7 @@ static void fill_desc(Eng& e, int k, sph_ctx* c, int count, double dt, double ti
     d.ppe = ppe_view(c);
     for (int f = 0; f < 3; f++) d.xnew[f] = c->xnew[f];
     d.rec = c->rec;
-    const bool compact = c->prm.precision == SPH_MIXED && c->pos_f32 && !c->prm.ale_positions && c->prm.compact_records;
+    const bool compact = c->compact();
     d.crec = compact ? c->crec : nullptr;
     d.crec_adv = compact ? c->crec_adv : nullptr;
     d.ibm_near = c->ibm_near_gen == c->generation ? c->ibm_near : nullptr;
@@ -559,10 +559,10 @@ static int step_body(Eng& e, sph_ctx* const* cases, int nc, const int* count, co
         sph_ctx* c = cases[k];
         if (c->prm.ale_positions && !c->xnew[0])
             for (int f = 0; f < 3; f++) SPH_TRY(dalloc(c, &c->xnew[f], c->cap));
-        if (!c->rec) SPH_TRY(dalloc(c, &c->rec, (size_t)c->cap * REC_DOUBLES));
-        if (!c->crec && c->prm.precision == SPH_MIXED) SPH_TRY(dalloc(c, &c->crec, (size_t)c->cap * CREC_FLOATS));
-        if (!c->crec_adv && c->prm.precision == SPH_MIXED)
-            SPH_TRY(dalloc(c, &c->crec_adv, (size_t)c->cap * CREC_ADV_FLOATS));
+        // the records this case's passes read
+        if (!c->compact() && !c->rec) SPH_TRY(dalloc(c, &c->rec, (size_t)c->cap * REC_DOUBLES));
+        if (c->compact() && !c->crec) SPH_TRY(dalloc(c, &c->crec, (size_t)c->cap * CREC_FLOATS));
+        if (c->compact() && !c->crec_adv) SPH_TRY(dalloc(c, &c->crec_adv, (size_t)c->cap * CREC_ADV_FLOATS));
         if (count[k] == 0 || c->prm.ale_positions) {   // moving particles: a search every step
             SPH_TRY(set_ncell_run(c));
             SPH_TRY(nnps_run(c));
@@ -575,7 +575,7 @@ static int step_body(Eng& e, sph_ctx* const* cases, int nc, const int* count, co
         if (c->nmp_gen != c->generation || c->nmp_for != c->nm_list || c->nmp_prec != prec || c->prm.ale_positions)
             SPH_TRY(neumann_pairs(c));
         SPH_TRY(ibm_near_build(c));   // the spreading targets of this search
-        if (prec == SPH_MIXED && c->pos_f32 && !c->prm.ale_positions && c->prm.compact_records) SPH_TRY(tile_build(c));
+        if (c->compact()) SPH_TRY(tile_build(c));
     }
     // composition of the step: tables and graphs stay valid while it holds
     std::vector<long long> sig;

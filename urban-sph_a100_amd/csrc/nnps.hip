@@ -422,14 +422,17 @@ __global__ void __launch_bounds__(BLOCK) k_cells(int num_cells, const int* keys,
 // arrays a launch (their gathers in flight together, the permutation read
 // once).  One array a launch took 58 launches a search: 0.40 ms on the 1 M
 // canyon, and 0.14 ms of 3 us launches in each refinement pass of a small case.
+// The integers are gathered to scratch by one launch (INTS_OUT) and copied back
+// by the next (INTS_BACK).
 constexpr int GATHER_N = 16;
+enum GatherInts { INTS_NONE, INTS_OUT, INTS_BACK };
 struct GatherSet {
     const double* in[GATHER_N];
     double* out[GATHER_N];
     const int* iin[SPH_I_COUNT];
     int* iout[SPH_I_COUNT];
 };
-template <bool INTS>
+template <GatherInts INTS>
 __global__ void __launch_bounds__(BLOCK) k_gather(int n, const int* perm, GatherSet G, int nd) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -438,10 +441,11 @@ __global__ void __launch_bounds__(BLOCK) k_gather(int n, const int* perm, Gather
 #pragma unroll
     for (int f = 0; f < GATHER_N; f++)
         if (f < nd) v[f] = G.in[f][p];
-    if (INTS) {
+    if (INTS != INTS_NONE) {
+        const int from = INTS == INTS_OUT ? p : i;
         int w[SPH_I_COUNT];
 #pragma unroll
-        for (int f = 0; f < SPH_I_COUNT; f++) w[f] = G.iin[f][p];
+        for (int f = 0; f < SPH_I_COUNT; f++) w[f] = G.iin[f][from];
 #pragma unroll
         for (int f = 0; f < SPH_I_COUNT; f++) G.iout[f][i] = w[f];
     }
@@ -768,34 +772,34 @@ static int permute_state(sph_ctx* c) {
     for (int f = 0; f < 10; f++) arr.push_back(&c->p2[f]);
     for (int f = 15; f < 18; f++) arr.push_back(&c->q[f]);
     if (c->apr_target) arr.push_back(&c->apr_target);
-    // each state array is swapped for its gathered copy, so the copies keep
-    // the context's capacity: refinement appends particles past n
-    double* tmp[GATHER_N] = {};
-    int* itmp[SPH_I_COUNT] = {};
-    for (auto& t : tmp) SPH_TRY(dalloc(c, &t, c->cap));
-    for (auto& t : itmp) SPH_TRY(dalloc(c, &t, c->cap));
+    // Each state array is swapped for its gathered copy.  The copies go to the
+    // working copies' arrays, of the context's capacity like all state arrays
+    // (refinement appends particles past n): nothing reads those between a
+    // step's end and the next one's start, which writes them all.  (Blocks of
+    // its own took a search 152 bytes a particle, which stayed in the cache.)
+    static_assert(MF_COUNT >= GATHER_N + (SPH_I_COUNT + 1) / 2, "room for the copies");
+    int* itmp[SPH_I_COUNT];
+    for (int f = 0; f < SPH_I_COUNT; f++) itmp[f] = (int*)c->sm[GATHER_N + f / 2] + (size_t)(f % 2) * c->cap;
     SPH_TRY(prof_begin(c, "permute", 0));
-    for (size_t a0 = 0; a0 < arr.size(); a0 += GATHER_N) {
+    const size_t launches = std::max<size_t>(2, (arr.size() + GATHER_N - 1) / GATHER_N);
+    for (size_t l = 0; l < launches; l++) {
+        const size_t a0 = std::min(arr.size(), l * GATHER_N);
         const int nd = (int)std::min<size_t>(GATHER_N, arr.size() - a0);
         GatherSet G{};
         for (int f = 0; f < nd; f++) {
             G.in[f] = *arr[a0 + f];
-            G.out[f] = tmp[f];
+            G.out[f] = c->sm[f];
         }
         for (int f = 0; f < SPH_I_COUNT; f++) {
-            G.iin[f] = c->pi[f];
-            G.iout[f] = itmp[f];
+            G.iin[f] = l == 0 ? c->pi[f] : itmp[f];
+            G.iout[f] = l == 0 ? itmp[f] : c->pi[f];
         }
-        if (a0 == 0) hipLaunchKernelGGL(k_gather<true>, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, n, (const int*)c->perm, G, nd);
-        else hipLaunchKernelGGL(k_gather<false>, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, n, (const int*)c->perm, G, nd);
+        auto* const kern = l == 0 ? k_gather<INTS_OUT> : l == 1 ? k_gather<INTS_BACK> : k_gather<INTS_NONE>;
+        hipLaunchKernelGGL(kern, dim3(grid1(n)), dim3(BLOCK), 0, c->stream, n, (const int*)c->perm, G, nd);
         SPH_TRY(launch_check(c, "permute"));
-        for (int f = 0; f < nd; f++) std::swap(*arr[a0 + f], tmp[f]);
-        if (a0 == 0)
-            for (int f = 0; f < SPH_I_COUNT; f++) std::swap(c->pi[f], itmp[f]);
+        for (int f = 0; f < nd; f++) std::swap(*arr[a0 + f], c->sm[f]);
     }
     SPH_TRY(prof_end(c));
-    for (auto t : tmp) dfree(c, t);
-    for (auto t : itmp) dfree(c, t);
     return 0;
 }
 
@@ -858,8 +862,7 @@ static int build_neighbor_list(sph_ctx* c) {
     Grid g = c->grid();
     const double *x = c->pf[SPH_F_X], *y = c->pf[SPH_F_Y], *z = c->pf[SPH_F_Z], *h = c->pf[SPH_F_H];
     const unsigned nlgrid = (unsigned)grid1(((long long)n + NL_P - 1) / NL_P * 64);
-    double* thr[4] = {};
-    for (auto& a : thr) SPH_TRY(dalloc(c, &a, c->cap));
+    double* const* const thr = c->sm;   // four arrays of the working copies (see permute_state)
     NLForm* form = nullptr;
     SPH_TRY(dalloc(c, &form, 1));
     SPH_HIP(c, hipMemsetAsync(form, 0, sizeof(NLForm), c->stream));
@@ -897,7 +900,6 @@ static int build_neighbor_list(sph_ctx* c) {
             SPH_TRY(launch_check(c, "slice_width"));
             c->nl_total = total;
             dfree(c, w);
-            for (auto a : thr) dfree(c, a);
             dfree(c, form);
             return build_porder(c);
         }
@@ -929,7 +931,6 @@ static int build_neighbor_list(sph_ctx* c) {
                        c->nl_cnt, (int*)nullptr);
     SPH_TRY(launch_check(c, "nl_fill"));
     SPH_TRY(prof_end(c));
-    for (auto a : thr) dfree(c, a);
     dfree(c, form);
     return build_porder(c);
 }

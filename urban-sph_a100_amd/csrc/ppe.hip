@@ -1630,14 +1630,20 @@ static int stencil_squeeze(sph_ctx* c, PPEState* P) {
     P->nnz = P->nnz - P->nnz_stencil + nz;
     P->nnz_stencil = nz;
     P->squeezed = true;
-    // the old layout's blocks would stay in the context's cache, counted in
-    // its device memory (the admission estimate bounds that); nothing in
-    // flight uses them after the synchronisation above.  The small blocks
-    // stay for the next search of this context: returning all of them cost a
-    // case that is uploaded again some 140 hipMalloc / hipFree pairs of
-    // 0.1-0.3 ms each
-    dcache_trim(c, (size_t)c->n * 640);
     return 0;
+}
+
+// The blocks of a search's set-up that its case no longer needs (the layout
+// before the squeeze, a hierarchy's temporaries) are in the context's cache,
+// counted in the device memory it holds, which servers admit by.  The smaller ones
+// stay for the next search of this context: 128 bytes a particle, and what a
+// hierarchy's set-up takes (some 320).  Returning all cost a 1 M canyon that
+// is uploaded again 4 ms of 35; keeping 640 bytes besides the hierarchy's held
+// 3365 bytes a particle and took 32.7 ms, this holds 2980 and takes 31.8 (the
+// hierarchy is built before, from the layout's blocks).
+static void trim_setup(sph_ctx* c) {
+    const bool mg = c->ppe && c->ppe->mg_state == 1;
+    dcache_trim(c, (size_t)c->n * (mg ? 448 : 128));
 }
 
 // Rows and column structure of a case's PPE from its neighbour list.
@@ -2116,29 +2122,6 @@ int ppe_solve(Eng& e) {
         SPH_TRY(tune_end(e));
         SPH_TRY(prof_end(e));
     }
-    // the values of a search's first step are written: its stencil slices
-    // drop their zero offsets, and the descriptors take the new layout
-    if (mixed && !jacobi) {
-        bool any = false;
-        for (int k = 0; k < nc; k++) {
-            sph_ctx* c = e.cs[k];
-            PPEState* P = c->ppe;
-            if (!P || !P->spat || P->squeezed || (!c->prm.ale_positions && c->vals_gen == c->generation)) continue;
-            if (!any) SPH_HIP(&e, hipStreamSynchronize(e.st));   // the assembly's values
-            any = true;
-            SPH_TRY(stencil_squeeze(c, P));
-            c->rep.nnz = P->nnz;
-            c->rep.slots = P->nnz_slots;
-            c->rep.stencil_nnz = P->nnz_stencil;
-        }
-        if (any) {
-            SPH_HIP(&e, hipEventSynchronize(e.up_ev));
-            for (int k = 0; k < nc; k++) e.h_desc[k].ppe = ppe_view(e.cs[k]);
-            ppe_streams(e);
-            SPH_HIP(&e, hipMemcpyAsync(e.d_desc, e.h_desc, sizeof(CaseDesc) * nc, hipMemcpyHostToDevice, e.st));
-            SPH_HIP(&e, hipEventRecord(e.up_ev, e.st));
-        }
-    }
     if (jacobi) {
         RL("ppe_scatter", 0, k_ppe_scatter, 1);
         for (sph_ctx* c : e.cs) {
@@ -2149,43 +2132,64 @@ int ppe_solve(Eng& e) {
         }
         return 0;
     }
+    // Case by case, so that one case's set-up blocks are given back before the
+    // next one's: the values of a search's first step are written and its stencil
+    // slices drop their zero offsets; then the multigrid preconditioner of every
+    // case that asks for it.  A hierarchy is built once per set of values (with
+    // fixed particles, at the first step of a search).  FP64 builds it from a
+    // float copy of its operator.
     std::vector<int> iters;
-    // the multigrid preconditioner of every case that asks for it; a
-    // hierarchy is built once per set of values (with fixed particles, at
-    // the first step of a search).  FP64 builds it from a float copy of its
-    // operator.
     std::vector<const MGState*> mgs(nc, nullptr);
-    bool any_mg = false;
+    bool any_mg = false, any_squeezed = false;
     for (int k = 0; k < nc; k++) {
         sph_ctx* c = e.cs[k];
         PPEState* P = c->ppe;
-        if (c->prm.ppe_precond != SPH_PRECOND_MULTIGRID || !P) continue;
+        if (!P) continue;
         const bool fresh = !c->prm.ale_positions && c->vals_gen == c->generation;
-        if (!fresh || P->mg_state == 0) {
-            mg_free(c, P->mg);
-            P->mg = nullptr;
-            P->mg_state = -1;
-            P->mg_why = SPH_MG_UNSUITED;
-            if (P->nr > MG_COARSE_MAX && (mixed || P->fp)) {
-                if (!mixed) {
-                    hipLaunchKernelGGL(k_vals_narrow, dim3(grid1(P->nnz_slots + 1)), dim3(BLOCK), 0, e.st,
-                                       P->nnz_slots + 1, (const double*)P->vals64, P->vals32);
-                    SPH_TRY(launch_check(&e, "vals_narrow"));
+        const bool squeeze = mixed && P->spat && !P->squeezed && !fresh;
+        if (squeeze) {
+            if (!any_squeezed) SPH_HIP(&e, hipStreamSynchronize(e.st));   // the assembly's values
+            any_squeezed = true;
+            SPH_TRY(stencil_squeeze(c, P));
+            c->rep.nnz = P->nnz;
+            c->rep.slots = P->nnz_slots;
+            c->rep.stencil_nnz = P->nnz_stencil;
+        }
+        if (c->prm.ppe_precond == SPH_PRECOND_MULTIGRID) {
+            if (!fresh || P->mg_state == 0) {
+                mg_free(c, P->mg);
+                P->mg = nullptr;
+                P->mg_state = -1;
+                P->mg_why = SPH_MG_UNSUITED;
+                if (P->nr > MG_COARSE_MAX && (mixed || P->fp)) {
+                    if (!mixed) {
+                        hipLaunchKernelGGL(k_vals_narrow, dim3(grid1(P->nnz_slots + 1)), dim3(BLOCK), 0, e.st,
+                                           P->nnz_slots + 1, (const double*)P->vals64, P->vals32);
+                        SPH_TRY(launch_check(&e, "vals_narrow"));
+                    }
+                    double q = 0.0;
+                    int ok = 0;
+                    SPH_TRY(finest_spacing(c, P, &q));
+                    SPH_TRY(mg_build(c, ppe_view(c), P->nnz_slots, q, &P->mg, &ok, &P->mg_why));
+                    P->mg_state = ok ? 1 : -1;
                 }
-                double q = 0.0;
-                int ok = 0;
-                SPH_TRY(finest_spacing(c, P, &q));
-                SPH_TRY(mg_build(c, ppe_view(c), P->nnz_slots, q, &P->mg, &ok, &P->mg_why));
-                P->mg_state = ok ? 1 : -1;
             }
+            if (P->mg_state == 1) {
+                mgs[k] = P->mg;
+                any_mg = true;
+                c->rep.mg_sorted_rows = mg_sorted_rows(P->mg);
+                c->rep.mg_long_rows = mg_long_rows(P->mg);
+            }
+            c->rep.mg_status = P->mg_state == -1 ? P->mg_why : SPH_MG_OK;
         }
-        if (P->mg_state == 1) {
-            mgs[k] = P->mg;
-            any_mg = true;
-            c->rep.mg_sorted_rows = mg_sorted_rows(P->mg);
-            c->rep.mg_long_rows = mg_long_rows(P->mg);
-        }
-        c->rep.mg_status = P->mg_state == -1 ? P->mg_why : SPH_MG_OK;
+        if (squeeze) trim_setup(c);
+    }
+    if (any_squeezed) {   // the descriptors take the new layouts
+        SPH_HIP(&e, hipEventSynchronize(e.up_ev));
+        for (int k = 0; k < nc; k++) e.h_desc[k].ppe = ppe_view(e.cs[k]);
+        ppe_streams(e);
+        SPH_HIP(&e, hipMemcpyAsync(e.d_desc, e.h_desc, sizeof(CaseDesc) * nc, hipMemcpyHostToDevice, e.st));
+        SPH_HIP(&e, hipEventRecord(e.up_ev, e.st));
     }
     auto mg_tables = [&]() -> int {
         bool changed = false;

@@ -159,8 +159,11 @@ long long sph_estimate_bytes(const sph_params* prm, int n) {
     const double val = mixed ? 4.0 : 8.0;
     const double krylov = mixed ? 10 * 4.0 : 8 * 8.0;
     double per = 96 * 8.0 + 6 * 4.0 + 16.0 + 160 * 4.0 + 128 * (4.0 + val) + 6 * 8.0 + krylov;
-    // neighbour records of the gathering passes: 128 bytes, plus the compact
-    // 32- and 64-byte records in MIXED
+    // neighbour records of the gathering passes: 112 bytes in double (counted
+    // as 128), in MIXED with fixed particles the compact 32- and 64-byte ones
+    // in their place (counted beside them: room for the blocks that the cache
+    // keeps for a next search, at most 128 bytes a particle and a hierarchy's
+    // temporaries)
     per += 128.0 + (mixed ? 96.0 : 0.0);
     // Neumann pairs of the boundary particles (a few hundred each, a few per
     // cent of the particles): about 32 four-byte pairs per particle, kept

@@ -697,6 +697,10 @@ struct sph_ctx {
 
     sph::PView pview() const;
     sph::PView sview() const;
+    // whether the gathering passes read the compact float records
+    bool compact() const {
+        return prm.precision == SPH_MIXED && pos_f32 && !prm.ale_positions && prm.compact_records;
+    }
     sph::P2View p2view() const;
     sph::P2View s2view() const;
     sph::QView qview() const;
