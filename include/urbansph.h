@@ -445,10 +445,9 @@ int sph_stats(sph_ctx* c, float* umax, float* drho_pct_max, float* fmax);
 /* sph_stats without any device allocation, memset or atomic: the same three
  * maxima, bit for bit.  No counterpart in the reference; for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
- * loops, harnesses that forbid hipMalloc).  Its working memory is one
- * library-owned array of about 768 KB per GPU, held until the process ends
- * and shared by every call on that GPU: calls that overlap on one GPU race.
- * Cases of more than 16,777,216 particles get SPH_E_ARG (use sph_stats). */
+ * loops, harnesses that forbid hipMalloc).  Its working memory is the
+ * context's, so calls on different contexts are independent.  Cases of more
+ * than 16,777,216 particles get SPH_E_ARG (use sph_stats). */
 int sph_stats_noalloc(sph_ctx* c, float* umax, float* drho_pct_max, float* fmax);
 
 /* Blocks until all enqueued work of the context is done; reports deferred

@@ -4,6 +4,7 @@
 // per-GPU thread ISPH_Calc owns them (ISPH_Calc.cuh:327-344,553-571), and
 // sph_step enqueues the step sequence of SOPHIA_single_ISPH
 // (ISPH_Calc.cuh:4-233) on the context's stream.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -287,7 +288,7 @@ int sph_create(const sph_params* prm, int n_part2, sph_ctx** out) {
     for (int f = 0; f < 10; f++) e = e ? e : A(&c->s2[f]);
     for (int f = 0; f < 18; f++) e = e ? e : A(&c->q[f]);
     for (int f = 0; f < 5; f++) e = e ? e : A(&c->snap[f]);
-    e = e ? e : dalloc(c, &c->stat_buf, 16);
+    e = e ? e : dalloc(c, &c->stat_buf, STAT_PARTS + 3 * (size_t)grid1(std::min<long long>(n_part2, NA_STATS_MAX_N)));
     if (e) { sph_destroy(c); return e; }
     *out = c;
     return 0;

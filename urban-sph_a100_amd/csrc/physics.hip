@@ -13,7 +13,6 @@
 // always accumulated in double.  Differences of positions and velocities are
 // taken in double and then rounded to R, so the float path loses no
 // significance to cancellation.
-#include <mutex>
 #include <string>
 
 #include "flags.h"
@@ -2362,15 +2361,10 @@ int stats_run(sph_ctx* c, float* umax, float* drho, float* fmax_) {
 }
 
 // ---- statistics without allocation (sph_stats_noalloc) -------------------
-// Per-workgroup maxima go to a file-scope device array instead of the
-// context's buffer, and a one-workgroup fold reduces them, so the call needs
-// no device allocation, no memset and no atomics.  The array is this
-// library's own on each GPU: every call on a GPU shares it, so calls that
-// overlap on one GPU race.  Particles up to NA_STATS_MAX_BLOCKS * BLOCK.
-constexpr int NA_STATS_MAX_BLOCKS = 1 << 16;
-constexpr int NA_STATS_OUT = 3 * NA_STATS_MAX_BLOCKS;   // first word of the 3 float results
-constexpr long long NA_STATS_MAX_N = (long long)NA_STATS_MAX_BLOCKS * BLOCK;
-static __device__ __align__(256) unsigned scratch[NA_STATS_OUT + 64];
+// Per-workgroup maxima go behind the context's accumulators (stat_buf, sized for
+// them when the context is made) and a one-workgroup fold reduces them, so the
+// call needs no device allocation, no memset and no atomics, and contexts share
+// nothing.
 
 // The maxima of k_stats for this workgroup's particles, stored at part[3b..3b+2].
 __global__ void __launch_bounds__(BLOCK) k_stats_part(int n, PView P, P2View S2, QView Q, unsigned* part) {
@@ -2413,42 +2407,17 @@ __global__ void __launch_bounds__(BLOCK) k_stats_fold(int nb, const unsigned* pa
     if (threadIdx.x < 3) out[threadIdx.x] = ord2f(s[threadIdx.x][0]);
 }
 
-// Device address of `scratch` on each GPU, looked up once per device with
-// that device current (the host-side name of the array is no device address).
-static std::mutex na_mu;
-static void* na_addr[64] = {};
-
-static int na_scratch(sph_ctx* c, unsigned** out) {
-    const int dev = c->device;
-    if (dev < 0 || dev >= 64) return fail(c, SPH_E_ARG, "sph_stats_noalloc: device index beyond 63");
-    std::lock_guard<std::mutex> lk(na_mu);
-    if (!na_addr[dev]) {
-        int cur = -1;
-        SPH_HIP(c, hipGetDevice(&cur));
-        if (cur != dev) SPH_HIP(c, hipSetDevice(dev));
-        void* p = nullptr;
-        const hipError_t er = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (cur != dev) SPH_HIP(c, hipSetDevice(cur));
-        if (er != hipSuccess || !p)
-            return fail(c, SPH_E_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(er));
-        na_addr[dev] = p;
-    }
-    *out = (unsigned*)na_addr[dev];
-    return 0;
-}
-
 int stats_run_noalloc(sph_ctx* c, float* umax, float* drho, float* fmax_) {
     const int n = c->n;
     if ((long long)n > NA_STATS_MAX_N)
         return fail(c, SPH_E_ARG, "sph_stats_noalloc: " + std::to_string(n) + " particles exceed its bound of " +
                                       std::to_string(NA_STATS_MAX_N) + " (use sph_stats)");
-    unsigned* sc = nullptr;
-    SPH_TRY(na_scratch(c, &sc));
+    unsigned* const part = (unsigned*)c->stat_buf + STAT_PARTS;
     const unsigned nb = grid1(n);
-    hipLaunchKernelGGL(k_stats_part, dim3(nb), dim3(BLOCK), 0, c->stream, n, c->pview(), c->s2view(), c->qview(), sc);
+    hipLaunchKernelGGL(k_stats_part, dim3(nb), dim3(BLOCK), 0, c->stream, n, c->pview(), c->s2view(), c->qview(), part);
     SPH_TRY(launch_check(c, "stats_part"));
-    float* res = (float*)(sc + NA_STATS_OUT);
-    hipLaunchKernelGGL(k_stats_fold, dim3(1), dim3(BLOCK), 0, c->stream, (int)nb, (const unsigned*)sc, res);
+    float* res = c->stat_buf + 4;
+    hipLaunchKernelGGL(k_stats_fold, dim3(1), dim3(BLOCK), 0, c->stream, (int)nb, (const unsigned*)part, res);
     SPH_TRY(launch_check(c, "stats_fold"));
     float h[3];
     SPH_HIP(c, hipMemcpyAsync(h, res, 3 * sizeof(float), hipMemcpyDeviceToHost, c->stream));

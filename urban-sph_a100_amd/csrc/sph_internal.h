@@ -684,7 +684,7 @@ struct sph_ctx {
     int nl_wprev_n = 0;              // its slices
     int* scan_tmp = nullptr; size_t scan_tmp_n = 0;
 
-    float* stat_buf = nullptr;           // stats reduction scratch
+    float* stat_buf = nullptr;           // statistics: accumulators, results, partials (STAT_PARTS)
     double* apr_target = nullptr;        // APR target level per particle (the reference's M_num)
     double* xnew[3] = {};                // ALE: corrector positions, committed at the end of the step
     double* rec = nullptr;               // neighbour records of the gathering passes (cap * REC_DOUBLES)
@@ -794,6 +794,10 @@ long long step_physics_back_key(const Eng& e);
 bool tune_pending(Eng& e);   // the autotuner still times candidates for this step's size class
 int stats_run(sph_ctx* c, float* umax, float* drho, float* fmax);
 int stats_run_noalloc(sph_ctx* c, float* umax, float* drho, float* fmax);
+// words of stat_buf before the per-workgroup maxima of sph_stats_noalloc, which
+// takes up to NA_STATS_MAX_N particles
+constexpr int STAT_PARTS = 16;
+constexpr long long NA_STATS_MAX_N = (1LL << 16) * BLOCK;
 
 // ppe.hip
 int ppe_build(sph_ctx* c);
