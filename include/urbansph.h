@@ -404,12 +404,13 @@ int sph_step(sph_ctx* c, int count, double dt, double time);
  * changes any result. */
 int sph_set_engine_options(sph_ctx* c, int use_graphs, int autotune);
 
-/* Workgroup sizes the autotuner picked: one row of 1 + SPH_TUNE_PASSES ints
+/* Workgroup sizes of the neighbour passes: one row of 1 + SPH_TUNE_PASSES ints
  * per size class (floor(log2(particles in the step)), then the size of each
- * tunable pass: grad_corr, prep, boundary3d, neumann, advection, freeslip,
+ * pass: grad_corr, prep, boundary3d, neumann, advection, freeslip,
  * pressure_force, ibm_force, ibm_spread, ppe_assemble; 0 while that class is
- * still being timed; neumann always runs one 64-thread wave per boundary
- * particle and reads 64).  Returns the number of rows written (<= max_rows). */
+ * still being timed).  The autotuner picks all but those of boundary3d, freeslip
+ * and ibm_force, which are 256, and of neumann, 64 in FP64 and 256 in MIXED (of
+ * the class's last steps).  Returns the number of rows written (<= max_rows). */
 #define SPH_TUNE_PASSES 10
 int sph_tuning(const sph_ctx* c, int* out, int max_rows);
 

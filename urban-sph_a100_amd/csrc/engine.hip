@@ -82,14 +82,19 @@ int prof_collect(Eng& e) {
 }
 
 // ---------------------------------------------------------------- tuning
+static bool tune_is_fixed(int kid) {
+    return kid == TK_BOUNDARY || kid == TK_NEUMANN || kid == TK_FREESLIP || kid == TK_IBM_FORCE;
+}
 static Eng::Tune& tune_for(Eng& e, int cls) {
     for (auto& t : e.tune)
         if (t.first == cls) return t.second;
     Eng::Tune t{};
-    for (int k = 0; k < TK_COUNT; k++) t.block[k] = BLOCK;
-    t.block[TK_NEUMANN] = 64;   // one wave per boundary particle, not tuned
+    for (int k = 0; k < TK_COUNT; k++) t.block[k] = tune_is_fixed(k) ? WAVE_BLOCK : BLOCK;
     e.tune.emplace_back(cls, t);
     return e.tune.back().second;
+}
+void tune_fixed(Eng& e, int kid, int block) {
+    if (e.autotune) tune_for(e, e.tune_class).block[kid] = block;
 }
 int tuned_block(Eng& e, int kid) {
     if (!e.autotune) return BLOCK;
@@ -141,7 +146,7 @@ static int tune_fold(Eng& e) {
         if (t.phase >= TUNE_CANDIDATES) continue;
         if (++t.phase < TUNE_CANDIDATES) continue;
         for (int k = 0; k < TK_COUNT; k++) {
-            if (k == TK_NEUMANN) continue;
+            if (tune_is_fixed(k)) continue;
             int best = -1;
             double best_ms = 0.0;
             for (int q = 0; q < TUNE_CANDIDATES; q++) {

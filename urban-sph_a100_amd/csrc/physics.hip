@@ -1,6 +1,8 @@
 // Per-step physics passes of the ISPH projection step on MI355X.
 //
-// One thread per particle over structure-of-arrays state.  Neighbour passes
+// Structure-of-arrays state; a thread per particle where a pass reads no
+// neighbours, else groups of lanes (GROUP; 16 or 32 for the boundary passes; a
+// wave for FP64 Neumann sums and heavy MIXED lists), which
 // walk the per-particle neighbour list built once by the count==0 search
 // (the reference rescans the 5^3 cell window every pass; in its Eulerian mode
 // positions never move, ISPH_Calc.cuh:23-63).  Each list entry carries
@@ -773,34 +775,33 @@ __global__ void __launch_bounds__(BLOCK) k_nmp_widen(int n, const int* a, long l
     if (r < n) b[r] = a[r];
 }
 
-template <class R>
-__global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_count0) {
-    // one 64-lane wave per boundary particle of the case's compact list
+// FP64: a 64-lane wave per boundary particle of the case's compact list, over
+// its listed pairs.  Each lane forms the terms of one pair exactly as a serial
+// scan does, and the sums are added in list order (OrderedSums).  (Each lane
+// adding the terms that a flag marked, one LDS read after another, took half of
+// the pass: 268 us on a 150 k canyon.)
+constexpr int NM_BLOCK = 64;
+__global__ void __launch_bounds__(NM_BLOCK) k_neumann(Seg sg, int which, int only_count0) {
     int first_;
     const int cid_ = seg_case(sg, first_);
     const CaseDesc& cd = sg.cd[cid_];
     const int u = first_ >> 6, lane = threadIdx.x;
     if (u >= cd.nm_count) return;
     if (only_count0 && cd.count != 0) return;   // the extra pre-advection call, ISPH_Calc.cuh:88-90
-    if (sizeof(R) == 4 && cd.nmp_off) return;   // k_neumann_mixed
     const KConst kc = cd.kc;
     const sph_params pr = cd.pr;
     const PView A = which ? cd.P : cd.S;
     const Grid g = cd.g;
     const double* pold = cd.snap[3];
     const int i = cd.nm_list[u];
-    const sph_domain& d = g.d;
-    R hi = (R)(2.0 * A.h[i]);
-    R tmp_A = calc_tmpA<R>(kc, hi);
-    R search_range = (R)kc.kappa * hi;
-    double xi = A.x[i], yi = A.y[i], zi = A.z[i];
+    const double hi = 2.0 * A.h[i], tmp_A = calc_tmpA<double>(kc, hi), search_range = kc.kappa * hi;
+    const double xi = A.x[i], yi = A.y[i], zi = A.z[i];
     double pres_g = 0;
-    int bt = A.buffer_type[i];
-    double xg = (bt == 1 || bt == -1) ? 2.0 * pr.L2 - xi : xi;
-    double yg = yi, zg = zi;
-    Cell c = query_cell(d, xg, yg, zg);
+    const int bt = A.buffer_type[i];
     // the ghost pressure and the gradient only enter the inlet formula
     const bool inlet = (bt == 1 || bt == -1);
+    const double xg = inlet ? 2.0 * pr.L2 - xi : xi, yg = yi, zg = zi;
+    const Cell c = query_cell(g.d, xg, yg, zg);
     // The window's cells of one x-row are consecutive in cell order, so
     // their particles form one range of the sorted order, visited in the
     // same order as cell by cell.  Lanes test consecutive candidates; the
@@ -814,62 +815,47 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
                 bool hit = false;
                 double pj = 0.0;
                 if (j < rg.y) {
-                    R dx = (R)(xg - A.x[j]), dy = (R)(yg - A.y[j]), dz = (R)(zg - A.z[j]);
-                    R dist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
-                    hit = dist < (R)pr.neumann_ghost_r;
+                    const double dx = xg - A.x[j], dy = yg - A.y[j], dz = zg - A.z[j];
+                    const double dist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
+                    hit = dist < pr.neumann_ghost_r;
                     pj = pold[j];
                 }
                 const unsigned long long m = __ballot(hit);
                 if (m) pres_g = __shfl(pj, 63 - __clzll(m), 64);
             }
         }
-    // FP64: each lane forms the terms of one candidate exactly as the serial
-    // scan does, and the sums are added in candidate order (OrderedSums).
-    // (Each lane adding the terms that a flag marked, one LDS read after
-    // another, took half of the pass: 268 us on a 150 k canyon.)
     __shared__ double terms[ord_doubles(8)];
     OrderedSums<8, 64> sums(terms);
-    const bool listed = cd.nmp_off != nullptr;
-    // one chunk of candidates v0 .. v0 + 63 of the window's flattened order:
-    // lane l holds candidate v0 + l (particle j, or j < 0 for none)
-    auto chunk = [&](int j, int) {
+    // (only fluid, non-buffer neighbours carry weight: the reference
+    // multiplies the others by 0, and leaving those exact zeros out of the
+    // list leaves every sum bit for bit the same)
+    const long long e0 = cd.nmp_off[u], e1 = cd.nmp_off[u + 1];
+    for (long long b = e0; b < e1; b += 64) {
         double v[8] = {};
-        // only fluid, non-buffer neighbours carry weight (the reference
-        // multiplies the others by 0; skipping those exact zeros leaves every
-        // sum bit for bit the same); the pair list holds only those
-        if (j >= 0 && (listed || (A.p_type[j] == 1 && A.buffer_type[j] == 0))) {
-            const R dx = (R)(xg - A.x[j]), dy = (R)(yg - A.y[j]), dz = (R)(zg - A.z[j]);
-            const R tdist = sqrt(dx * dx + dy * dy + dz * dz) - (R)1e-20;
+        if (b + lane < e1) {
+            const int j = cd.nmp_ent[b + lane];
+            const double dx = xg - A.x[j], dy = yg - A.y[j], dz = zg - A.z[j];
+            const double tdist = sqrt(dx * dx + dy * dy + dz * dz) - 1e-20;
             if (tdist < search_range) {
-                const R mj = (R)A.m[j], rhoj = (R)A.rho[j];
+                const double mj = A.m[j], rhoj = A.rho[j];
                 const double presj = pold[j];
-                const R twij = kernel_w<R>(kc, tmp_A, hi, tdist);
-                v[0] = (double)(mj / rhoj * (R)presj * twij);
-                v[1] = (double)(mj / rhoj * (R)A.ux[j] * twij);
-                v[2] = (double)(mj / rhoj * (R)A.uy[j] * twij);
-                v[3] = (double)(mj / rhoj * (R)A.uz[j] * twij);
-                v[4] = (double)(mj / rhoj * twij);
+                const double twij = kernel_w<double>(kc, tmp_A, hi, tdist);
+                v[0] = mj / rhoj * presj * twij;
+                v[1] = mj / rhoj * A.ux[j] * twij;
+                v[2] = mj / rhoj * A.uy[j] * twij;
+                v[3] = mj / rhoj * A.uz[j] * twij;
+                v[4] = mj / rhoj * twij;
                 if (inlet) {
-                    const R tdwij = kernel_dw<R>(kc, tmp_A, hi, tdist);
-                    const R tdwx = dx / tdist * tdwij, tdwy = dy / tdist * tdwij, tdwz = dz / tdist * tdwij;
-                    const R dp = (R)(presj - pres_g);
-                    v[5] = (double)(mj / rhoj * dp * tdwx);
-                    v[6] = (double)(mj / rhoj * dp * tdwy);
-                    v[7] = (double)(mj / rhoj * dp * tdwz);
+                    const double tdwij = kernel_dw<double>(kc, tmp_A, hi, tdist);
+                    const double tdwx = dx / tdist * tdwij, tdwy = dy / tdist * tdwij, tdwz = dz / tdist * tdwij;
+                    const double dp = presj - pres_g;
+                    v[5] = mj / rhoj * dp * tdwx;
+                    v[6] = mj / rhoj * dp * tdwy;
+                    v[7] = mj / rhoj * dp * tdwz;
                 }
             }
         }
         sums.add(v);
-    };
-    if (cd.nmp_off) {
-        // the pairs of this search (the window's weighted candidates, scan order)
-        const long long e0 = cd.nmp_off[u], e1 = cd.nmp_off[u + 1];
-        for (long long b = e0; b < e1; b += 64) {
-            const long long e = b + lane;
-            chunk(e < e1 ? cd.nmp_ent[e] : -1, (int)min((long long)64, e1 - b));
-        }
-    } else {
-        neumann_window(g, c, A.ncell[i], lane, chunk);
     }
     const double tpres = sums.sum(0), tux = sums.sum(1), tuy = sums.sum(2), tuz = sums.sum(3), tflt_s = sums.sum(4);
     const double grad_px = sums.sum(5), grad_py = sums.sum(6), grad_pz = sums.sum(7);
@@ -879,7 +865,7 @@ __global__ void __launch_bounds__(64) k_neumann(Seg sg, int which, int only_coun
     } else {
         A.pres[i] = tpres / tflt_s;
         if (A.p_type[i] == -1) { A.ux[i] = tux / tflt_s; A.uy[i] = tuy / tflt_s; A.uz[i] = tuz / tflt_s; }
-        if (bt == 1 || bt == -1) A.pres[i] = pres_g + (xi - xg) * grad_px + (yi - yg) * grad_py + (zi - zg) * grad_pz;
+        if (inlet) A.pres[i] = pres_g + (xi - xg) * grad_px + (yi - yg) * grad_py + (zi - zg) * grad_pz;
     }
 }
 
@@ -892,7 +878,7 @@ struct NMRow {
         return (unsigned)((const __attribute__((address_space(1))) int*)p)[k] | F_DP;
     }
 };
-// MIXED with listed pairs: NM_LANES lanes a boundary particle, each adding the
+// MIXED: NM_LANES lanes a boundary particle, each adding the
 // terms of pairs lane, lane + NM_LANES, ... in list order, then a fixed butterfly
 // (so the sums are the same on every call, alone or in a batch).  A wave a
 // particle spent most of its time on the loads before its few rounds.  By lanes
@@ -903,7 +889,6 @@ constexpr int NM_LANES = 32;
 __global__ void __launch_bounds__(WAVE_BLOCK) k_neumann_mixed(Seg sg, int which, int only_count0) {
     SEG_BOUNDARY_LANES(sg, NM_LANES);
     if (only_count0 && cd.count != 0) return;   // the extra pre-advection call, ISPH_Calc.cuh:88-90
-    if (!cd.nmp_off) return;                    // k_neumann
     const KConst kc = cd.kc;
     const sph_params& pr = cd.pr;
     const PView A = which ? cd.P : cd.S;
@@ -1951,8 +1936,7 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
 // tested inside the kernels, so one launch sequence serves any mix.
 // ========================================================================
 
-// launch over the particles of every case; tunable passes (kid >= 0) run at
-// the workgroup size the autotuner picked for this batch size
+// launches over the particles of every case
 // a boundary pass with `lanes` lanes per boundary particle of each case
 #define BOUNDL(name, kern, ...) BOUNDW(name, BLANES, kern, ##__VA_ARGS__)
 #define BOUNDW(name, lanes, kern, ...)                                                                        \
@@ -1993,8 +1977,8 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
             SPH_TRY(prof_end(e));                                                                   \
         }                                                                                           \
     } while (0)
-// the same with GROUP lanes a particle
-// (SEGO: FP64, with the LDS of nd doubles a wave for ordered sums)
+// GROUP lanes a particle, at the workgroup size the autotuner picked for this
+// batch size (SEGO: FP64, with the LDS of nd doubles a wave for ordered sums)
 #define SEGG(name, kid, kern, ...) SEGO(name, kid, 0, kern, ##__VA_ARGS__)
 #define SEGO(name, kid, nd, kern, ...)                                                                   \
     do {                                                                                            \
@@ -2010,17 +1994,14 @@ __global__ void k_stats_final(const unsigned* in, float* out) {
             SPH_TRY(prof_end(e));                                                                   \
         }                                                                                           \
     } while (0)
-#define SEGL(name, kid, kern, ...)                                                                   \
+#define SEGL(name, kern, ...)                                                                        \
     do {                                                                                            \
-        const int blk_ = (kid) >= 0 ? tuned_block(e, (kid)) : BLOCK;                                \
         Shape sh_;                                                                                  \
-        SPH_TRY(shape(e, 0, blk_, &sh_));                                                           \
+        SPH_TRY(shape(e, 0, BLOCK, &sh_));                                                          \
         if (sh_.grid > 0) {                                                                         \
             SPH_TRY(prof_begin(e, name, 0.0));                                                      \
-            if ((kid) >= 0) SPH_TRY(tune_begin(e, (kid), blk_));                                    \
-            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(blk_), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
+            hipLaunchKernelGGL(kern, dim3(sh_.grid), dim3(BLOCK), 0, e.st, Seg{e.d_desc, sh_.tab}, ##__VA_ARGS__); \
             SPH_TRY(launch_check(&e, name));                                                        \
-            if ((kid) >= 0) SPH_TRY(tune_end(e));                                                   \
             SPH_TRY(prof_end(e));                                                                   \
         }                                                                                           \
     } while (0)
@@ -2156,35 +2137,31 @@ int neumann_pairs(sph_ctx* c) {
 }
 
 static int run_neumann(Eng& e, int which, int only_count0) {
-    SEGL("snapshot", -1, k_snapshot, which, 1);
-    bool listed = false, general = !mixed_of(e);   // MIXED cases with and without listed pairs
-    for (size_t k = 0; k < e.cs.size() && mixed_of(e); k++)
-        (e.h_desc[k].nmp_off ? listed : general) = true;
-    if (listed) BOUNDW("neumann", NM_LANES, k_neumann_mixed, which, only_count0);
-    // one 64-thread block (one wave) per boundary particle of each case
-    Shape sh;
-    SPH_TRY(shape(e, 3, 64, &sh));
-    if (general && sh.grid > 0) {
+    SEGL("snapshot", k_snapshot, which, 1);
+    if (mixed_of(e)) {
+        tune_fixed(e, TK_NEUMANN, WAVE_BLOCK);
+        BOUNDW("neumann", NM_LANES, k_neumann_mixed, which, only_count0);
+        return 0;
+    }
+    tune_fixed(e, TK_NEUMANN, NM_BLOCK);
+    Shape sh;   // a block per boundary particle of each case
+    SPH_TRY(shape(e, 3, NM_BLOCK, &sh));
+    if (sh.grid > 0) {
         SPH_TRY(prof_begin(e, "neumann", 0.0));
-        if (mixed_of(e))
-            hipLaunchKernelGGL(k_neumann<float>, dim3(sh.grid), dim3(64), 0, e.st, Seg{e.d_desc, sh.tab}, which,
-                               only_count0);
-        else
-            hipLaunchKernelGGL(k_neumann<double>, dim3(sh.grid), dim3(64), 0, e.st, Seg{e.d_desc, sh.tab}, which,
-                               only_count0);
+        hipLaunchKernelGGL(k_neumann, dim3(sh.grid), dim3(NM_BLOCK), 0, e.st, Seg{e.d_desc, sh.tab}, which, only_count0);
         SPH_TRY(launch_check(&e, "neumann"));
         SPH_TRY(prof_end(e));
     }
     return 0;
 }
 static int run_outlet(Eng& e, int which) {
-    SEGL("snapshot", -1, k_snapshot, which, 0);
-    SEGL("outlet", -1, k_outlet, which);
+    SEGL("snapshot", k_snapshot, which, 0);
+    SEGL("outlet", k_outlet, which);
     return 0;
 }
 static int run_periodic(Eng& e, int which) {
-    SEGL("snapshot", -1, k_snapshot, which, 0);
-    SEGL("periodic", -1, k_periodic, which);
+    SEGL("snapshot", k_snapshot, which, 0);
+    SEGL("periodic", k_periodic, which);
     return 0;
 }
 static int run_freeslip(Eng& e, int which) {
@@ -2199,12 +2176,12 @@ int pack_records(Eng& e, int which) {
     if (which == REC_PRE) {
         bool any = false;
         for (size_t k = 0; k < e.cs.size(); k++) any |= e.h_desc[k].crec_adv != nullptr;
-        if (any) SEGL("pack_records", -1, k_pack_records<REC_PRE>);
+        if (any) SEGL("pack_records", k_pack_records<REC_PRE>);
         return 0;
     }
-    if (which == REC_PQ) SEGL("pack_records", -1, k_pack_records<REC_PQ>);
-    else if (which == REC_VEL_PQ) SEGL("pack_records", -1, k_pack_records<REC_VEL_PQ>);
-    else SEGL("pack_records", -1, k_pack_records<REC_ALL>);
+    if (which == REC_PQ) SEGL("pack_records", k_pack_records<REC_PQ>);
+    else if (which == REC_VEL_PQ) SEGL("pack_records", k_pack_records<REC_VEL_PQ>);
+    else SEGL("pack_records", k_pack_records<REC_ALL>);
     return 0;
 }
 
@@ -2270,13 +2247,13 @@ int step_physics_front(Eng& e) {
     const bool mixed = mixed_of(e);
     bool any_count0 = false;
     for (size_t k = 0; k < e.cs.size(); k++) any_count0 |= e.h_desc[k].count == 0;
-    SEGL("step_begin", -1, k_step_begin);
+    SEGL("step_begin", k_step_begin);
     bool any_nrm = false;   // a case whose marker normals this step sets
     for (size_t k = 0; k < e.cs.size(); k++) {
         const int m = e.cs[k]->prm.ib_normals;
         any_nrm |= m == SPH_IBN_REFERENCE || (m == SPH_IBN_PLANES && e.h_desc[k].count == 0);
     }
-    if (any_nrm) SEGL("ib_normals", -1, k_ib_normals);
+    if (any_nrm) SEGL("ib_normals", k_ib_normals);
     bool any_gc = false;
     for (size_t k = 0; k < e.cs.size(); k++) any_gc |= !e.h_desc[k].gc_fresh;
     if (any_gc) {
@@ -2291,8 +2268,8 @@ int step_physics_front(Eng& e) {
     } else SEGO("prep", TK_PREP, ord_doubles(PREP_SUMS), k_prep);
     if (mixed) BOUNDL("boundary3d", k_boundary3d_mixed);
     else BOUNDL("boundary3d", k_boundary3d);
-    SEGL("most_self", -1, k_most_self);
-    SEGL("most_deposit", -1, k_most_deposit);
+    SEGL("most_self", k_most_self);
+    SEGL("most_deposit", k_most_deposit);
     if (any_count0) SPH_TRY(run_neumann(e, 0, 1));
     SPH_TRY(pack_records(e, REC_ALL));
     bool scal = false;   // scalar transport or buoyancy in some case of the step
@@ -2312,7 +2289,7 @@ int step_physics_front(Eng& e) {
         if (scal) SEGO("advection", TK_ADVECTION, ord_doubles(adv_sums<true>(), ADV_SECOND), k_advection<true>);
         else SEGO("advection", TK_ADVECTION, ord_doubles(adv_sums<false>(), ADV_SECOND), k_advection<false>);
     }
-    SEGL("projection", -1, k_projection);
+    SEGL("projection", k_projection);
     SPH_TRY(run_periodic(e, 0));
     SPH_TRY(run_freeslip(e, 0));
     return 0;
@@ -2334,14 +2311,14 @@ int step_physics_back(Eng& e) {
     else BOUNDL("ibm_force", k_ibm_force);
     if (mixed) SEGG("ibm_spread", TK_IBM_SPREAD, k_ibm_spread_mixed);
     else SEGO("ibm_spread", TK_IBM_SPREAD, ord_doubles(4), k_ibm_spread);
-    SEGL("time_update", -1, k_time_update);
+    SEGL("time_update", k_time_update);
     SPH_TRY(run_neumann(e, 1, 0));
     SPH_TRY(run_outlet(e, 1));
     SPH_TRY(run_periodic(e, 1));
     SPH_TRY(run_freeslip(e, 1));
     bool ale = false;
     for (sph_ctx* c : e.cs) ale |= c->prm.ale_positions != 0;
-    if (ale) SEGL("commit_positions", -1, k_commit_positions);
+    if (ale) SEGL("commit_positions", k_commit_positions);
     return 0;
 }
 

@@ -216,8 +216,8 @@ struct Seg {
     const CaseDesc* cd;
     const int2* tab;
 };
-// The passes that give a boundary particle or a heavy list a 64-lane wave
-// run four waves (four particles) to a workgroup.  The waves share nothing.
+// The passes that give a heavy list a 64-lane wave, or a boundary particle 16
+// or 32 lanes, run four waves to a workgroup.  The waves share nothing.
 constexpr int WAVE_BLOCK = 256;
 // MIXED passes over the particles' lists: GROUP lanes a particle, lane g_
 // taking entries g_, g_ + GROUP, ... of its list, a fixed butterfly adding
@@ -303,7 +303,9 @@ __device__ __forceinline__ int seg_case(const Seg& s, int& first) {
 }
 
 
-// launch tuning: the neighbour passes whose workgroup size the autotuner picks
+// launch tuning: the passes of the public report.  The boundary passes
+// (TK_BOUNDARY, TK_NEUMANN, TK_FREESLIP, TK_IBM_FORCE) run at fixed sizes, which
+// it reports; the autotuner picks the others'.
 enum TuneKernel {
     TK_GRAD_CORR, TK_PREP, TK_BOUNDARY, TK_NEUMANN, TK_ADVECTION, TK_FREESLIP, TK_PRESSURE, TK_IBM_FORCE,
     TK_IBM_SPREAD, TK_ASSEMBLE, TK_COUNT
@@ -777,6 +779,7 @@ int engine_step(Eng& e, sph_ctx* const* cases, int nc, const int* count, const d
 struct Shape { unsigned grid; int block; const int2* tab; };
 int shape(Eng& e, int kind, int block, Shape* out);
 int tuned_block(Eng& e, int kid);
+void tune_fixed(Eng& e, int kid, int block);   // the report's size of a pass that is not tuned
 int tune_begin(Eng& e, int kid, int block);
 int tune_end(Eng& e);
 size_t tile_lds_bytes(const Eng& e, int recf);
