@@ -890,7 +890,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_post(const CaseDesc* cds, const MG
 // little company to hide its chain of dependent gathers.  Lane g adds
 // entries g, g + MG_G, ... in order, then a fixed shuffle tree adds the
 // group's sums, so the result does not depend on the launch.  A long row's
-// product comes from k_mg_clong.  tab: BLOCK / MG_G rows per block; every
+// product comes from k_mg_clong.  tab: blockDim / MG_G rows a block; every
 // lane of a group has the same row, so a group returns or stays whole.
 // sum of entries k0, k0 + step, ... < m of a coarse row, in that order
 __device__ __forceinline__ double coarse_sum(const MGLv& L, long long base, int k0, int m, int step) {
@@ -967,6 +967,9 @@ constexpr int RR_LANES = 32;
 // The limit counts the rows of all the step's cases on the level.  Below it a
 // launch saved is worth more than coalesced rows (200 k request 51.4 -> 50.2 ms);
 // a level of 240 k rows is 9 us slower in one pass, its members' rows scattered.
+// Between them it matters little: residual and restriction of a step's V-cycles
+// together 508 us in one pass and 542 in two with a level of 67 k rows, 504 and 539
+// with 115 k, of steps of 4.85 and 7.36 ms that do not differ.
 constexpr long long RR_ROWS = 40000;
 __global__ void __launch_bounds__(BLOCK) k_mg_res_restrict(const CaseDesc* cds, const MGLv* lv, const int2* tab, int l,
                                                            int sc_done) {

@@ -133,9 +133,13 @@ __device__ __forceinline__ R kernel_dwp(const KConst& k, R tA, R tH, R rr) {
 // a quotient is three: the product with the reciprocal, the exact remainder,
 // the correction (Markstein, IBM J. Res. Dev. 34(1), 1990).  It is the
 // correctly rounded quotient of normal-range operands (none of 4e8 random pairs
-// differed on the CPU, reciprocal started one ulp off; the root differs in
-// one of 1.4 million), so the pair terms keep the accuracy and, but for those,
-// the bits of the IEEE operations.
+// differed on the CPU, reciprocal started one ulp off), so the pair terms keep
+// the accuracy of the IEEE operations, and their bits but for these:
+// - the root of a squared distance differs in one of 1.4 million, and a distance
+//   is at least 1e-15 (dist_of);
+// - divisors below 2^-126 or above 2^126 (products of two densities below 1e-19),
+//   whose reciprocal overflows or is subnormal, give NaN or infinities;
+// - a zero or infinite operand gives NaN (quot; quot_any has the division's).
 __device__ __forceinline__ float fma1(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ float recip(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
